@@ -364,6 +364,7 @@ static void launch_persistent(K kernel, int tiles, const GemmParams& q, hipStrea
 }
 
 #include "pw_stream.hpp"
+#include "igemm_slice.hpp"
 
 static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
@@ -678,6 +679,14 @@ static int autotune(const GemmParams& q, bool conv, int batch, int unit, hipStre
             best = general_cfg;
         }
     }
+    for (int c = kSliceCfg; c < kSliceCfg + kSliceForms && batch == 1; ++c) {
+        slice_launch(c, q, conv, s);
+        const float ms = timed([&] { slice_launch(c, q, conv, s); });
+        if (ms < best_ms) {
+            best_ms = ms;
+            best = c;
+        }
+    }
     if (stream_ok) {
         stream_launch();
         const float ms = timed(stream_launch);
@@ -754,9 +763,12 @@ static fdx_status run_igemm(GemmParams& p, bool conv, int batch, const char* fam
             unpack();
         if (cfg == kStreamCfg && !stream_ok)
             cfg = -1;
-        if (cfg >= 10 && cfg != kStreamCfg && (!fast_ok || (cfg >= 13 && unit % 32 != 0)))
+        const bool slice = cfg >= kSliceCfg && cfg < kSliceCfg + kSliceForms;
+        if (slice && (!fast_ok || batch != 1))
             cfg = -1;
-        if (cfg < 10 || mode > 2 || mode < 0 || splits < 0 || splits > 64 || cfg == kStreamCfg) {
+        if (cfg >= 10 && cfg != kStreamCfg && !slice && (!fast_ok || cfg > 18 || (cfg >= 13 && unit % 32 != 0)))
+            cfg = -1;
+        if (cfg < 10 || mode > 2 || mode < 0 || splits < 0 || splits > 64 || cfg == kStreamCfg || slice) {
             splits = 1;
             mode = 0;
         }
@@ -800,10 +812,12 @@ static fdx_status run_igemm(GemmParams& p, bool conv, int batch, const char* fam
         }
         p.a2_records = (uint32_t)a2_bytes;
         const bool slab32 = p.K % 32 == 0 && p.K1 % 32 == 0;
-        if (cfg < 10 || cfg > 15 || (cfg >= 13 && !slab32))
+        if (cfg < 10 || (cfg > 15 && cfg < kSliceCfg) || (cfg >= 13 && cfg <= 15 && !slab32))
             cfg = -1;
         splits = 1;
         mode = 0;
+        if (cfg < 0)
+            cfg = slice_pick(conv, p.M, p.N, p.K);
         if (cfg < 0) {
             if (p.K >= 1024 && p.N % 128 == 0 && blocks(128, 128) >= 2048)
                 cfg = slab32 ? 13 : 10;
@@ -825,6 +839,8 @@ static fdx_status run_igemm(GemmParams& p, bool conv, int batch, const char* fam
                 [&] { pw_stream_launch(p, a_bytes, b_bytes, s); });
             settle();
         }
+        if (cfg < 0 && fast_ok && batch == 1)
+            cfg = slice_pick(conv, p.M, p.N, p.K);
         static const bool closed_cuts = [] { const char* e = std::getenv("FDX_CLOSED_SPLIT"); return !(e && e[0] == '0'); }();
         if (cfg >= 0) {
         } else if (stream_ok && p.K <= 32 && p.N <= 160 && p.M >= 65536) {
@@ -893,7 +909,9 @@ static fdx_status run_igemm(GemmParams& p, bool conv, int batch, const char* fam
         q.a_records = (uint32_t)a_bytes;
         q.b_records = (uint32_t)b_bytes;
         q.batch = batch;
-        if (!launch_fast(cfg, splits, mode, q, conv, batch, s))
+        if (cfg >= kSliceCfg)
+            slice_launch(cfg, q, conv, s);
+        else if (!launch_fast(cfg, splits, mode, q, conv, batch, s))
             launch_fast(cfg, 1, 0, q, conv, batch, s); // the requested cut does not fit the scratch
     } else {
         launch_general(cfg);

@@ -1,0 +1,317 @@
+// Problems with few output tiles (included inside namespace fdx by igemm.hip after igemm_fast.hpp): a network at batch 1,
+// short sequences, the last stages of a small batch.
+//
+// There the tiled kernel leaves most of the chip idle: a 64 x 64 tile of a 14 x 14 map walks K = 2304 slab by slab, each
+// slab a round trip to memory, an LDS pass and a barrier (one image, weights out of memory, per launch: 14 x 14 3x3
+// 256 -> 256 19.6 us, 1x1 1024 -> 256 13.6, 7 x 7 3x3 512 -> 512 26.8; here 9.4, 4.7, 13.2, of which 3.5 are the launch
+// itself; ResNet50 at batch 1 761 -> 390 us).  What bounds it is the path from L2 into a CU.  Here the eight (or sixteen) waves of a workgroup share one
+// small output tile and cut its K range between them, every wave on its own:
+//
+//  * a wave loads its units (UK consecutive k of all tile rows) as runs of 64 or 128 bytes per row, DEPTH units in flight from
+//    the first instruction on, and turns them into MFMA operands through a strip of LDS of its own: no barrier in the loop.
+//    (Loaded straight in operand order, 16x16x4 MFMA's neighbouring lanes lie in different rows, which the address unit
+//    takes one lane at a time: 77 cycles per 16-byte load and CU measured, whatever the rows' pitch.)
+//  * the waves' partial tiles meet once in LDS and are added in wave order (the sum does not depend on timing), the
+//    epilogue runs on the sum.  Bias and residual are requested in front of the K walk.
+//  * tiles are numbered so that an XCD owns neighbours that share the larger operand's rows: it passes through one L2.
+template <int TM, int TN, int NW, int UK, bool CONV, bool DUAL>
+__global__ __launch_bounds__(64 * NW) void igemm_slice_kernel(GemmParams p)
+{
+    constexpr int BM = 16 * TM, BN = 16 * TN;
+    constexpr int CPR = UK / 4, RPI = 64 / CPR;         // 16-byte chunks per row and unit; rows per load instruction
+    constexpr int AL = BM / RPI, BL = BN / RPI;         // load instructions per unit
+    constexpr int DEPTH = AL + BL <= 2 ? 8 : AL + BL <= 4 ? 4 : AL + BL <= 8 ? 2 : 1; // units in flight: up to 64 registers
+    constexpr int US = UK + 4, RS = BN + 4;             // LDS rows: a staged unit, a partial tile
+    constexpr int STRIP = (BM + BN) * US > BM * RS ? (BM + BN) * US : BM * RS;
+    constexpr uint32_t OOB = 0x80000000u;
+    static_assert(!DUAL || !CONV, "two sources: GEMM form only");
+    __shared__ __attribute__((aligned(16))) float smem[NW * STRIP];
+
+    const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int fr = lane & 15, fg = lane >> 4;
+    const int lrow = lane / CPR, lchunk = lane % CPR;
+    float* strip = smem + wave * STRIP;
+    const int tiles_m = (p.M + BM - 1) / BM, tiles_n = (p.N + BN - 1) / BN;
+    int id = blockIdx.x;
+    {
+        const int total = tiles_m * tiles_n, xcd = id & 7, per = total >> 3, rem = total & 7;
+        id = xcd * per + (xcd < rem ? xcd : rem) + (id >> 3);
+    }
+    int mt, nt;
+    if (p.M >= p.N) {
+        mt = id / tiles_n;
+        nt = id - mt * tiles_n;
+    } else {
+        nt = id / tiles_m;
+        mt = id - nt * tiles_m;
+    }
+    const int m0 = mt * BM, n0 = nt * BN;
+
+    uint32_t a_voff[AL], a2_voff[DUAL ? AL : 1], b_voff[BL];
+    uint64_t a_mask[AL];
+#pragma unroll
+    for (int i = 0; i < AL; ++i) {
+        const int m = m0 + i * RPI + lrow;
+        a_voff[i] = OOB;
+        a_mask[i] = 0;
+        if (DUAL)
+            a2_voff[i] = OOB;
+        if (m < p.M) {
+            if (CONV) {
+                const int img = m / (p.OH * p.OW), rm = m - img * (p.OH * p.OW);
+                const int oy = rm / p.OW, ox = rm - oy * p.OW;
+                const int iy0 = oy * p.sy - p.pad_top, ix0 = ox * p.sx - p.pad_left;
+                a_voff[i] = (uint32_t)(((img * p.H + oy * p.sy) * p.W + ox * p.sx) * p.pix_stride) * 4u + lchunk * 16;
+                uint64_t mk = 0;
+                for (int y = 0; y < p.kh; ++y) {
+                    const int iy = iy0 + y * p.dy;
+                    for (int x = 0; x < p.kw; ++x) {
+                        const int ix = ix0 + x * p.dx;
+                        if (iy >= 0 && iy < p.H && ix >= 0 && ix < p.W)
+                            mk |= 1ull << (y * p.kw + x);
+                    }
+                }
+                a_mask[i] = mk;
+            } else {
+                a_voff[i] = (uint32_t)((int64_t)m * p.lda) * 4u + lchunk * 16;
+                if (DUAL) {
+                    const int img = m / (p.OH * p.OW), rm = m - img * (p.OH * p.OW);
+                    const int oy = rm / p.OW, ox = rm - oy * p.OW;
+                    a2_voff[DUAL ? i : 0] = (uint32_t)(((img * p.H2 + oy * p.s2y) * p.W2 + ox * p.s2x) * p.C2) * 4u + lchunk * 16;
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < BL; ++j) {
+        const int n = n0 + j * RPI + lrow;
+        b_voff[j] = n < p.N ? (uint32_t)((int64_t)n * p.ldb) * 4u + lchunk * 16 : OOB;
+    }
+
+    // this wave's units of 16 k
+    const int units = p.K / UK;
+    const int u_lo = (int)((int64_t)units * wave / NW), u_n = (int)((int64_t)units * (wave + 1) / NW) - u_lo;
+    int issued = 0, soff_b = u_lo * (UK * 4), soff_a = soff_b, tap = 0, fx = 0, fy = 0, c0 = 0;
+    if (CONV) {
+        const int k = u_lo * UK;
+        tap = k / p.Cin;
+        c0 = k - tap * p.Cin;
+        fy = tap / p.kw;
+        fx = tap - fy * p.kw;
+        soff_a = ((fy * p.dy * p.W + fx * p.dx) * p.pix_stride + c0) * 4;
+    }
+    f32x4 ra[DEPTH][AL], rb[DEPTH][BL];
+    uint32_t a_eff[CONV ? AL : 1]; // a_voff under the current filter tap: out of range where the tap lies outside the image
+    auto enter_tap = [&]() {
+        if (CONV) {
+#pragma unroll
+            for (int i = 0; i < AL; ++i)
+                a_eff[CONV ? i : 0] = ((a_mask[i] >> tap) & 1) ? a_voff[i] : OOB;
+        }
+    };
+    enter_tap();
+    auto issue = [&](int d) {
+        // Loads are unconditional: behind a branch the compiler would have to assume the fewest loads in flight at every
+        // wait.  A unit beyond the range reads through a descriptor of extent zero, which answers zeros without traffic.
+        const bool live = issued < u_n;
+        const __amdgpu_buffer_rsrc_t srd_b = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p.B), 0, live ? (int)p.b_records : 0, 0x00020000);
+        if (DUAL && soff_b >= p.K1 * 4) {
+            const __amdgpu_buffer_rsrc_t srd_a2 = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p.A2), 0, live ? (int)p.a2_records : 0, 0x00020000);
+#pragma unroll
+            for (int i = 0; i < AL; ++i)
+                ra[d][i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(srd_a2, (int)a2_voff[DUAL ? i : 0], soff_b - p.K1 * 4, 0));
+        } else {
+            const __amdgpu_buffer_rsrc_t srd_a = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p.A), 0, live ? (int)p.a_records : 0, 0x00020000);
+#pragma unroll
+            for (int i = 0; i < AL; ++i)
+                ra[d][i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(srd_a, (int)(CONV ? a_eff[CONV ? i : 0] : a_voff[i]), soff_a, 0));
+        }
+#pragma unroll
+        for (int j = 0; j < BL; ++j)
+            rb[d][j] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(srd_b, (int)b_voff[j], soff_b, 0));
+        ++issued;
+        soff_b += UK * 4;
+        if (CONV) {
+            c0 += UK;
+            if (c0 == p.Cin) {
+                c0 = 0;
+                ++tap;
+                if (++fx == p.kw) {
+                    fx = 0;
+                    ++fy;
+                }
+                enter_tap();
+            }
+            soff_a = ((fy * p.dy * p.W + fx * p.dx) * p.pix_stride + c0) * 4;
+        } else {
+            soff_a += UK * 4;
+        }
+    };
+#pragma unroll
+    for (int d = 0; d < DEPTH; ++d)
+        issue(d);
+
+    // what the epilogue reads, requested behind the first operands
+    constexpr int QUADS = BM * BN / 4, QPT = (QUADS + 64 * NW - 1) / (64 * NW);
+    f32x4 bias4[QPT], res4[QPT];
+#pragma unroll
+    for (int q = 0; q < QPT; ++q) {
+        const int quad = t + q * 64 * NW, row = quad / (BN / 4), col = (quad % (BN / 4)) * 4;
+        const bool ok = quad < QUADS && m0 + row < p.M && n0 + col < p.N; // N is a multiple of 4 on this path
+        bias4[q] = res4[q] = f32x4 { 0.f, 0.f, 0.f, 0.f };
+        if (ok && p.bias)
+            bias4[q] = *reinterpret_cast<const f32x4*>(p.bias + n0 + col);
+        if (ok && p.residual)
+            res4[q] = *reinterpret_cast<const f32x4*>(p.residual + (int64_t)(m0 + row) * p.ldc + n0 + col);
+    }
+
+    f32x4 acc[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+            acc[i][j] = f32x4 { 0.f, 0.f, 0.f, 0.f };
+    for (int u = 0; u < u_n; u += DEPTH) {
+#pragma unroll
+        for (int d = 0; d < DEPTH; ++d) {
+            // a wave's LDS accesses complete in order, so the strip needs no second buffer
+#pragma unroll
+            for (int i = 0; i < AL; ++i)
+                *reinterpret_cast<f32x4*>(&strip[(i * RPI + lrow) * US + lchunk * 4]) = ra[d][i];
+#pragma unroll
+            for (int j = 0; j < BL; ++j)
+                *reinterpret_cast<f32x4*>(&strip[(BM + j * RPI + lrow) * US + lchunk * 4]) = rb[d][j];
+            issue(d);
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            if (u + d < u_n) { // uniform over the wave
+                f32x4 af[TM][UK / 16], bf[TN][UK / 16];
+#pragma unroll
+                for (int h = 0; h < UK / 16; ++h) {
+#pragma unroll
+                    for (int i = 0; i < TM; ++i)
+                        af[i][h] = *reinterpret_cast<const f32x4*>(&strip[(i * 16 + fr) * US + h * 16 + fg * 4]);
+#pragma unroll
+                    for (int j = 0; j < TN; ++j)
+                        bf[j][h] = *reinterpret_cast<const f32x4*>(&strip[(BM + j * 16 + fr) * US + h * 16 + fg * 4]);
+                }
+#pragma unroll
+                for (int h = 0; h < UK / 16; ++h)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+#pragma unroll
+                        for (int i = 0; i < TM; ++i)
+#pragma unroll
+                            for (int j = 0; j < TN; ++j)
+                                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(af[i][h][e], bf[j][h][e], acc[i][j], 0, 0, 0);
+            }
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        }
+    }
+
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                strip[(i * 16 + 4 * fg + e) * RS + j * 16 + fr] = acc[i][j][e];
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < QPT; ++q) {
+        const int quad = t + q * 64 * NW, row = quad / (BN / 4), col = (quad % (BN / 4)) * 4;
+        if (quad >= QUADS || m0 + row >= p.M || n0 + col >= p.N)
+            continue;
+        f32x4 s = *reinterpret_cast<const f32x4*>(&smem[row * RS + col]);
+#pragma unroll
+        for (int w = 1; w < NW; ++w)
+            s += *reinterpret_cast<const f32x4*>(&smem[w * STRIP + row * RS + col]);
+        float r[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            r[e] = s[e] * p.alpha + bias4[q][e] + res4[q][e];
+        apply_act_block(r, p.act);
+        *reinterpret_cast<f32x4*>(p.C + (int64_t)(m0 + row) * p.ldc + n0 + col) = f32x4 { r[0], r[1], r[2], r[3] };
+    }
+}
+
+// (rows / 16, columns / 16, waves) of the forms, by configuration number - kSliceCfg
+constexpr int kSliceCfg = 40, kSliceForms = 5;
+struct SliceForm {
+    int tm, tn, nw;
+};
+constexpr SliceForm kSliceForm[kSliceForms] = { { 1, 1, 8 }, { 1, 2, 8 }, { 2, 2, 8 }, { 2, 2, 4 }, { 4, 2, 8 } };
+
+// The form for a problem, or -1 where the tiled kernel is the better one.  Both sides were timed on 483 problems (M 1-16384,
+// N 16-3072, K 32-4608, up to 6 GFLOP, GEMM and convolution, operands out of memory, launches back to back) and follow, in
+// microseconds, with w = tiles per CU rounded up:
+//     slice forms:   t0 + w (c1 + c2 (rows + columns of the tile) K / 10^4), c2 larger for a convolution's addressing
+//     64 x 64 tiles: 4.8 + w (0.44 + 4.9 K / 1000) + t (12.3 K / 1000) + min(t, 1) 5.1 K / 1000,  t = tiles / 256
+// (8-13 % rms the slice forms, 20 % the tiled ones): a workgroup costs what it pulls through its CU's path from L2, about
+// 36 cycles per KB.  By this rule the timed problems take half the time of the tiled kernel alone (geometric mean), and
+// none takes more than 5 % longer.  Below 48 columns the other side is the general kernel's narrow tile, which wins from
+// about 600 row blocks of 64 on (N = 32, K = 144-192: 20000 rows 8.2-9.7 against 6.3-7.2 us here, 50000 rows 11.0-14.5
+// against 11.1-14.0, convolutions 13.9 against 17.1).
+static int slice_pick(bool conv, int M, int N, int K)
+{
+    static const float kCost[kSliceForms][4] = { // t0, c1, c2 of a GEMM, c2 of a convolution
+        { 2.18f, 1.29f, 0.42f, 0.59f }, { 2.13f, 1.07f, 0.50f, 0.62f }, { 2.24f, 1.47f, 0.64f, 1.02f }, { 2.52f, 0.71f, 0.76f, 0.92f },
+        { 1.52f, 2.43f, 0.83f, 1.25f }
+    };
+    const auto tiles_of = [&](int bm, int bn) { return (int64_t)((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
+    const auto per_cu = [](int64_t tiles) { return (float)((tiles + 255) / 256); };
+    const int64_t t64 = tiles_of(64, 64);
+    const bool narrow = N < 48;
+    if (narrow && t64 > 512)
+        return -1;
+    const float k = 1e-3f * K, t = (float)t64 / 256.f;
+    const float tiled = 4.8f + per_cu(t64) * (0.44f + 4.9f * k) + 12.3f * t * k + 5.1f * std::min(t, 1.f) * k;
+    int best = -1;
+    float best_cost = narrow ? 1e30f : (t64 <= 256 ? 0.85f : 0.75f) * tiled; // past a round of tiles operands re-read cost the neighbours, too
+    for (int i = 0; i < kSliceForms; ++i) {
+        const int bm = 16 * kSliceForm[i].tm, bn = 16 * kSliceForm[i].tn;
+        const float cost = kCost[i][0] + per_cu(tiles_of(bm, bn)) * (kCost[i][1] + kCost[i][conv ? 3 : 2] * 0.1f * (bm + bn) * k);
+        if (cost < best_cost) {
+            best_cost = cost;
+            best = kSliceCfg + i;
+        }
+    }
+    return best;
+}
+
+template <int I, int UK>
+static void slice_launch_form(const GemmParams& q, bool conv, hipStream_t s)
+{
+    constexpr SliceForm f = kSliceForm[I];
+    const dim3 grid((unsigned)(((q.M + 16 * f.tm - 1) / (16 * f.tm)) * ((q.N + 16 * f.tn - 1) / (16 * f.tn)))), block(64u * f.nw);
+    if (conv)
+        hipLaunchKernelGGL((igemm_slice_kernel<f.tm, f.tn, f.nw, UK, true, false>), grid, block, 0, s, q);
+    else if (q.A2)
+        hipLaunchKernelGGL((igemm_slice_kernel<f.tm, f.tn, f.nw, UK, false, true>), grid, block, 0, s, q);
+    else
+        hipLaunchKernelGGL((igemm_slice_kernel<f.tm, f.tn, f.nw, UK, false, false>), grid, block, 0, s, q);
+}
+
+static void slice_launch(int cfg, const GemmParams& q, bool conv, hipStream_t s)
+{
+    // the longer unit where a unit stays inside a filter tap / one of two sources
+    const bool wide = (conv ? q.Cin : q.A2 ? (q.K | q.K1) : q.K) % 32 == 0;
+    switch (cfg - kSliceCfg) {
+#define FDX_SLICE(I_)                                \
+    case I_:                                         \
+        if (wide)                                    \
+            slice_launch_form<I_, 32>(q, conv, s);   \
+        else                                         \
+            slice_launch_form<I_, 16>(q, conv, s);   \
+        break;
+        FDX_SLICE(0)
+        FDX_SLICE(1)
+        FDX_SLICE(2)
+        FDX_SLICE(3)
+        FDX_SLICE(4)
+#undef FDX_SLICE
+    }
+}

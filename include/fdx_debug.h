@@ -41,7 +41,8 @@ fdx_status fdx_profile_get_executed(int index, double* executed_flops);
  * every tile configuration and scheduling form of the convolution / GEMM kernels on small problems, where the tuner
  * would never pick them.
  *   fdx_debug_force_tile: -1 = tuner decides; 0..3 general kernel tiles; 10..18 fast-path tiles; 30 = the row-streaming
- *     kernel for K <= 128 (where it does not apply the tuner decides); + 100 * splits
+ *     kernel for K <= 128 (where it does not apply the tuner decides); 40..44 = the forms of the kernel for few output
+ *     tiles; + 100 * splits
  *     (every tile cut into `splits` K ranges), + 10000 (only the last partial round is cut), 20000 + tile = stream-K.
  *   fdx_debug_persist_cap: caps the persistent grid at `workgroups` (at least 8; 0 = the resident count).
  *   fdx_debug_force_strips: whole-tile launches of the fast path number their output tiles in this many column strips

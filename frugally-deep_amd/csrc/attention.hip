@@ -279,9 +279,191 @@ __global__ __launch_bounds__(256) void flash_prefill_kernel(FlashParams p)
     }
 }
 
+// The same products for launches with few queries in flight: one workgroup = 32 query rows of one (sequence, head), its
+// four waves take every fourth block of 32 keys, each with a running maximum, sum and output of its own, and meet once at
+// the end.  What bounds a short launch of the kernel above is one wave's serial walk over the keys (a block of 32 keys
+// costs it D MFMAs of 64 cycles, 1.7 us at depth 64) and CUs without a workgroup: one sequence of 77 / 256 / 512 tokens
+// with 8 heads of 64 takes 13.0 / 23.2 / 42.6 us there and 6.3 / 9.8 / 16.2 here (launches back to back).
+// A wave stages its key / value block through a strip of LDS of its own, so the loop has no barrier; the next block's
+// loads are in flight while a block is worked on.
+template <int D>
+__global__ __launch_bounds__(256) void flash_keysplit_kernel(FlashParams p)
+{
+    constexpr int KS = D + 4, VS = D + 8;  // as above
+    constexpr int LD = D / 8;              // 16-byte loads per lane for a block of 32 rows
+    constexpr int RPL = 256 / D;           // rows per load
+    constexpr int STRIP = 32 * (KS + VS), OS = D + 4;
+    __shared__ __attribute__((aligned(16))) float smem[4 * STRIP];
+    __shared__ float part_m[4][32], part_l[4][32];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int c = lane & 31, half = lane >> 5;
+    const int b = blockIdx.y / p.heads, h = blockIdx.y % p.heads;
+    const int q_first = blockIdx.x * 32, query = q_first + c;
+    const bool q_ok = query < p.t;
+    const int shift = p.s - p.t; // causal: query i sees keys 0 .. i + shift
+    float* ks = smem + wave * STRIP;
+    float* vs = ks + 32 * KS;
+
+    int s_end = p.s;
+    if (p.causal) {
+        const int q_last = (q_first + 32 < p.t ? q_first + 32 : p.t) - 1;
+        s_end = q_last + shift + 1 < p.s ? q_last + shift + 1 : p.s;
+    }
+    const int blocks = (s_end + 31) / 32;
+
+    const float* kbase = p.k + (int64_t)b * p.k_batch + h * D;
+    const float* vbase = p.v + (int64_t)b * p.v_batch + h * D;
+    const int lrow = lane / (D / 4), lcol = 4 * (lane % (D / 4));
+    f32x4 kst[LD], vst[LD];
+    auto fetch = [&](int blk) {
+#pragma unroll
+        for (int i = 0; i < LD; ++i) {
+            const int row = blk * 32 + i * RPL + lrow;
+            kst[i] = vst[i] = f32x4 { 0.f, 0.f, 0.f, 0.f };
+            if (row < p.s) {
+                kst[i] = *reinterpret_cast<const f32x4*>(kbase + (int64_t)row * p.ldk + lcol);
+                vst[i] = *reinterpret_cast<const f32x4*>(vbase + (int64_t)row * p.ldv + lcol);
+            }
+        }
+    };
+    if (wave < blocks)
+        fetch(wave);
+
+    // this lane's half of its query row: depth 8u + 4*half .. + 3, the same split the key fragments use
+    f32x4 qreg[D / 8];
+    {
+        const float* qrow = p.q + (int64_t)b * p.q_batch + (int64_t)(q_ok ? query : 0) * p.ldq + h * D + 4 * half;
+#pragma unroll
+        for (int u = 0; u < D / 8; ++u)
+            qreg[u] = q_ok ? *reinterpret_cast<const f32x4*>(qrow + 8 * u) : f32x4 { 0.f, 0.f, 0.f, 0.f };
+    }
+
+    f32x16 oacc[D / 32];
+#pragma unroll
+    for (int d = 0; d < D / 32; ++d)
+#pragma unroll
+        for (int e = 0; e < 16; ++e)
+            oacc[d][e] = 0.f;
+    float m_run = -INFINITY, l_run = 0.f;
+    const int key_limit = p.causal ? (query + shift < p.s - 1 ? query + shift : p.s - 1) : p.s - 1;
+
+    for (int blk = wave; blk < blocks; blk += 4) { // uniform over the wave
+        // a wave's LDS accesses complete in order, so the strip needs no second buffer
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+        for (int i = 0; i < LD; ++i) {
+            *reinterpret_cast<f32x4*>(&ks[(i * RPL + lrow) * KS + lcol]) = kst[i];
+            *reinterpret_cast<f32x4*>(&vs[(i * RPL + lrow) * VS + lcol]) = vst[i];
+        }
+        if (blk + 4 < blocks)
+            fetch(blk + 4);
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+
+        // S^T block: 32 keys x 32 queries
+        f32x16 sacc;
+#pragma unroll
+        for (int e = 0; e < 16; ++e)
+            sacc[e] = 0.f;
+#pragma unroll
+        for (int u = 0; u < D / 8; ++u) {
+            const f32x4 kf = *reinterpret_cast<const f32x4*>(&ks[c * KS + 8 * u + 4 * half]);
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                sacc = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[e], qreg[u][e], sacc, 0, 0, 0);
+        }
+        float mx = -INFINITY;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            const int key = blk * 32 + 8 * (e >> 2) + 4 * half + (e & 3);
+            sacc[e] = key <= key_limit ? sacc[e] * p.scale : -INFINITY;
+            mx = fmaxf(mx, sacc[e]);
+        }
+        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        const float m_new = fmaxf(m_run, mx);
+        const float m_use = m_new == -INFINITY ? 0.f : m_new; // no visible key yet
+        const float corr = expf(m_run - m_use);
+        float rs = 0.f;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            sacc[e] = __expf(sacc[e] - m_use);
+            rs += sacc[e];
+        }
+        rs += __shfl_xor(rs, 32, 64);
+        l_run = l_run * corr + rs;
+        m_run = m_new;
+#pragma unroll
+        for (int d = 0; d < D / 32; ++d)
+#pragma unroll
+            for (int e = 0; e < 16; ++e)
+                oacc[d][e] *= corr;
+        // O^T += V^T P^T
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            const float* vrow = &vs[(8 * (e >> 2) + 4 * half + (e & 3)) * VS + c];
+#pragma unroll
+            for (int d = 0; d < D / 32; ++d)
+                oacc[d] = __builtin_amdgcn_mfma_f32_32x32x2f32(vrow[32 * d], sacc[e], oacc[d], 0, 0, 0);
+        }
+    }
+
+    // the waves' shares meet: [query][depth] in the wave's own strip
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+    for (int d = 0; d < D / 32; ++d)
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+            *reinterpret_cast<f32x4*>(&ks[c * OS + 32 * d + 8 * g + 4 * half])
+                = f32x4 { oacc[d][4 * g], oacc[d][4 * g + 1], oacc[d][4 * g + 2], oacc[d][4 * g + 3] };
+    if (half == 0) {
+        part_m[wave][c] = m_run;
+        part_l[wave][c] = l_run;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < D / 32; ++i) {
+        const int idx = tid + 256 * i, row = idx / (D / 4), col = 4 * (idx % (D / 4));
+        if (q_first + row >= p.t)
+            continue;
+        float m = fmaxf(fmaxf(part_m[0][row], part_m[1][row]), fmaxf(part_m[2][row], part_m[3][row]));
+        m = m == -INFINITY ? 0.f : m;
+        float l = 0.f;
+        f32x4 o = { 0.f, 0.f, 0.f, 0.f };
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+            const float f = expf(part_m[w][row] - m);
+            l += f * part_l[w][row];
+            o += f * *reinterpret_cast<const f32x4*>(&smem[w * STRIP + row * OS + col]);
+        }
+        *reinterpret_cast<f32x4*>(p.out + (int64_t)b * p.o_batch + (int64_t)(q_first + row) * p.ldo + h * D + col)
+            = o * (l > 0.f ? 1.0f / l : 0.f);
+    }
+}
+
+// Which of the two, from 292 timed problems (4 to 16 heads of 32, 64 and 128, 1 to 64 sequences of 16 to 512 tokens, causal
+// and not).  Up to 32 queries the kernel above has work for one of its four waves: 1.2 to 1.8 times faster here, at depth
+// 128 (one workgroup per CU by LDS) as long as every CU takes one.  Beyond, a workgroup here reads keys and values for 32
+// queries instead of 128, which shows as soon as CUs take turns: with one workgroup per CU 1.2 to 2.7 times faster; up to
+// 448 with more than one 64-key tile 1.1 to 1.7 times (two keys' blocks only, 384 workgroups: 9.6 against 8.2 us); from 512
+// on 0.6 to 1.3 times.
+static bool keysplit_better(const FlashParams& p, int batch, int d)
+{
+    const int64_t groups = (int64_t)((p.t + 31) / 32) * batch * p.heads;
+    return groups <= 256 || (p.t <= 32 && d < 128) || (groups <= 448 && p.s > 64);
+}
+
 template <int DK, int DV>
 static void flash_launch(const FlashParams& p, int batch)
 {
+    if (DK == DV && keysplit_better(p, batch, DK)) {
+        hipLaunchKernelGGL(flash_keysplit_kernel<DK>, dim3((unsigned)((p.t + 31) / 32), (unsigned)(batch * p.heads)), dim3(256), 0, stream(), p);
+        return;
+    }
     const dim3 grid((unsigned)((p.t + 127) / 128), (unsigned)(batch * p.heads));
     hipLaunchKernelGGL((flash_prefill_kernel<DK, DV>), grid, dim3(256), 0, stream(), p);
 }

@@ -722,10 +722,13 @@ __global__ __launch_bounds__(256) void mha_decode_dyn_kernel(const float* __rest
 }
 
 // Packs (value, column) so that an unsigned 64-bit max picks the largest value and, among equal values,
-// the smallest column: the first maximum wins, as in the reference's tensor_max_pos.
+// the smallest column: the first maximum wins, as in the reference's tensor_max_pos.  As there, -0 equals 0 and a value
+// that does not exceed the lowest float (NaN included) never wins: 0 = "no value", column 0 if there is no other.
 __device__ __forceinline__ unsigned long long pack_max(float v, int col)
 {
-    unsigned int u = __float_as_uint(v);
+    if (!(v > -3.402823466e+38f))
+        return 0ull;
+    unsigned int u = __float_as_uint(v + 0.0f);
     u = (u & 0x80000000u) ? ~u : (u | 0x80000000u); // order-preserving map of floats to unsigned
     return ((unsigned long long)u << 32) | (unsigned long long)(0xFFFFFFFFu - (unsigned int)col);
 }

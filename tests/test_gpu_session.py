@@ -269,3 +269,28 @@ def test_greedy_loop_with_the_embedding_in_the_previous_steps_last_launch(fdx, m
     for i in range(6):
         _, cur = single.decode_step(cur)
         assert np.array_equal(part3[i], cur), i
+
+
+@pytest.mark.parametrize("heads,d_model,vocab", [(1, 64, 40009), (3, 192, 33000)])
+def test_prompts_last_position_runs_through_the_decode_launches(fdx, oracle, modelgen, heads, d_model, vocab):
+    """Behind the last attention layer's keys and values a prompt goes on for its last position only, on the decode
+    launches: against the oracle, for a first prompt, a continued one and prompts of 1 and 2 tokens, then greedy tokens from
+    there; and against a session too long for the decode attention's single pass, which keeps the general launches."""
+    say("prompt tail on decode launches", heads, d_model, vocab)
+    js = modelgen.dumps(modelgen.gpt2(seed=71, layers=2, d_model=d_model, heads=heads, vocab=vocab, max_pos=96, bias_std=0.1,
+                                      random_affine=True, std=0.2))
+    model, ref = fdx.Model(js), oracle.OracleModel(js)
+    for B in (1, 5, 16):
+        ids = np.random.default_rng(72 + B).integers(0, vocab, (B, 50))
+        short, long = fdx.Session(model, B, 64), fdx.Session(model, B, 16384)
+        for lo, hi in ((0, 37), (37, 38), (38, 40), (40, 50)):
+            logits, nxt = short.prefill(ids[:, lo:hi])
+            general, _ = long.prefill(ids[:, lo:hi])
+            assert np.array_equal(nxt, np.argmax(logits, -1).astype(nxt.dtype)), (B, hi)
+            assert rel(logits, general) <= 1e-5, (B, hi)
+        assert short.length() == 50
+        want = oracle_logits(ref, ids[B - 1].astype(np.float32))[-1]
+        assert rel(logits[B - 1], want) <= TOL
+        tokens, last = short.decode_greedy(nxt, 3)
+        seq = np.concatenate([ids[0], nxt[:1], tokens[:2, 0]]).astype(np.float32)
+        assert rel(last[0], oracle_logits(ref, seq)[-1]) <= TOL

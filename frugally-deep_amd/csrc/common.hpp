@@ -132,6 +132,14 @@ __device__ __forceinline__ float row16_sum(float v)
 }
 #endif
 
+// A column range of a GEMM's output with a tensor of its own (gemm_segments_launch): `cols` columns, rows `ld` floats apart
+// inside a sequence, sequences `stride` floats apart.
+struct GemmSegment {
+    float* ptr;
+    int64_t ld, stride;
+    int cols;
+};
+
 // activations an epilogue can carry
 inline bool epilogue_act_ok(const fdx_act* a) { return !a || a->kind == FDX_ACT_NONE || a->kind == FDX_ACT_RELU || a->kind == FDX_ACT_GELU; }
 

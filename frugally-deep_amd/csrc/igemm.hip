@@ -1051,6 +1051,62 @@ fdx_status gemm_ln_launch(const float* x, int64_t m, int k, const float* w, cons
     p.ln_eps = eps;
     return run_igemm(p, false, 1, "gemm_ln_f32");
 }
+// C = A . W^T + bias with the columns of C in up to three tensors and the rows of each in sequences of `rows` that lie apart
+// (see SEG in igemm_fast.hpp).  Segments start at multiples of 64 columns (a tile has one segment), K is a multiple of the
+// 32-float slab and every segment stays below 2 GiB (32-bit offsets in the epilogue).
+bool gemm_segments_supported(const GemmSegment* seg, int n_seg, int m, int rows, int k, const float* a, const float* w, const float* bias)
+{
+    if (n_seg < 1 || n_seg > 3 || m <= 0 || rows <= 0 || m % rows != 0 || k <= 0 || k % 32 != 0 || (int64_t)m * k >= (1LL << 29)
+        || !aligned16(a) || !aligned16(w) || (bias && !aligned16(bias)))
+        return false;
+    int64_t n = 0;
+    for (int i = 0; i < n_seg; ++i) {
+        n += seg[i].cols;
+        if (seg[i].cols <= 0 || seg[i].cols % 64 != 0 || !aligned16(seg[i].ptr) || seg[i].ld % 4 != 0 || seg[i].stride % 4 != 0
+            || seg[i].ld < seg[i].cols || seg[i].stride < 0
+            || (int64_t)(m / rows - 1) * seg[i].stride + (int64_t)(rows - 1) * seg[i].ld + seg[i].cols >= (1LL << 29))
+            return false;
+    }
+    return n * k < (1LL << 29);
+}
+
+fdx_status gemm_segments_launch(const float* a, const float* w, const float* bias, int m, int rows, int k, const GemmSegment* seg, int n_seg)
+{
+    FDX_REQUIRE(a && w && gemm_segments_supported(seg, n_seg, m, rows, k, a, w, bias), "gemm_segments: bad arguments");
+    std::lock_guard<std::mutex> lock(g_igemm_mutex);
+    GemmParams p {};
+    p.A = a; p.B = w; p.bias = bias;
+    p.M = m; p.K = k; p.lda = k; p.ldb = k;
+    p.alpha = 1.f; p.act = make_act(nullptr);
+    p.inner = 1; p.batch = 1; p.splits = 1;
+    p.seg_rows = rows;
+    for (int i = 0; i < 3; ++i) {
+        if (i < n_seg) {
+            p.N += seg[i].cols;
+            p.seg_ptr[i] = seg[i].ptr;
+            p.seg_ld[i] = seg[i].ld;
+            p.seg_stride[i] = seg[i].stride;
+        }
+        p.seg_col[i] = p.N;
+    }
+    p.ldc = p.N; // the tile walk's own arithmetic
+    p.a_records = (uint32_t)((int64_t)m * k * 4);
+    p.b_records = (uint32_t)((int64_t)p.N * k * 4);
+    profile_begin();
+    switch (slice_pick(false, m, p.N, k)) {
+    case kSliceCfg: slice_launch_seg<0>(p, stream()); break;
+    case kSliceCfg + 1: slice_launch_seg<1>(p, stream()); break;
+    case kSliceCfg + 2: slice_launch_seg<2>(p, stream()); break;
+    case kSliceCfg + 3: slice_launch_seg<3>(p, stream()); break;
+    case kSliceCfg + 4: slice_launch_seg<4>(p, stream()); break;
+    default:
+        launch_persistent(igemm_fast_kernel<64, 64, 2, 2, 32, false, false, false, false, false, true>, ((m + 63) / 64) * ((p.N + 63) / 64), p,
+            stream(), 256, 64, 64);
+    }
+    profile_end("gemm_f32", 2.0 * m * (double)p.N * k, 0.0);
+    FDX_LAUNCH_CHECK();
+    return FDX_OK;
+}
 } // namespace fdx
 
 extern "C" fdx_status fdx_debug_dual_conv(int one_launch)

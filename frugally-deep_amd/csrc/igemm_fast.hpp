@@ -31,6 +31,15 @@
 //    and their workspace slots computed from the cut points.
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
+// Where row m, column n of a tile whose first column is n0 lies with SEG, in bytes from the start of its segment; segments
+// begin at multiples of the tile width, so a tile's segment is uniform.
+__device__ __forceinline__ uint32_t seg_offset(const GemmParams& p, int sg, int m, int n)
+{
+    const int seq = m / p.seg_rows, row = m - seq * p.seg_rows;
+    return (uint32_t)(seq * p.seg_stride[sg] + row * p.seg_ld[sg] + n - (sg ? p.seg_col[sg - 1] : 0)) * 4u;
+}
+__device__ __forceinline__ int seg_of(const GemmParams& p, int n0) { return (n0 >= p.seg_col[0]) + (n0 >= p.seg_col[1]); }
+
 //  * DUAL (GEMM form, whole tiles only): the rows of A come from two tensors -- the first K1 columns from A with row
 //    stride lda, the other K - K1 from A2, whose row for output pixel (image, y, x) is pixel (y * s2y, x * s2x) of an
 //    [H2][W2][C2] map.  That is the sum of two pointwise convolutions as one GEMM over the concatenated channels
@@ -43,8 +52,11 @@ typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 //    the lanes that share a row after the loop, and applied in the epilogue as
 //        rstd * (acc - mean * rowsum(B)) + bias:
 //    no pass over A of its own, and the normalised tensor never exists.
+//  * SEG (GEMM form, whole tiles only): the columns of C go to up to three tensors, the rows of each in sequences that lie
+//    apart: the stacked query / key / value projection of prompts, keys and values straight into their cache rows (2048 rows, 768 -> 3 x 768:
+//    69 us instead of three launches of 29.6, which leave 384 tiles on 256 CUs each).
 template <int BM, int BN, int WAVES_M, int WAVES_N, int BKT, bool CONV, bool SPLIT = false, bool STREAMK = false, bool DUAL = false,
-    bool LNF = false>
+    bool LNF = false, bool SEG = false>
 // (the second bound asks for two waves per SIMD where the split variant of the largest four-wave tile would otherwise
 // settle for one: its reduction holds the accumulators in ordinary registers next to the prefetched operands)
 __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, (SPLIT && WAVES_M * WAVES_N == 4 && BM * BN >= 128 * 128) ? 2 : 1)
@@ -54,6 +66,7 @@ void igemm_fast_kernel(GemmParams p)
     static_assert(NT == 256 || NT == 512, "four or eight waves");
     static_assert(!DUAL || (!CONV && !SPLIT), "the two-source form is a whole-tile GEMM");
     static_assert(!LNF || (!CONV && !SPLIT && !DUAL), "the normalising form is a whole-tile GEMM");
+    static_assert(!SEG || (!CONV && !SPLIT && !DUAL && !LNF), "the form with segmented outputs is a whole-tile GEMM");
     constexpr int STRIDE = BKT + 4;
     constexpr int CPR = BKT / 4;  // 16-byte chunks per tile row
     constexpr int RPP = NT / CPR; // tile rows filled per loader pass
@@ -536,7 +549,13 @@ void igemm_fast_kernel(GemmParams p)
 #pragma unroll
             for (int ps = 0; ps < 32 / RPS; ++ps) {
                 const int m = em0 + wm * WTM + i * 32 + ps * RPS + srow;
-                if (m < p.M && n_ok) {
+                if (SEG) {
+                    if (m < p.M && n_ok) {
+                        const int sg = seg_of(p, en0);
+                        const __amdgpu_buffer_rsrc_t srd_c = __builtin_amdgcn_make_buffer_rsrc(p.seg_ptr[sg], 0, -1, 0x00020000);
+                        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, done[ps]), srd_c, (int)seg_offset(p, sg, m, n), 0, 16);
+                    }
+                } else if (m < p.M && n_ok) {
                     // written through to memory (agent scope) rather than left dirty in this XCD's L2: the next layer's
                     // workgroups run on all XCDs, and what a kernel leaves dirty is written back at its end with nothing
                     // else running (ResNet50 +0.4 %; the non-temporal hint instead: -0.8 %).  A buffer store because that

@@ -52,6 +52,11 @@ struct GemmParams {
     // ln_wsum = per output column the sum of its (gamma-folded) filter row, nullptr = no normalisation
     const float* ln_wsum;
     float ln_eps;
+    // fast path, GEMM form, whole tiles (see SEG in igemm_fast.hpp): output columns [seg_col[i - 1], seg_col[i]) go to
+    // seg_ptr[i], row m as row m % seg_rows of sequence m / seg_rows; C and ldc are not used
+    float* seg_ptr[3];
+    int64_t seg_ld[3], seg_stride[3]; // floats between rows of a sequence, between sequences
+    int seg_col[3], seg_rows;
 };
 
 // Key of the per-process tuning table (igemm.hip).  conv = 0 / 1: a GEMM / convolution shape and its tile choice

@@ -14,7 +14,7 @@
 //  * the waves' partial tiles meet once in LDS and are added in wave order (the sum does not depend on timing), the
 //    epilogue runs on the sum.  Bias and residual are requested in front of the K walk.
 //  * tiles are numbered so that an XCD owns neighbours that share the larger operand's rows: it passes through one L2.
-template <int TM, int TN, int NW, int UK, bool CONV, bool DUAL>
+template <int TM, int TN, int NW, int UK, bool CONV, bool DUAL, bool SEG = false>
 __global__ __launch_bounds__(64 * NW) void igemm_slice_kernel(GemmParams p)
 {
     constexpr int BM = 16 * TM, BN = 16 * TN;
@@ -25,6 +25,7 @@ __global__ __launch_bounds__(64 * NW) void igemm_slice_kernel(GemmParams p)
     constexpr int STRIP = (BM + BN) * US > BM * RS ? (BM + BN) * US : BM * RS;
     constexpr uint32_t OOB = 0x80000000u;
     static_assert(!DUAL || !CONV, "two sources: GEMM form only");
+    static_assert(!SEG || (!CONV && !DUAL), "segmented outputs: GEMM form only");
     __shared__ __attribute__((aligned(16))) float smem[NW * STRIP];
 
     const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -234,7 +235,11 @@ __global__ __launch_bounds__(64 * NW) void igemm_slice_kernel(GemmParams p)
         for (int e = 0; e < 4; ++e)
             r[e] = s[e] * p.alpha + bias4[q][e] + res4[q][e];
         apply_act_block(r, p.act);
-        *reinterpret_cast<f32x4*>(p.C + (int64_t)(m0 + row) * p.ldc + n0 + col) = f32x4 { r[0], r[1], r[2], r[3] };
+        if (SEG) {
+            const int sg = seg_of(p, n0);
+            *reinterpret_cast<f32x4*>(reinterpret_cast<char*>(p.seg_ptr[sg]) + seg_offset(p, sg, m0 + row, n0 + col)) = f32x4 { r[0], r[1], r[2], r[3] };
+        } else
+            *reinterpret_cast<f32x4*>(p.C + (int64_t)(m0 + row) * p.ldc + n0 + col) = f32x4 { r[0], r[1], r[2], r[3] };
     }
 }
 
@@ -293,6 +298,15 @@ static void slice_launch_form(const GemmParams& q, bool conv, hipStream_t s)
         hipLaunchKernelGGL((igemm_slice_kernel<f.tm, f.tn, f.nw, UK, false, true>), grid, block, 0, s, q);
     else
         hipLaunchKernelGGL((igemm_slice_kernel<f.tm, f.tn, f.nw, UK, false, false>), grid, block, 0, s, q);
+}
+
+// the form for outputs in segments, K a multiple of 32
+template <int I>
+static void slice_launch_seg(const GemmParams& q, hipStream_t s)
+{
+    constexpr SliceForm f = kSliceForm[I];
+    const dim3 grid((unsigned)(((q.M + 16 * f.tm - 1) / (16 * f.tm)) * ((q.N + 16 * f.tn - 1) / (16 * f.tn)))), block(64u * f.nw);
+    hipLaunchKernelGGL((igemm_slice_kernel<f.tm, f.tn, f.nw, 32, false, false, true>), grid, block, 0, s, q);
 }
 
 static void slice_launch(int cfg, const GemmParams& q, bool conv, hipStream_t s)

@@ -168,5 +168,7 @@ fdx_status mha_prefill_strided(const float* q, int64_t ldq, int64_t q_batch, con
     float* out, int64_t ldo, int64_t o_batch, void* scratch_dev);
 fdx_status argmax_launch(const float* x, int64_t rows, int depth, int32_t* out_idx, float* out_val, float* out_idx_f);
 fdx_status einsum_launch(EinsumSpec& spec, const float* in, const float* kernel, const float* bias, const Act& act, float* out);
+bool gemm_segments_supported(const GemmSegment* seg, int n_seg, int m, int rows, int k, const float* a, const float* w, const float* bias);
+fdx_status gemm_segments_launch(const float* a, const float* w, const float* bias, int m, int rows, int k, const GemmSegment* seg, int n_seg);
 fdx_status gather_rows_launch(const float* in, int64_t rows, int depth, int64_t row_stride, int64_t offset, float* out);
 }

@@ -24,6 +24,7 @@ struct fdx_session {
     int last_mha_pos = -1;
     int vocab = 0;
     std::map<int, float*> kc, vc; // per MultiHeadAttention op
+    std::map<int, std::pair<const float*, const float*>> qkv; // stacked query / key / value filters and biases of the fast path
     // bump arena for activations of one call; chunks are kept and reused by later calls
     struct Chunk {
         void* p;
@@ -254,20 +255,43 @@ fdx_status run(fdx_session* s, const float* ids_dev, int T, float* logits_dev, f
             bool by_steps = T > 1 && (int)p == s->last_mha_pos && s->tail_step >= 0;
             for (const auto& ti : s->tail_inputs)
                 by_steps = by_steps && buf[ti.op] && rows[ti.op] == (int64_t)B * T;
-            if (by_steps) {
-                // keys / values of all rows; query, attention and everything behind it for the last position (the decode
-                // launches write that position's keys / values once more).  Where the head has 50257 columns this
-                // replaces a 115 us GEMM, a 55 us pass over its logits and the layer's two projections and attention
-                // over all rows (16 prompts of 128 tokens, 12 layers of 768: 3768 -> 3569 us; one of 37 tokens: 240 us less).
+            // projections of the new rows: one GEMM over the stacked filters where the fast path has them, keys / values
+            // straight into their cache rows; otherwise a launch each
+            auto project = [&](float* q) -> fdx_status { // q null: keys and values only
+                float* kdst = kc + (int64_t)s->len * nk;
+                float* vdst = vc + (int64_t)s->len * nv;
+                const auto stacked = s->qkv.find(idx);
+                if (stacked != s->qkv.end()) {
+                    const float* w = stacked->second.first + (q ? 0 : nk * D);
+                    const float* bias = stacked->second.second + (q ? 0 : nk);
+                    const GemmSegment seg[3] = { { q, nk, T * nk, (int)nk }, { kdst, nk, s->max_len * nk, (int)nk },
+                        { vdst, nv, s->max_len * nv, (int)nv } };
+                    const GemmSegment* first = q ? seg : seg + 1;
+                    const int n_seg = q ? 3 : 2;
+                    if (B * (int64_t)T < (1LL << 31) && gemm_segments_supported(first, n_seg, B * T, T, D, in0, w, bias))
+                        return gemm_segments_launch(in0, w, bias, B * T, T, D, first, n_seg);
+                }
+                fdx_status ps = FDX_OK;
+                if (q)
+                    ps = fdx_gemm_bias_act_f32(in0, D, o.dw[0], D, B * T, (int)nk, D, 1.f, o.dw[1], 0, nullptr, nullptr, q, nk, nullptr);
                 fdx_gemm_batch bt {};
                 bt.batch = B;
                 bt.inner = 1;
                 bt.a_outer = (int64_t)T * D;
                 bt.c_outer = (int64_t)s->max_len * nk;
-                st = fdx_gemm_bias_act_f32(in0, D, o.dw[2], D, T, (int)nk, D, 1.f, o.dw[3], 0, nullptr, nullptr, kc + (int64_t)s->len * nk, nk, &bt);
+                if (ps == FDX_OK)
+                    ps = fdx_gemm_bias_act_f32(in0, D, o.dw[2], D, T, (int)nk, D, 1.f, o.dw[3], 0, nullptr, nullptr, kdst, nk, &bt);
                 bt.c_outer = (int64_t)s->max_len * nv;
-                if (st == FDX_OK)
-                    st = fdx_gemm_bias_act_f32(in0, D, o.dw[4], D, T, (int)nv, D, 1.f, o.dw[5], 0, nullptr, nullptr, vc + (int64_t)s->len * nv, nv, &bt);
+                if (ps == FDX_OK)
+                    ps = fdx_gemm_bias_act_f32(in0, D, o.dw[4], D, T, (int)nv, D, 1.f, o.dw[5], 0, nullptr, nullptr, vdst, nv, &bt);
+                return ps;
+            };
+            if (by_steps) {
+                // keys / values of all rows; query, attention and everything behind it for the last position (the decode
+                // launches write that position's keys / values once more).  Where the head has 50257 columns this
+                // replaces a 115 us GEMM, a 55 us pass over its logits and the layer's two projections and attention
+                // over all rows (16 prompts of 128 tokens, 12 layers of 768: 3768 -> 3569 us; one of 37 tokens: 240 us less).
+                st = project(nullptr);
                 for (const auto& ti : s->tail_inputs)
                     if (st == FDX_OK)
                         st = gather_rows_launch(buf[ti.op], B, ti.depth, (int64_t)T * ti.depth, (int64_t)(T - 1) * ti.depth, ti.dst);
@@ -288,27 +312,19 @@ fdx_status run(fdx_session* s, const float* ids_dev, int T, float* logits_dev, f
                 set_error("session: out of device memory");
                 return FDX_ERR_HIP;
             }
-            if ((st = fdx_gemm_bias_act_f32(in0, D, o.dw[0], D, (int)R, (int)nk, D, 1.f, o.dw[1], 0, nullptr, nullptr, q, nk, nullptr)) != FDX_OK)
-                return st;
             // keys / values of the new tokens go straight into their cache rows
             float* kdst = kc + (int64_t)s->len * nk;
             float* vdst = vc + (int64_t)s->len * nv;
             if (T == 1) {
+                if ((st = fdx_gemm_bias_act_f32(in0, D, o.dw[0], D, B, (int)nk, D, 1.f, o.dw[1], 0, nullptr, nullptr, q, nk, nullptr)) != FDX_OK)
+                    return st;
                 st = fdx_gemm_bias_act_f32(in0, D, o.dw[2], D, B, (int)nk, D, 1.f, o.dw[3], 0, nullptr, nullptr, kdst, (int64_t)s->max_len * nk, nullptr);
                 if (st == FDX_OK)
                     st = fdx_gemm_bias_act_f32(in0, D, o.dw[4], D, B, (int)nv, D, 1.f, o.dw[5], 0, nullptr, nullptr, vdst, (int64_t)s->max_len * nv, nullptr);
                 if (st == FDX_OK)
                     st = fdx_mha_decode_f32(q, kc, vc, B, H, o.dk, o.dv, s->len + 1, s->max_len, merged);
             } else {
-                fdx_gemm_batch bt {};
-                bt.batch = B;
-                bt.inner = 1;
-                bt.a_outer = (int64_t)T * D;
-                bt.c_outer = (int64_t)s->max_len * nk;
-                st = fdx_gemm_bias_act_f32(in0, D, o.dw[2], D, T, (int)nk, D, 1.f, o.dw[3], 0, nullptr, nullptr, kdst, nk, &bt);
-                bt.c_outer = (int64_t)s->max_len * nv;
-                if (st == FDX_OK)
-                    st = fdx_gemm_bias_act_f32(in0, D, o.dw[4], D, T, (int)nv, D, 1.f, o.dw[5], 0, nullptr, nullptr, vdst, nv, &bt);
+                st = project(q);
                 if (st == FDX_OK) {
                     const int S = s->len + T;
                     void* scratch = s->arena(fdx_mha_scratch_bytes(B, H, T, S, o.dv));
@@ -552,6 +568,7 @@ bool build_fast_plan(fdx_session* s)
                 || hipMemcpyAsync(bqkv + nk, o.dw[3], f * nk, hipMemcpyDeviceToDevice, cs) != hipSuccess
                 || hipMemcpyAsync(bqkv + 2 * nk, o.dw[5], f * nv, hipMemcpyDeviceToDevice, cs) != hipSuccess)
                 return false;
+            s->qkv[idx] = { wqkv, bqkv };
             fdx_session::Step pr;
             pr.kind = fdx_session::Step::Gemm;
             pr.op = idx;

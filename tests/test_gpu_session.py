@@ -294,3 +294,27 @@ def test_prompts_last_position_runs_through_the_decode_launches(fdx, oracle, mod
         tokens, last = short.decode_greedy(nxt, 3)
         seq = np.concatenate([ids[0], nxt[:1], tokens[:2, 0]]).astype(np.float32)
         assert rel(last[0], oracle_logits(ref, seq)[-1]) <= TOL
+
+
+@pytest.mark.parametrize("heads,d_model,chunks", [(3, 192, (37, 5, 2)), (12, 768, (130, 63)), (2, 64, (3, 2))])
+def test_stacked_projection_writes_the_cache_like_three_launches(fdx, modelgen, heads, d_model, chunks):
+    """Sessions of up to 16 sequences project queries, keys and values of a prompt with one GEMM whose column ranges go to
+    the query buffer and the two caches; one of 17 sequences takes a launch for each.  Same prompts through both, in ragged
+    pieces (tiles that cross sequences, few and many tiles), then greedy tokens, which read every cached row."""
+    say("stacked projection", heads, d_model, chunks)
+    js = modelgen.dumps(modelgen.gpt2(seed=91, layers=2, d_model=d_model, heads=heads, vocab=307, max_pos=256, bias_std=0.1,
+                                      random_affine=True, std=0.1))
+    model = fdx.Model(js, verify=False)
+    ids = np.random.default_rng(92).integers(0, 307, (17, sum(chunks)))
+    wide, stacked, one = fdx.Session(model, 17, 256), fdx.Session(model, 16, 256), fdx.Session(model, 1, 256)
+    lo = 0
+    for n in chunks:
+        want, _ = wide.prefill(ids[:, lo:lo + n])
+        got, nxt = stacked.prefill(ids[:16, lo:lo + n])
+        single, _ = one.prefill(ids[:1, lo:lo + n])
+        assert rel(got, want[:16]) <= 1e-5 and rel(single, want[:1]) <= 1e-5, lo
+        lo += n
+    cur = np.concatenate([nxt, nxt[:1]])
+    want, _ = wide.decode_step(cur)
+    got, _ = stacked.decode_step(nxt)
+    assert rel(got, want[:16]) <= 1e-5

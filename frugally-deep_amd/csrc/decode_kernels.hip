@@ -32,6 +32,7 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int SK_WAVES = 8;
 constexpr int SK_CHUNK = 8;       // slabs of 16 k-values whose loads are issued together (8 waves x 8 x 16 = 1024 k)
+constexpr int kViaLdsRows = 8;    // see skinny_gemm_launch
 constexpr int SK_CHUNK_LONG = 24; // long-K launches (up to 3072) still issue everything at once, one workgroup per CU
 
 // SINGLE: the workgroup's K range fits one chunk per wave (only one register set is live, which
@@ -39,21 +40,25 @@ constexpr int SK_CHUNK_LONG = 24; // long-K launches (up to 3072) still issue ev
 // tiles go to a workspace and the last workgroup to arrive at a column group (atomic ticket) adds
 // them in split order -- deterministic, no spinning -- and runs the epilogue.
 // LDS of one workgroup of the Dense kernel
+// (CHUNK = 0: no strips)
+template <int CHUNK>
 struct SkinnyShared {
     float red[SK_WAVES * 256];
     int is_last;
     float stat[SK_WAVES * 16], stat2[SK_WAVES * 16]; // per-wave row sums / sums of squared deviations
+    __attribute__((aligned(16))) float strip[SK_WAVES][CHUNK ? 16 * (CHUNK * 16 + 4) : 4]; // per-wave activation rows
 };
 
 // The work of workgroup (bx, by) of a (gx, gy) grid.
 // EMB: the instantiation that knows the embedding prologue (SkinnyParams::emb_x / emb_res); the others carry none of its code
-template <int CHUNK, bool SINGLE, bool EMB = false>
-__device__ __forceinline__ void skinny_gemm_body(const SkinnyParams& p, int bx, int by, int gx, int gy, SkinnyShared& sh)
+template <int CHUNK, bool SINGLE, bool EMB, bool VIA_LDS>
+__device__ __forceinline__ void skinny_gemm_body(const SkinnyParams& p, int bx, int by, int gx, int gy, SkinnyShared<VIA_LDS ? CHUNK : 0>& sh)
 {
     float* red = sh.red;
     float* stat = sh.stat;
     float* stat2 = sh.stat2;
     int& is_last = sh.is_last;
+    static_assert(!VIA_LDS || (SINGLE && !EMB), "the strip holds one chunk of rows that lie in memory");
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const int i = lane & 15, kq = lane >> 4;
     const int n0 = bx * 16;
@@ -73,7 +78,7 @@ __device__ __forceinline__ void skinny_gemm_body(const SkinnyParams& p, int bx, 
     const bool n_ok = n < p.N, m_ok = i < p.M;
     const gptr<const float> Wg = as_global(p.W);
     const gptr<const float> wrow = Wg + (int64_t)(n_ok ? n : 0) * p.ldw;
-    const int spw = per_wave / 16; // slabs per wave in the packed layout
+    const int spk = ((K + SK_WAVES * 16 - 1) / (SK_WAVES * 16)) * SK_WAVES; // slabs of a column group in the packed layout
     const bool emb = EMB && p.emb_x != 0;
     const bool emb_res = EMB && p.emb_res != 0;
     // embedding rows of this lane's activation row: token id (a float in the model's input) and position, both checked
@@ -99,12 +104,12 @@ __device__ __forceinline__ void skinny_gemm_body(const SkinnyParams& p, int bx, 
             const bool k_ok = s0 + s < slabs && k < k_end;
             f32x4 wv = { 0.f, 0.f, 0.f, 0.f }, av = { 0.f, 0.f, 0.f, 0.f };
             if (p.packed) {
-                // pre-packed operand: this wave's slab is one contiguous 1 KB run, zeros baked in
-                if (s0 + s < spw)
-                    wv = __builtin_nontemporal_load(reinterpret_cast<gptr<const f32x4>>(Wg) + (((int64_t)bx * SK_WAVES + wave) * spw + (s0 + s)) * 64 + lane);
+                // pre-packed operand: a slab is one contiguous 1 KB run, zeros baked in
+                if (s0 + s < slabs)
+                    wv = __builtin_nontemporal_load(reinterpret_cast<gptr<const f32x4>>(Wg) + ((int64_t)bx * spk + (k_begin >> 4) + s0 + s) * 64 + lane);
             } else if (n_ok && k_ok)
                 wv = __builtin_nontemporal_load(reinterpret_cast<gptr<const f32x4>>(wrow + k)); // every weight is used once per launch
-            if (m_ok && k_ok) {
+            if (!VIA_LDS && m_ok && k_ok) {
                 av = *reinterpret_cast<gptr<const f32x4>>(xrow + k);
                 if (emb) {
                     const f32x4 bv = *reinterpret_cast<gptr<const f32x4>>(xrow_b + k);
@@ -115,8 +120,20 @@ __device__ __forceinline__ void skinny_gemm_body(const SkinnyParams& p, int bx, 
             areg[s] = av;
         }
     };
+    // VIA_LDS: the activation rows are fetched as runs of whole rows, in front of the weights (loads complete in order), and
+    // change into operand order in a strip of LDS of this wave's own: in operand order sixteen neighbouring lanes lie in
+    // sixteen rows, which the address unit takes lane by lane.
+    f32x4 x0[VIA_LDS ? CHUNK : 1];
+    if constexpr (VIA_LDS) {
+#pragma unroll
+        for (int s = 0; s < CHUNK; ++s) {
+            const int c = s * 64 + lane, row = c / (4 * CHUNK), col = (c - row * (4 * CHUNK)) * 4;
+            x0[s] = f32x4 { 0.f, 0.f, 0.f, 0.f };
+            if (row < p.M && k_begin + col < k_end)
+                x0[s] = *reinterpret_cast<gptr<const f32x4>>(as_global(p.X) + (int64_t)row * p.ldx + k_begin + col);
+        }
+    }
     load_chunk(w0, a0, 0);
-
     // epilogue operands of this thread's output element travel with the weights instead of costing a
     // second dependent round trip after the reduction
     const int em = t >> 4, ecol = n0 + (t & 15);
@@ -141,6 +158,21 @@ __device__ __forceinline__ void skinny_gemm_body(const SkinnyParams& p, int bx, 
             e_seg = 2;
         if (p.seg[e_seg].len_stride)
             e_shift = (int64_t)(*as_global(p.len_dev)) * p.seg[e_seg].len_stride;
+    }
+
+    if constexpr (VIA_LDS) {
+        float* strip = sh.strip[wave];
+#pragma unroll
+        for (int s = 0; s < CHUNK; ++s) {
+            const int c = s * 64 + lane, row = c / (4 * CHUNK), col = (c - row * (4 * CHUNK)) * 4;
+            *reinterpret_cast<f32x4*>(&strip[row * (CHUNK * 16 + 4) + col]) = x0[s];
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+        for (int s = 0; s < CHUNK; ++s)
+            a0[s] = *reinterpret_cast<const f32x4*>(&strip[i * (CHUNK * 16 + 4) + s * 16 + kq * 4]);
     }
 
     // 16x16x4 MFMA: A operand lane (m = i, k slot = kq), B operand lane (n = i, k slot = kq);
@@ -320,11 +352,11 @@ __device__ __forceinline__ void skinny_gemm_body(const SkinnyParams& p, int bx, 
     }
 }
 
-template <int CHUNK, bool SINGLE, bool EMB = false>
+template <int CHUNK, bool SINGLE, bool EMB = false, bool VIA_LDS = false>
 __global__ __launch_bounds__(512) void skinny_gemm_kernel(SkinnyParams p)
 {
-    __shared__ SkinnyShared sh;
-    skinny_gemm_body<CHUNK, SINGLE, EMB>(p, blockIdx.x, blockIdx.y, gridDim.x, gridDim.y, sh);
+    __shared__ SkinnyShared<VIA_LDS ? CHUNK : 0> sh;
+    skinny_gemm_body<CHUNK, SINGLE, EMB, VIA_LDS>(p, blockIdx.x, blockIdx.y, gridDim.x, gridDim.y, sh);
 }
 
 
@@ -932,7 +964,7 @@ fdx_status argmax_parts_embed_launch(const unsigned long long* amax_parts, int p
     return FDX_OK;
 }
 
-// K ranges per column group of a launch without LayerNorm prologue and pre-packed operand
+// K ranges per column group of a launch without LayerNorm prologue
 static int skinny_ksplit(int K, int tiles)
 {
     // spread a narrow projection over the chip: a CU pulls only a few tens of GB/s on its own
@@ -963,7 +995,7 @@ fdx_status skinny_gemm_launch(const SkinnyParams& p)
     SkinnyParams q = p;
     // the caller's workspace (the entry point that allocates nothing brings its own) or the library's, allocated on first use
     const bool own_ws = p.workspace && p.tickets;
-    if (!p.ln && !p.packed && (own_ws || ensure_splitk_workspace())) {
+    if (!p.ln && (own_ws || ensure_splitk_workspace())) {
         const int64_t ws_floats = own_ws ? p.workspace_floats : kSplitWsFloats;
         const int ticket_count = own_ws ? p.ticket_count : kSplitTickets;
         ksplit = skinny_ksplit(p.K, tiles);
@@ -999,9 +1031,17 @@ fdx_status skinny_gemm_launch(const SkinnyParams& p)
         FDX_LAUNCH_CHECK();
         return FDX_OK;
     }
+    // Activation rows through LDS from eight rows on, next to packed weights (12 layers of 768, per step: 16 rows 366 us
+    // against 393, 12 rows 358 / 375, 8 rows 351 / 358, but 4 rows 345 / 337 and one row 335 / 320, where few lanes load
+    // rows at all and the exchange is what remains; row-major weights keep the address unit busy themselves: no gain).
+    const bool via_lds = p.packed && p.M >= kViaLdsRows && per_wg <= SK_WAVES * SK_CHUNK * 16;
     // every load of a workgroup in flight at once when its K range fits 8 (or 24) slabs per wave
     if (p.emb_x || p.emb_res)
         hipLaunchKernelGGL((skinny_gemm_kernel<6, true, true>), grid, dim3(512), 0, stream(), q);
+    else if (via_lds && per_wg <= SK_WAVES * 6 * 16)
+        hipLaunchKernelGGL((skinny_gemm_kernel<6, true, false, true>), grid, dim3(512), 0, stream(), q);
+    else if (via_lds)
+        hipLaunchKernelGGL((skinny_gemm_kernel<SK_CHUNK, true, false, true>), grid, dim3(512), 0, stream(), q);
     else if (per_wg <= SK_WAVES * 6 * 16) // K = 768 and the halves / quarters of longer rows: no empty register slots
         hipLaunchKernelGGL((skinny_gemm_kernel<6, true>), grid, dim3(512), 0, stream(), q);
     else if (per_wg <= SK_WAVES * SK_CHUNK * 16)

@@ -681,16 +681,12 @@ bool build_fast_plan(fdx_session* s)
     }
     for (auto& stp : s->steps)
         if (stp.kind == fdx_session::Step::Gemm) {
-            // decode-time copy of the operand in the order the kernel's lanes read it; narrow or long-K
-            // projections without LayerNorm stay row-major because they run split along K instead
-            const bool split_candidate = !stp.g.ln && stp.g.K > 1024;
-            if (!split_candidate) {
-                float* packed = alloc((size_t)packed_weight_floats(stp.g.N, stp.g.K));
-                if (!packed || pack_weights_launch(stp.g.W, stp.g.N, stp.g.K, stp.g.ldw, packed) != FDX_OK)
-                    return false;
-                stp.g.W = packed;
-                stp.g.packed = 1;
-            }
+            // decode-time copy of the operand in the order the kernel's lanes read it
+            float* packed = alloc((size_t)packed_weight_floats(stp.g.N, stp.g.K));
+            if (!packed || pack_weights_launch(stp.g.W, stp.g.N, stp.g.K, stp.g.ldw, packed) != FDX_OK)
+                return false;
+            stp.g.W = packed;
+            stp.g.packed = 1;
             stp.g.workspace = nullptr; // launches that split K take the library's workspace and tickets
             stp.g.workspace_floats = fdx_session::kWsFloats;
             stp.g.tickets = s->splitk_tickets;

@@ -745,8 +745,11 @@ extern "C" fdx_status fdx_dwconv2d_nhwc_f32(const float* in, int n, int h, int w
     profile_begin();
     const bool k3 = vec && kh == 3 && kw == 3 && dy == 1 && dx == 1 && sy == sx && (sy == 1 || sy == 2) && (!bias || al16(bias))
         && (uint64_t)n * out_h * ((out_w + 3) / 4) * (c / 4) < (1ull << 31); // 32-bit item index in the 3x3 kernel
-    // the sliding-window form wherever its (image, row tile, column tile, channel quad) items fill the chip; tiles of 7
-    // where they divide the extent and 8 does not (14 x 14, 7 x 7), row tiles of 4 where taller ones leave too few items
+    // Stride 1: the sliding-window form from 750000 output vectors on, tiles of 7 where they divide the extent and 8 does not
+    // (14 x 14, 7 x 7), row tiles of 4 where taller ones leave too few items.  Below, its items (16 to 64 vectors each) are a
+    // few dozen workgroups that walk rows one after the other while most CUs have none: 0.12-0.26 million vectors (21 x 21 x
+    // 192 to 11 x 11 x 576, 7 images) 7.3-8.1 us against 4.8-5.1 row by row in fours, 0.3-0.7 million 7.8-9.0 against 5.4-8.6;
+    // 0.79 million 9.1 against 11.0, 1.7 million 13.2 against 18.1.
     static const bool slide_on = [] { const char* e = std::getenv("FDX_DW_SLIDE"); return !(e && e[0] == '0'); }();
     const int tx_s = out_w % 7 == 0 && out_w % 8 != 0 ? 7 : 8;
     int ry_s = out_h % 7 == 0 && out_h % 8 != 0 ? 7 : 8;
@@ -754,7 +757,7 @@ extern "C" fdx_status fdx_dwconv2d_nhwc_f32(const float* in, int n, int h, int w
     if (slide_items_for(ry_s) < 256 * 256)
         ry_s = 4;
     const size_t slide_items = slide_items_for(ry_s);
-    const bool slide = k3 && sy == 1 && slide_on && slide_items >= 256 * 16;
+    const bool slide = k3 && sy == 1 && slide_on && items >= 750000;
 #define FDX_DW_SLIDE_LAUNCH(TX_, RY_)                                                                                                  \
     hipLaunchKernelGGL((dwconv3x3_slide_kernel<TX_, RY_>), dim3(grid_for(slide_items, 256)), dim3(256), 0, stream(), in, weights_hwc, bias, out, \
         n, h, w, c, pad_top, pad_left, out_h, out_w, a)
@@ -772,7 +775,7 @@ extern "C" fdx_status fdx_dwconv2d_nhwc_f32(const float* in, int n, int h, int w
         FDX_DW_SLIDE_LAUNCH(8, 4);
 #undef FDX_DW_SLIDE_LAUNCH
     else if (k3 && sy == 1)
-        hipLaunchKernelGGL((dwconv3x3_kernel<1, 8>), dim3(grid_for((size_t)n * out_h * ((out_w + 7) / 8) * (c / 4), 256)), dim3(256), 0,
+        hipLaunchKernelGGL((dwconv3x3_kernel<1, 4>), dim3(grid_for((size_t)n * out_h * ((out_w + 3) / 4) * (c / 4), 256)), dim3(256), 0,
             stream(), in, weights_hwc, bias, out, n, h, w, c, pad_top, pad_left, out_h, out_w, a);
     else if (k3)
         hipLaunchKernelGGL((dwconv3x3_kernel<2, 4>), dim3(grid_for((size_t)n * out_h * ((out_w + 3) / 4) * (c / 4), 256)), dim3(256), 0,

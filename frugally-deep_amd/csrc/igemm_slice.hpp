@@ -4,8 +4,8 @@
 // There the tiled kernel leaves most of the chip idle: a 64 x 64 tile of a 14 x 14 map walks K = 2304 slab by slab, each
 // slab a round trip to memory, an LDS pass and a barrier (one image, weights out of memory, per launch: 14 x 14 3x3
 // 256 -> 256 19.6 us, 1x1 1024 -> 256 13.6, 7 x 7 3x3 512 -> 512 26.8; here 9.4, 4.7, 13.2, of which 3.5 are the launch
-// itself; ResNet50 at batch 1 761 -> 390 us).  What bounds it is the path from L2 into a CU.  Here the eight (or sixteen) waves of a workgroup share one
-// small output tile and cut its K range between them, every wave on its own:
+// itself; ResNet50 at batch 1 761 -> 390 us).  What bounds it is the path from L2 into a CU.  Here the eight (or four) waves
+// of a workgroup share one small output tile and cut its K range between them, every wave on its own:
 //
 //  * a wave loads its units (UK consecutive k of all tile rows) as runs of 64 or 128 bytes per row, DEPTH units in flight from
 //    the first instruction on, and turns them into MFMA operands through a strip of LDS of its own: no barrier in the loop.
@@ -89,7 +89,7 @@ __global__ __launch_bounds__(64 * NW) void igemm_slice_kernel(GemmParams p)
         b_voff[j] = n < p.N ? (uint32_t)((int64_t)n * p.ldb) * 4u + lchunk * 16 : OOB;
     }
 
-    // this wave's units of 16 k
+    // this wave's units of UK k
     const int units = p.K / UK;
     const int u_lo = (int)((int64_t)units * wave / NW), u_n = (int)((int64_t)units * (wave + 1) / NW) - u_lo;
     int issued = 0, soff_b = u_lo * (UK * 4), soff_a = soff_b, tap = 0, fx = 0, fy = 0, c0 = 0;

@@ -445,7 +445,7 @@ bool build_fast_plan(fdx_session* s)
         st.op = idx;
         st.depth = depth;
         // operand of a weight-streaming GEMM; a pending LayerNorm is folded into copies of the weights
-        // (W * gamma, row sums, bias + W beta) so the launch works on the raw rows
+        // (W * gamma, bias + W beta) so the launch works on the raw rows
         auto gemm_input = [&](int src, SkinnyParams& g, const float* w, const float* bias, int n, int k) -> bool {
             g.W = w;
             g.bias = bias;
@@ -456,15 +456,13 @@ bool build_fast_plan(fdx_session* s)
             }
             const Op& ln = m.ops[src];
             float* wf = alloc((size_t)n * k);
-            float* ws = alloc((size_t)n);
             float* bf = alloc((size_t)n);
-            if (!wf || !ws || !bf || fold_layernorm_launch(ln.dw[0], ln.dw[1], w, bias, n, k, wf, ws, bf) != FDX_OK)
+            if (!wf || !bf || fold_layernorm_launch(ln.dw[0], ln.dw[1], w, bias, n, k, wf, nullptr, bf) != FDX_OK)
                 return false;
             g.X = buf[ln.in[0]];
             g.ln = 1;
             g.ln_eps = ln.eps;
             g.W = wf;
-            g.w_rowsum = ws;
             g.bias = bf;
             return g.X != nullptr;
         };

@@ -24,7 +24,6 @@ struct SkinnyParams {
     Act act;
     int ln;             // rows of X are layer-normalised over K before the product
     float ln_eps;
-    const float* w_rowsum; // [N] row sums of the folded W, needed when ln != 0
     int n_seg;
     SkinnySegment seg[3];
     const int* len_dev; // device int read by segments with len_stride != 0

@@ -219,8 +219,9 @@ fdx_status fdx_dense_rows_noalloc_f32(const float* x, int m, int k, const float*
  * LayerNormalization followed by Dense in one launch (layers/layer_normalization_layer.hpp:37-63 then
  * layers/dense_layer.hpp:76-86).  fdx_fold_layernorm_f32 prepares, once per layer pair,
  *   w_folded[n][k] = w[n][k] * gamma[k],  w_rowsum[n] = sum_k w_folded[n][k],  bias_folded[n] = bias[n] + sum_k w[n][k] * beta[k]
- * (gamma / beta / bias may be NULL); the launch then computes rstd[m] * (x w_folded^T - mean[m] * w_rowsum) + bias_folded
- * with each row's mean and biased two-pass variance taken from x itself.  k <= 1024.
+ * (gamma / beta / bias may be NULL); the launch then computes rstd[m] * ((x - mean[m]) w_folded^T) + bias_folded with each
+ * row's mean and biased two-pass variance taken from x itself (the row sums stay in the interface; centred rows need none).
+ * k <= 1024.
  */
 fdx_status fdx_fold_layernorm_f32(const float* gamma, const float* beta, const float* w_nk, const float* bias, int n,
     int k, float* w_folded, float* w_rowsum, float* bias_folded);

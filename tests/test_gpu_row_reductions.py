@@ -37,6 +37,41 @@ def test_softmax(fdx, oracle, rows, depth):
     assert rel(fdx.softmax(x), oracle.softmax(x)) <= 1e-5
 
 
+@pytest.mark.parametrize("rows,depth", [(999, 257), (1000, 257), (1001, 512), (1999, 513), (2000, 513), (2003, 1024), (5000, 300), (2000, 1025)])
+def test_softmax_many_rows(fdx, oracle, rows, depth):
+    """Rows of 257 to 1024 entries on both sides of the lines between a workgroup and a wave per row."""
+    print("softmax many rows", rows, depth, flush=True)
+    x = np.random.default_rng(6).normal(0, 3, (rows, depth)).astype(np.float32)
+    x[-1, -1] = 60.0
+    # at most depth roundings of 2^-24 in the sum, a few units in the last place of expf and logf on each side
+    assert rel(fdx.softmax(x), oracle.softmax(x)) <= 1e-5
+    t = min(rows, 7)
+    got = fdx.softmax(x[: rows // t * t], causal_period=t, causal_offset=depth - t)
+    for row in (0, 1, rows // t * t - 1):
+        visible = row % t + 1 + depth - t
+        assert rel(got[row, :visible], oracle.softmax(x[row, :visible])) <= 1e-5
+        assert not got[row, visible:].any()
+
+
+def test_softmax_of_more_rows_than_a_launch_has_workgroups_of_256(fdx, oracle):
+    """2^24 rows and more of 257 entries (17 GB, in place): a workgroup of 256 threads for each would be 2^32 threads.  The
+    rows looked at are written, the others hold whatever the memory held."""
+    c = fdx.ctypes
+    rows, depth = (1 << 24) + 3, 257
+    print("softmax", rows, depth, flush=True)
+    buf = fdx.DevBuf(4 * rows * depth)
+    at = [0, 1, 4095, (1 << 23) + 1, (1 << 24) - 1, 1 << 24, rows - 1]
+    x = np.random.default_rng(7).normal(0, 3, (len(at), depth)).astype(np.float32)
+    got = np.empty_like(x)
+    place = lambda i: c.c_void_p(buf.ptr.value + 4 * depth * at[i])
+    for i in range(len(at)):
+        fdx.check(fdx.lib.fdx_h2d(place(i), x[i].ctypes.data_as(c.c_void_p), c.c_size_t(4 * depth)))
+    fdx.check(fdx.lib.fdx_softmax_f32(fdx._dp(buf), c.c_int64(rows), depth, 0, 0, fdx._dp(buf)))
+    for i in range(len(at)):
+        fdx.check(fdx.lib.fdx_d2h(got[i].ctypes.data_as(c.c_void_p), place(i), c.c_size_t(4 * depth)))
+    assert rel(got, oracle.softmax(x)) <= 1e-5
+
+
 @pytest.mark.parametrize("t,s", [(3, 60), (5, 200), (7, 700)])
 def test_softmax_causal(fdx, oracle, t, s):
     print("softmax causal", t, s, flush=True)

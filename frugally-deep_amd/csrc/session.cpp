@@ -113,12 +113,20 @@ struct fdx_session {
     }
 };
 
+static int g_fail_step = -1;  // test hook: launch_steps reports an error in front of this step, or behind the last launch
 static int g_embed_fold = -1; // test hook: -1 = the environment decides, 0 / 1 = sessions created from now on
 
 extern "C" fdx_status fdx_debug_decode_embed_fold(int mode)
 {
     FDX_REQUIRE(mode >= -1 && mode <= 1, "fdx_debug_decode_embed_fold: mode must be -1, 0 or 1");
     g_embed_fold = mode;
+    return FDX_OK;
+}
+
+extern "C" fdx_status fdx_debug_fail_session_step(int step)
+{
+    FDX_REQUIRE(step >= -1, "fdx_debug_fail_session_step: -1 or the number of a step");
+    g_fail_step = step;
     return FDX_OK;
 }
 
@@ -819,7 +827,15 @@ fdx_status launch_steps(fdx_session* s, const float* ids_dev, float* next_dev, i
     fdx_model& m = *s->m;
     const int B = s->batch;
     fdx_status st = FDX_OK;
+    auto refused = [](size_t si) {
+        if ((int)si != g_fail_step)
+            return false;
+        set_error("session: step %d refused by fdx_debug_fail_session_step", g_fail_step);
+        return true;
+    };
     for (size_t si = first; si < s->steps.size(); ++si) {
+        if (refused(si))
+            return FDX_ERR_HIP;
         const auto& step = s->steps[si];
         const Op& o = m.ops[step.op];
         const fdx_act act = to_c(o.act);
@@ -867,12 +883,27 @@ fdx_status launch_steps(fdx_session* s, const float* ids_dev, float* next_dev, i
     // length on the device
     if (merged) {
         const auto& e = s->steps[0];
-        return argmax_parts_embed_launch(s->amax_parts, s->amax_part_count, B, next_dev, s->len_dev, s->history, e.a, e.g.M, e.b, e.g.N, e.depth,
+        st = argmax_parts_embed_launch(s->amax_parts, s->amax_part_count, B, next_dev, s->len_dev, s->history, e.a, e.g.M, e.b, e.g.N, e.depth,
             e.out, m.err_flag);
-    }
-    if (s->amax_part_count > 0)
-        return argmax_parts_launch(s->amax_parts, s->amax_part_count, B, next_dev, s->len_dev, s->history);
-    return argmax_bump_launch(s->logits_buf, B, s->vocab, next_dev, s->len_dev, s->amax, s->history);
+    } else if (s->amax_part_count > 0)
+        st = argmax_parts_launch(s->amax_parts, s->amax_part_count, B, next_dev, s->len_dev, s->history);
+    else
+        st = argmax_bump_launch(s->logits_buf, B, s->vocab, next_dev, s->len_dev, s->amax, s->history);
+    return st == FDX_OK && refused(s->steps.size()) ? FDX_ERR_HIP : st;
+}
+
+// The decode launches move the device's copy of the length on their own; behind a call that failed half way it goes back to
+// the length the session has (a later step would write its keys and values too far on, and attend over rows of no token).
+fdx_status settle_length(fdx_session* s, fdx_status st)
+{
+    if (!s->len_dev)
+        return st;
+    const std::string reason = st == FDX_OK ? std::string() : fdx_last_error();
+    const fdx_status ls = set_int_launch(s->len_dev, s->len);
+    if (st == FDX_OK)
+        return ls;
+    set_error("%s", reason.c_str());
+    return st;
 }
 
 // one decode step, eager launches
@@ -1009,8 +1040,11 @@ extern "C" fdx_status fdx_session_create(fdx_model* m, int batch, int max_len, f
     std::vector<int> memo(m->ops.size(), -1);
     s->vocab = depth_of(*m, m->outputs[0], memo);
     s->fast = build_fast_plan(s.get());
-    if (!s->fast)
+    if (!s->fast) {
         s->steps.clear();
+        s->tail_step = -1;
+        s->tail_inputs.clear();
+    }
     *out = s.release();
     return FDX_OK;
 }
@@ -1040,17 +1074,16 @@ extern "C" fdx_status fdx_session_length(const fdx_session* s, int* len)
 extern "C" fdx_status fdx_session_prefill(fdx_session* s, const float* ids_dev, int t, float* logits_dev, float* next_ids_dev)
 {
     FDX_REQUIRE(s, "session_prefill: null session");
-    fdx_status st = run(s, ids_dev, t, logits_dev, next_ids_dev);
-    if (st == FDX_OK && s->len_dev)
-        st = set_int_launch(s->len_dev, s->len);
-    return st;
+    return settle_length(s, run(s, ids_dev, t, logits_dev, next_ids_dev));
 }
 
 extern "C" fdx_status fdx_session_decode_step(fdx_session* s, const float* ids_dev, float* logits_dev, float* next_ids_dev)
 {
     FDX_REQUIRE(s, "session_decode_step: null session");
-    if (s->fast)
-        return run_fast(s, ids_dev, logits_dev, next_ids_dev);
+    if (s->fast) {
+        const fdx_status st = run_fast(s, ids_dev, logits_dev, next_ids_dev);
+        return st == FDX_OK ? st : settle_length(s, st);
+    }
     return run(s, ids_dev, 1, logits_dev, next_ids_dev);
 }
 
@@ -1063,15 +1096,17 @@ extern "C" fdx_status fdx_session_decode_greedy(fdx_session* s, const float* fir
         const char* e = std::getenv("FDX_DECODE_GRAPH");
         return !(e && e[0] == '0');
     }();
-    if (s->fast && use_graph && !profiling())
-        return run_fast_greedy(s, first_ids_dev, steps, tokens_dev, last_logits_dev);
+    if (s->fast && use_graph && !profiling()) {
+        const fdx_status st = run_fast_greedy(s, first_ids_dev, steps, tokens_dev, last_logits_dev);
+        return st == FDX_OK ? st : settle_length(s, st);
+    }
     for (int i = 0; i < steps; ++i) {
         const float* ids = i == 0 ? first_ids_dev : tokens_dev + (size_t)(i - 1) * s->batch;
         float* logits = i + 1 == steps ? last_logits_dev : nullptr;
         float* next = tokens_dev + (size_t)i * s->batch;
         fdx_status st = s->fast ? run_fast(s, ids, logits, next) : run(s, ids, 1, logits, next);
         if (st != FDX_OK)
-            return st;
+            return s->fast ? settle_length(s, st) : st;
     }
     return FDX_OK;
 }

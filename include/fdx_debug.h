@@ -74,6 +74,9 @@ fdx_status fdx_debug_force_ln_fold(int mode);
  * that read its result (measured slower than the launch it saves, hence not the default), 0 = never, -1 = as the
  * environment says (FDX_DECODE_EMBED_FOLD=1) */
 fdx_status fdx_debug_decode_embed_fold(int mode);
+/* decode sessions: the launches of a step (or of the end of a prompt) stop with an error in front of step `step` of the
+ * plan, or behind its last launch if the plan has `step` steps; -1 = never (the default) */
+fdx_status fdx_debug_fail_session_step(int step);
 fdx_status fdx_debug_persist_cap(int workgroups);
 fdx_status fdx_debug_force_strips(int strips);
 fdx_status fdx_debug_force_dw_fusion(int mode);

@@ -318,3 +318,37 @@ def test_stacked_projection_writes_the_cache_like_three_launches(fdx, modelgen, 
     want, _ = wide.decode_step(cur)
     got, _ = stacked.decode_step(nxt)
     assert rel(got, want[:16]) <= 1e-5
+
+
+@pytest.mark.parametrize("step", [6, 9, 11, 12])
+def test_a_call_that_fails_half_way_leaves_the_length_alone(fdx, modelgen, step):
+    """Prompts and steps move the device's copy of the session length by launches of their own.  Stopped in the last layer, in
+    the head or behind the arg-max, they leave the session where it was: what follows equals a session that never failed."""
+    say("failing step", step)
+    js = modelgen.dumps(modelgen.gpt2(seed=121, layers=2, d_model=192, heads=3, vocab=33000, max_pos=64, bias_std=0.1, std=0.1))
+    model = fdx.Model(js, verify=False)
+    ids = np.random.default_rng(122).integers(0, 33000, (5, 40))
+    hurt, sound = fdx.Session(model, 5, 40), fdx.Session(model, 5, 40)
+
+    def fails(call):
+        fdx.check(fdx.lib.fdx_debug_fail_session_step(step))
+        try:
+            with pytest.raises(fdx.FdxError, match="refused"):
+                call()
+        finally:
+            fdx.check(fdx.lib.fdx_debug_fail_session_step(-1))
+
+    fails(lambda: hurt.prefill(ids[:, :30]))
+    assert hurt.length() == 0
+    for s in (hurt, sound):
+        s.prefill(ids[:, :12])
+    fails(lambda: hurt.prefill(ids[:, 12:39]))
+    fails(lambda: hurt.decode_step(ids[:, 12]))
+    assert hurt.length() == 12
+    for s in (hurt, sound):
+        s.last = s.decode_step(ids[:, 12])
+    assert np.array_equal(hurt.last[0], sound.last[0]) and np.array_equal(hurt.last[1], sound.last[1])
+    fails(lambda: hurt.decode_greedy(hurt.last[1], 4))
+    a, b = hurt.decode_greedy(hurt.last[1], 4), sound.decode_greedy(sound.last[1], 4)
+    assert np.array_equal(a[0], b[0]) and np.array_equal(a[1], b[1])
+    assert hurt.length() == sound.length() == 17

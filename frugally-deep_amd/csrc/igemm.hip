@@ -680,6 +680,10 @@ static int autotune(const GemmParams& q, bool conv, int batch, int unit, hipStre
         }
     }
     for (int c = kSliceCfg; c < kSliceCfg + kSliceForms && batch == 1; ++c) {
+        // only forms that a grid can hold (a refused launch would time as nothing) and that may win
+        if (!slice_fits(c - kSliceCfg, q.M, q.N)
+            || slice_cost(c - kSliceCfg, conv, q.M, q.N, q.K) > 1.5f * slice_tiled_cost(q.M, q.N, q.K))
+            continue;
         slice_launch(c, q, conv, s);
         const float ms = timed([&] { slice_launch(c, q, conv, s); });
         if (ms < best_ms) {
@@ -764,7 +768,7 @@ static fdx_status run_igemm(GemmParams& p, bool conv, int batch, const char* fam
         if (cfg == kStreamCfg && !stream_ok)
             cfg = -1;
         const bool slice = cfg >= kSliceCfg && cfg < kSliceCfg + kSliceForms;
-        if (slice && (!fast_ok || batch != 1))
+        if (slice && (!fast_ok || batch != 1 || !slice_fits(cfg - kSliceCfg, p.M, p.N)))
             cfg = -1;
         if (cfg >= 10 && cfg != kStreamCfg && !slice && (!fast_ok || cfg > 18 || (cfg >= 13 && unit % 32 != 0)))
             cfg = -1;

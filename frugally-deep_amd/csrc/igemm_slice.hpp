@@ -260,26 +260,42 @@ constexpr SliceForm kSliceForm[kSliceForms] = { { 1, 1, 8 }, { 1, 2, 8 }, { 2, 2
 // none takes more than 5 % longer.  Below 48 columns the other side is the general kernel's narrow tile, which wins from
 // about 600 row blocks of 64 on (N = 32, K = 144-192: 20000 rows 8.2-9.7 against 6.3-7.2 us here, 50000 rows 11.0-14.5
 // against 11.1-14.0, convolutions 13.9 against 17.1).
-static int slice_pick(bool conv, int M, int N, int K)
+// Large problems are few in this sense, too, where the last column block of 64 would be half empty: N = 80, 96, 144, 160 or
+// 208 and long rows, up to 118000 rows of K = 3520 with N = 96 792 -> 687 us; 160 such problems 0.93-2.1 times, 1.33 on average.
+static int64_t slice_tiles(int M, int N, int bm, int bn) { return (int64_t)((M + bm - 1) / bm) * ((N + bn - 1) / bn); }
+static float slice_rounds(int64_t tiles) { return (float)((tiles + 255) / 256); }
+static float slice_cost(int form, bool conv, int M, int N, int K)
 {
     static const float kCost[kSliceForms][4] = { // t0, c1, c2 of a GEMM, c2 of a convolution
         { 2.18f, 1.29f, 0.42f, 0.59f }, { 2.13f, 1.07f, 0.50f, 0.62f }, { 2.24f, 1.47f, 0.64f, 1.02f }, { 2.52f, 0.71f, 0.76f, 0.92f },
         { 1.52f, 2.43f, 0.83f, 1.25f }
     };
-    const auto tiles_of = [&](int bm, int bn) { return (int64_t)((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
-    const auto per_cu = [](int64_t tiles) { return (float)((tiles + 255) / 256); };
-    const int64_t t64 = tiles_of(64, 64);
+    const int bm = 16 * kSliceForm[form].tm, bn = 16 * kSliceForm[form].tn;
+    return kCost[form][0] + slice_rounds(slice_tiles(M, N, bm, bn)) * (kCost[form][1] + kCost[form][conv ? 3 : 2] * 1e-4f * (bm + bn) * K);
+}
+static float slice_tiled_cost(int M, int N, int K)
+{
+    const int64_t t64 = slice_tiles(M, N, 64, 64);
+    const float k = 1e-3f * K, t = (float)t64 / 256.f;
+    return 4.8f + slice_rounds(t64) * (0.44f + 4.9f * k) + 12.3f * t * k + 5.1f * std::min(t, 1.f) * k;
+}
+// whether a launch of this form stays below the 2^32 threads a grid can have
+static bool slice_fits(int form, int M, int N)
+{
+    const SliceForm& f = kSliceForm[form];
+    return slice_tiles(M, N, 16 * f.tm, 16 * f.tn) * 64 * f.nw < (1LL << 32);
+}
+static int slice_pick(bool conv, int M, int N, int K)
+{
+    const int64_t t64 = slice_tiles(M, N, 64, 64);
     const bool narrow = N < 48;
     if (narrow && t64 > 512)
         return -1;
-    const float k = 1e-3f * K, t = (float)t64 / 256.f;
-    const float tiled = 4.8f + per_cu(t64) * (0.44f + 4.9f * k) + 12.3f * t * k + 5.1f * std::min(t, 1.f) * k;
     int best = -1;
-    float best_cost = narrow ? 1e30f : (t64 <= 256 ? 0.85f : 0.75f) * tiled; // past a round of tiles operands re-read cost the neighbours, too
+    float best_cost = narrow ? 1e30f : (t64 <= 256 ? 0.85f : 0.75f) * slice_tiled_cost(M, N, K); // past a round of tiles operands re-read cost the neighbours, too
     for (int i = 0; i < kSliceForms; ++i) {
-        const int bm = 16 * kSliceForm[i].tm, bn = 16 * kSliceForm[i].tn;
-        const float cost = kCost[i][0] + per_cu(tiles_of(bm, bn)) * (kCost[i][1] + kCost[i][conv ? 3 : 2] * 0.1f * (bm + bn) * k);
-        if (cost < best_cost) {
+        const float cost = slice_cost(i, conv, M, N, K);
+        if (cost < best_cost && slice_fits(i, M, N)) {
             best_cost = cost;
             best = kSliceCfg + i;
         }

@@ -83,3 +83,29 @@ def test_residual_block_with_shortcut_convolution_few_tiles(fdx, oracle, modelge
     finally:
         fdx.lib.fdx_debug_force_tile(-1)
     assert rel(got, want) <= 2 * TOL
+
+
+def test_more_tiles_than_a_launch_can_hold(fdx):
+    """131072 x 16384 outputs (8.6 GB): a workgroup of 512 threads for each 16 x 16 of them would be 2^32 threads.  Neither
+    the timing runs nor a forced form takes that form."""
+    m, n, k = 131072, 16384, 16
+    c = fdx.ctypes
+    print("gemm", m, n, k, flush=True)
+    r = np.random.default_rng(12)
+    a, w = r.standard_normal((m, k)).astype(np.float32), r.standard_normal((n, k)).astype(np.float32)
+    da, dw, out = fdx.DevBuf.from_host(a), fdx.DevBuf.from_host(w), fdx.DevBuf(4 * m * n)
+    rows = [0, 1, m // 2, m - 1]
+    got = np.empty((len(rows), n), np.float32)
+    for timing, tile in ((False, -1), (False, 40), (True, -1), (True, -1)):
+        fdx.tuner_timing(timing)
+        fdx.lib.fdx_debug_force_tile(tile)
+        try:
+            fdx.check(fdx.lib.fdx_gemm_bias_act_f32(fdx._dp(da), c.c_int64(k), fdx._dp(dw), c.c_int64(k), m, n, k, c.c_float(1), None, 0, None,
+                                                    None, fdx._dp(out), c.c_int64(n), None))
+            fdx.sync()
+        finally:
+            fdx.lib.fdx_debug_force_tile(-1)
+            fdx.tuner_timing(False)
+        for i, row in enumerate(rows):
+            fdx.check(fdx.lib.fdx_d2h(got[i].ctypes.data_as(c.c_void_p), c.c_void_p(out.ptr.value + 4 * n * row), c.c_size_t(4 * n)))
+        assert rel(got, a[rows].astype(np.float64) @ w.astype(np.float64).T) <= TOL

@@ -582,6 +582,24 @@ bool tune_frozen()
 }
 static int g_split_enabled = 1; // FDX_SPLITK=0 keeps the tuner to one K range per tile
 
+// Three launches back to back, the faster of two such rounds: candidates within a percent of each other are common, and a
+// single round of a 30 us kernel is too short a window to tell them apart.
+template <typename F>
+static float time_rounds(hipEvent_t a, hipEvent_t b, hipStream_t s, F&& launch)
+{
+    float best_round = 1e30f;
+    for (int round = 0; round < 2; ++round) {
+        (void)hipEventRecord(a, s);
+        for (int r = 0; r < 3; ++r)
+            launch();
+        (void)hipEventRecord(b, s);
+        float ms = 1e30f;
+        if (hipEventSynchronize(b) == hipSuccess && hipEventElapsedTime(&ms, a, b) == hipSuccess && ms < best_round)
+            best_round = ms;
+    }
+    return best_round;
+}
+
 // general_cfg >= 0: the general kernel's configuration for this shape competes too (narrow outputs, where half of a
 // 64-wide fast tile is idle); general_launch runs it once on the caller's unshifted parameters
 // stream_ok: the row-streaming short-K kernel (configuration 30, pw_stream.hpp) competes as well
@@ -607,21 +625,7 @@ static int autotune(const GemmParams& q, bool conv, int batch, int unit, hipStre
     int best = -1, best_split = -1;
     float best_ms = 1e30f, best_split_ms = 1e30f;
     const bool can_split = g_split_enabled && split_prepare();
-    // three launches back to back, the faster of two such rounds: candidates within a percent of each other are
-    // common, and a single round of a 30 us kernel is too short a window to tell them apart
-    auto timed = [&](auto&& launch) -> float {
-        float best_round = 1e30f;
-        for (int round = 0; round < 2; ++round) {
-            (void)hipEventRecord(a, s);
-            for (int r = 0; r < 3; ++r)
-                launch();
-            (void)hipEventRecord(b, s);
-            float ms = 1e30f;
-            if (hipEventSynchronize(b) == hipSuccess && hipEventElapsedTime(&ms, a, b) == hipSuccess && ms < best_round)
-                best_round = ms;
-        }
-        return best_round;
-    };
+    auto timed = [&](auto&& launch) -> float { return time_rounds(a, b, s, launch); };
     bool clock_settled = false;
     for (int cfg = 10; cfg <= 18; ++cfg) {
         if (cfg >= 13 && unit % 32 != 0)
@@ -1096,17 +1100,57 @@ fdx_status gemm_segments_launch(const float* a, const float* w, const float* bia
     p.ldc = p.N; // the tile walk's own arithmetic
     p.a_records = (uint32_t)((int64_t)m * k * 4);
     p.b_records = (uint32_t)((int64_t)p.N * k * 4);
-    profile_begin();
-    switch (slice_pick(false, m, p.N, k)) {
-    case kSliceCfg: slice_launch_seg<0>(p, stream()); break;
-    case kSliceCfg + 1: slice_launch_seg<1>(p, stream()); break;
-    case kSliceCfg + 2: slice_launch_seg<2>(p, stream()); break;
-    case kSliceCfg + 3: slice_launch_seg<3>(p, stream()); break;
-    case kSliceCfg + 4: slice_launch_seg<4>(p, stream()); break;
-    default:
-        launch_persistent(igemm_fast_kernel<64, 64, 2, 2, 32, false, false, false, false, false, true>, ((m + 63) / 64) * ((p.N + 63) / 64), p,
-            stream(), 256, 64, 64);
+    hipStream_t s = stream();
+    constexpr int kTiled = 15; // the 64 x 64 tile with the 32-float slab
+    auto launch = [&](int cfg) {
+        switch (cfg) {
+        case kSliceCfg: slice_launch_seg<0>(p, s); break;
+        case kSliceCfg + 1: slice_launch_seg<1>(p, s); break;
+        case kSliceCfg + 2: slice_launch_seg<2>(p, s); break;
+        case kSliceCfg + 3: slice_launch_seg<3>(p, s); break;
+        case kSliceCfg + 4: slice_launch_seg<4>(p, s); break;
+        default:
+            launch_persistent(igemm_fast_kernel<64, 64, 2, 2, 32, false, false, false, false, false, true>, ((m + 63) / 64) * ((p.N + 63) / 64), p,
+                s, 256, 64, 64);
+        }
+    };
+    // The form comes from a test hook, the tuning table, a timing run where those are asked for, or the closed rule.
+    auto usable = [&](int cfg) {
+        return cfg == kTiled || (cfg >= kSliceCfg && cfg < kSliceCfg + kSliceForms && slice_fits(cfg - kSliceCfg, m, p.N));
+    };
+    int cfg = g_forced_tile;
+    if (!usable(cfg)) {
+        TuneKey key;
+        std::memset(&key, 0, sizeof key);
+        key.conv = 4; key.M = m; key.N = p.N; key.K = k; key.Cin = n_seg; key.batch = m / rows;
+        hipEvent_t ea = nullptr, eb = nullptr;
+        if (tune_lookup(key, &cfg)) {
+        } else if (!tune_frozen() && 2.0 * m * (double)p.N * k >= 2e8 && hipEventCreate(&ea) == hipSuccess && hipEventCreate(&eb) == hipSuccess) {
+            float best_ms = 1e30f;
+            for (int c : { kTiled, kSliceCfg, kSliceCfg + 1, kSliceCfg + 2, kSliceCfg + 3, kSliceCfg + 4 }) {
+                if (!usable(c) || (c != kTiled && slice_cost(c - kSliceCfg, false, m, p.N, k) > 1.5f * slice_tiled_cost(m, p.N, k)))
+                    continue;
+                if (c == kTiled)
+                    tune_settle_clock([&] { launch(c); return true; });
+                launch(c);
+                const float ms = time_rounds(ea, eb, s, [&] { launch(c); });
+                if (ms < best_ms) {
+                    best_ms = ms;
+                    cfg = c;
+                }
+            }
+            tune_mark();
+            tune_store(key, cfg);
+        }
+        if (ea)
+            (void)hipEventDestroy(ea);
+        if (eb)
+            (void)hipEventDestroy(eb);
     }
+    if (!usable(cfg))
+        cfg = slice_pick(false, m, p.N, k);
+    profile_begin();
+    launch(cfg);
     profile_end("gemm_f32", 2.0 * m * (double)p.N * k, 0.0);
     FDX_LAUNCH_CHECK();
     return FDX_OK;
@@ -1305,7 +1349,7 @@ extern "C" fdx_status fdx_tuner_import(const char* text)
         if (got <= 0)
             break; // trailing white space
         FDX_REQUIRE(got == 12, "tuner_import: malformed line near offset %d", (int)(p - text));
-        FDX_REQUIRE(k.conv >= 0 && k.conv <= 3 && choice >= -1, "tuner_import: value out of range near offset %d", (int)(p - text));
+        FDX_REQUIRE(k.conv >= 0 && k.conv <= 4 && choice >= -1, "tuner_import: value out of range near offset %d", (int)(p - text));
         rows.emplace_back(k, choice);
         p += used;
         while (*p == '\n' || *p == '\r' || *p == ' ')

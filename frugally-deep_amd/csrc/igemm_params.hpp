@@ -64,7 +64,8 @@ struct GemmParams {
 // K = channels, N = filters, sy = stride, res = residual, kh = input channels of a whole block) and the form it runs
 // in (1 = depthwise + projection as one launch, 2 = a launch per layer, 3 = the whole block as one launch);
 // conv = 3: a 3x3 stride-1 convolution (M = output pixels of the batch, kh / kw = input height / width, sy / sx = top /
-// left padding) and its kernel (0 = direct, 1 = Winograd).
+// left padding) and its kernel (0 = direct, 1 = Winograd); conv = 4: a GEMM whose columns go to several tensors (Cin = how many,
+// batch = sequences) and its configuration (15 or a form of the few-tiles kernel).
 struct TuneKey {
     int conv, M, N, K, Cin, kh, kw, sy, sx, batch, res;
     bool operator<(const TuneKey& o) const { return std::memcmp(this, &o, sizeof(TuneKey)) < 0; }

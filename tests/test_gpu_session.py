@@ -352,3 +352,57 @@ def test_a_call_that_fails_half_way_leaves_the_length_alone(fdx, modelgen, step)
     a, b = hurt.decode_greedy(hurt.last[1], 4), sound.decode_greedy(sound.last[1], 4)
     assert np.array_equal(a[0], b[0]) and np.array_equal(a[1], b[1])
     assert hurt.length() == sound.length() == 17
+
+
+@pytest.mark.parametrize("tile", [15, 40, 41, 42, 43, 44])
+def test_every_form_of_the_stacked_projection(fdx, modelgen, tile):
+    """The stacked projection's forms one by one: three tensors in the first layer, keys and values only in the last, from one
+    row block to tiles that cross sequences, against a session of 17 sequences, which takes a launch for each."""
+    say("stacked projection", tile)
+    js = modelgen.dumps(modelgen.gpt2(seed=131, layers=2, d_model=192, heads=3, vocab=33000, max_pos=128, bias_std=0.1,
+                                      random_affine=True, std=0.1))
+    model = fdx.Model(js, verify=False)
+    ids = np.random.default_rng(132).integers(0, 33000, (17, 90))
+    wide = fdx.Session(model, 17, 96)
+    some = {B: fdx.Session(model, B, 96) for B in (1, 5, 16)}
+    lo = 0
+    for n in (2, 3, 16, 63):
+        want, _ = wide.prefill(ids[:, lo:lo + n])
+        fdx.lib.fdx_debug_force_tile(tile)
+        try:
+            got = {B: s.prefill(ids[:B, lo:lo + n])[0] for B, s in some.items()}
+        finally:
+            fdx.lib.fdx_debug_force_tile(-1)
+        for B in some:
+            assert rel(got[B], want[:B]) <= 1e-5, (B, n)
+        lo += n
+
+
+def test_stacked_projection_timed_and_from_a_table(fdx, modelgen):
+    """With timing asked for, the stacked projection's form is timed once per shape and exported; the table comes back in and
+    holds for a frozen process."""
+    say("stacked projection, timed")
+    js = modelgen.dumps(modelgen.gpt2(seed=133, layers=2, d_model=192, heads=3, vocab=307, max_pos=128, bias_std=0.1, std=0.1))
+    model = fdx.Model(js, verify=False)
+    ids = np.random.default_rng(134).integers(0, 307, (16, 111))
+    s = fdx.Session(model, 16, 111)
+    want, _ = s.prefill(ids)
+    rows = lambda: [r for r in fdx.tuner_export().splitlines() if r.startswith("4 1776 576 192 3 ")]
+    assert not rows()
+    fdx.tuner_timing(True)
+    try:
+        s.reset()
+        timed, _ = s.prefill(ids)
+    finally:
+        fdx.tuner_timing(False)
+    row, = rows()
+    assert int(row.split()[-1]) in (15, 40, 41, 42, 43, 44)
+    head = row.rsplit(" ", 1)[0]
+    try:
+        for choice in (40, 44, 15, 39, 99):  # the last two are no forms: the closed rule
+            fdx.tuner_import("%s %d\n" % (head, choice))
+            s.reset()
+            got, _ = s.prefill(ids)
+            assert rel(got, want) <= 1e-5 and rel(timed, want) <= 1e-5, choice
+    finally:
+        fdx.tuner_import(row + "\n")

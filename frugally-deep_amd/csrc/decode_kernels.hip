@@ -34,7 +34,7 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int SK_WAVES = 8;
 constexpr int SK_CHUNK = 8;       // slabs of 16 k-values whose loads are issued together (8 waves x 8 x 16 = 1024 k)
-constexpr int kViaLdsRows = 8;    // see skinny_gemm_launch
+constexpr int kViaLdsRows = 8, kViaLdsK = 448; // see skinny_gemm_launch
 constexpr int SK_CHUNK_LONG = 24; // long-K launches (up to 3072) still issue everything at once, one workgroup per CU
 
 // SINGLE: the workgroup's K range fits one chunk per wave (only one register set is live, which
@@ -1028,8 +1028,12 @@ fdx_status skinny_gemm_launch(const SkinnyParams& p)
     }
     // Activation rows through LDS from eight rows on, next to packed weights (12 layers of 768, per step: 16 rows 366 us
     // against 393, 12 rows 358 / 375, 8 rows 351 / 358, but 4 rows 345 / 337 and one row 335 / 320, where few lanes load
-    // rows at all and the exchange is what remains; row-major weights keep the address unit busy themselves: no gain).
-    const bool via_lds = p.packed && p.M >= kViaLdsRows && per_wg <= SK_WAVES * SK_CHUNK * 16;
+    // rows at all and the exchange is what remains; row-major weights keep the address unit busy themselves: no gain), and
+    // from 448 floats of a workgroup's K range on: below, a wave has fewer than four slabs of 16 to turn, and the exchange
+    // costs what it costs (6 layers, per step in us, through LDS against directly: width 256 with 16 rows 143.9 / 135.9,
+    // with 8 rows 139.6 / 134.2; 384: 151.4 / 152.3 and 144.0 / 139.0; 448: 153.8 / 159.4 and 147.5 / 147.7; 512: 157.4 /
+    // 162.9 and 149.3 / 149.0; 640: 163.8 / 175.6 and 156.8 / 159.2).
+    const bool via_lds = p.packed && p.M >= kViaLdsRows && per_wg >= kViaLdsK && per_wg <= SK_WAVES * SK_CHUNK * 16;
     // every load of a workgroup in flight at once when its K range fits 8 (or 24) slabs per wave
     if (p.emb_x || p.emb_res)
         hipLaunchKernelGGL((skinny_gemm_kernel<6, true, true>), grid, dim3(512), 0, stream(), q);

@@ -306,8 +306,7 @@ __global__ void pool2d_kernel(const float* __restrict__ in, float* __restrict__ 
 
 // One workgroup per (sample, group of G * VEC channels): a lane owns VEC channels, 256 / G positions are read at once, four
 // steps ahead.  Bound by the latency of the walk over positions, hence the many slots: with four positions at a time
-// (a wave each) the pass took 12.4 us on one 16 x 16 x 32 map and 14.1 us on 256 of them, here 2.8 and 4.4;
-// 49 positions of 2048 channels 5.8 -> 3.6.
+// (a wave each) the pass took 12.4 us on one 16 x 16 x 32 map and 14.1 us on 256 of them, here 2.8 and 4.4.
 template <int VEC>
 __global__ __launch_bounds__(256) void global_pool_kernel(const float* __restrict__ in, float* __restrict__ out,
     int positions, int c, int group_log2, int mode)
@@ -364,6 +363,49 @@ __global__ __launch_bounds__(256) void global_pool_kernel(const float* __restric
                 r = mode == 0 ? fmaxf(r, part[w][lane][v]) : r + part[w][lane][v];
             out[(int64_t)img * c + (int64_t)cq * VEC + v] = mode == 0 ? r : r / (float)positions;
         }
+}
+
+// The same for few positions: one workgroup per (sample, 64 channels), a wave takes every fourth position, up to four loads
+// in flight.  There is little to read side by side there, and the kernel above pays for shuffles and idle slots (kernel
+// time: 1000 maps of 2 x 2 x 512 6.0 us here, 8.2 there; 258 of 8 x 1152 4.4 / 6.0; 7 of 6 x 6 x 1280 2.7 / 3.0).
+__global__ __launch_bounds__(256) void global_pool_few_kernel(const float* __restrict__ in, float* __restrict__ out,
+    int positions, int c, int mode)
+{
+    __shared__ float part[4][64];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int groups = (c + 63) / 64;
+    const int img = blockIdx.x / groups, ch = (blockIdx.x - img * groups) * 64 + lane;
+    float val = mode == 0 ? -FLT_MAX : 0.f;
+    if (ch < c && wave < positions) {
+        const float* p = in + ((int64_t)img * positions + wave) * c + ch;
+        const int64_t step = 4LL * c;
+        auto take = [&](auto steps) {
+            float cur[steps()];
+#pragma unroll
+            for (int u = 0; u < steps(); ++u, p += step)
+                cur[u] = *p;
+#pragma unroll
+            for (int u = 0; u < steps(); ++u)
+                val = mode == 0 ? fmaxf(val, cur[u]) : val + cur[u];
+        };
+        int left = (positions - wave + 3) >> 2; // uniform over the wave
+        for (; left >= 4; left -= 4)
+            take(std::integral_constant<int, 4>());
+        if (left == 1)
+            take(std::integral_constant<int, 1>());
+        else if (left == 2)
+            take(std::integral_constant<int, 2>());
+        else if (left == 3)
+            take(std::integral_constant<int, 3>());
+    }
+    part[wave][lane] = val;
+    __syncthreads();
+    if (wave == 0 && ch < c) {
+        float r = part[0][lane];
+        for (int w = 1; w < 4; ++w)
+            r = mode == 0 ? fmaxf(r, part[w][lane]) : r + part[w][lane];
+        out[(int64_t)img * c + ch] = mode == 0 ? r : r / (float)positions;
+    }
 }
 
 // ------------------------------------------------------------------ element-wise
@@ -827,7 +869,12 @@ extern "C" fdx_status fdx_global_pool_f32(const float* in, int n, int positions,
     while (g < most && (1 << g) < cv)
         ++g;
     const dim3 grid((unsigned)((int64_t)n * ((cv + (1 << g) - 1) >> g)));
-    if (vec)
+    // Few positions: up to 64 (a wave per fourth of them, kernel time against the form with many slots: 25 positions 1500 x
+    // 128 channels 4.4 / 5.6 us, 49 positions 128 x 1280 5.9 / 6.1, 81 positions 20 x 30 3.0 / 2.7), or 32 where a wave has
+    // less than its 64 channels (36 positions 42 x 14: 2.7 / 2.5)
+    if (positions <= (c >= 64 ? 64 : 32))
+        hipLaunchKernelGGL(global_pool_few_kernel, dim3((unsigned)((int64_t)n * ((c + 63) / 64))), dim3(256), 0, stream(), in, out, positions, c, mode);
+    else if (vec)
         hipLaunchKernelGGL(global_pool_kernel<4>, grid, dim3(256), 0, stream(), in, out, positions, c, g, mode);
     else
         hipLaunchKernelGGL(global_pool_kernel<1>, grid, dim3(256), 0, stream(), in, out, positions, c, g, mode);

@@ -13,7 +13,10 @@ def rel(a, b):
 
 
 @pytest.mark.parametrize("n,h,w,c", [(1, 1, 1, 4), (2, 7, 7, 1), (1, 16, 16, 32), (3, 5, 13, 30), (1, 7, 7, 2048), (5, 33, 31, 68),
-                                     (130, 3, 3, 128), (2, 9, 5, 67)])
+                                     (130, 3, 3, 128), (2, 9, 5, 67),
+                                     # both sides of the lines to the form for few positions, every number of its last loads
+                                     (3, 8, 8, 64), (3, 5, 13, 64), (3, 4, 8, 63), (3, 3, 11, 63), (700, 2, 2, 130), (2, 1, 2, 200), (2, 1, 3, 64),
+                                     (2, 1, 5, 12), (2, 3, 3, 65), (2, 13, 1, 96), (2, 1, 17, 64), (2, 3, 7, 64)])
 @pytest.mark.parametrize("mode", ["avg", "max"])
 def test_global_pool(fdx, oracle, n, h, w, c, mode):
     print("global pool", n, h, w, c, mode, flush=True)

@@ -172,9 +172,9 @@ __global__ __launch_bounds__(256) void dwconv3x3_kernel(const float* __restrict_
 // The same 3x3 stride-1 stencil with a window that slides down the image: a lane owns TX output columns of four
 // channels and walks RY output rows, keeping three input rows in registers, so every input value is loaded once per
 // column tile (plus its two frame columns) instead of once per output row that touches it -- 1.3 to 1.7 loads per
-// output where the row-at-a-time kernel above issues 3.75.  Meant for the small feature maps (14 x 14, 7 x 7) with
-// many channels, where that kernel's three-fold row reuse has to come from the caches; it needs enough (image, row
-// tile, column tile, channel quad) items to fill the chip, which the launcher checks.
+// output where the row-at-a-time kernel above issues 3.75.  Meant for large batches of feature maps, where that kernel's
+// three-fold row reuse has to come from the caches; it needs enough (image, row tile, column tile, channel quad) items to
+// fill the chip, which the launcher sees to with a least number of output vectors.
 template <int TX, int RY>
 __global__ __launch_bounds__(256) void dwconv3x3_slide_kernel(const float* __restrict__ in, const float* __restrict__ wts,
     const float* __restrict__ bias, float* __restrict__ out, int n, int h, int w, int c, int pad_top, int pad_left,
@@ -791,7 +791,10 @@ extern "C" fdx_status fdx_dwconv2d_nhwc_f32(const float* in, int n, int h, int w
     // (14 x 14, 7 x 7), row tiles of 4 where taller ones leave too few items.  Below, its items (16 to 64 vectors each) are a
     // few dozen workgroups that walk rows one after the other while most CUs have none: 0.12-0.26 million vectors (21 x 21 x
     // 192 to 11 x 11 x 576, 7 images) 7.3-8.1 us against 4.8-5.1 row by row in fours, 0.3-0.7 million 7.8-9.0 against 5.4-8.6;
-    // 0.79 million 9.1 against 11.0, 1.7 million 13.2 against 18.1.
+    // 0.79 million 9.1 against 11.0, 1.7 million 13.2 against 18.1.  Where the rows' fours reach beyond the map the line is drawn
+    // through what they compute, if a row of the map is more than a workgroup's lanes: the three rows that read an input row then
+    // sit in workgroups on different XCDs (40 images of 10 x 10 x 700, 0.70 million vectors, 0.84 in fours: 8.9 against 10.3; 5 of
+    // 56 x 21 x 480 8.1 / 10.6; but 79 of 41 x 9 x 88, 66 items a row, 8.7 / 7.2).
     static const bool slide_on = [] { const char* e = std::getenv("FDX_DW_SLIDE"); return !(e && e[0] == '0'); }();
     const int tx_s = out_w % 7 == 0 && out_w % 8 != 0 ? 7 : 8;
     int ry_s = out_h % 7 == 0 && out_h % 8 != 0 ? 7 : 8;
@@ -799,7 +802,8 @@ extern "C" fdx_status fdx_dwconv2d_nhwc_f32(const float* in, int n, int h, int w
     if (slide_items_for(ry_s) < 256 * 256)
         ry_s = 4;
     const size_t slide_items = slide_items_for(ry_s);
-    const bool slide = k3 && sy == 1 && slide_on && items >= 750000;
+    const size_t row_items = (size_t)((out_w + 3) / 4) * (c / 4);
+    const bool slide = k3 && sy == 1 && slide_on && (items >= 750000 || ((size_t)n * out_h * row_items * 4 >= 750000 && row_items >= 320));
 #define FDX_DW_SLIDE_LAUNCH(TX_, RY_)                                                                                                  \
     hipLaunchKernelGGL((dwconv3x3_slide_kernel<TX_, RY_>), dim3(grid_for(slide_items, 256)), dim3(256), 0, stream(), in, weights_hwc, bias, out, \
         n, h, w, c, pad_top, pad_left, out_h, out_w, a)

@@ -137,7 +137,7 @@ def test_gemm_vs_oracle_dense(fdx, oracle, m, n, k, tile):
     # the column-tiled 3x3 kernel: widths that are not a multiple of its four-column tile, one-column images, same / valid
     (2, 7, 7, 32, 3, 3, (1, 1), (1, 1), "same"), (1, 5, 1, 8, 3, 3, (1, 1), (1, 1), "same"), (2, 9, 13, 16, 3, 3, (2, 2), (1, 1), "same"),
     (1, 8, 10, 12, 3, 3, (1, 1), (1, 1), "valid"), (1, 3, 3, 4, 3, 3, (2, 2), (1, 1), "valid"), (2, 6, 5, 8, 5, 5, (1, 1), (1, 1), "same"),
-    # enough items for the sliding-window 3x3 kernel with row tiles of 4: column tiles of 7 and of 8, extents that end inside a tile
+    # the row-by-row 3x3 kernel with more channels than a workgroup's lanes, extents that end inside a tile
     (16, 14, 14, 256, 3, 3, (1, 1), (1, 1), "same"), (32, 7, 7, 480, 3, 3, (1, 1), (1, 1), "same"), (8, 9, 11, 512, 3, 3, (1, 1), (1, 1), "same"),
     (8, 21, 16, 256, 3, 3, (1, 1), (1, 1), "valid")])
 def test_dwconv_vs_oracle(fdx, oracle, case):

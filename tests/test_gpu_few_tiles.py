@@ -85,6 +85,32 @@ def test_residual_block_with_shortcut_convolution_few_tiles(fdx, oracle, modelge
     assert rel(got, want) <= 2 * TOL
 
 
+@pytest.mark.parametrize("tile", [40, 41, 42, 43, 44])
+@pytest.mark.parametrize("mid,cin,n,size", [(16, 48, 1, 9), (48, 16, 3, 5), (48, 80, 1, 14), (32, 64, 2, 7), (160, 32, 1, 3)])
+def test_both_units_of_the_two_source_form(fdx, oracle, modelgen, tile, mid, cin, n, size):
+    """The sum of two pointwise convolutions as one GEMM: channel counts that are multiples of 16 only (the 16-float unit) and
+    of 32 (the 32-float one) in either source, waves whose share of K lies in one source, in both, or is empty."""
+    print("two sources", tile, mid, cin, n, size, flush=True)
+    b = modelgen.Builder("dual", 15)
+    x = b.input((size, size, cin), "x")
+    y = b.conv2d(x, mid, 1, "c1", strides=2, activation="relu", bias_std=0.1)
+    y = b.conv2d(y, 52, 1, "c2", bias_std=0.1)
+    s = b.conv2d(x, 52, 1, "c0", strides=2, bias_std=0.1)
+    js = modelgen.dumps(b.finish([b.add([s, y], "sum")]))
+    xs = np.random.default_rng(16).standard_normal((n, size, size, cin)).astype(np.float32)
+    ref = oracle.OracleModel(js)
+    want = np.stack([ref.predict([xs[i]])[0] for i in range(n)])
+    model = fdx.Model(js, verify=False)
+    fdx.lib.fdx_debug_force_tile(tile)
+    try:
+        got = model.predict([xs])[0]
+        again = model.predict([xs])[0]
+    finally:
+        fdx.lib.fdx_debug_force_tile(-1)
+    assert rel(got, want) <= 2 * TOL
+    assert np.array_equal(got, again)
+
+
 def test_more_tiles_than_a_launch_can_hold(fdx):
     """131072 x 16384 outputs (8.6 GB): a workgroup of 512 threads for each 16 x 16 of them would be 2^32 threads.  Neither
     the timing runs nor a forced form takes that form."""

@@ -406,3 +406,75 @@ def test_stacked_projection_timed_and_from_a_table(fdx, modelgen):
             assert rel(got, want) <= 1e-5 and rel(timed, want) <= 1e-5, choice
     finally:
         fdx.tuner_import(row + "\n")
+
+
+LOWEST = np.float32(-3.4028234663852886e38)
+HEADS = {
+    "NaN among numbers": lambda b: b.__setitem__(slice(3, 40, 9), np.nan),
+    "NaN only": lambda b: b.fill(np.nan),
+    "-inf only": lambda b: b.fill(-np.inf),
+    "the lowest float only": lambda b: b.fill(LOWEST),
+    "the lowest float, then NaN": lambda b: (b.fill(LOWEST), b.__setitem__(7, np.nan)),
+    "-inf but for one": lambda b: (b.fill(-np.inf), b.__setitem__(17, -1e38)),
+    "inf twice": lambda b: b.__setitem__([20, 25], np.inf),
+    "0 everywhere": lambda b: b.fill(0),
+    "-0 in front of 0": lambda b: (b.fill(-1), b.__setitem__(11, -0.0), b.__setitem__(13, 0.0)),
+    "equal largest values": lambda b: b.__setitem__([30, 31, 39], 99),
+}
+
+
+@pytest.mark.parametrize("vocab", [40, 33000])
+@pytest.mark.parametrize("head", list(HEADS))
+def test_greedy_ids_of_special_logits(fdx, oracle, modelgen, vocab, head):
+    """What a prompt, a step and the greedy loop pick follows the reference's scan for the first value above all before it,
+    which starts at the lowest float: NaN, -inf and the lowest float never win, id 0 stands for no winner.  With a small head
+    the ids come from a pass over the logits, with a large one from the maxima its launch leaves."""
+    say("special logits", vocab, head)
+    spec = modelgen.gpt2(seed=151, layers=1, d_model=64, heads=1, vocab=vocab, max_pos=32, bias_std=0.1, std=0.1)
+    lm = spec["trainable_params"]["lm_head"]
+    lm["weights"][:] = 0  # the logits are the bias
+    HEADS[head](lm["bias"])
+    model = fdx.Model(modelgen.dumps(spec), verify=False)
+    want, best = 0, LOWEST
+    for i, v in enumerate(lm["bias"]):
+        if v > best:
+            want, best = i, v
+    assert want == oracle.argmax(lm["bias"])
+    for B in (1, 5, 17):
+        s = fdx.Session(model, B, 32)
+        ids = np.random.default_rng(152).integers(0, vocab, (B, 6))
+        logits, nxt = s.prefill(ids)
+        assert np.array_equal(logits, np.tile(lm["bias"], (B, 1)), equal_nan=True)
+        assert nxt.tolist() == [want] * B
+        assert s.decode_step(nxt)[1].tolist() == [want] * B
+        assert s.decode_greedy(nxt, 3)[0].tolist() == [[want] * B] * 3
+
+
+def test_prompts_take_the_decode_launches_behind_the_last_cache_rows(fdx, modelgen):
+    """Which launches a prompt's last position takes, from the profile: the projections of the decode kernels where the plan
+    allows them (its last layer's three and the head, one attention launch and the arg-max of the head's maxima), none of them
+    in a session that is too long for the decode attention."""
+    say("launches of a prompt")
+    c = fdx.ctypes
+    model = fdx.Model(modelgen.dumps(modelgen.gpt2(seed=161, layers=2, d_model=192, heads=3, vocab=33000, max_pos=64, std=0.1)), verify=False)
+
+    def families(max_len):
+        s = fdx.Session(model, 4, max_len)
+        fdx.check(fdx.lib.fdx_profile_enable(1))
+        try:
+            fdx.check(fdx.lib.fdx_profile_reset())
+            s.prefill(np.arange(4 * 9).reshape(4, 9))
+            fdx.sync()
+            seen, i = {}, 0
+            name, n, ms, fl, by = c.create_string_buffer(128), c.c_uint64(), c.c_double(), c.c_double(), c.c_double()
+            while fdx.lib.fdx_profile_get(i, name, 128, c.byref(n), c.byref(ms), c.byref(fl), c.byref(by)) == 0:
+                seen[name.value.decode()] = n.value
+                i += 1
+        finally:
+            fdx.check(fdx.lib.fdx_profile_enable(0))
+        return seen
+
+    short, long = families(64), families(16384)
+    print(short, long, flush=True)
+    assert short.get("dense_rows_f32") == 5 and short.get("mha_decode_f32") == 1 and short.get("mha_flash_f32") == 1
+    assert "dense_rows_f32" not in long and "mha_decode_f32" not in long and long.get("mha_flash_f32") == 2

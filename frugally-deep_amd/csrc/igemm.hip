@@ -387,19 +387,17 @@ static bool split_prepare()
     return true;
 }
 
-static void tile_of(int cfg, int& bm, int& bn, int& bk)
+// Tile configurations of the fast kernel; the numbers are what tuning tables hold (10, 11, 12 and 17 were forms of the
+// tiles of 13, 14, 15 and 13 and stand for them).
+static int canonical_tile(int cfg) { return cfg >= 10 && cfg <= 12 ? cfg + 3 : cfg == 17 ? 13 : cfg; }
+constexpr int kSlab = 32;
+static void tile_of(int cfg, int& bm, int& bn)
 {
-    switch (cfg) {
-    case 10: bm = 128; bn = 128; bk = 16; break;
-    case 11: bm = 128; bn = 64; bk = 16; break;
-    case 12: bm = 64; bn = 64; bk = 16; break;
-    case 13: bm = 128; bn = 128; bk = 32; break;
-    case 14: bm = 128; bn = 64; bk = 32; break;
-    case 15: bm = 64; bn = 64; bk = 32; break;
-    case 16: bm = 128; bn = 128; bk = 32; break;
-    case 17: bm = 128; bn = 128; bk = 32; break;
-    case 18: bm = 256; bn = 128; bk = 32; break;
-    default: bm = 64; bn = 64; bk = 32; break;
+    switch (canonical_tile(cfg)) {
+    case 14: bm = 128; bn = 64; break;
+    case 15: bm = 64; bn = 64; break;
+    case 18: bm = 256; bn = 128; break;
+    default: bm = 128; bn = 128; break;
     }
 }
 
@@ -407,9 +405,9 @@ static void tile_of(int cfg, int& bm, int& bn, int& bk)
 // range, and the partial tiles and tickets fit the scratch
 static bool split_fits(int cfg, int splits, int64_t split_tiles, const GemmParams& q)
 {
-    int bm, bn, bk;
-    tile_of(cfg, bm, bn, bk);
-    return splits >= 2 && q.K / bk >= 2 * splits && split_tiles <= kSplitTickets
+    int bm, bn;
+    tile_of(cfg, bm, bn);
+    return splits >= 2 && (q.K + kSlab - 1) / kSlab >= 2 * splits && split_tiles <= kSplitTickets
         && (size_t)split_tiles * splits * bm * bn * sizeof(float) <= kSplitWsBytes && split_tiles * splits < (1 << 30);
 }
 
@@ -419,19 +417,19 @@ static bool split_fits(int cfg, int splits, int64_t split_tiles, const GemmParam
 // mode 2 (stream-K, splits == 0): one workgroup per resident slot, each with an equal stretch of the slabs of all tiles;
 // needs two workspace slots per workgroup and a ticket per tile.
 template <typename K>
-static bool launch_split(K kernel, int tiles, int splits, int mode, int cfg, GemmParams& q, hipStream_t s)
+static bool launch_split(K kernel, int tiles, int splits, int mode, int cfg, GemmParams& q, hipStream_t s, int threads)
 {
-    const int resident = g_persist_scale > 0 ? g_persist_scale : resident_workgroups(kernel, 256);
+    const int resident = g_persist_scale > 0 ? g_persist_scale : resident_workgroups(kernel, threads);
     if (mode == 2) {
-        int bm, bn, bk;
-        tile_of(cfg, bm, bn, bk);
-        const int64_t slabs = (int64_t)tiles * (q.K / bk);
+        int bm, bn;
+        tile_of(cfg, bm, bn);
+        const int64_t slabs = (int64_t)tiles * ((q.K + kSlab - 1) / kSlab);
         const int grid = (int)std::min<int64_t>(resident, slabs);
         if (tiles > kSplitTickets || (size_t)grid * 2 * bm * bn * sizeof(float) > kSplitWsBytes || slabs >= (1LL << 40))
             return false;
         q.splits = 0;
         q.split_dp_tiles = 0;
-        hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(256), 0, s, q);
+        hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3((unsigned)threads), 0, s, q);
         return true;
     }
     const bool hybrid = mode == 1;
@@ -439,7 +437,7 @@ static bool launch_split(K kernel, int tiles, int splits, int mode, int cfg, Gem
     if (tiles - dp > 0 && !split_fits(cfg, splits, tiles - dp, q))
         return false;
     q.split_dp_tiles = dp;
-    launch_persistent(kernel, dp + (tiles - dp) * splits, q, s);
+    launch_persistent(kernel, dp + (tiles - dp) * splits, q, s, threads);
     return true;
 }
 
@@ -453,61 +451,118 @@ static bool launch_fast(int cfg, int splits, int mode, const GemmParams& q0, boo
     q.strip_w = 0; // set per whole-tile launch
 
     bool ok = true;
-#define FDX_FAST(BM_, BN_, BK_)                                                                                  \
+#define FDX_FAST(BM_, BN_, WM_, WN_)                                                                             \
     {                                                                                                            \
+        constexpr int nt = 64 * WM_ * WN_;                                                                       \
         const int tiles = ((q.M + BM_ - 1) / BM_) * ((q.N + BN_ - 1) / BN_) * batch;                             \
         if (mode == 2) {                                                                                         \
             if (conv)                                                                                            \
-                ok = launch_split(igemm_fast_kernel<BM_, BN_, 2, 2, BK_, true, true, true>, tiles, splits, mode, cfg, q, s); \
+                ok = launch_split(igemm_fast_kernel<BM_, BN_, WM_, WN_, true, true, true>, tiles, splits, mode, cfg, q, s, nt); \
             else                                                                                                 \
-                ok = launch_split(igemm_fast_kernel<BM_, BN_, 2, 2, BK_, false, true, true>, tiles, splits, mode, cfg, q, s); \
+                ok = launch_split(igemm_fast_kernel<BM_, BN_, WM_, WN_, false, true, true>, tiles, splits, mode, cfg, q, s, nt); \
         } else if (splits > 1) {                                                                                 \
             if (conv)                                                                                            \
-                ok = launch_split(igemm_fast_kernel<BM_, BN_, 2, 2, BK_, true, true>, tiles, splits, mode, cfg, q, s); \
+                ok = launch_split(igemm_fast_kernel<BM_, BN_, WM_, WN_, true, true>, tiles, splits, mode, cfg, q, s, nt); \
             else                                                                                                 \
-                ok = launch_split(igemm_fast_kernel<BM_, BN_, 2, 2, BK_, false, true>, tiles, splits, mode, cfg, q, s); \
-        } else if (conv)                                                                                         \
-            launch_persistent(igemm_fast_kernel<BM_, BN_, 2, 2, BK_, true>, tiles, q, s, 256, BM_, BN_);         \
-        else if (q.A2)                                                                                           \
-            launch_persistent(igemm_fast_kernel<BM_, BN_, 2, 2, BK_, false, false, false, true>, tiles, q, s, 256, BM_, BN_); \
-        else                                                                                                     \
-            launch_persistent(igemm_fast_kernel<BM_, BN_, 2, 2, BK_, false>, tiles, q, s, 256, BM_, BN_);        \
+                ok = launch_split(igemm_fast_kernel<BM_, BN_, WM_, WN_, false, true>, tiles, splits, mode, cfg, q, s, nt); \
+        } else                                                                                                   \
+            FDX_FAST_WHOLE(BM_, BN_, WM_, WN_)                                                                   \
     }
-        // eight-wave variants: more waves per SIMD to cover LDS and global latency, or a 256-row tile that halves the
-        // operand traffic per FLOP
-#define FDX_FAST8(BM_, BN_, WM_, WN_)                                                                            \
+#define FDX_FAST_WHOLE(BM_, BN_, WM_, WN_)                                                                       \
     {                                                                                                            \
-        const int tiles = ((q.M + BM_ - 1) / BM_) * ((q.N + BN_ - 1) / BN_) * batch;                             \
+        constexpr int wnt = 64 * WM_ * WN_;                                                                      \
+        const int wtiles = ((q.M + BM_ - 1) / BM_) * ((q.N + BN_ - 1) / BN_) * batch;                            \
         if (conv)                                                                                                \
-            launch_persistent(igemm_fast_kernel<BM_, BN_, WM_, WN_, 32, true>, tiles, q, s, 512, BM_, BN_);      \
+            launch_persistent(igemm_fast_kernel<BM_, BN_, WM_, WN_, true>, wtiles, q, s, wnt, BM_, BN_);         \
+        else if (q.A2)                                                                                           \
+            launch_persistent(igemm_fast_kernel<BM_, BN_, WM_, WN_, false, false, false, true>, wtiles, q, s, wnt, BM_, BN_); \
         else                                                                                                     \
-            launch_persistent(igemm_fast_kernel<BM_, BN_, WM_, WN_, 32, false>, tiles, q, s, 512, BM_, BN_);     \
+            launch_persistent(igemm_fast_kernel<BM_, BN_, WM_, WN_, false>, wtiles, q, s, wnt, BM_, BN_);        \
     }
-    if (q.ln_wsum) { // rows normalised on the way: whole tiles of the 32-float slab configurations
-        switch (cfg) {
-        case 13: launch_persistent(igemm_fast_kernel<128, 128, 2, 2, 32, false, false, false, false, true>,
-            ((q.M + 127) / 128) * ((q.N + 127) / 128) * batch, q, s, 256, 128, 128); break;
-        case 14: launch_persistent(igemm_fast_kernel<128, 64, 2, 2, 32, false, false, false, false, true>,
+    if (q.ln_wsum) { // rows normalised on the way: whole tiles
+        switch (canonical_tile(cfg)) {
+        case 13: launch_persistent(igemm_fast_kernel<128, 128, 4, 2, false, false, false, false, true>,
+            ((q.M + 127) / 128) * ((q.N + 127) / 128) * batch, q, s, 512, 128, 128); break;
+        case 14: launch_persistent(igemm_fast_kernel<128, 64, 2, 2, false, false, false, false, true>,
             ((q.M + 127) / 128) * ((q.N + 63) / 64) * batch, q, s, 256, 128, 64); break;
-        default: launch_persistent(igemm_fast_kernel<64, 64, 2, 2, 32, false, false, false, false, true>,
+        default: launch_persistent(igemm_fast_kernel<64, 64, 2, 2, false, false, false, false, true>,
             ((q.M + 63) / 64) * ((q.N + 63) / 64) * batch, q, s, 256, 64, 64); break;
         }
         return true;
     }
-        switch (cfg) {
-        case 10: FDX_FAST(128, 128, 16) break;
-        case 11: FDX_FAST(128, 64, 16) break;
-        case 12: FDX_FAST(64, 64, 16) break;
-        case 13: FDX_FAST(128, 128, 32) break;
-        case 14: FDX_FAST(128, 64, 32) break;
-        case 16: FDX_FAST8(128, 128, 2, 4) break;
-        case 17: FDX_FAST8(128, 128, 4, 2) break;
-        case 18: FDX_FAST8(256, 128, 4, 2) break;
-        default: FDX_FAST(64, 64, 32) break;
-        }
+    switch (canonical_tile(cfg)) {
+    case 13: FDX_FAST(128, 128, 4, 2) break;
+    case 14: FDX_FAST(128, 64, 2, 2) break;
+    case 16: FDX_FAST_WHOLE(128, 128, 2, 2) break;
+    case 18: FDX_FAST_WHOLE(256, 128, 4, 2) break;
+    default: FDX_FAST(64, 64, 2, 2) break;
+    }
 #undef FDX_FAST
-#undef FDX_FAST8
+#undef FDX_FAST_WHOLE
     return ok;
+}
+
+// The closed rule of the fast kernel: which tile, and whether K is cut.  Costs fitted to 240 timed problems (M 200-200000,
+// N 48-3200, K 32-5000, 0.2-40 GFLOP, two thirds GEMM, a third convolutions; rms 5-8 %); by them 240 others of the same ranges take
+// 4 % longer than the fastest of all forms (20 % in the worst case).
+//     whole tiles    t0 + w (e + a k) + r (f + b k) + c k t + g k min(t, 1) + d k w (convolution) + io
+//     K ranges       the same on S times the tiles and a range's k, plus 0.9 per range and 0.75 per MB of partial tiles
+//     stream-K       11 + 44 k per stretch + 2.2 per contributor of a tile + 1.7 t + io
+// in microseconds, with k = K / 1000 in whole slabs, t = tiles (or ranges) / CUs, w = t rounded up, r = rounds of the workgroups
+// that are resident, io = the floats read of A, of the residual and written, per million.
+struct TileCost {
+    int cfg, resident;
+    float t0, e, a, f, b, c, g, d, io;
+};
+static const TileCost kTileCost[] = {
+    { 13, 256, 1.90f, 0.f, 33.1f, 2.97f, 0.f, 5.54f, 0.f, 2.72f, 0.194f },
+    { 14, 512, 2.22f, 0.98f, 10.9f, 0.73f, 17.9f, 1.65f, 0.f, 2.75f, 0.195f },
+    { 15, 768, 1.84f, 0.76f, 5.15f, 0.f, 15.0f, 1.50f, 0.f, 1.08f, 0.152f },
+    { 16, 512, 3.47f, 2.09f, 19.9f, 0.90f, 19.5f, 3.38f, 0.f, 6.64f, 0.320f },
+    { 18, 256, 1.02f, 0.f, 54.5f, 5.86f, 0.f, 8.00f, 0.f, 5.93f, 0.279f },
+};
+static float tile_cost(const TileCost& c, bool conv, int64_t units, float k, float io)
+{
+    const float t = (float)units / 256.f, w = (float)((units + 255) / 256), r = (float)((units + c.resident - 1) / c.resident);
+    return c.t0 + w * (c.e + (c.a + (conv ? c.d : 0.f)) * k) + r * (c.f + c.b * k) + c.c * k * t + c.g * k * std::min(t, 1.f) + c.io * io;
+}
+struct TileChoice {
+    int cfg, splits, mode;
+    float cost;
+};
+static TileChoice tile_pick(bool conv, int M, int N, int K, int64_t a_floats, bool residual, int batch, bool cuts)
+{
+    const int slabs = (K + kSlab - 1) / kSlab;
+    const float k = (float)slabs * (kSlab * 1e-3f);
+    const float io = 1e-6f * (float)batch * ((float)a_floats + (residual ? 2.f : 1.f) * (float)M * (float)N);
+    auto tiles = [&](int cfg) {
+        int bm, bn;
+        tile_of(cfg, bm, bn);
+        return (int64_t)((M + bm - 1) / bm) * ((N + bn - 1) / bn) * batch;
+    };
+    TileChoice best { 15, 1, 0, 1e30f };
+    auto consider = [&](int cfg, int splits, int mode, float cost, float handicap) {
+        if (cost * handicap < best.cost)
+            best = { cfg, splits, mode, cost * handicap };
+    };
+    for (const TileCost& c : kTileCost)
+        consider(c.cfg, 1, 0, tile_cost(c, conv, tiles(c.cfg), k, io), 1.f);
+    if (!cuts)
+        return best;
+    // A cut costs more than its own time (partial tiles through memory; stretches read operands at a K phase of their own, so
+    // that neighbours do not share them in L2): handicaps of 4 and 3 %.
+    const int64_t t64 = tiles(15);
+    static const TileCost kRange = { 15, 768, 0.71f, 0.18f, 6.22f, 2.49f, 14.1f, 1.21f, 0.f, 1.61f, 0.02f };
+    for (int S : { 2, 3, 4, 6, 8 })
+        if (t64 <= 768 && slabs >= 2 * S)
+            consider(15, S, 0, tile_cost(kRange, conv, t64 * S, (float)((slabs + S - 1) / S) * (kSlab * 1e-3f), io) + 0.91f * S
+                    + 0.755f * (float)(t64 * S) * (64 * 64 * 1e-6f), 1.04f);
+    const int64_t t128 = tiles(13);
+    if (t128 >= 86 && t128 <= 512 && K >= 256) {
+        const float stretch = (float)(t128 * slabs) / (float)std::min<int64_t>(256, t128 * slabs);
+        consider(13, 0, 2, 11.1f + 44.4f * stretch * (kSlab * 1e-3f) + 0.49f * io + 2.21f * 256.f / (float)t128 + 1.74f * (float)t128 / 256.f, 1.03f);
+    }
+    return best;
 }
 
 // First sight of a problem shape on the fast path: time every tile configuration once on the
@@ -605,7 +660,7 @@ static float time_rounds(hipEvent_t a, hipEvent_t b, hipStream_t s, F&& launch)
 // stream_ok: the row-streaming short-K kernel (configuration 30, pw_stream.hpp) competes as well
 constexpr int kStreamCfg = 30;
 template <typename F, typename G>
-static int autotune(const GemmParams& q, bool conv, int batch, int unit, hipStream_t s, int general_cfg, F general_launch,
+static int autotune(const GemmParams& q, bool conv, int batch, hipStream_t s, int general_cfg, F general_launch,
     bool stream_ok, G stream_launch)
 {
     static const bool split_env = [] { const char* sp = std::getenv("FDX_SPLITK"); return !(sp && sp[0] == '0'); }();
@@ -627,11 +682,9 @@ static int autotune(const GemmParams& q, bool conv, int batch, int unit, hipStre
     const bool can_split = g_split_enabled && split_prepare();
     auto timed = [&](auto&& launch) -> float { return time_rounds(a, b, s, launch); };
     bool clock_settled = false;
-    for (int cfg = 10; cfg <= 18; ++cfg) {
-        if (cfg >= 13 && unit % 32 != 0)
-            continue;
-        int bm, bn, bk;
-        tile_of(cfg, bm, bn, bk);
+    for (int cfg : { 13, 14, 15, 16, 18 }) {
+        int bm, bn;
+        tile_of(cfg, bm, bn);
         const int64_t tiles = (int64_t)((q.M + bm - 1) / bm) * ((q.N + bn - 1) / bn) * batch;
         if (bn > 64 && q.N <= bn / 2)
             continue; // a tile at least twice as wide as the output only idles half of every MFMA
@@ -686,7 +739,7 @@ static int autotune(const GemmParams& q, bool conv, int batch, int unit, hipStre
     for (int c = kSliceCfg; c < kSliceCfg + kSliceForms && batch == 1; ++c) {
         // only forms that a grid can hold (a refused launch would time as nothing) and that may win
         if (!slice_fits(c - kSliceCfg, q.M, q.N)
-            || slice_cost(c - kSliceCfg, conv, q.M, q.N, q.K) > 1.5f * slice_tiled_cost(q.M, q.N, q.K))
+            || slice_cost(c - kSliceCfg, conv, q.M, q.N, q.K) > 1.5f * tile_pick(conv, q.M, q.N, q.K, (int64_t)q.M * q.K, q.residual != nullptr, 1, true).cost)
             continue;
         slice_launch(c, q, conv, s);
         const float ms = timed([&] { slice_launch(c, q, conv, s); });
@@ -754,7 +807,6 @@ static fdx_status run_igemm(GemmParams& p, bool conv, int batch, const char* fam
         a_ok = a_mode == A_ROWS_VEC && p.K % 16 == 0;
     }
     const bool fast_ok = out_ok && a_ok && b_vec && a_bytes < (1LL << 31) && b_bytes < (1LL << 31) && p.ldc < (1LL << 24);
-    const int unit = conv ? p.Cin : p.K;
 
     int cfg = g_forced_tile, splits = 1, mode = 0;
     auto unpack = [&]() { // configuration + 100 * splits + 10000 * mode
@@ -774,13 +826,13 @@ static fdx_status run_igemm(GemmParams& p, bool conv, int batch, const char* fam
         const bool slice = cfg >= kSliceCfg && cfg < kSliceCfg + kSliceForms;
         if (slice && (!fast_ok || batch != 1 || !slice_fits(cfg - kSliceCfg, p.M, p.N)))
             cfg = -1;
-        if (cfg >= 10 && cfg != kStreamCfg && !slice && (!fast_ok || cfg > 18 || (cfg >= 13 && unit % 32 != 0)))
+        if (cfg >= 10 && cfg != kStreamCfg && !slice && (!fast_ok || cfg > 18))
             cfg = -1;
         if (cfg < 10 || mode > 2 || mode < 0 || splits < 0 || splits > 64 || cfg == kStreamCfg || slice) {
             splits = 1;
             mode = 0;
         }
-        if (cfg >= 10 && splits != 1 && (cfg > 15 || !split_prepare())) {
+        if (cfg >= 10 && splits != 1 && (canonical_tile(cfg) > 15 || !split_prepare())) {
             splits = 1;
             mode = 0;
         }
@@ -801,6 +853,7 @@ static fdx_status run_igemm(GemmParams& p, bool conv, int batch, const char* fam
             set_error("igemm: this normalising problem needs the fast path");
             return FDX_ERR_UNSUPPORTED;
         }
+        cfg = canonical_tile(cfg);
         if (cfg < 13 || cfg > 15)
             cfg = -1;
         splits = 1;
@@ -819,18 +872,15 @@ static fdx_status run_igemm(GemmParams& p, bool conv, int batch, const char* fam
             return FDX_ERR_UNSUPPORTED;
         }
         p.a2_records = (uint32_t)a2_bytes;
-        const bool slab32 = p.K % 32 == 0 && p.K1 % 32 == 0;
-        if (cfg < 10 || (cfg > 15 && cfg < kSliceCfg) || (cfg >= 13 && cfg <= 15 && !slab32))
+        if (cfg < 10 || (cfg > 18 && cfg < kSliceCfg))
             cfg = -1;
         splits = 1;
         mode = 0;
-        if (cfg < 0)
-            cfg = slice_pick(conv, p.M, p.N, p.K);
         if (cfg < 0) {
-            if (p.K >= 1024 && p.N % 128 == 0 && blocks(128, 128) >= 2048)
-                cfg = slab32 ? 13 : 10;
-            else
-                cfg = (slab32 && p.K >= 128) ? 15 : 12;
+            const TileChoice tile = tile_pick(conv, p.M, p.N, p.K, (int64_t)p.M * p.K, false, 1, false);
+            cfg = slice_pick(conv, p.M, p.N, p.K, tile.cost);
+            if (cfg < 0)
+                cfg = tile.cfg;
         }
     } else if (cfg < 0) {
         if (fast_ok && p.N >= 16 && 2.0 * p.M * (double)p.N * p.K * batch >= 2e8) {
@@ -843,51 +893,26 @@ static fdx_status run_igemm(GemmParams& p, bool conv, int batch, const char* fam
             // fast path can read this operand
             const bool general_ok = p.N < 64 && p.a_valid_k == 0 && !(conv && p.pix_stride != p.Cin);
             const int general_cfg = !general_ok ? -1 : p.N <= 32 ? 2 : (blocks(128, 64) >= 512 ? 1 : 3);
-            cfg = autotune(q, conv, batch, unit, s, general_cfg, [&] { launch_general(general_cfg); }, stream_ok,
+            cfg = autotune(q, conv, batch, s, general_cfg, [&] { launch_general(general_cfg); }, stream_ok,
                 [&] { pw_stream_launch(p, a_bytes, b_bytes, s); });
             settle();
         }
-        if (cfg < 0 && fast_ok && batch == 1)
-            cfg = slice_pick(conv, p.M, p.N, p.K);
         static const bool closed_cuts = [] { const char* e = std::getenv("FDX_CLOSED_SPLIT"); return !(e && e[0] == '0'); }();
+        TileChoice tile { -1, 1, 0, 1e30f };
+        if (cfg < 0 && fast_ok) {
+            tile = tile_pick(conv, p.M, p.N, p.K, conv ? a_bytes / 4 : (int64_t)p.M * p.K, p.residual != nullptr, batch, closed_cuts);
+            if (batch == 1)
+                cfg = slice_pick(conv, p.M, p.N, p.K, tile.cost);
+        }
         if (cfg >= 0) {
         } else if (stream_ok && p.K <= 32 && p.N <= 160 && p.M >= 65536) {
             // very short rows over a long map (MobileNetV2's first expansions): the row-streaming kernel
             cfg = kStreamCfg;
-        } else if (fast_ok && p.N >= 64) {
-            // what the timing runs pick most often: the 64 x 64 tile at four or five workgroups per CU, with the
-            // 32-float slab where K is long enough for it; the 128 x 128 tile only for problems that are large in
-            // every dimension; the 128 x 64 tile with the short slab for wide outputs from short rows, where the
-            // stores dominate
-            if (p.K >= 1024 && p.N % 128 == 0 && blocks(128, 128) >= 2048)
-                cfg = unit % 32 == 0 ? 13 : 10;
-            else if (p.K <= 96 && p.N >= 128 && blocks(128, 64) >= 1024)
-                cfg = 11;
-            else
-                cfg = (unit % 32 == 0 && p.K >= 128) ? 15 : 12;
-            // Fewer 64 x 64 tiles than one round of resident workgroups (four per CU) and a long K: the chip is filled
-            // by cutting K instead.  Below one tile per CU every tile is cut into equal K ranges, about two workgroups
-            // per CU in total (a Dense with few rows: 2.8 times faster at 64 x 1000 x 2048); from there up to one
-            // round the stream-K form spreads the slabs of all tiles evenly over the resident workgroups (10-12 %
-            // faster on ResNet50's 14 x 14 and 7 x 7 1x1 layers).  Both forms add their partial tiles in a fixed order.
-            if (closed_cuts && (cfg == 15 || cfg == 12)) {
-                const int64_t t64 = blocks(64, 64);
-                const int slabs = p.K / (cfg == 15 ? 32 : 16);
-                if (t64 < 256 && p.K >= 512) {
-                    int want = (int)std::min<int64_t>(8, (512 + t64 - 1) / t64);
-                    while (want >= 2 && slabs < 4 * want)
-                        --want;
-                    if (want >= 2) {
-                        splits = want;
-                        mode = 0;
-                    }
-                } else if (t64 < 1024 && p.K >= 1024 && cfg == 15) {
-                    splits = 0;
-                    mode = 2;
-                }
-                if (splits != 1)
-                    settle(); // the cut needs its workspace
-            }
+        } else if (fast_ok && p.N > 32) {
+            cfg = tile.cfg;
+            splits = tile.splits;
+            mode = tile.mode;
+            settle(); // a cut needs its workspace
         } else if (p.N <= 32)
             cfg = 2;
         else if (p.N <= 64)
@@ -1110,7 +1135,7 @@ fdx_status gemm_segments_launch(const float* a, const float* w, const float* bia
         case kSliceCfg + 3: slice_launch_seg<3>(p, s); break;
         case kSliceCfg + 4: slice_launch_seg<4>(p, s); break;
         default:
-            launch_persistent(igemm_fast_kernel<64, 64, 2, 2, 32, false, false, false, false, false, true>, ((m + 63) / 64) * ((p.N + 63) / 64), p,
+            launch_persistent(igemm_fast_kernel<64, 64, 2, 2, false, false, false, false, false, true>, ((m + 63) / 64) * ((p.N + 63) / 64), p,
                 s, 256, 64, 64);
         }
     };
@@ -1128,7 +1153,7 @@ fdx_status gemm_segments_launch(const float* a, const float* w, const float* bia
         } else if (!tune_frozen() && 2.0 * m * (double)p.N * k >= 2e8 && hipEventCreate(&ea) == hipSuccess && hipEventCreate(&eb) == hipSuccess) {
             float best_ms = 1e30f;
             for (int c : { kTiled, kSliceCfg, kSliceCfg + 1, kSliceCfg + 2, kSliceCfg + 3, kSliceCfg + 4 }) {
-                if (!usable(c) || (c != kTiled && slice_cost(c - kSliceCfg, false, m, p.N, k) > 1.5f * slice_tiled_cost(m, p.N, k)))
+                if (!usable(c) || (c != kTiled && slice_cost(c - kSliceCfg, false, m, p.N, k) > 1.5f * tile_cost(kTileCost[2], false, (int64_t)((m + 63) / 64) * ((p.N + 63) / 64), 1e-3f * k, 1e-6f * m * (float)(k + p.N))))
                     continue;
                 if (c == kTiled)
                     tune_settle_clock([&] { launch(c); return true; });
@@ -1148,7 +1173,7 @@ fdx_status gemm_segments_launch(const float* a, const float* w, const float* bia
             (void)hipEventDestroy(eb);
     }
     if (!usable(cfg))
-        cfg = slice_pick(false, m, p.N, k);
+        cfg = slice_pick(false, m, p.N, k, tile_cost(kTileCost[2], false, (int64_t)((m + 63) / 64) * ((p.N + 63) / 64), 1e-3f * k, 1e-6f * m * (float)(k + p.N)));
     profile_begin();
     launch(cfg);
     profile_end("gemm_f32", 2.0 * m * (double)p.N * k, 0.0);

@@ -1,8 +1,28 @@
 // Fast path of the implicit-GEMM Conv2D / GEMM (included inside namespace fdx by igemm.hip).
 //
-// Same tiling and MFMA schedule as igemm_kernel, with the per-slab overhead stripped for the
-// shapes that dominate real networks (Cin, or K for a plain GEMM, a multiple of the slab; N a
-// multiple of 4), and the workgroups made persistent:
+// For the shapes that dominate real networks (Cin, or K for a plain GEMM, a multiple of 16; N a multiple of 4).  fp32
+// operands, fp32 accumulators and fp32 accuracy, on the bf16 matrix cores:
+//
+//  * The fp32 MFMA (157 TFLOP/s) is what bounds this work; the bf16 one has 16 times its rate.  An fp32 value is exactly
+//    the sum of three bf16 values (8 + 8 + 8 bits, each the rounding of what the ones before leave), so a product of two
+//    is nine bf16 products, of which the three smallest (a1 b2, a2 b1, a2 b2 with planes counted from 0: 2^-27 of the
+//    result and below) are left out: six MFMAs for sixteen steps of K instead of eight fp32 ones of twice the length.
+//    The MFMA adds exact products in fp32, to nearest.  The leading product has accumulators of its own, so a result is
+//    rounded at its own size once per 16 steps of K where the fp32 MFMA does so eight times: against 64-bit sums the
+//    relative error (2-norm, normal operands, K = 64 / 512 / 4608) is 0.5 / 1.3 / 4.2 e-7, with the fp32 MFMA 1.4 / 4.1 / 12 e-7.
+//    8192 x 2048 x 512: 147 -> 93 us, 186 TFLOP/s; with nothing but its MFMAs the kernel runs at 302 and the clock falls to
+//    1.9 GHz: the power limit, not the issue rate, is the next bound.
+//  * Both operands are split by the threads that stage them, on the way from registers to LDS (5.5 vector instructions a
+//    value, hidden behind the MFMAs): operands stay fp32 in memory, nothing is prepared or kept.  Splitting the filter once
+//    at load instead was measured slower (half as many vector instructions, but 6 bytes a value through L2 instead of 4).
+//  * A row of a slab (32 floats) is fetched by four lanes, two 16-byte chunks each (k = 4q.. and 16 + 4q.. for lane q); the
+//    eight values are one MFMA operand (16 bytes) in each plane.  The matrix product does not care which k sit together as
+//    long as both operands agree.  LDS holds blocks of one lane number: block q of a plane = 16 bytes per tile row, so that
+//    a wave's operand reads are two runs of 512 bytes, and blocks are offset by 32 bytes against each other, so that a
+//    wave's writes meet each bank once.
+//  * The largest four-wave tile keeps one slab in LDS (two workgroups on a CU then: one's staging beside the other's
+//    products); its operands go to registers in front of a barrier.  The others keep two.
+//  * Workgroups are persistent:
 //
 //  * Operands are fetched with raw buffer loads: each lane keeps ONE 32-bit byte offset per
 //    tile row for the whole K loop, the walk along K is a scalar offset shared by the
@@ -30,6 +50,80 @@
 //    same workspace / ticket / ordered-sum path, with the number of contributors of a tile
 //    and their workspace slots computed from the cut points.
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+
+__device__ __forceinline__ uint32_t bf16_pair(float a, float b)
+{
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2 { a, b }), bf16x2));
+}
+// Two floats as three pairs of bf16 that add up to them exactly (below 2^-110 the last bits fall under bf16's subnormals).
+__device__ __forceinline__ void split3(float a, float b, uint32_t& p0, uint32_t& p1, uint32_t& p2)
+{
+    p0 = bf16_pair(a, b);
+    a -= __builtin_bit_cast(float, p0 << 16);
+    b -= __builtin_bit_cast(float, p0 & 0xffff0000u);
+    p1 = bf16_pair(a, b);
+    a -= __builtin_bit_cast(float, p1 << 16);
+    b -= __builtin_bit_cast(float, p1 & 0xffff0000u);
+    p2 = bf16_pair(a, b);
+}
+
+// LDS slabs per workgroup and waves per SIMD (the register budget) of a tile.
+constexpr int split_tile_buffers(int bm, int bn, int waves_m, int waves_n)
+{
+    return waves_m * waves_n == 4 && bm * bn >= 128 * 128 ? 1 : 2;
+}
+constexpr int split_tile_waves(int bm, int bn, int waves_m, int waves_n)
+{
+    return waves_m * waves_n == 8 || bm * bn > 64 * 64 ? 2 : 3;
+}
+
+// Element (m, n) of problem z as a plain fp32 sum over K: the value that infinite or NaN operands (or ones beyond the
+// largest bf16) give.
+template <bool CONV, bool DUAL>
+__device__ __forceinline__ float plain_dot(const GemmParams& p, int z, int m, int n)
+{
+    const float* A = p.A + (z / p.inner) * p.a_outer + (z % p.inner) * p.a_inner;
+    const float* B = p.B + (z / p.inner) * p.b_outer + (z % p.inner) * p.b_inner + (int64_t)n * p.ldb;
+    const float* A2 = p.A2;
+    int iy0 = 0, ix0 = 0;
+    if (CONV || DUAL) {
+        const int img = m / (p.OH * p.OW), rm = m - img * (p.OH * p.OW), oy = rm / p.OW, ox = rm - oy * p.OW;
+        if (CONV) {
+            A += ((int64_t)(img * p.H + oy * p.sy) * p.W + ox * p.sx) * p.pix_stride; // A starts (pad_top, pad_left) early
+            iy0 = oy * p.sy - p.pad_top;
+            ix0 = ox * p.sx - p.pad_left;
+        } else {
+            A2 += ((int64_t)(img * p.H2 + oy * p.s2y) * p.W2 + ox * p.s2x) * p.C2;
+        }
+    }
+    if (!CONV)
+        A += (int64_t)m * p.lda;
+    float s = 0.f;
+    int fy = 0, fx = 0, c = 0;
+    const int k_end = p.a_valid_k > 0 ? p.a_valid_k : p.K;
+#pragma clang loop unroll(disable)
+    for (int k = 0; k < k_end; ++k) {
+        float a;
+        if (CONV) {
+            const int iy = iy0 + fy * p.dy, ix = ix0 + fx * p.dx;
+            a = iy >= 0 && iy < p.H && ix >= 0 && ix < p.W ? A[((int64_t)fy * p.dy * p.W + fx * p.dx) * p.pix_stride + c] : 0.f;
+            if (++c == p.Cin) {
+                c = 0;
+                if (++fx == p.kw) {
+                    fx = 0;
+                    ++fy;
+                }
+            }
+        } else {
+            a = DUAL && k >= p.K1 ? A2[k - p.K1] : A[k];
+        }
+        s = fmaf(a, B[k], s);
+    }
+    return s;
+}
 
 // Where row m, column n of a tile whose first column is n0 lies with SEG, in bytes from the start of its segment; segments
 // begin at multiples of the tile width, so a tile's segment is uniform.
@@ -55,11 +149,9 @@ __device__ __forceinline__ int seg_of(const GemmParams& p, int n0) { return (n0 
 //  * SEG (GEMM form, whole tiles only): the columns of C go to up to three tensors, the rows of each in sequences that lie
 //    apart: the stacked query / key / value projection of prompts, keys and values straight into their cache rows (2048 rows, 768 -> 3 x 768:
 //    69 us instead of three launches of 29.6, which leave 384 tiles on 256 CUs each).
-template <int BM, int BN, int WAVES_M, int WAVES_N, int BKT, bool CONV, bool SPLIT = false, bool STREAMK = false, bool DUAL = false,
+template <int BM, int BN, int WAVES_M, int WAVES_N, bool CONV, bool SPLIT = false, bool STREAMK = false, bool DUAL = false,
     bool LNF = false, bool SEG = false>
-// (the second bound asks for two waves per SIMD where the split variant of the largest four-wave tile would otherwise
-// settle for one: its reduction holds the accumulators in ordinary registers next to the prefetched operands)
-__global__ __launch_bounds__(64 * WAVES_M * WAVES_N, (SPLIT && WAVES_M * WAVES_N == 4 && BM * BN >= 128 * 128) ? 2 : 1)
+__global__ __launch_bounds__(64 * WAVES_M * WAVES_N, split_tile_waves(BM, BN, WAVES_M, WAVES_N))
 void igemm_fast_kernel(GemmParams p)
 {
     constexpr int NT = 64 * WAVES_M * WAVES_N;
@@ -67,24 +159,28 @@ void igemm_fast_kernel(GemmParams p)
     static_assert(!DUAL || (!CONV && !SPLIT), "the two-source form is a whole-tile GEMM");
     static_assert(!LNF || (!CONV && !SPLIT && !DUAL), "the normalising form is a whole-tile GEMM");
     static_assert(!SEG || (!CONV && !SPLIT && !DUAL && !LNF), "the form with segmented outputs is a whole-tile GEMM");
-    constexpr int STRIDE = BKT + 4;
-    constexpr int CPR = BKT / 4;  // 16-byte chunks per tile row
-    constexpr int RPP = NT / CPR; // tile rows filled per loader pass
-    constexpr int A_LOADS = BM / RPP, B_LOADS = BN / RPP;
+    constexpr int BKT = 32;
+    constexpr bool DB = split_tile_buffers(BM, BN, WAVES_M, WAVES_N) == 2;
+    constexpr int RPP = NT / 4; // tile rows filled per loader pass: four lanes per row, two 16-byte chunks each
+    constexpr int A_UNITS = BM / RPP, B_UNITS = BN / RPP;
     static_assert(BM % RPP == 0 && BN % RPP == 0, "tile rows must be a multiple of the loader pass");
     constexpr int WTM = BM / WAVES_M, WTN = BN / WAVES_N;
     constexpr int TM = WTM / 32, TN = WTN / 32;
     constexpr int OSTRIDE = WTN + 4; // epilogue scratch row
-    static_assert(2 * (BM + BN) * STRIDE >= WAVES_M * WAVES_N * 32 * OSTRIDE, "epilogue scratch must fit in the operand buffers");
+    // LDS of one slab: per operand three planes of four blocks (one per lane of a row), a block = 16 bytes per tile row
+    constexpr int A_BLK = BM * 16 + 32, B_BLK = BN * 16 + 32, A_BYTES = 12 * A_BLK, BUF_BYTES = 12 * (A_BLK + B_BLK);
+    constexpr int SMEM_BYTES = (DB ? 2 : 1) * BUF_BYTES;
+    static_assert(SMEM_BYTES >= WAVES_M * WAVES_N * 32 * OSTRIDE * 4, "epilogue scratch must fit in the operand buffers");
     constexpr uint32_t OOB = 0x80000000u; // beyond any extent this path accepts: the load returns zeros
 
-    __shared__ __attribute__((aligned(16))) float smem[2 * (BM + BN) * STRIDE];
+    __shared__ __attribute__((aligned(16))) unsigned char smem_raw[SMEM_BYTES];
+    float* const smem = reinterpret_cast<float*>(smem_raw);
     __shared__ int last_flag;
     __shared__ float ln_stats[LNF ? 2 * BM : 2]; // (mean, 1 / sqrt(var + eps)) per tile row
 
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const int wm = wave / WAVES_N, wn = wave % WAVES_N;
-    const int kq = t % CPR, r0 = t / CPR;
+    const int kq = t & 3, r0 = t >> 2;
     const int fr = lane & 31, fh = lane >> 5;
 
     const int tiles_m = (p.M + BM - 1) / BM, tiles_n = (p.N + BN - 1) / BN;
@@ -101,7 +197,7 @@ void igemm_fast_kernel(GemmParams p)
     const int alo = xcd * (n_dp >> 3) + (xcd < (n_dp & 7) ? xcd : (n_dp & 7)), na = (n_dp >> 3) + (xcd < (n_dp & 7) ? 1 : 0);
     const int blo = xcd * (n_su >> 3) + (xcd < (n_su & 7) ? xcd : (n_su & 7)), nb = (n_su >> 3) + (xcd < (n_su & 7) ? 1 : 0);
     const int hi = na + nb; // local unit indices [0, hi)
-    const int KT = p.K / BKT;
+    const int KT = (p.K + BKT - 1) / BKT; // the second half of the last slab may lie behind the end of K: zeros
 
     // stream-K: workgroup g (numbered XCD by XCD, so an XCD owns a contiguous stretch of tiles) takes the slabs
     // [g * W / G, (g + 1) * W / G) of the W = tiles * KT slabs; its units are the tiles that stretch touches
@@ -117,14 +213,15 @@ void igemm_fast_kernel(GemmParams p)
     const int sk_units = (sk && sk_hi > sk_lo) ? (int)((sk_hi - 1) / KT) - sk_first + 1 : 0;
 
     // ---- per-tile loader state
-    uint32_t a_voff[A_LOADS], b_voff[B_LOADS];
-    uint32_t a2_voff[DUAL ? A_LOADS : 1];
-    uint64_t a_mask[A_LOADS];
+    uint32_t a_voff[A_UNITS], b_voff[B_UNITS];
+    uint32_t a2_voff[DUAL ? A_UNITS : 1];
+    uint64_t a_mask[A_UNITS];
     __amdgpu_buffer_rsrc_t srd_a, srd_b;
     const __amdgpu_buffer_rsrc_t srd_a2 = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(DUAL ? p.A2 : p.A), 0,
         DUAL ? (int)p.a2_records : 0, 0x00020000);
+    // the walk along K goes by half slabs of 16 floats; in a convolution one half slab lies within one filter tap
     int tap, fx, fy, c0, soff_a, soff_b;
-    f32x4 ra[A_LOADS], rb[B_LOADS];
+    f32x4 ra[A_UNITS][2], rb[B_UNITS][2];
     int kt_n = KT; // slabs of the current unit
 
     int cur_su = -1;  // workspace slot of the current work item's partial tile, -1 for a whole tile
@@ -171,7 +268,7 @@ void igemm_fast_kernel(GemmParams p)
         srd_a = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(A), 0, (int)p.a_records, 0x00020000);
         srd_b = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(B), 0, (int)p.b_records, 0x00020000);
 #pragma unroll
-        for (int i = 0; i < A_LOADS; ++i) {
+        for (int i = 0; i < A_UNITS; ++i) {
             const int m = m0 + r0 + i * RPP;
             a_voff[i] = OOB;
             a_mask[i] = 0;
@@ -207,7 +304,7 @@ void igemm_fast_kernel(GemmParams p)
             }
         }
 #pragma unroll
-        for (int i = 0; i < B_LOADS; ++i) {
+        for (int i = 0; i < B_UNITS; ++i) {
             const int n = n0 + r0 + i * RPP;
             b_voff[i] = n < p.N ? (uint32_t)((int64_t)n * p.ldb) * 4u + kq * 16 : OOB;
         }
@@ -227,24 +324,28 @@ void igemm_fast_kernel(GemmParams p)
             }
         }
     };
-    auto load_tiles = [&]() {
-        if (DUAL && soff_b >= p.K1 * 4) { // the slab lies in the second tensor's columns (uniform over the workgroup)
+    const int k_bytes = p.K * 4;
+    // Requests half h of the next slab; dead: no such slab, the offsets are out of range and nothing is fetched.
+    auto load_half = [&](int h, bool live) {
+        const bool in_k = live && soff_b < k_bytes;
+        const uint32_t off = in_k ? 0u : OOB;
+        if (DUAL && soff_b >= p.K1 * 4) { // the half slab lies in the second tensor's columns (uniform over the workgroup)
 #pragma unroll
-            for (int i = 0; i < A_LOADS; ++i)
-                ra[i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(srd_a2, (int)a2_voff[DUAL ? i : 0], soff_b - p.K1 * 4, 0));
+            for (int i = 0; i < A_UNITS; ++i)
+                ra[i][h] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(srd_a2, (int)(a2_voff[DUAL ? i : 0] | off), soff_b - p.K1 * 4, 0));
         } else {
 #pragma unroll
-            for (int i = 0; i < A_LOADS; ++i) {
-                const uint32_t vo = CONV ? (((a_mask[i] >> tap) & 1) ? a_voff[i] : OOB) : a_voff[i];
-                ra[i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(srd_a, (int)vo, soff_a, 0));
+            for (int i = 0; i < A_UNITS; ++i) {
+                const uint32_t vo = CONV ? (in_k && ((a_mask[i] >> tap) & 1) ? a_voff[i] : OOB) : (a_voff[i] | off);
+                ra[i][h] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(srd_a, (int)vo, soff_a, 0));
             }
         }
 #pragma unroll
-        for (int i = 0; i < B_LOADS; ++i)
-            rb[i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(srd_b, (int)b_voff[i], soff_b, 0));
-        soff_b += BKT * 4;
+        for (int i = 0; i < B_UNITS; ++i)
+            rb[i][h] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(srd_b, (int)(b_voff[i] | off), soff_b, 0));
+        soff_b += 64;
         if (CONV) {
-            c0 += BKT;
+            c0 += 16;
             if (c0 == p.Cin) {
                 c0 = 0;
                 ++tap;
@@ -255,35 +356,50 @@ void igemm_fast_kernel(GemmParams p)
             }
             soff_a = ((fy * p.dy * p.W + fx * p.dx) * p.pix_stride + c0) * 4;
         } else {
-            soff_a += BKT * 4;
+            soff_a += 64;
         }
     };
-    float ln_shift[LNF ? A_LOADS : 1], ln_s[LNF ? A_LOADS : 1], ln_q[LNF ? A_LOADS : 1];
-    auto store_tiles = [&](int buf, bool first = false) {
-        float* as = smem + buf * (BM + BN) * STRIDE;
-        float* bs = as + BM * STRIDE;
+    auto load_tiles = [&](bool live) {
+        load_half(0, live);
+        load_half(1, live);
+    };
+    float ln_shift[LNF ? A_UNITS : 1], ln_s[LNF ? A_UNITS : 1], ln_q[LNF ? A_UNITS : 1];
+    // eight floats of a row (chunks kq and 4 + kq of the slab) -> 16 bytes of each plane
+    auto put = [&](unsigned char* dst, int plane_bytes, const f32x4& lo, const f32x4& hi) {
+        uint32_t w[3][4];
+        split3(lo[0], lo[1], w[0][0], w[1][0], w[2][0]);
+        split3(lo[2], lo[3], w[0][1], w[1][1], w[2][1]);
+        split3(hi[0], hi[1], w[0][2], w[1][2], w[2][2]);
+        split3(hi[2], hi[3], w[0][3], w[1][3], w[2][3]);
+#pragma unroll
+        for (int q = 0; q < 3; ++q)
+            *reinterpret_cast<u32x4*>(dst + q * plane_bytes) = u32x4 { w[q][0], w[q][1], w[q][2], w[q][3] };
+    };
+    auto store_a = [&](int buf, bool first = false) {
         if (LNF) {
 #pragma unroll
-            for (int i = 0; i < A_LOADS; ++i) {
+            for (int i = 0; i < A_UNITS; ++i) {
                 if (first) {
-                    ln_shift[LNF ? i : 0] = ra[i][0];
+                    ln_shift[LNF ? i : 0] = ra[i][0][0];
                     ln_s[LNF ? i : 0] = 0.f;
                     ln_q[LNF ? i : 0] = 0.f;
                 }
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const float dlt = ra[i][e] - ln_shift[LNF ? i : 0];
+                for (int e = 0; e < 8; ++e) {
+                    const float dlt = ra[i][e >> 2][e & 3] - ln_shift[LNF ? i : 0];
                     ln_s[LNF ? i : 0] += dlt;
                     ln_q[LNF ? i : 0] += dlt * dlt;
                 }
             }
         }
 #pragma unroll
-        for (int i = 0; i < A_LOADS; ++i)
-            *reinterpret_cast<f32x4*>(&as[(r0 + i * RPP) * STRIDE + kq * 4]) = ra[i];
+        for (int i = 0; i < A_UNITS; ++i)
+            put(smem_raw + buf * BUF_BYTES + kq * A_BLK + (r0 + i * RPP) * 16, 4 * A_BLK, ra[i][0], ra[i][1]);
+    };
+    auto store_b = [&](int buf) {
 #pragma unroll
-        for (int i = 0; i < B_LOADS; ++i)
-            *reinterpret_cast<f32x4*>(&bs[(r0 + i * RPP) * STRIDE + kq * 4]) = rb[i];
+        for (int i = 0; i < B_UNITS; ++i)
+            put(smem_raw + buf * BUF_BYTES + A_BYTES + kq * B_BLK + (r0 + i * RPP) * 16, 4 * B_BLK, rb[i][0], rb[i][1]);
     };
 
     int tile = sk ? 0 : wg_in_xcd; // local unit index
@@ -293,75 +409,91 @@ void igemm_fast_kernel(GemmParams p)
     int m0, n0;
     int64_t c_off;
     setup(tile, m0, n0, c_off);
-    load_tiles();
+    load_tiles(true);
 
     for (;;) {
-        f32x16 acc[TM][TN];
+        // the leading products of a tile in one set of accumulators, the five small ones in a second: a result is rounded
+        // against its own size once per 16 steps of K instead of once per product
+        f32x16 acc[TM][TN], acc_lo[TM][TN];
 #pragma unroll
         for (int i = 0; i < TM; ++i)
 #pragma unroll
             for (int j = 0; j < TN; ++j)
 #pragma unroll
                 for (int e = 0; e < 16; ++e)
-                    acc[i][j][e] = 0.f;
+                    acc[i][j][e] = acc_lo[i][j][e] = 0.f;
 
-        store_tiles(0, true);
-        __syncthreads();
         const int kt_end = kt_n;
-        for (int kt = 0; kt < kt_end; ++kt) {
-            const int buf = kt & 1;
-            if (kt + 1 < kt_end)
-                load_tiles();
-            const float* as = smem + buf * (BM + BN) * STRIDE;
-            const float* bs = as + BM * STRIDE;
-            if (TM == 1 && TN == 1) {
-                // one 32 x 32 piece per wave: the fragments of the whole slab are requested from LDS before the first MFMA
-                // (read two groups at a time, the second pair of groups waited out its LDS latency with the pipe drained: the
-                // encoder's GEMMs 1 % faster this way)
-                f32x4 af[BKT / 8], bf[BKT / 8];
+        store_a(0, true);
+        store_b(0);
+        load_tiles(1 < kt_end);
+        __syncthreads();
+        bf16x8 af[2][TM][3], bf[2][TN][3];
+        auto read_frags = [&](int s, int buf) {
+            const unsigned char* as = smem_raw + buf * BUF_BYTES + (2 * s + fh) * A_BLK + (wm * WTM + fr) * 16;
+            const unsigned char* bs = smem_raw + buf * BUF_BYTES + A_BYTES + (2 * s + fh) * B_BLK + (wn * WTN + fr) * 16;
 #pragma unroll
-                for (int k8 = 0; k8 < BKT / 8; ++k8) {
-                    af[k8] = *reinterpret_cast<const f32x4*>(&as[(wm * WTM + fr) * STRIDE + k8 * 8 + fh * 4]);
-                    bf[k8] = *reinterpret_cast<const f32x4*>(&bs[(wn * WTN + fr) * STRIDE + k8 * 8 + fh * 4]);
-                }
-                __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                for (int k8 = 0; k8 < BKT / 8; ++k8)
-#pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(af[k8][e], bf[k8][e], acc[0][0], 0, 0, 0);
-            } else {
-#pragma unroll
-            for (int k8 = 0; k8 < BKT / 8; ++k8) {
-                f32x4 af[TM], bf[TN];
+            for (int q = 0; q < 3; ++q) {
 #pragma unroll
                 for (int i = 0; i < TM; ++i)
-                    af[i] = *reinterpret_cast<const f32x4*>(&as[(wm * WTM + i * 32 + fr) * STRIDE + k8 * 8 + fh * 4]);
+                    af[s][i][q] = *reinterpret_cast<const bf16x8*>(as + q * 4 * A_BLK + i * 512);
 #pragma unroll
                 for (int j = 0; j < TN; ++j)
-                    bf[j] = *reinterpret_cast<const f32x4*>(&bs[(wn * WTN + j * 32 + fr) * STRIDE + k8 * 8 + fh * 4]);
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-#pragma unroll
-                    for (int i = 0; i < TM; ++i)
-#pragma unroll
-                        for (int j = 0; j < TN; ++j)
-                            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(af[i][e], bf[j][e], acc[i][j], 0, 0, 0);
+                    bf[s][j][q] = *reinterpret_cast<const bf16x8*>(bs + q * 4 * B_BLK + j * 512);
             }
-            }
-            if (kt + 1 < kt_end)
-                store_tiles(buf ^ 1);
-            if (LNF && kt + 1 == kt_end) {
-                // Every slab has passed through store_tiles by now, so every thread has seen 4 * KT values of each of its
-                // rows.  The eight lanes that share a row (consecutive lanes, CPR = 8) merge their means and sums of
-                // squared deviations pairwise, equal counts on both sides at every step, on the VALU's lane swaps: inside
-                // quads twice, then with the mirrored lane of the row's eight, whose quad holds the other half's result.
-                // Done here, behind the last slab's MFMAs and in front of the loop's last barrier, it costs no barrier of
-                // its own.
-                static_assert(!LNF || CPR == 8, "the merge below is written for eight lanes per row");
+        };
+        auto product = [&](int s, int x, int y, f32x16(&d)[TM][TN]) {
 #pragma unroll
-                for (int i = 0; i < A_LOADS; ++i) {
-                    float cnt = 4.0f * (float)KT;
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j)
+                    d[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[s][i][x], bf[s][j][y], d[i][j], 0, 0, 0);
+        };
+        auto multiply = [&](int s) {
+            product(s, 0, 0, acc);
+            product(s, 0, 1, acc_lo);
+            product(s, 1, 0, acc_lo);
+            product(s, 1, 1, acc_lo);
+            product(s, 0, 2, acc_lo);
+            product(s, 2, 0, acc_lo);
+        };
+        // all slabs but the last: the next slab goes to LDS between the two halves of this one's products, and the one
+        // after that is requested into the registers this frees
+        for (int kt = 0; kt + 1 < kt_end; ++kt) {
+            const int buf = DB ? kt & 1 : 0;
+            if (DB) {
+                read_frags(0, buf);
+                multiply(0);
+                store_a(buf ^ 1);
+                read_frags(1, buf);
+                multiply(1);
+                store_b(buf ^ 1);
+            } else {
+                read_frags(0, 0);
+                read_frags(1, 0);
+                __syncthreads();
+                multiply(0);
+                store_a(0);
+                multiply(1);
+                store_b(0);
+            }
+            load_tiles(kt + 2 < kt_end);
+            __syncthreads();
+        }
+        {
+            const int buf = DB ? (kt_end - 1) & 1 : 0;
+            read_frags(0, buf);
+            multiply(0);
+            read_frags(1, buf);
+            multiply(1);
+            if (LNF) {
+                // Every slab has passed through store_tiles by now, so every thread has seen 8 * KT values of each of its
+                // rows.  The four lanes that share a row (a quad) merge their means and sums of
+                // squared deviations pairwise, equal counts on both sides at each step, on the VALU's lane swaps.  Done here,
+                // behind the last slab's MFMAs and in front of the barrier below, it costs no barrier of its own.
+#pragma unroll
+                for (int i = 0; i < A_UNITS; ++i) {
+                    float cnt = 8.0f * (float)KT;
                     float mean = ln_shift[LNF ? i : 0] + ln_s[LNF ? i : 0] / cnt;
                     float m2 = ln_q[LNF ? i : 0] - ln_s[LNF ? i : 0] * ln_s[LNF ? i : 0] / cnt;
                     auto merge = [&](float om, float o2) {
@@ -372,7 +504,6 @@ void igemm_fast_kernel(GemmParams p)
                     };
                     merge(dpp_move<0xB1>(mean), dpp_move<0xB1>(m2));   // quad_perm [1, 0, 3, 2]
                     merge(dpp_move<0x4E>(mean), dpp_move<0x4E>(m2));   // quad_perm [2, 3, 0, 1]
-                    merge(dpp_move<0x141>(mean), dpp_move<0x141>(m2)); // row_half_mirror
                     if (kq == 0) {
                         ln_stats[2 * (r0 + i * RPP)] = mean;
                         ln_stats[2 * (r0 + i * RPP) + 1] = 1.0f / sqrtf(fmaxf(m2, 0.f) / cnt + p.ln_eps);
@@ -381,7 +512,13 @@ void igemm_fast_kernel(GemmParams p)
             }
             __syncthreads();
         }
-
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+#pragma unroll
+                for (int e = 0; e < 16; ++e)
+                    acc[i][j][e] += acc_lo[i][j][e];
 
         // this tile's coordinates for the epilogue; the loader state moves on to the next tile
         const int em0 = m0, en0 = n0;
@@ -423,7 +560,7 @@ void igemm_fast_kernel(GemmParams p)
         const bool more = tile < unit_end;
         if (more) {
             setup(tile, m0, n0, c_off);
-            load_tiles(); // in flight while this tile is written out
+            load_tiles(true); // in flight while this tile is written out
         }
 
         if (SPLIT && su_done >= 0) {
@@ -524,6 +661,27 @@ void igemm_fast_kernel(GemmParams p)
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
             __builtin_amdgcn_wave_barrier();
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            // Inf and NaN do not survive the split (Inf - Inf in the remainders), and a value that rounds up to an infinite
+            // bf16 makes one: such elements are summed again in plain fp32.  (A band of huge finite values may come here too
+            // and finds nothing to do.)
+            float size = 0.f;
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+#pragma unroll
+                for (int e = 0; e < 16; ++e)
+                    size += fabsf(acc[i][j][e]);
+            if (__builtin_expect(__any(!(size < INFINITY)), 0)) {
+#pragma clang loop unroll(disable)
+                for (int o = lane; o < 32 * WTN; o += 64) {
+                    const int m = em0 + wm * WTM + i * 32 + o / WTN, nn = en0 + wn * WTN + o % WTN;
+                    float& v = scratch[(o / WTN) * OSTRIDE + o % WTN];
+                    if (!(fabsf(v) < INFINITY) && m < p.M && nn < p.N)
+                        v = plain_dot<CONV, DUAL>(p, tile_done / per_problem, m, nn);
+                }
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            }
             // all rows of the band are finished in registers before the first of them is stored: the wait for the
             // residual loads would otherwise also wait, pass after pass, for the store of the pass before
             f32x4 done[32 / RPS];

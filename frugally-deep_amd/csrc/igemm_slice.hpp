@@ -250,18 +250,14 @@ struct SliceForm {
 };
 constexpr SliceForm kSliceForm[kSliceForms] = { { 1, 1, 8 }, { 1, 2, 8 }, { 2, 2, 8 }, { 2, 2, 4 }, { 4, 2, 8 } };
 
-// The form for a problem, or -1 where the tiled kernel is the better one.  Both sides were timed on 483 problems (M 1-16384,
-// N 16-3072, K 32-4608, up to 6 GFLOP, GEMM and convolution, operands out of memory, launches back to back) and follow, in
-// microseconds, with w = tiles per CU rounded up:
-//     slice forms:   t0 + w (c1 + c2 (rows + columns of the tile) K / 10^4), c2 larger for a convolution's addressing
-//     64 x 64 tiles: 4.8 + w (0.44 + 4.9 K / 1000) + t (12.3 K / 1000) + min(t, 1) 5.1 K / 1000,  t = tiles / 256
-// (8-13 % rms the slice forms, 20 % the tiled ones): a workgroup costs what it pulls through its CU's path from L2, about
-// 36 cycles per KB.  By this rule the timed problems take half the time of the tiled kernel alone (geometric mean), and
-// none takes more than 5 % longer.  Below 48 columns the other side is the general kernel's narrow tile, which wins from
-// about 600 row blocks of 64 on (N = 32, K = 144-192: 20000 rows 8.2-9.7 against 6.3-7.2 us here, 50000 rows 11.0-14.5
-// against 11.1-14.0, convolutions 13.9 against 17.1).
-// Large problems are few in this sense, too, where the last column block of 64 would be half empty: N = 80, 96, 144, 160 or
-// 208 and long rows, up to 118000 rows of K = 3520 with N = 96 792 -> 687 us; 160 such problems 0.93-2.1 times, 1.33 on average.
+// The form for a problem, or -1 where the tiled kernel (its cost by tile_pick) is the better one.  The forms were timed on 483
+// problems (M 1-16384, N 16-3072, K 32-4608, up to 6 GFLOP, GEMM and convolution, operands out of memory, launches back to
+// back) and follow, in microseconds, with w = tiles per CU rounded up, to 8-13 % rms
+//     t0 + w (c1 + c2 (rows + columns of the tile) K / 10^4), c2 larger for a convolution's addressing:
+// a workgroup costs what it pulls through its CU's path from L2, about 36 cycles per KB.  Up to 32 columns the other side is the
+// general kernel's narrow tile, which wins from about 600 row blocks of 64 on (N = 32, K = 144-192: 20000 rows 8.2-9.7 against
+// 6.3-7.2 us here, 50000 rows 11.0-14.5 against 11.1-14.0, convolutions 13.9 against 17.1); between 32 and 64 columns the tiled
+// kernel's half empty 64-column tile beats it (97733 x 40 x 288 31.5 against 40.9 us, 24000 x 36 x 512 17.4 / 21.7).
 static int64_t slice_tiles(int M, int N, int bm, int bn) { return (int64_t)((M + bm - 1) / bm) * ((N + bn - 1) / bn); }
 static float slice_rounds(int64_t tiles) { return (float)((tiles + 255) / 256); }
 static float slice_cost(int form, bool conv, int M, int N, int K)
@@ -273,26 +269,20 @@ static float slice_cost(int form, bool conv, int M, int N, int K)
     const int bm = 16 * kSliceForm[form].tm, bn = 16 * kSliceForm[form].tn;
     return kCost[form][0] + slice_rounds(slice_tiles(M, N, bm, bn)) * (kCost[form][1] + kCost[form][conv ? 3 : 2] * 1e-4f * (bm + bn) * K);
 }
-static float slice_tiled_cost(int M, int N, int K)
-{
-    const int64_t t64 = slice_tiles(M, N, 64, 64);
-    const float k = 1e-3f * K, t = (float)t64 / 256.f;
-    return 4.8f + slice_rounds(t64) * (0.44f + 4.9f * k) + 12.3f * t * k + 5.1f * std::min(t, 1.f) * k;
-}
 // whether a launch of this form stays below the 2^32 threads a grid can have
 static bool slice_fits(int form, int M, int N)
 {
     const SliceForm& f = kSliceForm[form];
     return slice_tiles(M, N, 16 * f.tm, 16 * f.tn) * 64 * f.nw < (1LL << 32);
 }
-static int slice_pick(bool conv, int M, int N, int K)
+static int slice_pick(bool conv, int M, int N, int K, float tiled_cost)
 {
     const int64_t t64 = slice_tiles(M, N, 64, 64);
-    const bool narrow = N < 48;
+    const bool narrow = N <= 32;
     if (narrow && t64 > 512)
         return -1;
     int best = -1;
-    float best_cost = narrow ? 1e30f : (t64 <= 256 ? 0.85f : 0.75f) * slice_tiled_cost(M, N, K); // past a round of tiles operands re-read cost the neighbours, too
+    float best_cost = narrow ? 1e30f : (t64 <= 256 ? 0.95f : 0.85f) * tiled_cost; // past a round of tiles operands re-read cost the neighbours, too
     for (int i = 0; i < kSliceForms; ++i) {
         const float cost = slice_cost(i, conv, M, N, K);
         if (cost < best_cost && slice_fits(i, M, N)) {

@@ -1,0 +1,105 @@
+"""The tiled GEMM / convolution kernel (configurations 13-18, cut along K in several ways): fp32 operands as exact sums of three
+bf16 values on the bf16 matrix instructions.
+
+Error bound: every 16 steps of K round the main sum once (at most 2^-24 of the running sum, itself at most the sum of the
+magnitudes S), the small products' sum and the final add a few times more, the products left out are below 3 * 2^-26 S; twice
+that is allowed: (K / 16 + 8) 2^-23 S for an element.  For the 2-norm, where roundings average out, twice what operands of
+unit variance show against 64 bits (6e-9 sqrt(K))."""
+import zlib
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+TILES = [-1, 13, 14, 15, 16, 18, 215, 815, 315 + 10000, 20013, 20015]
+
+
+def forced(fdx, tile, f):
+    fdx.lib.fdx_debug_force_tile(tile)
+    try:
+        return f()
+    finally:
+        fdx.lib.fdx_debug_force_tile(-1)
+
+
+def check(got, a, w, extra=0.0):
+    a, w = a.astype(np.float64), w.astype(np.float64)
+    want, size, k = a @ w.T + extra, np.abs(a) @ np.abs(w).T + np.abs(extra), a.shape[1]
+    err = np.abs(got - want)
+    assert (err <= (k / 16 + 8) * 2.0 ** -23 * size).all(), (err / size).max()
+    assert np.linalg.norm(err) <= (1.2e-8 * np.sqrt(k) + 1.2e-7) * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("tile", TILES)
+@pytest.mark.parametrize("m,n,k", [(1, 36, 16), (63, 64, 48), (129, 132, 32), (255, 100, 272), (257, 260, 512), (640, 64, 2320)])
+def test_gemm_edges(fdx, m, n, k, tile):
+    print("split products", m, n, k, tile, flush=True)
+    r = np.random.default_rng(zlib.crc32(repr((m, n, k)).encode()))
+    a, w = r.standard_normal((m, k)).astype(np.float32), (r.standard_normal((n, k)) / np.sqrt(k)).astype(np.float32)
+    b, res = r.standard_normal(n).astype(np.float32), r.standard_normal((m, n)).astype(np.float32)
+    plain, full, again = forced(fdx, tile, lambda: (fdx.gemm(a, w), fdx.gemm(a, w, b, residual=res), fdx.gemm(a, w, b, residual=res)))
+    check(plain, a, w)
+    check(full, a, w, (b + res).astype(np.float64))
+    assert np.array_equal(full, again)
+    # the split does not depend on the operands' scale
+    scaled = forced(fdx, tile, lambda: fdx.gemm(a * np.float32(2.0 ** 60), w * np.float32(2.0 ** -50)))
+    assert np.array_equal(scaled, plain * np.float32(2.0 ** 10))
+
+
+def special(a, w):
+    a[1, 3], a[2, -1], a[3, 0], a[4, 5] = np.inf, -np.inf, np.nan, 3.4e38   # 3.4e38 rounds up to an infinite bf16
+    a[5, 2], a[5, -2] = np.inf, -np.inf
+    w[0, 1], w[2, -3] = np.inf, np.nan
+    w[3, :] = 0                                                            # 0 * Inf
+    w[4, 5] = 0.25
+
+
+def check_special(got, a, w):
+    with np.errstate(all="ignore"):
+        want = a.astype(np.float64) @ w.astype(np.float64).T
+        want = np.where(np.abs(want) > np.finfo(np.float32).max, np.sign(want) * np.inf, want)
+    finite = np.isfinite(want)
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(got[~finite & ~np.isnan(want)], want[~finite & ~np.isnan(want)])
+    assert np.allclose(got[finite], want[finite], rtol=1e-4, atol=1e-4)
+
+
+@pytest.mark.parametrize("tile", TILES)
+def test_infinities_and_nan(fdx, tile):
+    print("special operands", tile, flush=True)
+    r = np.random.default_rng(5)
+    m, n, k = 140, 68, 336
+    a, w = r.standard_normal((m, k)).astype(np.float32), (r.standard_normal((n, k)) / 18).astype(np.float32)
+    special(a, w)
+    check_special(forced(fdx, tile, lambda: fdx.gemm(a, w)), a, w)
+    # a 3x3 convolution over a map of one row: the same products with zero taps above and below
+    x = a.reshape(1, m, 1, k).transpose(0, 2, 1, 3).copy()
+    wc = np.zeros((n, 3, 3, k), np.float32)
+    wc[:, 1, 1] = w
+    got = forced(fdx, tile, lambda: fdx.conv2d(x, wc, None, padding="same"))[0, 0]
+    with np.errstate(all="ignore"):
+        want = a.astype(np.float64) @ w.astype(np.float64).T
+    far = np.ones(m, bool)
+    far[:8] = False                       # zero taps of the neighbours meet infinities there: only positions past them compare
+    far_w = np.isfinite(w).all(1)
+    assert np.allclose(got[far][:, far_w], want[far][:, far_w], rtol=1e-4, atol=1e-4)
+    assert np.isnan(got[:, 2]).all() and not np.isfinite(got[far][:, 0]).any()
+
+
+def test_infinities_two_sources(fdx, modelgen):
+    """The sum of two 1x1 convolutions as one GEMM: an infinite pixel of either map gives that pixel's infinities and nothing else."""
+    b = modelgen.Builder("two_src", 7)
+    x = b.input((9, 7, 32), "img")
+    y = b.conv2d(x, 16, 1, "c1", strides=2, use_bias=False)
+    z = b.conv2d(y, 64, 1, "c3", bias_std=0.2)
+    sc = b.conv2d(x, 64, 1, "sc", strides=2, bias_std=0.1)
+    spec = b.finish([b.add([sc, z], "sum")])
+    xs = np.random.default_rng(3).standard_normal((4, 9, 7, 32)).astype(np.float32)
+    bad = xs.copy()
+    bad[2, 4, 2, 5] = np.inf
+    print("two sources", flush=True)
+    model = fdx.Model(modelgen.dumps(spec), verify=False)
+    for tile in (-1, 13, 14, 15, 16, 18):
+        want, got = forced(fdx, tile, lambda: (model.predict([xs])[0], model.predict([bad])[0]))
+        hit = np.zeros(want.shape[:3], bool)
+        hit[2, 2, 1] = True
+        assert np.array_equal(got[~hit], want[~hit]) and not np.isfinite(got[hit]).any()

@@ -12,6 +12,7 @@
 #include <cstdint>
 #include <cstdlib>
 
+#include "bf16_split.hpp"
 #include "common.hpp"
 
 namespace fdx {
@@ -100,6 +101,7 @@ __global__ __launch_bounds__(256) void mha_decode_kernel(const float* __restrict
 
 // ---- fused prefill attention: scores, softmax and P V in one pass, nothing but the output written --------------------
 //
+// Depth 128; depths 32 and 64 take flash_split_kernel below (its operands of depth 128 would not fit two waves per SIMD).
 // One workgroup = 128 query rows of one (sequence, head), one wave = 32 of them; keys / values pass through LDS in
 // tiles of 64.  The products are taken transposed on the 32x32x2 fp32 MFMA: S^T = K Q^T puts a query on a lane
 // (column) and keys on the accumulator registers, so the running maximum, the running sum and the rescaling of the
@@ -279,6 +281,264 @@ __global__ __launch_bounds__(256) void flash_prefill_kernel(FlashParams p)
     }
 }
 
+// The same recurrence with both products on the bf16 matrix instructions, every fp32 operand (queries, keys, values,
+// probabilities) as the exact sum of three bf16 values and six of the nine partial products taken (see igemm_fast.hpp): the
+// fp32 MFMA is what bounds the kernel above (its products alone are 8192 of a 64-key tile's cycles at depth 64; here 3072,
+// beside about 2600 of vector instructions).  32 sequences of 256 tokens, 8 heads of 64: 54.5 -> 37.9 us a
+// launch; error against 64-bit results (2-norm, unit operands) 3.3e-7 -> 1.4e-7.
+//  * Keys and values are split on their way into LDS, once for the workgroup's 128 queries.  LDS holds blocks of eight
+//    contraction indices: keys [plane][depth block][key][16 bytes], values [plane][key block][depth][16 bytes].
+//  * Depth block 4 g + l holds depths 32 g + 4 l .. + 3 and 32 g + 16 + 4 l .. + 3, the two 16-byte chunks that lane l of four
+//    fetches of a key row; a key block holds the eight keys whose probabilities one lane half has in eight consecutive
+//    accumulator registers: 16 s + 4 half + {0 .. 3, 8 .. 11}.
+//  * Scores and a tile's share of the output start from zero, small products first, and meet the running output in one
+//    multiply-add (its rescaling), so sums are rounded at their own size a few times per tile.
+//  * The scale of the scores is taken to base two, so a probability is one subtraction and one hardware exponential.
+//  * A query whose result is not finite (infinite or NaN operands do not survive the split) is taken again in plain fp32.
+template <int D>
+__global__ __launch_bounds__(256, 2) void flash_split_kernel(FlashParams p)
+{
+    constexpr int KB = D / 8;                // depth blocks
+    constexpr int KBLK = 64 * 16 + 32, VBLK = D * 16 + 32; // bytes of a block: 64 keys / D depths, offset against each other
+    constexpr int STEPS = D / 16;            // MFMA steps over the depth
+    constexpr int KL = D / 32;               // pairs of 16-byte key loads per thread
+    constexpr int VD = D / 32;               // depths per thread when values are staged
+    static_assert(D == 32 || D == 64, "depths whose operands fit two waves per SIMD");
+    __shared__ __attribute__((aligned(16))) unsigned char ks[3 * KB * KBLK];
+    __shared__ __attribute__((aligned(16))) unsigned char vs[3 * 8 * VBLK];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int c = lane & 31, half = lane >> 5;
+    const int b = blockIdx.y / p.heads, h = blockIdx.y % p.heads;
+    const int q_first = blockIdx.x * 128;
+    const int query = q_first + wave * 32 + c;
+    const bool q_ok = query < p.t;
+    const int shift = p.s - p.t; // causal: query i sees keys 0 .. i + shift
+    const float* qrow = p.q + (int64_t)b * p.q_batch + (int64_t)(q_ok ? query : 0) * p.ldq + h * D;
+
+    u32x4 qf[STEPS][3];
+#pragma unroll
+    for (int u = 0; u < STEPS; ++u) { // depth block 2 u + half
+        const int blk = 2 * u + half, d0 = 32 * (blk >> 2) + 4 * (blk & 3);
+        f32x4 lo = { 0.f, 0.f, 0.f, 0.f }, hi = lo;
+        if (q_ok) {
+            lo = *reinterpret_cast<const f32x4*>(qrow + d0);
+            hi = *reinterpret_cast<const f32x4*>(qrow + d0 + 16);
+        }
+        const float x[8] = { lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3] };
+        split3x8(x, qf[u]);
+    }
+
+    int s_end = p.s;
+    if (p.causal) {
+        const int q_last = (q_first + 128 < p.t ? q_first + 128 : p.t) - 1;
+        s_end = q_last + shift + 1 < p.s ? q_last + shift + 1 : p.s;
+    }
+    const int tiles = (s_end + 63) / 64;
+    const int wave_q_first = q_first + wave * 32, wave_q_last = wave_q_first + 31;
+
+    const float* kbase = p.k + (int64_t)b * p.k_batch + h * D;
+    const float* vbase = p.v + (int64_t)b * p.v_batch + h * D;
+    // keys: lane l of four has chunks l and 4 + l of each 32-float run of its key; values: VD depths of one block's eight keys
+    const int krow = tid >> 2, kl = tid & 3;
+    const int vblk = tid >> 5, vd = (tid & 31) * VD;
+    f32x4 kst[KL][2];
+    float vst[8][VD];
+    auto fetch = [&](int j0) {
+#pragma unroll
+        for (int g = 0; g < KL; ++g)
+#pragma unroll
+            for (int e = 0; e < 2; ++e)
+                kst[g][e] = j0 + krow < p.s ? *reinterpret_cast<const f32x4*>(kbase + (int64_t)(j0 + krow) * p.ldk + 32 * g + 16 * e + 4 * kl)
+                                            : f32x4 { 0.f, 0.f, 0.f, 0.f };
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const int key = j0 + 16 * (vblk >> 1) + 4 * (vblk & 1) + 8 * (j >> 2) + (j & 3);
+#pragma unroll
+            for (int d = 0; d < VD; ++d)
+                vst[j][d] = key < p.s ? vbase[(int64_t)key * p.ldv + vd + d] : 0.f;
+        }
+    };
+    auto stage = [&]() {
+#pragma unroll
+        for (int g = 0; g < KL; ++g) {
+            const float x[8] = { kst[g][0][0], kst[g][0][1], kst[g][0][2], kst[g][0][3], kst[g][1][0], kst[g][1][1], kst[g][1][2], kst[g][1][3] };
+            u32x4 planes[3];
+            split3x8(x, planes);
+#pragma unroll
+            for (int q = 0; q < 3; ++q)
+                *reinterpret_cast<u32x4*>(&ks[(q * KB + 4 * g + kl) * KBLK + krow * 16]) = planes[q];
+        }
+#pragma unroll
+        for (int d = 0; d < VD; ++d) {
+            const float x[8] = { vst[0][d], vst[1][d], vst[2][d], vst[3][d], vst[4][d], vst[5][d], vst[6][d], vst[7][d] };
+            u32x4 planes[3];
+            split3x8(x, planes);
+#pragma unroll
+            for (int q = 0; q < 3; ++q)
+                *reinterpret_cast<u32x4*>(&vs[(q * 8 + vblk) * VBLK + (vd + d) * 16]) = planes[q];
+        }
+    };
+    auto mfma = [](const u32x4& a, const u32x4& bb, const f32x16& acc) {
+        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, bb), acc, 0, 0, 0);
+    };
+    constexpr f32x16 kZero = { 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f };
+
+    f32x16 oacc[D / 32];
+#pragma unroll
+    for (int d = 0; d < D / 32; ++d)
+        oacc[d] = kZero;
+    const float scale2 = p.scale * 1.44269504088896340736f;
+    const int key_limit = p.causal ? (query + shift < p.s - 1 ? query + shift : p.s - 1) : p.s - 1;
+    float m_run = -INFINITY, l_run = 0.f; // maximum in units of log2
+
+    if (tiles > 0)
+        fetch(0);
+    for (int tile = 0; tile < tiles; ++tile) {
+        const int j0 = tile * 64;
+        __syncthreads(); // every wave is done with the previous tile
+        stage();
+        __syncthreads();
+        if (tile + 1 < tiles)
+            fetch(j0 + 64); // in flight while this tile is worked on
+        if (p.causal && j0 > wave_q_last + shift)
+            continue; // nothing in this tile is visible to any of this wave's queries (wave-uniform)
+
+        // S^T tile: 64 keys x 32 queries
+        f32x16 sacc[2];
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb) {
+            f32x16 lo = kZero, hi = kZero;
+#pragma unroll
+            for (int u = 0; u < STEPS; ++u) {
+                u32x4 kf[3];
+#pragma unroll
+                for (int q = 0; q < 3; ++q)
+                    kf[q] = *reinterpret_cast<const u32x4*>(&ks[(q * KB + 2 * u + half) * KBLK + (kb * 32 + c) * 16]);
+                hi = mfma(kf[0], qf[u][0], hi);
+                lo = mfma(kf[2], qf[u][0], lo);
+                lo = mfma(kf[1], qf[u][1], lo);
+                lo = mfma(kf[0], qf[u][2], lo);
+                lo = mfma(kf[1], qf[u][0], lo);
+                lo = mfma(kf[0], qf[u][1], lo);
+            }
+#pragma unroll
+            for (int e = 0; e < 16; ++e)
+                sacc[kb][e] = (hi[e] + lo[e]) * scale2;
+        }
+        // mask where a query of this wave does not see the whole tile, running maximum
+        if (j0 + 64 > p.s || (p.causal && j0 + 63 > wave_q_first + shift)) {
+#pragma unroll
+            for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+                for (int e = 0; e < 16; ++e)
+                    if (j0 + kb * 32 + 8 * (e >> 2) + 4 * half + (e & 3) > key_limit)
+                        sacc[kb][e] = -INFINITY;
+        }
+        float mx = -INFINITY;
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+            for (int e = 0; e < 16; ++e)
+                mx = fmaxf(mx, sacc[kb][e]);
+        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        const float m_new = fmaxf(m_run, mx);
+        // a query that has seen no key yet (rows past the end of the sequence) keeps zeros instead of NaNs
+        const float m_use = m_new == -INFINITY ? 0.f : m_new;
+        const float corr = __builtin_amdgcn_exp2f(m_run - m_use);
+        float rs = 0.f;
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                sacc[kb][e] = __builtin_amdgcn_exp2f(sacc[kb][e] - m_use);
+                rs += sacc[kb][e];
+            }
+        rs += __shfl_xor(rs, 32, 64);
+        l_run = l_run * corr + rs;
+        m_run = m_new;
+        // O^T = O^T corr + V^T P^T
+        f32x16 hi[D / 32], lo[D / 32];
+#pragma unroll
+        for (int d = 0; d < D / 32; ++d)
+            hi[d] = lo[d] = kZero;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) { // keys of block 2 u + half: registers 8 (u % 2) .. + 7 of half tile u / 2
+            float x[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                x[j] = sacc[u >> 1][8 * (u & 1) + j];
+            u32x4 pf[3];
+            split3x8(x, pf);
+#pragma unroll
+            for (int d = 0; d < D / 32; ++d) {
+                u32x4 vf[3];
+#pragma unroll
+                for (int q = 0; q < 3; ++q)
+                    vf[q] = *reinterpret_cast<const u32x4*>(&vs[(q * 8 + 2 * u + half) * VBLK + (d * 32 + c) * 16]);
+                hi[d] = mfma(vf[0], pf[0], hi[d]);
+                lo[d] = mfma(vf[2], pf[0], lo[d]);
+                lo[d] = mfma(vf[1], pf[1], lo[d]);
+                lo[d] = mfma(vf[0], pf[2], lo[d]);
+                lo[d] = mfma(vf[1], pf[0], lo[d]);
+                lo[d] = mfma(vf[0], pf[1], lo[d]);
+            }
+        }
+#pragma unroll
+        for (int d = 0; d < D / 32; ++d)
+#pragma unroll
+            for (int e = 0; e < 16; ++e)
+                oacc[d][e] = oacc[d][e] * corr + (hi[d][e] + lo[d][e]);
+    }
+
+    float size = l_run;
+#pragma unroll
+    for (int d = 0; d < D / 32; ++d)
+#pragma unroll
+        for (int e = 0; e < 16; ++e)
+            size += fabsf(oacc[d][e]);
+    if (__builtin_expect(q_ok && !(size < INFINITY), 0)) {
+        // both halves of the lane pair may not come here together, so each walks the keys for itself
+        auto score = [&](int key) {
+            const float* krow_p = kbase + (int64_t)key * p.ldk;
+            float s = 0.f;
+#pragma clang loop unroll(disable)
+            for (int d = 0; d < D; ++d)
+                s = fmaf(krow_p[d], qrow[d], s);
+            return s * p.scale;
+        };
+        float m = -INFINITY;
+        for (int key = 0; key <= key_limit; ++key)
+            m = fmaxf(m, score(key));
+        m = m == -INFINITY ? 0.f : m;
+        l_run = 0.f;
+#pragma unroll
+        for (int d = 0; d < D / 32; ++d)
+            oacc[d] = kZero;
+#pragma clang loop unroll(disable)
+        for (int key = 0; key <= key_limit; ++key) {
+            const float pv = __expf(score(key) - m);
+            l_run += pv;
+            const float* vrow = vbase + (int64_t)key * p.ldv + 4 * half;
+#pragma unroll
+            for (int d = 0; d < D / 32; ++d)
+#pragma unroll
+                for (int e = 0; e < 16; ++e)
+                    oacc[d][e] = fmaf(pv, vrow[32 * d + 8 * (e >> 2) + (e & 3)], oacc[d][e]);
+        }
+    }
+    if (q_ok) {
+        const float inv = l_run > 0.f ? 1.0f / l_run : 0.f;
+        float* orow = p.out + (int64_t)b * p.o_batch + (int64_t)query * p.ldo + h * D + 4 * half;
+#pragma unroll
+        for (int d = 0; d < D / 32; ++d)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const f32x4 o = { oacc[d][4 * g] * inv, oacc[d][4 * g + 1] * inv, oacc[d][4 * g + 2] * inv, oacc[d][4 * g + 3] * inv };
+                *reinterpret_cast<f32x4*>(orow + 32 * d + 8 * g) = o;
+            }
+    }
+}
+
 // The same products for launches with few queries in flight: one workgroup = 32 query rows of one (sequence, head), its
 // four waves take every fourth block of 32 keys, each with a running maximum, sum and output of its own, and meet once at
 // the end.  What bounds a short launch of the kernel above is one wave's serial walk over the keys (a block of 32 keys
@@ -450,7 +710,8 @@ __global__ __launch_bounds__(256) void flash_keysplit_kernel(FlashParams p)
 // 128 (one workgroup per CU by LDS) as long as every CU takes one.  Beyond, a workgroup here reads keys and values for 32
 // queries instead of 128, which shows as soon as CUs take turns: with one workgroup per CU 1.2 to 2.7 times faster; up to
 // 448 with more than one 64-key tile 1.1 to 1.7 times (two keys' blocks only, 384 workgroups: 9.6 against 8.2 us); from 512
-// on 0.6 to 1.3 times.
+// on 0.6 to 1.3 times.  Against the split form at depths 32 and 64 (110 problems) the line lies in the same place: 1.0 to 1.9 times
+// faster below it, 0.97 to 1.05 above.
 static bool keysplit_better(const FlashParams& p, int batch, int d)
 {
     const int64_t groups = (int64_t)((p.t + 31) / 32) * batch * p.heads;
@@ -465,7 +726,10 @@ static void flash_launch(const FlashParams& p, int batch)
         return;
     }
     const dim3 grid((unsigned)((p.t + 127) / 128), (unsigned)(batch * p.heads));
-    hipLaunchKernelGGL((flash_prefill_kernel<DK, DV>), grid, dim3(256), 0, stream(), p);
+    if constexpr (DK == DV && DK <= 64)
+        hipLaunchKernelGGL(flash_split_kernel<DK>, grid, dim3(256), 0, stream(), p);
+    else
+        hipLaunchKernelGGL((flash_prefill_kernel<DK, DV>), grid, dim3(256), 0, stream(), p);
 }
 
 static bool flash_enabled()

@@ -49,27 +49,6 @@
 //    whole tiles and the beginning of another; the (at most two) partial tiles go through the
 //    same workspace / ticket / ordered-sum path, with the number of contributors of a tile
 //    and their workspace slots computed from the cut points.
-typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef float f32x2 __attribute__((ext_vector_type(2)));
-
-__device__ __forceinline__ uint32_t bf16_pair(float a, float b)
-{
-    return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2 { a, b }), bf16x2));
-}
-// Two floats as three pairs of bf16 that add up to them exactly (below 2^-110 the last bits fall under bf16's subnormals).
-__device__ __forceinline__ void split3(float a, float b, uint32_t& p0, uint32_t& p1, uint32_t& p2)
-{
-    p0 = bf16_pair(a, b);
-    a -= __builtin_bit_cast(float, p0 << 16);
-    b -= __builtin_bit_cast(float, p0 & 0xffff0000u);
-    p1 = bf16_pair(a, b);
-    a -= __builtin_bit_cast(float, p1 << 16);
-    b -= __builtin_bit_cast(float, p1 & 0xffff0000u);
-    p2 = bf16_pair(a, b);
-}
-
 // LDS slabs per workgroup and waves per SIMD (the register budget) of a tile.
 constexpr int split_tile_buffers(int bm, int bn, int waves_m, int waves_n)
 {
@@ -366,14 +345,12 @@ void igemm_fast_kernel(GemmParams p)
     float ln_shift[LNF ? A_UNITS : 1], ln_s[LNF ? A_UNITS : 1], ln_q[LNF ? A_UNITS : 1];
     // eight floats of a row (chunks kq and 4 + kq of the slab) -> 16 bytes of each plane
     auto put = [&](unsigned char* dst, int plane_bytes, const f32x4& lo, const f32x4& hi) {
-        uint32_t w[3][4];
-        split3(lo[0], lo[1], w[0][0], w[1][0], w[2][0]);
-        split3(lo[2], lo[3], w[0][1], w[1][1], w[2][1]);
-        split3(hi[0], hi[1], w[0][2], w[1][2], w[2][2]);
-        split3(hi[2], hi[3], w[0][3], w[1][3], w[2][3]);
+        const float x[8] = { lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3] };
+        u32x4 planes[3];
+        split3x8(x, planes);
 #pragma unroll
         for (int q = 0; q < 3; ++q)
-            *reinterpret_cast<u32x4*>(dst + q * plane_bytes) = u32x4 { w[q][0], w[q][1], w[q][2], w[q][3] };
+            *reinterpret_cast<u32x4*>(dst + q * plane_bytes) = planes[q];
     };
     auto store_a = [&](int buf, bool first = false) {
         if (LNF) {

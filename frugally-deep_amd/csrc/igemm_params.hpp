@@ -2,6 +2,7 @@
 #pragma once
 #include <cstring>
 #include <functional>
+#include "bf16_split.hpp"
 #include "common.hpp"
 
 namespace fdx {

@@ -502,12 +502,13 @@ static bool launch_fast(int cfg, int splits, int mode, const GemmParams& q0, boo
     return ok;
 }
 
-// The closed rule of the fast kernel: which tile, and whether K is cut.  Costs fitted to 240 timed problems (M 200-200000,
-// N 48-3200, K 32-5000, 0.2-40 GFLOP, two thirds GEMM, a third convolutions; rms 5-8 %); by them 240 others of the same ranges take
-// 4 % longer than the fastest of all forms (20 % in the worst case).
+// The closed rule of the fast kernel: which tile, and whether K is cut.  Costs fitted to 500 timed problems (M 200-200000,
+// N 16-3200, K 32-5000, 0.2-40 GFLOP, two thirds GEMM, a third convolutions; rms 5-8 %); the choice takes 2 % longer than the
+// fastest of all forms (problems left out of the fit).
 //     whole tiles    t0 + w (e + a k) + r (f + b k) + c k t + g k min(t, 1) + d k w (convolution) + io
-//     K ranges       the same on S times the tiles and a range's k, plus 0.9 per range and 0.75 per MB of partial tiles
-//     stream-K       11 + 44 k per stretch + 2.2 per contributor of a tile + 1.7 t + io
+//     K ranges       the same on S times the tiles and a range's k, plus 0.85 per range and 1.1 per MB of partial tiles
+//     stream-K       5 + 38 k t + 3.8 contributors of a tile + 6.8 t
+//     hybrid         whole rounds and a cut last one, a sum over both (128 x 128 tiles, one workgroup per CU)
 // in microseconds, with k = K / 1000 in whole slabs, t = tiles (or ranges) / CUs, w = t rounded up, r = rounds of the workgroups
 // that are resident, io = the floats read of A, of the residual and written, per million.
 struct TileCost {
@@ -515,11 +516,11 @@ struct TileCost {
     float t0, e, a, f, b, c, g, d, io;
 };
 static const TileCost kTileCost[] = {
-    { 13, 256, 1.90f, 0.f, 33.1f, 2.97f, 0.f, 5.54f, 0.f, 2.72f, 0.194f },
-    { 14, 512, 2.22f, 0.98f, 10.9f, 0.73f, 17.9f, 1.65f, 0.f, 2.75f, 0.195f },
-    { 15, 768, 1.84f, 0.76f, 5.15f, 0.f, 15.0f, 1.50f, 0.f, 1.08f, 0.152f },
-    { 16, 512, 3.47f, 2.09f, 19.9f, 0.90f, 19.5f, 3.38f, 0.f, 6.64f, 0.320f },
-    { 18, 256, 1.02f, 0.f, 54.5f, 5.86f, 0.f, 8.00f, 0.f, 5.93f, 0.279f },
+    { 13, 256, 1.72f, 0.f, 26.7f, 3.49f, 0.f, 8.22f, 0.f, 4.25f, 0.153f },
+    { 14, 512, 2.41f, 0.58f, 11.9f, 1.46f, 13.5f, 3.18f, 0.f, 1.51f, 0.176f },
+    { 15, 768, 2.48f, 0.51f, 6.05f, 0.17f, 11.6f, 2.44f, 0.f, 0.76f, 0.153f },
+    { 16, 512, 3.82f, 1.30f, 19.4f, 1.63f, 19.2f, 4.11f, 0.f, 7.21f, 0.364f },
+    { 18, 256, 1.16f, 0.f, 54.1f, 5.83f, 0.f, 10.8f, 0.f, 6.07f, 0.254f },
 };
 static float tile_cost(const TileCost& c, bool conv, int64_t units, float k, float io)
 {
@@ -550,18 +551,25 @@ static TileChoice tile_pick(bool conv, int M, int N, int K, int64_t a_floats, bo
     if (!cuts)
         return best;
     // A cut costs more than its own time (partial tiles through memory; stretches read operands at a K phase of their own, so
-    // that neighbours do not share them in L2): handicaps of 4 and 3 %.
+    // that neighbours do not share them in L2): handicaps of 2 to 4 %.
     const int64_t t64 = tiles(15);
-    static const TileCost kRange = { 15, 768, 0.71f, 0.18f, 6.22f, 2.49f, 14.1f, 1.21f, 0.f, 1.61f, 0.02f };
+    static const TileCost kRange = { 15, 768, 0.51f, 0.f, 7.04f, 2.76f, 11.3f, 0.47f, 0.24f, 1.17f, 0.063f };
     for (int S : { 2, 3, 4, 6, 8 })
         if (t64 <= 768 && slabs >= 2 * S)
-            consider(15, S, 0, tile_cost(kRange, conv, t64 * S, (float)((slabs + S - 1) / S) * (kSlab * 1e-3f), io) + 0.91f * S
-                    + 0.755f * (float)(t64 * S) * (64 * 64 * 1e-6f), 1.04f);
+            consider(15, S, 0, tile_cost(kRange, conv, t64 * S, (float)((slabs + S - 1) / S) * (kSlab * 1e-3f), io) + 0.85f * S
+                    + 1.09f * (float)(t64 * S) * (64 * 64 * 1e-6f), 1.04f);
     const int64_t t128 = tiles(13);
-    if (t128 >= 86 && t128 <= 512 && K >= 256) {
-        const float stretch = (float)(t128 * slabs) / (float)std::min<int64_t>(256, t128 * slabs);
-        consider(13, 0, 2, 11.1f + 44.4f * stretch * (kSlab * 1e-3f) + 0.49f * io + 2.21f * 256.f / (float)t128 + 1.74f * (float)t128 / 256.f, 1.03f);
-    }
+    const float t = (float)t128 / 256.f;
+    if (t128 >= 86 && t128 <= 512 && K >= 256)
+        consider(13, 0, 2, 4.96f + (conv ? 39.f : 37.9f) * k * t + 3.76f / t + 6.75f * t, 1.03f);
+    if (t128 <= 1024 && t128 % 256 != 0)
+        for (int S : { 2, 3, 4 })
+            if (slabs >= 4 * S) {
+                const int64_t whole = t128 / 256, units = (t128 % 256) * S, w = (units + 255) / 256;
+                const float ks = (float)((slabs + S - 1) / S) * (kSlab * 1e-3f);
+                consider(13, S, 1, (float)whole * (4.56f + 27.1f * k) + (float)w * (7.43f + 27.4f * ks)
+                        + (conv ? 2.82f * ((float)whole * k + (float)w * ks) : 0.f) + 9.87f * k * t + 0.135f * (float)units * (128 * 128 * 1e-6f) + 1.07f * S, 1.02f);
+            }
     return best;
 }
 

@@ -391,9 +391,17 @@ static bool split_prepare()
 // tiles of 13, 14, 15 and 13 and stand for them).
 static int canonical_tile(int cfg) { return cfg >= 10 && cfg <= 12 ? cfg + 3 : cfg == 17 ? 13 : cfg; }
 constexpr int kSlab = 32;
+// 23, 24, 28: the tiles of 13, 14, 18 in the halo form of convolutions (see HALO in igemm_fast.hpp)
+constexpr int kHaloCfg = 10;
+static bool halo_cfg(int cfg) { return cfg == 23 || cfg == 24 || cfg == 28; }
+static bool halo_ok(const GemmParams& p, bool conv)
+{
+    return conv && p.sy == 1 && p.sx == 1 && p.OH == p.H && p.OW == p.W && p.pix_stride == p.Cin && p.Cin % kSlab == 0
+        && p.kh * p.kw >= 2 && p.kh * p.kw <= 32 && (int64_t)(p.kh - 1) * p.dy * p.W + (int64_t)(p.kw - 1) * p.dx <= kHaloSpan;
+}
 static void tile_of(int cfg, int& bm, int& bn)
 {
-    switch (canonical_tile(cfg)) {
+    switch (canonical_tile(halo_cfg(cfg) ? cfg - kHaloCfg : cfg)) {
     case 14: bm = 128; bn = 64; break;
     case 15: bm = 64; bn = 64; break;
     case 18: bm = 256; bn = 128; break;
@@ -490,6 +498,24 @@ static bool launch_fast(int cfg, int splits, int mode, const GemmParams& q0, boo
         }
         return true;
     }
+    if (halo_cfg(cfg)) {
+#define FDX_HALO(BM_, BN_, WM_, WN_)                                                                                           \
+    {                                                                                                                          \
+        constexpr int nt = 64 * WM_ * WN_;                                                                                     \
+        const int tiles = ((q.M + BM_ - 1) / BM_) * ((q.N + BN_ - 1) / BN_) * batch;                                           \
+        if (splits > 1)                                                                                                        \
+            ok = launch_split(igemm_fast_kernel<BM_, BN_, WM_, WN_, true, true, false, false, false, false, true>, tiles, splits, mode, cfg, q, s, nt); \
+        else                                                                                                                   \
+            launch_persistent(igemm_fast_kernel<BM_, BN_, WM_, WN_, true, false, false, false, false, false, true>, tiles, q, s, nt, BM_, BN_); \
+    }
+        switch (cfg) {
+        case 23: FDX_HALO(128, 128, 4, 2) break;
+        case 24: FDX_HALO(128, 64, 2, 2) break;
+        default: FDX_HALO(256, 128, 4, 2) break;
+        }
+#undef FDX_HALO
+        return ok;
+    }
     switch (canonical_tile(cfg)) {
     case 13: FDX_FAST(128, 128, 4, 2) break;
     case 14: FDX_FAST(128, 64, 2, 2) break;
@@ -509,6 +535,7 @@ static bool launch_fast(int cfg, int splits, int mode, const GemmParams& q0, boo
 //     K ranges       the same on S times the tiles and a range's k, plus 0.85 per range and 1.1 per MB of partial tiles
 //     stream-K       5 + 38 k t + 3.8 contributors of a tile + 6.8 t
 //     hybrid         whole rounds and a cut last one, a sum over both (128 x 128 tiles, one workgroup per CU)
+// and the same for the halo form (220 3x3 convolutions of 0.1-25 GFLOP on maps of 6 to 62 pixels, rms 2-4 %).
 // in microseconds, with k = K / 1000 in whole slabs, t = tiles (or ranges) / CUs, w = t rounded up, r = rounds of the workgroups
 // that are resident, io = the floats read of A, of the residual and written, per million.
 struct TileCost {
@@ -531,7 +558,7 @@ struct TileChoice {
     int cfg, splits, mode;
     float cost;
 };
-static TileChoice tile_pick(bool conv, int M, int N, int K, int64_t a_floats, bool residual, int batch, bool cuts)
+static TileChoice tile_pick(bool conv, int M, int N, int K, int64_t a_floats, bool residual, int batch, bool cuts, bool halo = false)
 {
     const int slabs = (K + kSlab - 1) / kSlab;
     const float k = (float)slabs * (kSlab * 1e-3f);
@@ -548,6 +575,14 @@ static TileChoice tile_pick(bool conv, int M, int N, int K, int64_t a_floats, bo
     };
     for (const TileCost& c : kTileCost)
         consider(c.cfg, 1, 0, tile_cost(c, conv, tiles(c.cfg), k, io), 1.f);
+    static const TileCost kHaloCost[] = {
+        { 23, 256, 1.29f, 5.12f, 25.5f, 0.f, 0.f, 7.84f, 0.f, 0.f, 0.085f },
+        { 24, 512, 4.47f, 1.34f, 11.6f, 0.71f, 9.35f, 2.17f, 0.f, 0.f, 0.f },
+        { 28, 256, 2.76f, 0.f, 49.5f, 8.55f, 0.f, 10.4f, 0.f, 0.f, 0.307f },
+    };
+    if (halo)
+        for (const TileCost& c : kHaloCost)
+            consider(c.cfg, 1, 0, tile_cost(c, false, tiles(c.cfg), k, io), 1.f);
     if (!cuts)
         return best;
     // A cut costs more than its own time (partial tiles through memory; stretches read operands at a K phase of their own, so
@@ -562,14 +597,35 @@ static TileChoice tile_pick(bool conv, int M, int N, int K, int64_t a_floats, bo
     const float t = (float)t128 / 256.f;
     if (t128 >= 86 && t128 <= 512 && K >= 256)
         consider(13, 0, 2, 4.96f + (conv ? 39.f : 37.9f) * k * t + 3.76f / t + 6.75f * t, 1.03f);
-    if (t128 <= 1024 && t128 % 256 != 0)
+    // whole rounds at (e0 + a0 k) each, then the last one in S ranges
+    auto hybrid = [&](int cfg, float e0, float a0, float e1, float a1, float c, float part, float per_range) {
         for (int S : { 2, 3, 4 })
             if (slabs >= 4 * S) {
                 const int64_t whole = t128 / 256, units = (t128 % 256) * S, w = (units + 255) / 256;
                 const float ks = (float)((slabs + S - 1) / S) * (kSlab * 1e-3f);
-                consider(13, S, 1, (float)whole * (4.56f + 27.1f * k) + (float)w * (7.43f + 27.4f * ks)
-                        + (conv ? 2.82f * ((float)whole * k + (float)w * ks) : 0.f) + 9.87f * k * t + 0.135f * (float)units * (128 * 128 * 1e-6f) + 1.07f * S, 1.02f);
+                consider(cfg, S, 1, (float)whole * (e0 + a0 * k) + (float)w * (e1 + a1 * ks) + c * k * t + part * (float)units * (128 * 128 * 1e-6f)
+                        + per_range * S, 1.02f);
             }
+    };
+    if (t128 <= 1024 && t128 % 256 != 0) {
+        const float d = conv ? 2.82f : 0.f;
+        hybrid(13, 4.56f, 27.1f + d, 7.43f, 27.4f + d, 9.87f, 0.135f, 1.07f);
+        if (halo)
+            hybrid(23, 3.85f, 26.4f, 8.58f, 25.1f, 7.31f, 0.161f, 1.12f);
+    }
+    static const TileCost kHaloRange[] = {
+        { 23, 256, 0.78f, 0.f, 25.3f, 8.20f, 0.f, 7.65f, 0.f, 0.f, 0.f },
+        { 24, 512, 1.08f, 0.64f, 10.0f, 5.60f, 10.3f, 2.17f, 0.f, 0.f, 0.f },
+    };
+    if (halo && t128 <= 256)
+        for (const TileCost& c : kHaloRange)
+            for (int S : { 2, 3, 4 })
+                if (slabs >= 2 * S && (c.cfg == 23 || S < 4)) {
+                    int bm, bn;
+                    tile_of(c.cfg, bm, bn);
+                    consider(c.cfg, S, 0, tile_cost(c, false, tiles(c.cfg) * S, (float)((slabs + S - 1) / S) * (kSlab * 1e-3f), io)
+                            + (c.cfg == 23 ? 1.01f : 1.7f) * S + (c.cfg == 23 ? 0.209f : 0.288f) * (float)(tiles(c.cfg) * S * bm * bn) * 1e-6f, 1.02f);
+                }
     return best;
 }
 
@@ -690,7 +746,9 @@ static int autotune(const GemmParams& q, bool conv, int batch, hipStream_t s, in
     const bool can_split = g_split_enabled && split_prepare();
     auto timed = [&](auto&& launch) -> float { return time_rounds(a, b, s, launch); };
     bool clock_settled = false;
-    for (int cfg : { 13, 14, 15, 16, 18 }) {
+    for (int cfg : { 13, 14, 15, 16, 18, 23, 24, 28 }) {
+        if (halo_cfg(cfg) && !halo_ok(q, conv))
+            continue;
         int bm, bn;
         tile_of(cfg, bm, bn);
         const int64_t tiles = (int64_t)((q.M + bm - 1) / bm) * ((q.N + bn - 1) / bn) * batch;
@@ -700,7 +758,7 @@ static int autotune(const GemmParams& q, bool conv, int batch, hipStream_t s, in
         for (const auto& ch : kChoices) {
             const int splits = ch[0], mode = ch[1];
             const bool hybrid = mode == 1;
-            if (splits != 1 && !(can_split && cfg <= 15))
+            if (splits != 1 && !(can_split && (cfg <= 15 || (halo_cfg(cfg) && mode != 2))))
                 continue;
             static const bool streamk_on = [] { const char* e = std::getenv("FDX_STREAMK"); return !(e && e[0] == '0'); }();
             if (mode == 2 && !streamk_on)
@@ -834,13 +892,13 @@ static fdx_status run_igemm(GemmParams& p, bool conv, int batch, const char* fam
         const bool slice = cfg >= kSliceCfg && cfg < kSliceCfg + kSliceForms;
         if (slice && (!fast_ok || batch != 1 || !slice_fits(cfg - kSliceCfg, p.M, p.N)))
             cfg = -1;
-        if (cfg >= 10 && cfg != kStreamCfg && !slice && (!fast_ok || cfg > 18))
+        if (cfg >= 10 && cfg != kStreamCfg && !slice && (!fast_ok || (cfg > 18 && !(halo_cfg(cfg) && halo_ok(p, conv) && mode < 2))))
             cfg = -1;
         if (cfg < 10 || mode > 2 || mode < 0 || splits < 0 || splits > 64 || cfg == kStreamCfg || slice) {
             splits = 1;
             mode = 0;
         }
-        if (cfg >= 10 && splits != 1 && (canonical_tile(cfg) > 15 || !split_prepare())) {
+        if (cfg >= 10 && splits != 1 && ((canonical_tile(cfg) > 15 && !halo_cfg(cfg)) || !split_prepare())) {
             splits = 1;
             mode = 0;
         }
@@ -908,7 +966,8 @@ static fdx_status run_igemm(GemmParams& p, bool conv, int batch, const char* fam
         static const bool closed_cuts = [] { const char* e = std::getenv("FDX_CLOSED_SPLIT"); return !(e && e[0] == '0'); }();
         TileChoice tile { -1, 1, 0, 1e30f };
         if (cfg < 0 && fast_ok) {
-            tile = tile_pick(conv, p.M, p.N, p.K, conv ? a_bytes / 4 : (int64_t)p.M * p.K, p.residual != nullptr, batch, closed_cuts);
+            tile = tile_pick(conv, p.M, p.N, p.K, conv ? a_bytes / 4 : (int64_t)p.M * p.K, p.residual != nullptr, batch, closed_cuts,
+                halo_ok(p, conv) && p.kh * p.kw >= 6);
             if (batch == 1)
                 cfg = slice_pick(conv, p.M, p.N, p.K, tile.cost);
         }
@@ -1210,6 +1269,20 @@ extern "C" fdx_status fdx_debug_persist_cap(int workgroups)
     fdx::g_persist_scale = workgroups > 0 && workgroups < 8 ? 8 : workgroups;
     return FDX_OK;
 }
+
+namespace fdx {
+// Predicted time (us) of a 3x3 stride-1 convolution as a direct sum, by the closed rule's costs.
+float conv3x3_direct_cost(int n, int h, int w, int cin, int cout, int oh, int ow, bool residual)
+{
+    const int64_t m = std::min<int64_t>((int64_t)n * oh * ow, INT32_MAX); // larger ones are refused by either kernel
+    const bool halo = oh == h && ow == w && cin % kSlab == 0 && 2 * w + 2 <= kHaloSpan;
+    const TileChoice tile = tile_pick(true, (int)m, cout, 9 * cin, (int64_t)n * h * w * cin, residual, 1, true, halo);
+    float best = tile.cost;
+    for (int i = 0; i < kSliceForms; ++i)
+        best = std::min(best, slice_cost(i, true, (int)m, cout, 9 * cin));
+    return best;
+}
+} // namespace fdx
 
 extern "C" fdx_status fdx_conv2d_nhwc_f32(const float* in, int n, int h, int w, int cin,
     const float* weights, const float* bias, int cout, int kh, int kw,

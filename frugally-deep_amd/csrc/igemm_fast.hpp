@@ -54,6 +54,7 @@ constexpr int split_tile_buffers(int bm, int bn, int waves_m, int waves_n)
 {
     return waves_m * waves_n == 4 && bm * bn >= 128 * 128 ? 1 : 2;
 }
+constexpr int kHaloSpan = 128; // HALO: pixels of a slab of A beyond the tile's rows
 constexpr int split_tile_waves(int bm, int bn, int waves_m, int waves_n)
 {
     return waves_m * waves_n == 8 || bm * bn > 64 * 64 ? 2 : 3;
@@ -128,8 +129,15 @@ __device__ __forceinline__ int seg_of(const GemmParams& p, int n0) { return (n0 
 //  * SEG (GEMM form, whole tiles only): the columns of C go to up to three tensors, the rows of each in sequences that lie
 //    apart: the stacked query / key / value projection of prompts, keys and values straight into their cache rows (2048 rows, 768 -> 3 x 768:
 //    69 us instead of three launches of 29.6, which leave 384 tiles on 256 CUs each).
+//  * HALO (convolution whose map keeps its size, stride 1): K is walked channel slab by channel slab and tap by tap inside a
+//    slab, and a slab of A is the run of input pixels that all taps of the tile's rows touch (rows of a tile are neighbours in
+//    raster order, so is what they read: BM + (kh - 1) dy W + (kw - 1) dx pixels).  It is fetched and split once for all taps
+//    instead of once per tap -- nine times less of that work, and of the traffic from L2, for a 3x3 filter -- and a tap's
+//    operands are read from LDS at its distance; a lane whose row has no such pixel (the convolution's padding) reads a
+//    pixel of zeros kept behind the run.  64 images: 28 x 28 x 128 -> 128 84 -> 77 us, 14 x 14 x 256 -> 256 87 -> 77,
+//    56 x 56 x 64 -> 64 113 -> 85; 16 images 32 -> 29, 35 (few-tiles ranges) -> 36, 34 -> 26.
 template <int BM, int BN, int WAVES_M, int WAVES_N, bool CONV, bool SPLIT = false, bool STREAMK = false, bool DUAL = false,
-    bool LNF = false, bool SEG = false>
+    bool LNF = false, bool SEG = false, bool HALO = false>
 __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, split_tile_waves(BM, BN, WAVES_M, WAVES_N))
 void igemm_fast_kernel(GemmParams p)
 {
@@ -141,14 +149,18 @@ void igemm_fast_kernel(GemmParams p)
     constexpr int BKT = 32;
     constexpr bool DB = split_tile_buffers(BM, BN, WAVES_M, WAVES_N) == 2;
     constexpr int RPP = NT / 4; // tile rows filled per loader pass: four lanes per row, two 16-byte chunks each
-    constexpr int A_UNITS = BM / RPP, B_UNITS = BN / RPP;
-    static_assert(BM % RPP == 0 && BN % RPP == 0, "tile rows must be a multiple of the loader pass");
+    static_assert(!HALO || (CONV && !STREAMK && DB), "the halo form is a convolution with whole tiles or K ranges");
+    constexpr int ROWS_A = HALO ? BM + kHaloSpan : BM; // pixels of A in LDS
+    constexpr int A_UNITS = ROWS_A / RPP, B_UNITS = BN / RPP;
+    static_assert(ROWS_A % RPP == 0 && BN % RPP == 0, "tile rows must be a multiple of the loader pass");
     constexpr int WTM = BM / WAVES_M, WTN = BN / WAVES_N;
     constexpr int TM = WTM / 32, TN = WTN / 32;
     constexpr int OSTRIDE = WTN + 4; // epilogue scratch row
     // LDS of one slab: per operand three planes of four blocks (one per lane of a row), a block = 16 bytes per tile row
-    constexpr int A_BLK = BM * 16 + 32, B_BLK = BN * 16 + 32, A_BYTES = 12 * A_BLK, BUF_BYTES = 12 * (A_BLK + B_BLK);
-    constexpr int SMEM_BYTES = (DB ? 2 : 1) * BUF_BYTES;
+    // (HALO: one slab of A, whose last 16 bytes of a block are the pixel of zeros, and two of B)
+    constexpr int A_BLK = ROWS_A * 16 + 32, B_BLK = BN * 16 + 32, A_BYTES = 12 * A_BLK;
+    constexpr int A_STEP = HALO ? 0 : A_BYTES + 12 * B_BLK, B_STEP = HALO ? 12 * B_BLK : A_STEP; // from buffer 0 to buffer 1
+    constexpr int SMEM_BYTES = A_BYTES + 12 * B_BLK + (DB ? B_STEP : 0);
     static_assert(SMEM_BYTES >= WAVES_M * WAVES_N * 32 * OSTRIDE * 4, "epilogue scratch must fit in the operand buffers");
     constexpr uint32_t OOB = 0x80000000u; // beyond any extent this path accepts: the load returns zeros
 
@@ -194,7 +206,11 @@ void igemm_fast_kernel(GemmParams p)
     // ---- per-tile loader state
     uint32_t a_voff[A_UNITS], b_voff[B_UNITS];
     uint32_t a2_voff[DUAL ? A_UNITS : 1];
-    uint64_t a_mask[A_UNITS];
+    uint64_t a_mask[HALO ? 1 : A_UNITS];
+    uint32_t row_mask[TM]; // HALO: taps of this lane's operand rows that lie inside the image
+    const int taps = HALO ? p.kh * p.kw : 1;
+    int slab_c = 0;        // HALO: first channel of the next slab of A
+    int read_tap = 0, read_fx = 0, read_shift = 0; // HALO: the tap whose operands are read next and its distance in pixels
     __amdgpu_buffer_rsrc_t srd_a, srd_b;
     const __amdgpu_buffer_rsrc_t srd_a2 = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(DUAL ? p.A2 : p.A), 0,
         DUAL ? (int)p.a2_records : 0, 0x00020000);
@@ -244,13 +260,40 @@ void igemm_fast_kernel(GemmParams p)
         const float* A = p.A + (z / p.inner) * p.a_outer + (z % p.inner) * p.a_inner;
         const float* B = p.B + (z / p.inner) * p.b_outer + (z % p.inner) * p.b_inner;
         c_off = (z / p.inner) * p.c_outer + (z % p.inner) * p.c_inner;
-        srd_a = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(A), 0, (int)p.a_records, 0x00020000);
+        const int halo_lo = HALO ? p.pad_top * p.W + p.pad_left : 0;
+        if (HALO) // A starts halo_lo pixels early
+            srd_a = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(A) + (int64_t)halo_lo * p.Cin, 0, (int)((uint32_t)p.M * p.Cin * 4u), 0x00020000);
+        else
+            srd_a = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(A), 0, (int)p.a_records, 0x00020000);
         srd_b = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(B), 0, (int)p.b_records, 0x00020000);
+        if (HALO) {
+            const int span = (p.kh - 1) * p.dy * p.W + (p.kw - 1) * p.dx;
+#pragma unroll
+            for (int i = 0; i < A_UNITS; ++i) {
+                const int slot = r0 + i * RPP, px = m0 - halo_lo + slot;
+                a_voff[i] = slot < BM + span && px >= 0 && px < p.M ? (uint32_t)px * p.Cin * 4u + kq * 16 : OOB;
+            }
+#pragma unroll
+            for (int i = 0; i < TM; ++i) {
+                const int m = m0 + wm * WTM + i * 32 + fr;
+                const int rm = m % (p.OH * p.OW), oy = rm / p.OW, ox = rm - oy * p.OW;
+                uint32_t mk = 0;
+                for (int y = 0; y < p.kh; ++y) {
+                    const int iy = oy - p.pad_top + y * p.dy;
+                    for (int x = 0; x < p.kw; ++x) {
+                        const int ix = ox - p.pad_left + x * p.dx;
+                        if (m < p.M && iy >= 0 && iy < p.H && ix >= 0 && ix < p.W)
+                            mk |= 1u << (y * p.kw + x);
+                    }
+                }
+                row_mask[i] = mk;
+            }
+        } else
 #pragma unroll
         for (int i = 0; i < A_UNITS; ++i) {
             const int m = m0 + r0 + i * RPP;
             a_voff[i] = OOB;
-            a_mask[i] = 0;
+            a_mask[HALO ? 0 : i] = 0;
             if (m < p.M) {
                 if (CONV) {
                     const int img = m / (p.OH * p.OW), rm = m - img * (p.OH * p.OW);
@@ -267,10 +310,10 @@ void igemm_fast_kernel(GemmParams p)
                                 mk |= 1ull << (y * p.kw + x);
                         }
                     }
-                    a_mask[i] = mk;
+                    a_mask[HALO ? 0 : i] = mk;
                 } else {
                     a_voff[i] = (uint32_t)((int64_t)m * p.lda) * 4u + kq * 16;
-                    a_mask[i] = ~0ull;
+                    a_mask[HALO ? 0 : i] = ~0ull;
                 }
             }
             if (DUAL) {
@@ -289,7 +332,15 @@ void igemm_fast_kernel(GemmParams p)
         }
         tap = fx = fy = c0 = 0;
         soff_a = soff_b = 0;
-        if (SPLIT && kt_lo > 0) {
+        if (HALO) {
+            const int cs = kt_lo / taps;
+            tap = read_tap = kt_lo - cs * taps;
+            slab_c = c0 = cs * BKT;
+            soff_b = (tap * p.Cin + c0) * 4;
+            const int y = tap / p.kw;
+            read_fx = tap - y * p.kw;
+            read_shift = y * p.dy * p.W + read_fx * p.dx;
+        } else if (SPLIT && kt_lo > 0) {
             const int k_start = kt_lo * BKT;
             soff_b = k_start * 4;
             if (CONV) {
@@ -315,7 +366,7 @@ void igemm_fast_kernel(GemmParams p)
         } else {
 #pragma unroll
             for (int i = 0; i < A_UNITS; ++i) {
-                const uint32_t vo = CONV ? (in_k && ((a_mask[i] >> tap) & 1) ? a_voff[i] : OOB) : (a_voff[i] | off);
+                const uint32_t vo = CONV ? (in_k && ((a_mask[HALO ? 0 : i] >> tap) & 1) ? a_voff[i] : OOB) : (a_voff[i] | off);
                 ra[i][h] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(srd_a, (int)vo, soff_a, 0));
             }
         }
@@ -338,7 +389,35 @@ void igemm_fast_kernel(GemmParams p)
             soff_a += 64;
         }
     };
+    // HALO: B of the next (channel slab, tap), A of the next channel slab
+    auto load_halo_b = [&](bool live) {
+        const uint32_t off = live ? 0u : OOB;
+#pragma unroll
+        for (int i = 0; i < B_UNITS; ++i)
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+                rb[i][h] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(srd_b, (int)(b_voff[i] | off), soff_b + 64 * h, 0));
+        soff_b += p.Cin * 4;
+        if (++tap == taps) {
+            tap = 0;
+            c0 += BKT;
+            soff_b = c0 * 4;
+        }
+    };
+    auto load_halo_a = [&]() { // behind the last slab nothing is fetched
+        const uint32_t off = slab_c < p.Cin ? 0u : OOB;
+#pragma unroll
+        for (int i = 0; i < A_UNITS; ++i)
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+                ra[i][h] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(srd_a, (int)(a_voff[i] | off), slab_c * 4 + 64 * h, 0));
+        slab_c += BKT;
+    };
     auto load_tiles = [&](bool live) {
+        if (HALO) {
+            load_halo_b(live);
+            return;
+        }
         load_half(0, live);
         load_half(1, live);
     };
@@ -371,12 +450,14 @@ void igemm_fast_kernel(GemmParams p)
         }
 #pragma unroll
         for (int i = 0; i < A_UNITS; ++i)
-            put(smem_raw + buf * BUF_BYTES + kq * A_BLK + (r0 + i * RPP) * 16, 4 * A_BLK, ra[i][0], ra[i][1]);
+            put(smem_raw + buf * A_STEP + kq * A_BLK + (r0 + i * RPP) * 16, 4 * A_BLK, ra[i][0], ra[i][1]);
+        if (HALO && t < 12)
+            *reinterpret_cast<u32x4*>(smem_raw + t * A_BLK + ROWS_A * 16) = u32x4 { 0u, 0u, 0u, 0u };
     };
     auto store_b = [&](int buf) {
 #pragma unroll
         for (int i = 0; i < B_UNITS; ++i)
-            put(smem_raw + buf * BUF_BYTES + A_BYTES + kq * B_BLK + (r0 + i * RPP) * 16, 4 * B_BLK, rb[i][0], rb[i][1]);
+            put(smem_raw + buf * B_STEP + A_BYTES + kq * B_BLK + (r0 + i * RPP) * 16, 4 * B_BLK, rb[i][0], rb[i][1]);
     };
 
     int tile = sk ? 0 : wg_in_xcd; // local unit index
@@ -386,6 +467,8 @@ void igemm_fast_kernel(GemmParams p)
     int m0, n0;
     int64_t c_off;
     setup(tile, m0, n0, c_off);
+    if (HALO)
+        load_halo_a();
     load_tiles(true);
 
     for (;;) {
@@ -404,16 +487,22 @@ void igemm_fast_kernel(GemmParams p)
         store_a(0, true);
         store_b(0);
         load_tiles(1 < kt_end);
+        if (HALO)
+            load_halo_a();
         __syncthreads();
         bf16x8 af[2][TM][3], bf[2][TN][3];
         auto read_frags = [&](int s, int buf) {
-            const unsigned char* as = smem_raw + buf * BUF_BYTES + (2 * s + fh) * A_BLK + (wm * WTM + fr) * 16;
-            const unsigned char* bs = smem_raw + buf * BUF_BYTES + A_BYTES + (2 * s + fh) * B_BLK + (wn * WTN + fr) * 16;
+            const unsigned char* as = smem_raw + buf * A_STEP + (2 * s + fh) * A_BLK + (HALO ? 0 : (wm * WTM + fr) * 16);
+            const unsigned char* bs = smem_raw + buf * B_STEP + A_BYTES + (2 * s + fh) * B_BLK + (wn * WTN + fr) * 16;
+            int row[TM]; // where operand row i lies
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+                row[i] = !HALO ? i * 512 : (row_mask[i] >> read_tap) & 1 ? (wm * WTM + i * 32 + fr + read_shift) * 16 : ROWS_A * 16;
 #pragma unroll
             for (int q = 0; q < 3; ++q) {
 #pragma unroll
                 for (int i = 0; i < TM; ++i)
-                    af[s][i][q] = *reinterpret_cast<const bf16x8*>(as + q * 4 * A_BLK + i * 512);
+                    af[s][i][q] = *reinterpret_cast<const bf16x8*>(as + q * 4 * A_BLK + row[i]);
 #pragma unroll
                 for (int j = 0; j < TN; ++j)
                     bf[s][j][q] = *reinterpret_cast<const bf16x8*>(bs + q * 4 * B_BLK + j * 512);
@@ -423,6 +512,10 @@ void igemm_fast_kernel(GemmParams p)
         // the second half's reads would wait for them, with the matrix pipe drained (128 x 128 tiles 7 % faster this way,
         // 128 x 64 2 %; the 256-row tile has no registers for it, 3 % slower).
         constexpr bool READ_AHEAD = BM <= 128;
+        // The halo form in eight waves of 128 rows: the barrier lies between the halves, and the next slab's first half is read
+        // under the second half's products (7 % faster; 128 x 64 tiles, two workgroups on a CU, gain nothing, the tiles that
+        // stage A for every slab lose 6 %).
+        constexpr bool CARRIED = HALO && READ_AHEAD && NT == 512;
         auto product = [&](int s, int x, int y, f32x16(&d)[TM][TN]) {
 #pragma unroll
             for (int i = 0; i < TM; ++i)
@@ -447,6 +540,36 @@ void igemm_fast_kernel(GemmParams p)
         // after that is requested into the registers this frees
         for (int kt = 0; kt + 1 < kt_end; ++kt) {
             const int buf = DB ? kt & 1 : 0;
+            if (HALO) {
+                if (!CARRIED || kt == 0)
+                    read_frags(0, buf);
+                if (READ_AHEAD)
+                    read_frags(1, buf);
+                multiply(0);
+                if (!READ_AHEAD)
+                    read_frags(1, buf);
+                store_b(buf ^ 1);
+                if (!CARRIED)
+                    multiply(1);
+                load_tiles(kt + 2 < kt_end);
+                read_shift += p.dx;
+                if (++read_fx == p.kw) {
+                    read_fx = 0;
+                    read_shift += p.dy * p.W - p.kw * p.dx;
+                }
+                if (++read_tap == taps) { // the next slab of channels
+                    read_tap = read_fx = read_shift = 0;
+                    __syncthreads();
+                    store_a(0);
+                    load_halo_a();
+                }
+                __syncthreads();
+                if (CARRIED) {
+                    read_frags(0, buf ^ 1);
+                    multiply(1);
+                }
+                continue;
+            }
             if (DB) {
                 read_frags(0, buf);
                 if (READ_AHEAD)
@@ -471,7 +594,8 @@ void igemm_fast_kernel(GemmParams p)
         }
         {
             const int buf = DB ? (kt_end - 1) & 1 : 0;
-            read_frags(0, buf);
+            if (!CARRIED || kt_end == 1)
+                read_frags(0, buf);
             if (READ_AHEAD)
                 read_frags(1, buf);
             multiply(0);
@@ -552,6 +676,8 @@ void igemm_fast_kernel(GemmParams p)
         const bool more = tile < unit_end;
         if (more) {
             setup(tile, m0, n0, c_off);
+            if (HALO)
+                load_halo_a();
             load_tiles(true); // in flight while this tile is written out
         }
 

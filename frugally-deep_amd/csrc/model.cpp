@@ -1794,6 +1794,16 @@ extern "C" fdx_status fdx_debug_force_chain(int mode)
 
 // test hook: -1 = a plan times the direct and the Winograd kernel of a 3x3 stride-1 convolution, 0 = always direct, 1 = Winograd
 // wherever it applies
+// Direct sum or Winograd form of a 3x3 stride-1 convolution by predicted cost.  Of 220 timed ones (maps of 6 to 62 pixels, 32 to
+// 512 channels, batches of 1 to 64) the choice takes 2 % longer than the faster form on average; Winograd from a gigaflop of
+// direct-sum work on, the line before the direct kernel took its products to the bf16 matrix instructions, took 11 % longer
+// (5 images, 32 x 32 x 256 -> 64: direct 22.5 us, Winograd 37.6; 24 images, 40 x 40 x 512 -> 64: 133 / 115).  The direct kernel
+// draws more power, which the layers around it pay for with clock: 3 % against it.
+static bool winograd_by_rule(int n, int h, int w, int cin, int cout, int oh, int ow, bool residual)
+{
+    return conv2d_winograd_cost(n, cin, cout, oh, ow) < 1.03f * conv3x3_direct_cost(n, h, w, cin, cout, oh, ow, residual);
+}
+
 static int g_force_winograd = -1;
 
 extern "C" fdx_status fdx_debug_force_winograd(int mode)
@@ -2009,7 +2019,8 @@ fdx_status get_plan(fdx_model* m, int batch, const std::vector<Shape>& in_shapes
             key.res = o.residual >= 0;
             int known = 0;
             const bool listed = tune_lookup(key, &known);
-            p->conv_form[idx] = (listed ? known == 1 : 2.0 * key.M * (double)key.N * key.K >= 1e9) ? 1 : 0;
+            p->conv_form[idx] = (listed ? known == 1
+                : winograd_by_rule(batch, (int)is[0], (int)is[1], (int)is[2], o.cout, g[4], g[5], o.residual >= 0)) ? 1 : 0;
         }
     m->plans.insert(m->plans.begin(), std::move(p));
     *out = m->plans[0].get();
@@ -2054,11 +2065,8 @@ namespace {
         if (listed || tune_frozen() || hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess) {
             if (e0)
                 (void)hipEventDestroy(e0);
-            // Nothing is timed and the shape is not in the table: the Winograd kernel from a gigaflop of direct-sum work
-            // up (every 3x3 layer of ResNet50 from batch 5; timed, it wins all four of its shapes at batch 64 by 1.4-1.8
-            // times), the direct kernel below that, where a launch is too short for the kernel's fixed costs to pay.
-            const bool by_rule = 2.0 * key.M * (double)key.N * key.K >= 1e9;
-            p.conv_form[idx] = (listed ? known == 1 : by_rule) ? 1 : 0;
+            // nothing is timed and the shape is not in the table
+            p.conv_form[idx] = (listed ? known == 1 : winograd_by_rule(B, h, w, c, o.cout, g[4], g[5], res != nullptr)) ? 1 : 0;
             fdx_status st = run(p.conv_form[idx]);
             if (st == FDX_ERR_UNSUPPORTED && p.conv_form[idx] == 1) {
                 p.conv_form[idx] = 0;

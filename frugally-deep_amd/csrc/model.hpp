@@ -159,6 +159,9 @@ fdx_status conv1x1_chain_launch(const float* a, int n, int oh, int ow, int k1, c
 bool gemm_ln_supported(int64_t m, int n, int k);
 fdx_status gemm_ln_launch(const float* x, int64_t m, int k, const float* w, const float* bias, const float* wsum, float eps, const float* residual,
     const fdx_act* act, float* out, int n);
+// predicted times of a 3x3 stride-1 convolution as a direct sum and in the Winograd form (igemm.hip, wino.hip)
+float conv3x3_direct_cost(int n, int h, int w, int cin, int cout, int oh, int ow, bool residual);
+float conv2d_winograd_cost(int n, int cin, int cout, int oh, int ow);
 fdx_status conv1x1_dual_launch(const float* in1, int n, int oh, int ow, int c1, const float* in2, int h2, int w2, int c2, int s2y, int s2x,
     const float* w_cat, const float* bias, int cout, const fdx_act* act, float* out);
 fdx_status conv1x1_padded_launch(const float* in, int64_t rows, int cin, const float* w_padded, int k_padded, const float* bias,

@@ -12,6 +12,7 @@ import pytest
 
 pytestmark = pytest.mark.gpu
 TILES = [-1, 13, 14, 15, 16, 18, 215, 815, 315 + 10000, 20013, 20015]
+HALO = [23, 24, 28, 223]
 
 
 def forced(fdx, tile, f):
@@ -63,23 +64,23 @@ def check_special(got, a, w):
     assert np.allclose(got[finite], want[finite], rtol=1e-4, atol=1e-4)
 
 
-@pytest.mark.parametrize("tile", TILES)
+@pytest.mark.parametrize("tile", TILES + HALO)
 def test_infinities_and_nan(fdx, tile):
     print("special operands", tile, flush=True)
     r = np.random.default_rng(5)
-    m, n, k = 140, 68, 336
+    m, n, k = 140, 68, 352
     a, w = r.standard_normal((m, k)).astype(np.float32), (r.standard_normal((n, k)) / 18).astype(np.float32)
     special(a, w)
     check_special(forced(fdx, tile, lambda: fdx.gemm(a, w)), a, w)
-    # a 3x3 convolution over a map of one row: the same products with zero taps above and below
-    x = a.reshape(1, m, 1, k).transpose(0, 2, 1, 3).copy()
+    # a 3x3 convolution over a map of ten positions a row: the same products with zero taps around
+    x = a.reshape(1, m // 10, 10, k).copy()
     wc = np.zeros((n, 3, 3, k), np.float32)
     wc[:, 1, 1] = w
-    got = forced(fdx, tile, lambda: fdx.conv2d(x, wc, None, padding="same"))[0, 0]
+    got = forced(fdx, tile, lambda: fdx.conv2d(x, wc, None, padding="same")).reshape(m, n)
     with np.errstate(all="ignore"):
         want = a.astype(np.float64) @ w.astype(np.float64).T
     far = np.ones(m, bool)
-    far[:8] = False                       # zero taps of the neighbours meet infinities there: only positions past them compare
+    far[:20] = False                      # zero taps of the neighbours meet infinities there: only positions past them compare
     far_w = np.isfinite(w).all(1)
     assert np.allclose(got[far][:, far_w], want[far][:, far_w], rtol=1e-4, atol=1e-4)
     assert np.isnan(got[:, 2]).all() and not np.isfinite(got[far][:, 0]).any()
@@ -103,3 +104,28 @@ def test_infinities_two_sources(fdx, modelgen):
         hit = np.zeros(want.shape[:3], bool)
         hit[2, 2, 1] = True
         assert np.array_equal(got[~hit], want[~hit]) and not np.isfinite(got[hit]).any()
+
+
+@pytest.mark.parametrize("tile", [23, 24, 28, 223, 10323, 424])
+@pytest.mark.parametrize("n,h,w,cin,cout,kh,kw,dil", [
+    (2, 9, 7, 32, 64, 3, 3, 1), (3, 14, 14, 64, 132, 3, 3, 1), (1, 28, 56, 32, 64, 3, 3, 1), (9, 7, 7, 96, 260, 3, 3, 1),
+    (2, 11, 63, 32, 68, 3, 3, 1),                               # the longest run of pixels: 128 beyond the tile's rows
+    (1, 20, 31, 64, 64, 5, 5, 1), (2, 17, 12, 32, 36, 1, 3, 1), (2, 16, 15, 64, 40, 3, 3, 2), (1, 5, 4, 32, 36, 3, 2, 1)])
+def test_convolution_halo(fdx, n, h, w, cin, cout, kh, kw, dil, tile):
+    """The form that fetches a tile's pixels once for all filter taps: rows of a tile over image borders and images, runs cut at
+    both ends of the batch, K ranges that begin inside a channel slab."""
+    import torch
+    print("halo", n, h, w, cin, cout, kh, kw, dil, tile, flush=True)
+    r = np.random.default_rng(zlib.crc32(repr((n, h, w, cin, cout)).encode()))
+    x = r.standard_normal((n, h, w, cin)).astype(np.float32)
+    wc = (r.standard_normal((cout, kh, kw, cin)) / np.sqrt(kh * kw * cin)).astype(np.float32)
+    b, res = r.standard_normal(cout).astype(np.float32), r.standard_normal((n, h, w, cout)).astype(np.float32)
+    got, again = forced(fdx, tile, lambda: [fdx.conv2d(x, wc, b, dilation=(dil, dil), padding="same", residual=res) for _ in range(2)])
+    eh, ew = (kh - 1) * dil, (kw - 1) * dil
+    xp = torch.nn.functional.pad(torch.from_numpy(x).double().permute(0, 3, 1, 2), (ew // 2, ew - ew // 2, eh // 2, eh - eh // 2))
+    conv = lambda a, f: torch.nn.functional.conv2d(a, f.permute(0, 3, 1, 2), dilation=dil).permute(0, 2, 3, 1).numpy()
+    want, size = conv(xp, torch.from_numpy(wc).double()) + b + res, conv(xp.abs(), torch.from_numpy(wc).double().abs()) + np.abs(b) + np.abs(res)
+    k = kh * kw * cin
+    assert (np.abs(got - want) <= (k / 16 + 8) * 2.0 ** -23 * size).all()
+    assert np.linalg.norm(got - want) <= (1.2e-8 * np.sqrt(k) + 1.2e-7) * np.linalg.norm(want)
+    assert np.array_equal(got, again)

@@ -2924,12 +2924,13 @@ namespace {
         // longest run of ops that can take a range of samples: device ops outside any fused block, every choice already made
         int longest = 0;
         double flops = 0, total = p.flops > 0 ? p.flops : 1;
-        // what the pieces behind the first need to travel (55 GB/s over the link) at the rate piece-sized launches compute
-        // at (75 TFLOP/s), and no more than a quarter of the model: ResNet50 b64 from host memory, prefix of 12 / 11 / 8 /
-        // 7 / 6 / 5 / 2 ops: 12.9 / 13.1-13.3 / 13.6 / 13.65 / 13.55 / 13.3 / 12.85 k img/s -- a longer prefix runs more
-        // of the model at a quarter of the batch than the copy can hide, a shorter one leaves the copy uncovered
+        // what the pieces behind the first need to travel (55 GB/s over the link) at 50 TFLOP/s, and no more than a quarter of
+        // the model: a longer prefix runs more of the model at a quarter of the batch than the copy can hide, a shorter one
+        // leaves the copy uncovered.  ResNet50 from host memory, us at 10 / 20 / 35 / 50 / 75 / 110 / 150 TFLOP/s: 16 images 1674 / 1683 /
+        // 1666 / 1672 / 1780 / 1792 / 1827 (two machines, scaled to one), 32 2535 / 2548 / 2520 / 2484 / 2535 / 2545 / 2607, 64 4370 / 4380 /
+        // 4317 / 4175 / 4180 / 4210 / 4280.
         const double in_bytes = 4.0 * (double)batch * (double)volume(p.shapes[(size_t)m.inputs[0]]);
-        const double enough = std::min(total / 4, in_bytes / 55e9 * 75e12);
+        const double enough = std::min(total / 4, in_bytes / 55e9 * 50e12);
         int wanted = -1;
         for (int pos = 0; pos < n_pos; ++pos) {
             const int idx = p.order[(size_t)pos];

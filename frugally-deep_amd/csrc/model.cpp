@@ -2926,9 +2926,9 @@ namespace {
         double flops = 0, total = p.flops > 0 ? p.flops : 1;
         // what the pieces behind the first need to travel (55 GB/s over the link) at 50 TFLOP/s, and no more than a quarter of
         // the model: a longer prefix runs more of the model at a quarter of the batch than the copy can hide, a shorter one
-        // leaves the copy uncovered.  ResNet50 from host memory, us at 10 / 20 / 35 / 50 / 75 / 110 / 150 TFLOP/s: 16 images 1674 / 1683 /
-        // 1666 / 1672 / 1780 / 1792 / 1827 (two machines, scaled to one), 32 2535 / 2548 / 2520 / 2484 / 2535 / 2545 / 2607, 64 4370 / 4380 /
-        // 4317 / 4175 / 4180 / 4210 / 4280.
+        // leaves the copy uncovered.  ResNet50 from host memory, 16 / 32 / 64 images, us: at 50 TFLOP/s 1711 / 2587 / 4355, 75 1780 / 2639 / 4352,
+        // 110 1792 / 2648 / 4386, 150 1828 / 2714 / 4454; on another machine 50 1672 / 2484 / 4175, 35 1666 / 2520 / 4318, 20 1684 / 2549 / 4380,
+        // 10 1674 / 2536 / 4371.
         const double in_bytes = 4.0 * (double)batch * (double)volume(p.shapes[(size_t)m.inputs[0]]);
         const double enough = std::min(total / 4, in_bytes / 55e9 * 50e12);
         int wanted = -1;

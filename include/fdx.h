@@ -74,7 +74,7 @@ fdx_status fdx_d2h(void* dst_host, const void* src_dev, size_t bytes);
 fdx_status fdx_sync(void);
 
 /*
- * Conv2D, cross-correlation, implicit GEMM on fp32 MFMA:
+ * Conv2D, cross-correlation, implicit GEMM in fp32 precision on the matrix cores:
  *   out[n][oy][ox][co] = act(bias[co] + sum_{fy,fx,ci} w[co][fy][fx][ci] * in[n][oy*sy+fy*dy-pad_top][ox*sx+fx*dx-pad_left][ci]
  *                            (+ residual[n][oy][ox][co]))
  * replaces convolve / convolve_accumulative (include/fdeep/convolution.hpp:398-429, 224-305).
@@ -177,7 +177,7 @@ fdx_status fdx_stem_block_nhwc_f32(const float* in, int n, int ih, int iw, int i
     const float* pw_weights_nc, const float* pw_bias, int n_out, const float* residual, const fdx_act* act, float* out);
 
 /*
- * Row-major GEMM with fused epilogue, fp32 MFMA:
+ * Row-major GEMM with fused epilogue, fp32 precision on the matrix cores:
  *   c[m][n] = act(alpha * sum_k a[m][k] * b_nk[n][k] + bias + residual[m][n])
  * replaces dense_layer::apply_impl (include/fdeep/layers/dense_layer.hpp:76-86; weights arrive
  * [in][out] and are transposed once at load to [out][in]) and dot_product_tensors

@@ -19,6 +19,7 @@
 #include <map>
 #include <mutex>
 
+#include "bf16_split.hpp"
 #include "common.hpp"
 #include "igemm_params.hpp"
 

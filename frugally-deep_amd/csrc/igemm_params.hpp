@@ -2,7 +2,6 @@
 #pragma once
 #include <cstring>
 #include <functional>
-#include "bf16_split.hpp"
 #include "common.hpp"
 
 namespace fdx {

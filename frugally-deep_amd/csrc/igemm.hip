@@ -499,6 +499,36 @@ static bool launch_fast(int cfg, int splits, int mode, const GemmParams& q0, boo
         }
         return true;
     }
+    if (q.seg_rows > 0) { // outputs in segments
+#define FDX_SEG(BM_, BN_, WM_, WN_)                                                                                            \
+    launch_persistent(igemm_fast_kernel<BM_, BN_, WM_, WN_, false, false, false, false, false, true>,                          \
+        ((q.M + BM_ - 1) / BM_) * ((q.N + BN_ - 1) / BN_), q, s, 64 * WM_ * WN_, BM_, BN_)
+#define FDX_SEG_CUT(BM_, BN_, WM_, WN_, STREAM_)                                                                               \
+    ok = launch_split(igemm_fast_kernel<BM_, BN_, WM_, WN_, false, true, STREAM_, false, false, true>,                         \
+        ((q.M + BM_ - 1) / BM_) * ((q.N + BN_ - 1) / BN_), splits, mode, cfg, q, s, 64 * WM_ * WN_)
+        const bool cut = mode == 2 || splits > 1;
+        switch (cfg) {
+        case 13:
+            if (mode == 2)
+                FDX_SEG_CUT(128, 128, 4, 2, true);
+            else if (cut)
+                FDX_SEG_CUT(128, 128, 4, 2, false);
+            else
+                FDX_SEG(128, 128, 4, 2);
+            break;
+        case 14: FDX_SEG(128, 64, 2, 2); break;
+        case 16: FDX_SEG(128, 128, 2, 2); break;
+        case 18: FDX_SEG(256, 128, 4, 2); break;
+        default:
+            if (cut)
+                FDX_SEG_CUT(64, 64, 2, 2, false);
+            else
+                FDX_SEG(64, 64, 2, 2);
+        }
+#undef FDX_SEG
+#undef FDX_SEG_CUT
+        return ok;
+    }
     if (halo_cfg(cfg)) {
 #define FDX_HALO(BM_, BN_, WM_, WN_)                                                                                           \
     {                                                                                                                          \
@@ -628,6 +658,13 @@ static TileChoice tile_pick(bool conv, int M, int N, int K, int64_t a_floats, bo
                             + (c.cfg == 23 ? 1.01f : 1.7f) * S + (c.cfg == 23 ? 0.209f : 0.288f) * (float)(tiles(c.cfg) * S * bm * bn) * 1e-6f, 1.02f);
                 }
     return best;
+}
+
+// whether the closed rule may cut K (FDX_CLOSED_SPLIT=0: whole tiles)
+static bool closed_cuts()
+{
+    static const bool on = [] { const char* e = std::getenv("FDX_CLOSED_SPLIT"); return !(e && e[0] == '0'); }();
+    return on;
 }
 
 // First sight of a problem shape on the fast path: time every tile configuration once on the
@@ -964,10 +1001,9 @@ static fdx_status run_igemm(GemmParams& p, bool conv, int batch, const char* fam
                 [&] { pw_stream_launch(p, a_bytes, b_bytes, s); });
             settle();
         }
-        static const bool closed_cuts = [] { const char* e = std::getenv("FDX_CLOSED_SPLIT"); return !(e && e[0] == '0'); }();
         TileChoice tile { -1, 1, 0, 1e30f };
         if (cfg < 0 && fast_ok) {
-            tile = tile_pick(conv, p.M, p.N, p.K, conv ? a_bytes / 4 : (int64_t)p.M * p.K, p.residual != nullptr, batch, closed_cuts,
+            tile = tile_pick(conv, p.M, p.N, p.K, conv ? a_bytes / 4 : (int64_t)p.M * p.K, p.residual != nullptr, batch, closed_cuts(),
                 halo_ok(p, conv) && p.kh * p.kw >= 6);
             if (batch == 1)
                 cfg = slice_pick(conv, p.M, p.N, p.K, tile.cost);
@@ -1194,23 +1230,51 @@ fdx_status gemm_segments_launch(const float* a, const float* w, const float* bia
     p.a_records = (uint32_t)((int64_t)m * k * 4);
     p.b_records = (uint32_t)((int64_t)p.N * k * 4);
     hipStream_t s = stream();
-    constexpr int kTiled = 15; // the 64 x 64 tile with the 32-float slab
-    auto launch = [&](int cfg) {
-        switch (cfg) {
+    constexpr int kTiled = 15; // the 64 x 64 tile
+    // A choice is packed as in the tuning table: cfg + 100 * splits + 10000 * mode, a bare number for whole tiles and slices.
+    auto unpack = [](int code) { return TileChoice { code % 100, code < 100 ? 1 : (code % 10000) / 100, code / 10000, 0.f }; };
+    auto launch = [&](int code) {
+        switch (code) {
         case kSliceCfg: slice_launch_seg<0>(p, s); break;
         case kSliceCfg + 1: slice_launch_seg<1>(p, s); break;
         case kSliceCfg + 2: slice_launch_seg<2>(p, s); break;
         case kSliceCfg + 3: slice_launch_seg<3>(p, s); break;
         case kSliceCfg + 4: slice_launch_seg<4>(p, s); break;
-        default:
-            launch_persistent(igemm_fast_kernel<64, 64, 2, 2, false, false, false, false, false, true>, ((m + 63) / 64) * ((p.N + 63) / 64), p,
-                s, 256, 64, 64);
+        default: {
+            const TileChoice c = unpack(code);
+            if (!launch_fast(c.cfg, c.splits, c.mode, p, false, 1, s))
+                launch_fast(c.cfg, 1, 0, p, false, 1, s); // the requested cut does not fit the scratch
+        }
         }
     };
+    // A tile has one segment: the 64 x 64 tile where a segment is no multiple of 128 columns, the general rule otherwise.  The
+    // small tile alone leaves rounds of workgroups part filled and does a third less per byte of LDS; 2304 columns, K = 768,
+    // 64 x 64 tiles against the rule: 2048 rows 56.6 -> 49.7 us (stream-K), 4800 rows 122 -> 100, 8000 rows 208 -> 166 (128 x
+    // 128 tiles), 1000 rows 33.8 -> 31.0, 400 rows (slices before) 21.2 -> 19.0 (K ranges).
+    bool wide = true;
+    for (int i = 0; i < n_seg; ++i)
+        wide = wide && seg[i].cols % 128 == 0;
     // The form comes from a test hook, the tuning table, a timing run where those are asked for, or the closed rule.
-    auto usable = [&](int cfg) {
-        return cfg == kTiled || (cfg >= kSliceCfg && cfg < kSliceCfg + kSliceForms && slice_fits(cfg - kSliceCfg, m, p.N));
+    auto usable = [&](int code) {
+        if (code >= kSliceCfg && code < kSliceCfg + kSliceForms)
+            return slice_fits(code - kSliceCfg, m, p.N);
+        const TileChoice c = unpack(code);
+        if (code == kTiled)
+            return true;
+        if (!wide || code < 0 || !(c.cfg == kTiled || c.cfg == 13 || c.cfg == 14 || c.cfg == 16 || c.cfg == 18))
+            return false;
+        if (code < 100)
+            return true;
+        const bool form = c.cfg == 13 ? (c.mode == 2 ? c.splits == 0 : c.mode < 2 && c.splits >= 2 && c.splits <= 64)
+                                      : c.cfg == kTiled && c.mode == 0 && c.splits >= 2 && c.splits <= 64;
+        return form && split_prepare();
     };
+    TileChoice tile { kTiled, 1, 0, 0.f };
+    if (wide)
+        tile = tile_pick(false, m, p.N, k, (int64_t)m * k, false, 1, closed_cuts());
+    else
+        tile.cost = tile_cost(kTileCost[2], false, (int64_t)((m + 63) / 64) * ((p.N + 63) / 64), 1e-3f * k, 1e-6f * m * (float)(k + p.N));
+    const int tiled = tile.splits == 1 ? tile.cfg : tile.cfg + 100 * tile.splits + 10000 * tile.mode;
     int cfg = g_forced_tile;
     if (!usable(cfg)) {
         TuneKey key;
@@ -1220,10 +1284,10 @@ fdx_status gemm_segments_launch(const float* a, const float* w, const float* bia
         if (tune_lookup(key, &cfg)) {
         } else if (!tune_frozen() && 2.0 * m * (double)p.N * k >= 2e8 && hipEventCreate(&ea) == hipSuccess && hipEventCreate(&eb) == hipSuccess) {
             float best_ms = 1e30f;
-            for (int c : { kTiled, kSliceCfg, kSliceCfg + 1, kSliceCfg + 2, kSliceCfg + 3, kSliceCfg + 4 }) {
-                if (!usable(c) || (c != kTiled && slice_cost(c - kSliceCfg, false, m, p.N, k) > 1.5f * tile_cost(kTileCost[2], false, (int64_t)((m + 63) / 64) * ((p.N + 63) / 64), 1e-3f * k, 1e-6f * m * (float)(k + p.N))))
+            for (int c : { kTiled, tiled, kSliceCfg, kSliceCfg + 1, kSliceCfg + 2, kSliceCfg + 3, kSliceCfg + 4 }) {
+                if (!usable(c) || (c >= kSliceCfg && c < kSliceCfg + kSliceForms && slice_cost(c - kSliceCfg, false, m, p.N, k) > 1.5f * tile.cost))
                     continue;
-                if (c == kTiled)
+                if (best_ms == 1e30f)
                     tune_settle_clock([&] { launch(c); return true; });
                 launch(c);
                 const float ms = time_rounds(ea, eb, s, [&] { launch(c); });
@@ -1240,8 +1304,11 @@ fdx_status gemm_segments_launch(const float* a, const float* w, const float* bia
         if (eb)
             (void)hipEventDestroy(eb);
     }
-    if (!usable(cfg))
-        cfg = slice_pick(false, m, p.N, k, tile_cost(kTileCost[2], false, (int64_t)((m + 63) / 64) * ((p.N + 63) / 64), 1e-3f * k, 1e-6f * m * (float)(k + p.N)));
+    if (!usable(cfg)) {
+        cfg = slice_pick(false, m, p.N, k, tile.cost);
+        if (cfg < 0)
+            cfg = usable(tiled) ? tiled : kTiled;
+    }
     profile_begin();
     launch(cfg);
     profile_end("gemm_f32", 2.0 * m * (double)p.N * k, 0.0);

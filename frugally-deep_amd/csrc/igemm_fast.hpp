@@ -126,7 +126,7 @@ __device__ __forceinline__ int seg_of(const GemmParams& p, int n0) { return (n0 
 //    the lanes that share a row after the loop, and applied in the epilogue as
 //        rstd * (acc - mean * rowsum(B)) + bias:
 //    no pass over A of its own, and the normalised tensor never exists.
-//  * SEG (GEMM form, whole tiles only): the columns of C go to up to three tensors, the rows of each in sequences that lie
+//  * SEG (GEMM form): the columns of C go to up to three tensors, the rows of each in sequences that lie
 //    apart: the stacked query / key / value projection of prompts, keys and values straight into their cache rows (2048 rows, 768 -> 3 x 768:
 //    69 us instead of three launches of 29.6, which leave 384 tiles on 256 CUs each).
 //  * HALO (convolution whose map keeps its size, stride 1): K is walked channel slab by channel slab and tap by tap inside a
@@ -145,7 +145,7 @@ void igemm_fast_kernel(GemmParams p)
     static_assert(NT == 256 || NT == 512, "four or eight waves");
     static_assert(!DUAL || (!CONV && !SPLIT), "the two-source form is a whole-tile GEMM");
     static_assert(!LNF || (!CONV && !SPLIT && !DUAL), "the normalising form is a whole-tile GEMM");
-    static_assert(!SEG || (!CONV && !SPLIT && !DUAL && !LNF), "the form with segmented outputs is a whole-tile GEMM");
+    static_assert(!SEG || (!CONV && !DUAL && !LNF), "the form with segmented outputs is a GEMM");
     constexpr int BKT = 32;
     constexpr bool DB = split_tile_buffers(BM, BN, WAVES_M, WAVES_N) == 2;
     constexpr int RPP = NT / 4; // tile rows filled per loader pass: four lanes per row, two 16-byte chunks each

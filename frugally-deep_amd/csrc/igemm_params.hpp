@@ -52,7 +52,7 @@ struct GemmParams {
     // ln_wsum = per output column the sum of its (gamma-folded) filter row, nullptr = no normalisation
     const float* ln_wsum;
     float ln_eps;
-    // fast path, GEMM form, whole tiles (see SEG in igemm_fast.hpp): output columns [seg_col[i - 1], seg_col[i]) go to
+    // fast path, GEMM form (see SEG in igemm_fast.hpp): output columns [seg_col[i - 1], seg_col[i]) go to
     // seg_ptr[i], row m as row m % seg_rows of sequence m / seg_rows; C and ldc are not used
     float* seg_ptr[3];
     int64_t seg_ld[3], seg_stride[3]; // floats between rows of a sequence, between sequences

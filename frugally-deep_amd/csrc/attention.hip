@@ -293,7 +293,8 @@ __global__ __launch_bounds__(256) void flash_prefill_kernel(FlashParams p)
 //    accumulator registers: 16 s + 4 half + {0 .. 3, 8 .. 11}.
 //  * Scores and a tile's share of the output start from zero, small products first, and meet the running output in one
 //    multiply-add (its rescaling), so sums are rounded at their own size a few times per tile.
-//  * The scale of the scores is taken to base two, so a probability is one subtraction and one hardware exponential.
+//  * The scale of the scores is taken to base two, so a probability is one subtraction and one hardware exponential.  It also takes
+//    back the factor of the split operands; the output keeps it until the end.
 //  * A query whose result is not finite (infinite or NaN operands do not survive the split) is taken again in plain fp32.
 template <int D>
 __global__ __launch_bounds__(256, 2) void flash_split_kernel(FlashParams p)
@@ -387,7 +388,7 @@ __global__ __launch_bounds__(256, 2) void flash_split_kernel(FlashParams p)
 #pragma unroll
     for (int d = 0; d < D / 32; ++d)
         oacc[d] = kZero;
-    const float scale2 = p.scale * 1.44269504088896340736f;
+    const float scale2 = p.scale * 1.44269504088896340736f * kSplitDown;
     const int key_limit = p.causal ? (query + shift < p.s - 1 ? query + shift : p.s - 1) : p.s - 1;
     float m_run = -INFINITY, l_run = 0.f; // maximum in units of log2
 
@@ -496,7 +497,9 @@ __global__ __launch_bounds__(256, 2) void flash_split_kernel(FlashParams p)
 #pragma unroll
         for (int e = 0; e < 16; ++e)
             size += fabsf(oacc[d][e]);
+    float unscale = kSplitDown;
     if (__builtin_expect(q_ok && !(size < INFINITY), 0)) {
+        unscale = 1.f;
         // both halves of the lane pair may not come here together, so each walks the keys for itself
         auto score = [&](int key) {
             const float* krow_p = kbase + (int64_t)key * p.ldk;
@@ -527,7 +530,7 @@ __global__ __launch_bounds__(256, 2) void flash_split_kernel(FlashParams p)
         }
     }
     if (q_ok) {
-        const float inv = l_run > 0.f ? 1.0f / l_run : 0.f;
+        const float inv = l_run > 0.f ? unscale / l_run : 0.f;
         float* orow = p.out + (int64_t)b * p.o_batch + (int64_t)query * p.ldo + h * D + 4 * half;
 #pragma unroll
         for (int d = 0; d < D / 32; ++d)

@@ -422,42 +422,50 @@ void igemm_fast_kernel(GemmParams p)
         load_half(1, live);
     };
     float ln_shift[LNF ? A_UNITS : 1], ln_s[LNF ? A_UNITS : 1], ln_q[LNF ? A_UNITS : 1];
-    // eight floats of a row (chunks kq and 4 + kq of the slab) -> 16 bytes of each plane
-    auto put = [&](unsigned char* dst, int plane_bytes, const f32x4& lo, const f32x4& hi) {
-        const float x[8] = { lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3] };
-        u32x4 planes[3];
-        split3x8(x, planes);
+    // The slab's staging in steps of two floats: a thread's unit of eight (chunks kq and 4 + kq of a row, 16 bytes of each plane)
+    // is written behind its last pair.  Units of A come before those of B.
+    constexpr int A_PAIRS = 4 * A_UNITS, PAIRS = A_PAIRS + 4 * B_UNITS;
+    uint32_t planes[3][4];
+    auto stage_pair = [&](int i, int buf) {
+        const int unit = i / 4, e = i % 4, b_unit = unit < A_UNITS ? 0 : unit - A_UNITS, a_unit = unit < A_UNITS ? unit : 0;
+        const f32x4(&r)[2] = unit < A_UNITS ? ra[a_unit] : rb[b_unit];
+        split3(r[e >> 1][2 * (e & 1)] * kSplitUp, r[e >> 1][2 * (e & 1) + 1] * kSplitUp, planes[0][e], planes[1][e], planes[2][e]);
+        if (e == 3) {
+            unsigned char* dst = unit < A_UNITS ? smem_raw + buf * A_STEP + kq * A_BLK + (r0 + a_unit * RPP) * 16
+                                                : smem_raw + buf * B_STEP + A_BYTES + kq * B_BLK + (r0 + b_unit * RPP) * 16;
 #pragma unroll
-        for (int q = 0; q < 3; ++q)
-            *reinterpret_cast<u32x4*>(dst + q * plane_bytes) = planes[q];
+            for (int q = 0; q < 3; ++q)
+                *reinterpret_cast<u32x4*>(dst + q * (unit < A_UNITS ? 4 * A_BLK : 4 * B_BLK)) = u32x4 { planes[q][0], planes[q][1], planes[q][2], planes[q][3] };
+        }
     };
-    auto store_a = [&](int buf, bool first = false) {
-        if (LNF) {
+    // LNF: the statistics of the slab that is staged next
+    auto gather_rows = [&](bool first) {
 #pragma unroll
-            for (int i = 0; i < A_UNITS; ++i) {
-                if (first) {
-                    ln_shift[LNF ? i : 0] = ra[i][0][0];
-                    ln_s[LNF ? i : 0] = 0.f;
-                    ln_q[LNF ? i : 0] = 0.f;
-                }
+        for (int i = 0; i < (LNF ? A_UNITS : 0); ++i) {
+            if (first) {
+                ln_shift[LNF ? i : 0] = ra[i][0][0];
+                ln_s[LNF ? i : 0] = 0.f;
+                ln_q[LNF ? i : 0] = 0.f;
+            }
 #pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const float dlt = ra[i][e >> 2][e & 3] - ln_shift[LNF ? i : 0];
-                    ln_s[LNF ? i : 0] += dlt;
-                    ln_q[LNF ? i : 0] += dlt * dlt;
-                }
+            for (int e = 0; e < 8; ++e) {
+                const float dlt = ra[i][e >> 2][e & 3] - ln_shift[LNF ? i : 0];
+                ln_s[LNF ? i : 0] += dlt;
+                ln_q[LNF ? i : 0] += dlt * dlt;
             }
         }
+    };
+    auto store_a = [&](int buf) {
 #pragma unroll
-        for (int i = 0; i < A_UNITS; ++i)
-            put(smem_raw + buf * A_STEP + kq * A_BLK + (r0 + i * RPP) * 16, 4 * A_BLK, ra[i][0], ra[i][1]);
+        for (int i = 0; i < A_PAIRS; ++i)
+            stage_pair(i, buf);
         if (HALO && t < 12)
             *reinterpret_cast<u32x4*>(smem_raw + t * A_BLK + ROWS_A * 16) = u32x4 { 0u, 0u, 0u, 0u };
     };
     auto store_b = [&](int buf) {
 #pragma unroll
-        for (int i = 0; i < B_UNITS; ++i)
-            put(smem_raw + buf * B_STEP + A_BYTES + kq * B_BLK + (r0 + i * RPP) * 16, 4 * B_BLK, rb[i][0], rb[i][1]);
+        for (int i = A_PAIRS; i < PAIRS; ++i)
+            stage_pair(i, buf);
     };
 
     int tile = sk ? 0 : wg_in_xcd; // local unit index
@@ -484,7 +492,8 @@ void igemm_fast_kernel(GemmParams p)
                     acc[i][j][e] = acc_lo[i][j][e] = 0.f;
 
         const int kt_end = kt_n;
-        store_a(0, true);
+        gather_rows(true);
+        store_a(0);
         store_b(0);
         load_tiles(1 < kt_end);
         if (HALO)
@@ -523,21 +532,33 @@ void igemm_fast_kernel(GemmParams p)
                 for (int j = 0; j < TN; ++j)
                     d[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[s][i][x], bf[s][j][y], d[i][j], 0, 0, 0);
         };
-        auto multiply = [&](int s) {
+        // The six products of half a slab; pairs [from, to) of the next slab's staging are spread over those from number `first` on:
+        // a wave issues a product's MFMAs and splits floats while they run (the empty asm pins a pair to its place: without it
+        // the compiler moves the splitting together).  The slab's first products stand alone, its loads arrive meanwhile.
+        auto multiply = [&](int s, int from = 0, int to = 0, int buf = 0, int first = 0) {
             // the 256-row tile keeps A's plane from one product to the next (2.6 % faster: fewer operand changes, and power is
             // what bounds it); where the next half's operands are at hand the other order is 2 % faster
-            product(s, 0, 0, acc);
-            product(s, 0, 1, acc_lo);
-            if (!READ_AHEAD)
-                product(s, 0, 2, acc_lo);
-            product(s, 1, 0, acc_lo);
-            product(s, 1, 1, acc_lo);
-            if (READ_AHEAD)
-                product(s, 0, 2, acc_lo);
-            product(s, 2, 0, acc_lo);
+            constexpr int X[6] = { 0, 0, READ_AHEAD ? 1 : 0, 1, READ_AHEAD ? 0 : 1, 2 };
+            constexpr int Y[6] = { 0, 1, READ_AHEAD ? 0 : 2, READ_AHEAD ? 1 : 0, READ_AHEAD ? 2 : 1, 0 };
+#pragma unroll
+            for (int q = 0; q < 6; ++q) {
+                product(s, X[q], Y[q], q == 0 ? acc : acc_lo);
+                if (to == from || q < first)
+                    continue;
+                const int lo = from + (to - from) * (q - first) / (6 - first), hi = from + (to - from) * (q + 1 - first) / (6 - first);
+#pragma unroll
+                for (int i = lo; i < hi; ++i) {
+                    stage_pair(i, buf);
+                    asm volatile("" : "+v"(planes[0][i % 4]), "+v"(planes[1][i % 4]), "+v"(planes[2][i % 4]));
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
         };
-        // all slabs but the last: the next slab goes to LDS between the two halves of this one's products, and the one
-        // after that is requested into the registers this frees
+        // all slabs but the last: the next slab goes to LDS beside this one's products, and the one after that is requested into
+        // the registers this frees.  Staging spread over the products, against all MFMAs in front of all the splitting as the
+        // compiler orders them, in the tiles that keep two slabs and read ahead: 8192 x 1536 x 512 in 128 x 128 tiles 81 -> 77 us,
+        // 8192 x 512 x 2048 97 -> 91, 2048 x 768 x 3072 120 -> 101, 128 x 64 tiles 2 to 9 %, 64 x 64 2 %; the 256-row tile and the
+        // halo form gain nothing or lose 2 to 8 %.
         for (int kt = 0; kt + 1 < kt_end; ++kt) {
             const int buf = DB ? kt & 1 : 0;
             if (HALO) {
@@ -574,16 +595,22 @@ void igemm_fast_kernel(GemmParams p)
                 read_frags(0, buf);
                 if (READ_AHEAD)
                     read_frags(1, buf);
-                multiply(0);
-                store_a(buf ^ 1);
-                if (!READ_AHEAD)
+                gather_rows(false);
+                if (READ_AHEAD) {
+                    multiply(0, 0, PAIRS / 3, buf ^ 1, 3);
+                    multiply(1, PAIRS / 3, PAIRS, buf ^ 1);
+                } else {
+                    multiply(0);
+                    store_a(buf ^ 1);
                     read_frags(1, buf);
-                multiply(1);
-                store_b(buf ^ 1);
+                    multiply(1);
+                    store_b(buf ^ 1);
+                }
             } else {
                 read_frags(0, 0);
                 read_frags(1, 0);
                 __syncthreads();
+                gather_rows(false);
                 multiply(0);
                 store_a(0);
                 multiply(1);
@@ -759,6 +786,15 @@ void igemm_fast_kernel(GemmParams p)
                     }
             }
         }
+
+        // the factor of the split operands (partial tiles keep it: a result among the subnormal numbers is rounded once)
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+#pragma unroll
+                for (int e = 0; e < 16; ++e)
+                    acc[i][j][e] *= kSplitDown;
 
         // ---- epilogue: accumulators -> per-wave LDS scratch [32][WTN] -> 16-byte row accesses
         float* scratch = smem + wave * 32 * OSTRIDE;

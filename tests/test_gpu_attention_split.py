@@ -36,6 +36,26 @@ def test_against_64_bits(fdx, b, t, s, heads, d, causal):
     assert np.linalg.norm(got - want) / np.linalg.norm(want) <= 4e-5
 
 
+@pytest.mark.parametrize("d", [32, 64])
+def test_tiny_operands(fdx, d):
+    """Keys, queries, values and probabilities whose last bits lie below bf16's range: the bound of ordinary operands."""
+    b, t, heads = 16, 128, 8
+    r = np.random.default_rng(2)
+    q, k, v = (r.standard_normal((b, t, heads * d)).astype(np.float32) for _ in range(3))
+    for eq, ek, ev in ((120, -122, 0), (-122, 120, 0), (0, 0, -122), (127 - 8, -137, 0)):
+        print("attention split tiny", d, eq, ek, ev, flush=True)
+        x = [np.ldexp(a.astype(np.float64), e).astype(np.float32) for a, e in ((q, eq), (k, ek), (v, ev))]
+        got, want = fdx.mha_prefill(*x, heads, d, d), reference(*x, heads, False)
+        got = got.astype(np.float64)
+        assert np.linalg.norm(got - want) / np.linalg.norm(want) <= 1e-6, (d, eq, ek, ev)
+    # One key with probability 1 and value 0, the others' probabilities e^-84 and below, which make the whole output.  An exponent
+    # of 84 log2(e) = 121 is held to 2^-18 in fp32: 4e-6 of a probability.
+    q, k, v = np.zeros_like(q), np.zeros_like(k), v * np.float32(2.0 ** 60)
+    q[:, :, ::d], k[:, 1:, ::d], v[:, 0] = np.sqrt(d), -84 - r.random((b, t - 1, heads)), 0
+    got, want = fdx.mha_prefill(q, k, v, heads, d, d), reference(q, k, v, heads, False)
+    assert np.linalg.norm(got - want) / np.linalg.norm(want) <= 8e-6
+
+
 def test_infinities_and_nan(fdx):
     """Operands that the split cannot hold: the queries they reach get the values of plain sums, the others stay as they are."""
     print("attention split special", flush=True)

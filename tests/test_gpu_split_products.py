@@ -47,6 +47,29 @@ def test_gemm_edges(fdx, m, n, k, tile):
     assert np.array_equal(scaled, plain * np.float32(2.0 ** 10))
 
 
+# exponents of A's and of W's values: one side, or both, around the smallest normal and among the subnormal numbers
+@pytest.mark.parametrize("ea,ew", [(-122, 110), (110, -122), (-127, 115), (-140, 120), (120, -140), (-75, -65)])
+@pytest.mark.parametrize("tile", [13, 14, 15, 16, 18, 215, 20013] + HALO)
+def test_tiny_operands(fdx, tile, ea, ew):
+    """Operands whose last bits lie below bf16's range keep all of them: the bound of ordinary operands.  (Results below 2^-126
+    are rounded once to multiples of 2^-149, which the last term allows; the kernels on fp32 instructions, which the closed rule
+    takes for a problem as small as this, round every partial sum there.)"""
+    print("tiny operands", tile, ea, ew, flush=True)
+    r = np.random.default_rng(11)
+    m, n, k = 130, 68, 352
+    a = np.ldexp(r.standard_normal((m, k)), ea).astype(np.float32)
+    w = np.ldexp(r.standard_normal((n, k)) / np.sqrt(k), ew).astype(np.float32)
+    if tile in HALO:   # a 1x3 filter over rows of 130 positions, only its middle tap not zero
+        wc = np.zeros((n, 1, 3, k), np.float32)
+        wc[:, 0, 1] = w
+        got = forced(fdx, tile, lambda: fdx.conv2d(a.reshape(1, 1, m, k), wc, None, padding="same")).reshape(m, n)
+    else:
+        got = forced(fdx, tile, lambda: fdx.gemm(a, w))
+    a, w = a.astype(np.float64), w.astype(np.float64)
+    want, size = a @ w.T, np.abs(a) @ np.abs(w).T
+    assert (np.abs(got - want) <= (k / 16 + 8) * 2.0 ** -23 * size + 2.0 ** -148).all(), (np.abs(got - want) / size).max()
+
+
 def special(a, w):
     a[1, 3], a[2, -1], a[3, 0], a[4, 5] = np.inf, -np.inf, np.nan, 3.4e38   # 3.4e38 rounds up to an infinite bf16
     a[5, 2], a[5, -2] = np.inf, -np.inf

@@ -60,11 +60,16 @@ constexpr int split_tile_waves(int bm, int bn, int waves_m, int waves_n)
     return waves_m * waves_n == 8 || bm * bn > 64 * 64 ? 2 : 3;
 }
 
-// Element (m, n) of problem z as a plain fp32 sum over K: the value that infinite or NaN operands (or ones beyond the
-// largest bf16) give.
+// The elements of a 32 x 32 block (its accumulators, rows from m0, columns from n0, of problem z) that are not finite, again as
+// plain fp32 sums on the fp32 MFMA: what infinite or NaN operands, or ones beyond the largest split value, give.  Lane (row or
+// column fr, half fh) takes four consecutive k of eight at a time straight from memory.  A running sum that is NaN stays so: the
+// walk ends where all of the elements that it is for are.  One whole wave comes here.  (One lane per element and one k at a time
+// took 15 ms for 8192 x 2048 x 512 of NaN, 137 us this way; the product of finite operands 87.)
 template <bool CONV, bool DUAL>
-__device__ __forceinline__ float plain_dot(const GemmParams& p, int z, int m, int n)
+__device__ __forceinline__ void plain_block(const GemmParams& p, int z, int m0, int n0, f32x16& acc)
 {
+    const int lane = threadIdx.x & 63, fh = lane >> 5, m = m0 + (lane & 31), n = n0 + (lane & 31);
+    const bool m_ok = m < p.M, n_ok = n < p.N;
     const float* A = p.A + (z / p.inner) * p.a_outer + (z % p.inner) * p.a_inner;
     const float* B = p.B + (z / p.inner) * p.b_outer + (z % p.inner) * p.b_inner + (int64_t)n * p.ldb;
     const float* A2 = p.A2;
@@ -81,28 +86,56 @@ __device__ __forceinline__ float plain_dot(const GemmParams& p, int z, int m, in
     }
     if (!CONV)
         A += (int64_t)m * p.lda;
-    float s = 0.f;
+    f32x16 sum = { 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f };
     int fy = 0, fx = 0, c = 0;
-    const int k_end = p.a_valid_k > 0 ? p.a_valid_k : p.K;
+    const int k_end = p.a_valid_k > 0 ? p.a_valid_k : p.K; // a multiple of 4
 #pragma clang loop unroll(disable)
-    for (int k = 0; k < k_end; ++k) {
-        float a;
+    for (int k = 0; k < k_end; k += 16) { // sixteen k lie within one filter tap, and in one source
+        bool a_ok = m_ok;
+        const float* a_at = A + k;
         if (CONV) {
             const int iy = iy0 + fy * p.dy, ix = ix0 + fx * p.dx;
-            a = iy >= 0 && iy < p.H && ix >= 0 && ix < p.W ? A[((int64_t)fy * p.dy * p.W + fx * p.dx) * p.pix_stride + c] : 0.f;
-            if (++c == p.Cin) {
+            a_ok = m_ok && iy >= 0 && iy < p.H && ix >= 0 && ix < p.W;
+            a_at = A + ((int64_t)fy * p.dy * p.W + fx * p.dx) * p.pix_stride + c;
+            c += 16;
+            if (c == p.Cin) {
                 c = 0;
                 if (++fx == p.kw) {
                     fx = 0;
                     ++fy;
                 }
             }
-        } else {
-            a = DUAL && k >= p.K1 ? A2[k - p.K1] : A[k];
+        } else if (DUAL && k >= p.K1) {
+            a_at = A2 + (k - p.K1);
         }
-        s = fmaf(a, B[k], s);
+        f32x4 a[2], b[2];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int at = 8 * u + 4 * fh;
+            const bool in_k = k + at < k_end;
+            a[u] = b[u] = f32x4 { 0.f, 0.f, 0.f, 0.f };
+            if (a_ok && in_k)
+                a[u] = *reinterpret_cast<const f32x4*>(a_at + at);
+            if (n_ok && in_k)
+                b[u] = *reinterpret_cast<const f32x4*>(B + k + at);
+        }
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                sum = __builtin_amdgcn_mfma_f32_32x32x2f32(a[u][e], b[u][e], sum, 0, 0, 0);
+        if ((k & 48) == 48) {
+            bool open = false;
+#pragma unroll
+            for (int e = 0; e < 16; ++e)
+                open = open || (!(fabsf(acc[e]) < INFINITY) && sum[e] == sum[e]);
+            if (!__any(open))
+                break;
+        }
     }
-    return s;
+#pragma unroll
+    for (int e = 0; e < 16; ++e)
+        acc[e] = fabsf(acc[e]) < INFINITY ? acc[e] : sum[e];
 }
 
 // Where row m, column n of a tile whose first column is n0 lies with SEG, in bytes from the start of its segment; segments
@@ -815,9 +848,9 @@ void igemm_fast_kernel(GemmParams p)
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
             __builtin_amdgcn_wave_barrier();
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-            // Inf and NaN do not survive the split (Inf - Inf in the remainders), and a value that rounds up to an infinite
-            // bf16 makes one: such elements are summed again in plain fp32.  (A band of huge finite values may come here too
-            // and finds nothing to do.)
+            // Inf and NaN do not survive the split (Inf - Inf in the remainders), and a value from 2^112 on makes an infinite bf16:
+            // such elements are summed again in plain fp32.  (A band of huge finite values may come here too and finds nothing to
+            // do.)  Behind the transposition, where the band's accumulators are free.
             float size = 0.f;
 #pragma unroll
             for (int j = 0; j < TN; ++j)
@@ -826,11 +859,21 @@ void igemm_fast_kernel(GemmParams p)
                     size += fabsf(acc[i][j][e]);
             if (__builtin_expect(__any(!(size < INFINITY)), 0)) {
 #pragma clang loop unroll(disable)
-                for (int o = lane; o < 32 * WTN; o += 64) {
-                    const int m = em0 + wm * WTM + i * 32 + o / WTN, nn = en0 + wn * WTN + o % WTN;
-                    float& v = scratch[(o / WTN) * OSTRIDE + o % WTN];
-                    if (!(fabsf(v) < INFINITY) && m < p.M && nn < p.N)
-                        v = plain_dot<CONV, DUAL>(p, tile_done / per_problem, m, nn);
+                for (int j = 0; j < TN; ++j) {
+                    float* const block = scratch + 4 * fh * OSTRIDE + j * 32 + fr;
+                    f32x16 v;
+                    float block_size = 0.f;
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) {
+                        v[e] = block[(8 * (e >> 2) + (e & 3)) * OSTRIDE];
+                        block_size += fabsf(v[e]);
+                    }
+                    if (!__any(!(block_size < INFINITY)))
+                        continue;
+                    plain_block<CONV, DUAL>(p, tile_done / per_problem, em0 + wm * WTM + i * 32, en0 + wn * WTN + j * 32, v);
+#pragma unroll
+                    for (int e = 0; e < 16; ++e)
+                        block[(8 * (e >> 2) + (e & 3)) * OSTRIDE] = v[e];
                 }
                 __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
                 __builtin_amdgcn_wave_barrier();

@@ -80,3 +80,27 @@ def test_infinities_and_nan(fdx):
     assert np.allclose(got[2, neg, 64:128], want[2, neg, 64:128], rtol=1e-4, atol=1e-5) and np.isnan(got[2, ~neg, 64:128]).all()
     assert np.isinf(got[3, :, 128]).all() and np.allclose(got[3, :, 129:192], clean[3, :, 129:192], rtol=1e-4, atol=1e-5)
     assert np.allclose(got[4, :, 192:], want[4, :, 192:], rtol=1e-4, atol=1e-5)
+
+
+@pytest.mark.parametrize("d", [32, 64])
+def test_infinities_under_the_causal_mask(fdx, d):
+    """A query takes no part of a key that it may not see, whatever the key and its value hold; in a wave of 32 queries any number
+    may be taken again, four at a time."""
+    print("attention split causal special", d, flush=True)
+    b, t, heads = 16, 150, 8         # enough queries for the kernel with split operands
+    r = np.random.default_rng(3)
+    q, k, v = (r.standard_normal((b, t, heads * d)).astype(np.float32) for _ in range(3))
+    clean = fdx.mha_prefill(q, k, v, heads, d, d, causal=True)
+    k[0, 71, 0] = np.nan             # sequence 0, head 0: queries from 71 on are NaN
+    v[1, 100, 1] = np.inf            # sequence 1, head 0, depth 1: infinite from 100 on
+    q[2, [3, 40, 41, 77, 78, 79, 80, 149], 0] = np.nan
+    got = fdx.mha_prefill(q, k, v, heads, d, d, causal=True)
+    same = np.ones((b, t, heads * d), bool)
+    same[0, 71:, :d] = same[1, 100:, :d] = same[2, [3, 40, 41, 77, 78, 79, 80, 149], :d] = False
+    assert np.isnan(got[0, 71:, :d]).all() and np.isnan(got[2, [3, 40, 41, 77, 78, 79, 80, 149], :d]).all()
+    assert np.isposinf(got[1, 100:, 1]).all()
+    rest = [0] + list(range(2, d))
+    assert np.allclose(got[1, 100:, rest], clean[1, 100:, rest], rtol=1e-4, atol=1e-5)
+    # a tile of 64 keys holds values that some of its queries may not see: those are taken again, to fp32 sums in another order
+    assert np.allclose(got[same], clean[same], rtol=1e-4, atol=1e-5)
+    assert np.array_equal(got[3:], clean[3:])

@@ -660,6 +660,40 @@ static TileChoice tile_pick(bool conv, int M, int N, int K, int64_t a_floats, bo
     return best;
 }
 
+// The closed rule of all forms of the fast path: a tile of the rule above, or a form of the kernel for few tiles.
+static TileChoice fast_pick(bool conv, int M, int N, int K, int64_t a_floats, bool residual, int batch, bool cuts, bool halo)
+{
+    TileChoice best = tile_pick(conv, M, N, K, a_floats, residual, batch, cuts, halo);
+    const int slice = batch == 1 ? slice_pick(conv, M, N, K, best.cost) : -1;
+    if (slice >= 0)
+        best = { slice, 1, 0, slice_cost(slice - kSliceCfg, conv, M, N, K) };
+    return best;
+}
+
+// The general kernel's tile for a problem outside the fast path.
+static int general_pick(int M, int N, int batch)
+{
+    auto blocks = [&](int bm, int bn) { return (int64_t)((M + bm - 1) / bm) * ((N + bn - 1) / bn) * batch; };
+    if (N <= 32)
+        return 2;
+    if (N <= 64)
+        return blocks(128, 64) >= 512 ? 1 : 3;
+    return blocks(128, 128) >= 512 ? 0 : blocks(128, 64) >= 512 ? 1 : 3;
+}
+// Its predicted time, fitted to 245 3x3 convolutions of 8 to 200 channels that are no multiple of 16 (3 to 4 % rms):
+//     t0 + w (e + a k) + f t + b k t + g k,  t = tiles / CUs, w = t rounded up, k = K / 1000.
+static float general_cost(int M, int N, int K)
+{
+    const int cfg = general_pick(M, N, 1);
+    static const float kCost[4][6] = { { 8.11f, 2.65f, 67.1f, 0.f, 16.2f, 0.f }, { 4.14f, 1.49f, 31.1f, 0.f, 12.5f, 0.f },
+        { 4.14f, 1.49f, 31.1f, 0.f, 12.5f, 0.f }, { 3.45f, 0.34f, 14.6f, 0.65f, 1.2f, 20.f } }; // cfg 2: not fitted, no 3x3 filter needs it
+    const int bm = cfg == 3 ? 64 : 128, bn = cfg == 0 ? 128 : cfg == 2 ? 32 : 64;
+    const int64_t tiles = (int64_t)((M + bm - 1) / bm) * ((N + bn - 1) / bn);
+    const float k = 1e-3f * BK * (float)((K + BK - 1) / BK), t = (float)tiles / 256.f, w = (float)((tiles + 255) / 256);
+    const float* c = kCost[cfg];
+    return c[0] + w * (c[1] + c[2] * k) + t * (c[3] + c[4] * k) + c[5] * k;
+}
+
 // whether the closed rule may cut K (FDX_CLOSED_SPLIT=0: whole tiles)
 static bool closed_cuts()
 {
@@ -981,10 +1015,7 @@ static fdx_status run_igemm(GemmParams& p, bool conv, int batch, const char* fam
         splits = 1;
         mode = 0;
         if (cfg < 0) {
-            const TileChoice tile = tile_pick(conv, p.M, p.N, p.K, (int64_t)p.M * p.K, false, 1, false);
-            cfg = slice_pick(conv, p.M, p.N, p.K, tile.cost);
-            if (cfg < 0)
-                cfg = tile.cfg;
+            cfg = fast_pick(conv, p.M, p.N, p.K, (int64_t)p.M * p.K, false, 1, false, false).cfg;
         }
     } else if (cfg < 0) {
         if (fast_ok && p.N >= 16 && 2.0 * p.M * (double)p.N * p.K * batch >= 2e8) {
@@ -1001,32 +1032,22 @@ static fdx_status run_igemm(GemmParams& p, bool conv, int batch, const char* fam
                 [&] { pw_stream_launch(p, a_bytes, b_bytes, s); });
             settle();
         }
-        TileChoice tile { -1, 1, 0, 1e30f };
-        if (cfg < 0 && fast_ok) {
-            tile = tile_pick(conv, p.M, p.N, p.K, conv ? a_bytes / 4 : (int64_t)p.M * p.K, p.residual != nullptr, batch, closed_cuts(),
+        TileChoice choice { -1, 1, 0, 1e30f };
+        if (cfg < 0 && fast_ok)
+            choice = fast_pick(conv, p.M, p.N, p.K, conv ? a_bytes / 4 : (int64_t)p.M * p.K, p.residual != nullptr, batch, closed_cuts(),
                 halo_ok(p, conv) && p.kh * p.kw >= 6);
-            if (batch == 1)
-                cfg = slice_pick(conv, p.M, p.N, p.K, tile.cost);
-        }
         if (cfg >= 0) {
-        } else if (stream_ok && p.K <= 32 && p.N <= 160 && p.M >= 65536) {
+        } else if (choice.cfg < kSliceCfg && stream_ok && p.K <= 32 && p.N <= 160 && p.M >= 65536) {
             // very short rows over a long map (MobileNetV2's first expansions): the row-streaming kernel
             cfg = kStreamCfg;
-        } else if (fast_ok && p.N > 32) {
-            cfg = tile.cfg;
-            splits = tile.splits;
-            mode = tile.mode;
+        } else if (fast_ok && (p.N > 32 || choice.cfg >= kSliceCfg)) {
+            cfg = choice.cfg;
+            splits = choice.splits;
+            mode = choice.mode;
             settle(); // a cut needs its workspace
-        } else if (p.N <= 32)
-            cfg = 2;
-        else if (p.N <= 64)
-            cfg = blocks(128, 64) >= 512 ? 1 : 3;
-        else if (blocks(128, 128) >= 512)
-            cfg = 0;
-        else if (blocks(128, 64) >= 512)
-            cfg = 1;
-        else
-            cfg = 3;
+        } else {
+            cfg = general_pick(p.M, p.N, batch);
+        }
     }
 
     if (cfg < 10 && p.a_valid_k > 0) { // only the buffer loads of the fast path stop at the real extent
@@ -1339,16 +1360,16 @@ extern "C" fdx_status fdx_debug_persist_cap(int workgroups)
 }
 
 namespace fdx {
-// Predicted time (us) of a 3x3 stride-1 convolution as a direct sum, by the closed rule's costs.
+// Predicted time (us) of a 3x3 stride-1 convolution as a direct sum: of the kernel that run_igemm launches by its closed rules (the
+// general one where the channels are no multiple of 16 or a tensor lies beyond the fast path's 2 GiB).
 float conv3x3_direct_cost(int n, int h, int w, int cin, int cout, int oh, int ow, bool residual)
 {
     const int64_t m = std::min<int64_t>((int64_t)n * oh * ow, INT32_MAX); // larger ones are refused by either kernel
+    const int64_t a_floats = (int64_t)n * h * w * cin;
+    if (cin % 16 != 0 || cout % 4 != 0 || a_floats + (int64_t)(w + 1) * cin >= (1LL << 29) - 16 || (int64_t)cout * 9 * cin >= (1LL << 29))
+        return general_cost((int)m, cout, 9 * cin);
     const bool halo = oh == h && ow == w && cin % kSlab == 0 && 2 * w + 2 <= kHaloSpan;
-    const TileChoice tile = tile_pick(true, (int)m, cout, 9 * cin, (int64_t)n * h * w * cin, residual, 1, true, halo);
-    float best = tile.cost;
-    for (int i = 0; i < kSliceForms; ++i)
-        best = std::min(best, slice_cost(i, true, (int)m, cout, 9 * cin));
-    return best;
+    return fast_pick(true, (int)m, cout, 9 * cin, a_floats, residual, 1, closed_cuts(), halo).cost;
 }
 } // namespace fdx
 

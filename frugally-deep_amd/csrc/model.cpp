@@ -1792,18 +1792,22 @@ extern "C" fdx_status fdx_debug_force_chain(int mode)
     return FDX_OK;
 }
 
-// test hook: -1 = a plan times the direct and the Winograd kernel of a 3x3 stride-1 convolution, 0 = always direct, 1 = Winograd
-// wherever it applies
-// Direct sum or Winograd form of a 3x3 stride-1 convolution by predicted cost.  Of 220 timed ones (maps of 6 to 62 pixels, 32 to
-// 512 channels, batches of 1 to 64) the choice takes 2 % longer than the faster form on average; Winograd from a gigaflop of
-// direct-sum work on, the line before the direct kernel took its products to the bf16 matrix instructions, took 11 % longer
-// (5 images, 32 x 32 x 256 -> 64: direct 22.5 us, Winograd 37.6; 24 images, 40 x 40 x 512 -> 64: 133 / 115).  The direct kernel
-// draws more power, which the layers around it pay for with clock: 3 % against it.
+// Direct sum or Winograd form of a 3x3 stride-1 convolution by predicted cost.  Of 300 timed ones that the costs were not fitted to
+// (maps of 6 to 62 pixels, 8 to 512 channels, batches of 1 to 64) the choice takes 0.6 % longer than the faster form on average, at
+// worst 21 %; Winograd from a gigaflop of direct-sum work on takes 8 %, always the direct kernel 13 % (36 % where the channels
+// are no multiple of 16: 8 images, 56 x 56 x 56 -> 128: direct 49.6 us, Winograd 31.2; 16 of 56 x 56 x 64 -> 64 29.7 / 35.1).  The
+// direct kernel draws more power, which the layers around it pay for with clock: 3 % against it.
 static bool winograd_by_rule(int n, int h, int w, int cin, int cout, int oh, int ow, bool residual)
 {
     return conv2d_winograd_cost(n, cin, cout, oh, ow) < 1.03f * conv3x3_direct_cost(n, h, w, cin, cout, oh, ow, residual);
 }
+extern "C" int fdx_debug_conv3x3_form(int n, int h, int w, int cin, int cout)
+{
+    return fdx_conv2d_winograd_supported(cin, cout) && winograd_by_rule(n, h, w, cin, cout, h, w, false) ? 1 : 0;
+}
 
+// test hook: -1 = a plan takes the direct or the Winograd kernel of a 3x3 stride-1 convolution by the rule (or times both, where
+// timing is asked for), 0 = always direct, 1 = Winograd wherever it applies
 static int g_force_winograd = -1;
 
 extern "C" fdx_status fdx_debug_force_winograd(int mode)

@@ -362,14 +362,29 @@ __global__ __launch_bounds__(256, 2) void wino_kernel(WinoParams p)
     }
 }
 
-// Predicted time (us), fitted to 220 convolutions of 0.1-25 GFLOP on maps of 6 to 62 pixels (10 % rms): a fixed part, the
-// exchange between the workgroups that share a unit, the filter out of memory, the steps.
+// How a launch's steps (8 input channels of a unit) are dealt to workgroups, every one at least four: two workgroups fit on a CU.
+// The second one pays where units are short (64 input channels: 8 steps per unit, -9 %; 128: -3 %): the end of one's unit runs
+// under the other's steps.  Units of 32 and 64 steps gain nothing there and lose 2-8 % to the shares of the units that twice as
+// many stretches cut: one workgroup per CU for them.  (The steps themselves do not get faster with a second wave on the SIMD:
+// their loads -- 16 per 32 MFMAs, the patch pieces 32 lines per instruction -- keep the CU's vector memory path as busy as the
+// MFMAs keep the matrix pipe.)
+static int wino_grid(int64_t total_steps, int cin, int cus)
+{
+    return (int)std::min<int64_t>(std::max<int64_t>(total_steps / 4, 1), cin <= 128 ? 2 * cus : cus);
+}
+
+// Predicted time (us), fitted to 750 convolutions of 8 to 512 channels and 0.1-25 GFLOP on maps of 6 to 62 pixels (9 % rms, within
+// 12 % on average at every channel count): a fixed part, more where workgroups' stretches cut units, the steps of a CU, the unit
+// ends of a CU, the exchange between the workgroups that share a unit.  16 images of 56 x 56 x 64 -> 64: 34.3, measured 35.1.
 float conv2d_winograd_cost(int n, int cin, int cout, int oh, int ow)
 {
-    const double tiles = (double)n * ((oh + 1) / 2) * ((ow + 1) / 2), units = std::ceil(tiles / WINO_TM) * (cout / 64);
-    const double spu = cin / 8, steps = units * spu, grid = std::min(std::max(std::floor(steps / 4), 1.0), cin <= 128 ? 512.0 : 256.0);
-    const double per = std::ceil(steps / grid);
-    return (float)(7.0 + 3.16 * std::max(spu / per, 1.0) + 0.53e-6 * cin * cout + 1.5 * steps / 256.0);
+    const int64_t tiles = (int64_t)n * ((oh + 1) / 2) * ((ow + 1) / 2), units = (tiles + WINO_TM - 1) / WINO_TM * (cout / 64), spu = cin / 8;
+    constexpr int cus = 256;
+    const int64_t total = units * spu, grid = wino_grid(total, cin, cus), per = total / grid, longer = total % grid;
+    const bool cut = per % spu != 0 || longer != 0;
+    const double most = (double)(per + (longer != 0)), on_cu = (double)((grid + cus - 1) / cus);
+    return (float)(4.68 + (cut ? 4.58 : 0.0) + 1.264 * most * on_cu + 1.734 * (most / (double)spu + (cut ? 1.0 : 0.0)) * on_cu
+        + 2.55 * std::max((double)spu / (double)per - 1.0, 0.0));
 }
 
 static size_t wino_lds_bytes(int nt) { return sizeof(float) * (size_t)8 * WINO_TM * (nt * 32 + WINO_PAD) + sizeof(int) * 2 * WINO_TM; }
@@ -509,14 +524,7 @@ extern "C" fdx_status fdx_conv2d_winograd_nhwc_f32(const float* in, int n, int h
     // every workgroup gets at least four steps; none gets an empty stretch
     const int64_t total_steps = (int64_t)p.units * (cin / 8);
     FDX_WINO_LIMIT(total_steps < (1LL << 30), "conv2d_winograd: too many steps for one launch");
-    const int64_t by_steps = total_steps / 4 > 0 ? total_steps / 4 : 1;
-    // Two workgroups fit on a CU.  The second one pays where units are short (64 input channels: 8 steps per unit, -9 %;
-    // 128: -3 %): the end of one's unit runs under the other's steps.  Units of 32 and 64 steps gain nothing there and
-    // lose 2-8 % to the shares of the units that twice as many stretches cut: one workgroup per CU for them.  (The
-    // steps themselves do not get faster with a second wave on the SIMD: their loads -- 16 per 32 MFMAs, the patch
-    // pieces 32 lines per instruction -- keep the CU's vector memory path as busy as the MFMAs keep the matrix pipe.)
-    const int resident = cin <= 128 ? g_wino_grid : g_wino_grid / 2;
-    const dim3 grid((unsigned)(by_steps < resident ? by_steps : resident));
+    const dim3 grid((unsigned)wino_grid(total_steps, cin, g_wino_grid / 2));
     p.per_wg = (int)(total_steps / grid.x);
     p.longer = (int)(total_steps % grid.x);
     const size_t lds = wino_lds_bytes(nt);

@@ -81,3 +81,19 @@ def test_model_check_runs_without_a_gpu(fdx, modelgen):
         fdx.model_check(b'{"image_data_format": "channels_first"}')
     with pytest.raises(fdx.FdxError):
         fdx.model_check(b'{"image_data_format": "channels_last", "architecture": {')
+
+
+@pytest.mark.parametrize("n,h,w,cin,cout,form", [
+    # measured, direct against Winograd kernel in us; channels that are no multiple of 16 run the general kernel as a direct sum
+    (8, 56, 56, 56, 128, 1),     # 49.6 / 31.2
+    (7, 26, 35, 104, 512, 1),    # 85.5 / 41.8
+    (1, 36, 59, 200, 128, 1),    # 67.0 / 35.0
+    (16, 28, 28, 72, 128, 1),    # 36.8 / 29.2
+    (16, 56, 56, 64, 64, 0),     # 29.7 / 35.1
+    (16, 28, 28, 128, 128, 0),   # 29.4 / 38.7
+    (4, 15, 15, 320, 128, 0),    # 12.7 / 39.6
+    (27, 36, 36, 320, 64, 1),    # 107 / 69
+])
+def test_direct_or_winograd(n, h, w, cin, cout, form):
+    lib = ctypes.CDLL(os.path.join(ROOT, "frugally-deep_amd", "libfdx.so"))
+    assert lib.fdx_debug_conv3x3_form(n, h, w, cin, cout) == form

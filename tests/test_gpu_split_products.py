@@ -2,8 +2,9 @@
 bf16 values on the bf16 matrix instructions.
 
 Error bound: every 16 steps of K round the main sum once (at most 2^-24 of the running sum, itself at most the sum of the
-magnitudes S), the small products' sum and the final add a few times more, the products left out are below 3 * 2^-26 S; twice
-that is allowed: (K / 16 + 8) 2^-23 S for an element.  For the 2-norm, where roundings average out, twice what operands of
+magnitudes S); the products left out are at most 2^-24 S (the second part of a value is at most 2^-8 of it, the third 2^-17, so
+a1 b2 and a2 b1 are 2^-25 of a b each; 2^-27.5 on average); bias, residual, the sum with the small products and those of partial
+tiles round a few times more, seven are allowed for; twice all that: (K / 16 + 8) 2^-23 S for an element.  For the 2-norm, where roundings average out, twice what operands of
 unit variance show against 64 bits (6e-9 sqrt(K))."""
 import zlib
 
@@ -45,6 +46,21 @@ def test_gemm_edges(fdx, m, n, k, tile):
     # the split does not depend on the operands' scale
     scaled = forced(fdx, tile, lambda: fdx.gemm(a * np.float32(2.0 ** 60), w * np.float32(2.0 ** -50)))
     assert np.array_equal(scaled, plain * np.float32(2.0 ** 10))
+
+
+@pytest.mark.parametrize("tile", [13, 14, 15, 16, 18, 215, 20013])
+@pytest.mark.parametrize("k", [16, 352])
+def test_left_out_products_that_add_up(fdx, tile, k):
+    """All operands close to 1 + 2^-8 - 2^-17, whose parts are the largest there are and have one sign: the products left out are
+    2^-24.02 of every product and do not average out.  Undoubled bound of an element."""
+    print("left out products", tile, k, flush=True)
+    r = np.random.default_rng(12)
+    m, n = 130, 68
+    near = lambda *shape: (float.fromhex("0x1.00fe8p0") + r.integers(-2, 3, shape) * 2.0 ** -23).astype(np.float32)
+    a, w = near(m, k), near(n, k)
+    got = forced(fdx, tile, lambda: fdx.gemm(a, w))
+    want = a.astype(np.float64) @ w.astype(np.float64).T
+    assert (np.abs(got - want) <= (k / 16 + 8) * 2.0 ** -24 * want).all()
 
 
 # exponents of A's and of W's values: one side, or both, around the smallest normal and among the subnormal numbers
@@ -201,6 +217,38 @@ def test_convolution_halo(fdx, n, h, w, cin, cout, kh, kw, dil, tile):
     conv = lambda a, f: torch.nn.functional.conv2d(a, f.permute(0, 3, 1, 2), dilation=dil).permute(0, 2, 3, 1).numpy()
     want, size = conv(xp, torch.from_numpy(wc).double()) + b + res, conv(xp.abs(), torch.from_numpy(wc).double().abs()) + np.abs(b) + np.abs(res)
     k = kh * kw * cin
+    assert (np.abs(got - want) <= (k / 16 + 8) * 2.0 ** -23 * size).all()
+    assert np.linalg.norm(got - want) <= (1.2e-8 * np.sqrt(k) + 1.2e-7) * np.linalg.norm(want)
+    assert np.array_equal(got, again)
+
+
+@pytest.mark.parametrize("cap", [8, 10])
+@pytest.mark.parametrize("tile", [23, 24, 28, 223, 424, 228, 10223, 10323, 10224, 10228])
+@pytest.mark.parametrize("kh,kw,cin,dil", [(3, 3, 64, 1), (1, 3, 128, 2), (3, 2, 96, 1)])
+def test_convolution_halo_several_tiles_a_workgroup(fdx, kh, kw, cin, dil, tile, cap):
+    """A grid of `cap` workgroups: each walks to tiles of another place and of another column block, the next tile's pixels requested
+    in front of the epilogue of the one before; the hybrid cuts leave whole tiles and a cut remainder (27 tiles of 128 x 128, 45 of
+    128 x 64, 15 of 256 x 128)."""
+    import torch
+    n, h, w, cout = 3, 20, 19, 260
+    bm, bn = {3: (128, 128), 4: (128, 64), 8: (256, 128)}[tile % 10]
+    tiles, splits = -(-n * h * w // bm) * -(-cout // bn), tile % 10000 // 100
+    assert tiles > cap and tiles % cap != 0 and (splits == 0 or kh * kw * cin // 32 >= 2 * splits)   # the cut is not refused
+    print("halo, several tiles", kh, kw, cin, dil, tile, cap, flush=True)
+    r = np.random.default_rng(zlib.crc32(repr((kh, kw, cin)).encode()))
+    x = r.standard_normal((n, h, w, cin)).astype(np.float32)
+    k = kh * kw * cin
+    wc = (r.standard_normal((cout, kh, kw, cin)) / np.sqrt(k)).astype(np.float32)
+    b, res = r.standard_normal(cout).astype(np.float32), r.standard_normal((n, h, w, cout)).astype(np.float32)
+    fdx.lib.fdx_debug_persist_cap(cap)
+    try:
+        got, again = forced(fdx, tile, lambda: [fdx.conv2d(x, wc, b, dilation=(dil, dil), padding="same", residual=res) for _ in range(2)])
+    finally:
+        fdx.lib.fdx_debug_persist_cap(0)
+    eh, ew = (kh - 1) * dil, (kw - 1) * dil
+    xp = torch.nn.functional.pad(torch.from_numpy(x).double().permute(0, 3, 1, 2), (ew // 2, ew - ew // 2, eh // 2, eh - eh // 2))
+    conv = lambda a, f: torch.nn.functional.conv2d(a, f.permute(0, 3, 1, 2), dilation=dil).permute(0, 2, 3, 1).numpy()
+    want, size = conv(xp, torch.from_numpy(wc).double()) + b + res, conv(xp.abs(), torch.from_numpy(wc).double().abs()) + np.abs(b) + np.abs(res)
     assert (np.abs(got - want) <= (k / 16 + 8) * 2.0 ** -23 * size).all()
     assert np.linalg.norm(got - want) <= (1.2e-8 * np.sqrt(k) + 1.2e-7) * np.linalg.norm(want)
     assert np.array_equal(got, again)

@@ -852,12 +852,12 @@ static int autotune(const GemmParams& q, bool conv, int batch, hipStream_t s, in
                     best = cfg;
                 }
             } else {
-                // What a cut costs beyond its own time: partial tiles written and read back (K ranges, and the last
-                // round of the hybrid form), and in the stream-K form every tile's operands fetched at a K phase of
-                // its own, so that tiles of one row block no longer share them in L2 (measured on ResNet50's
-                // 14 x 14 and 7 x 7 1x1 layers: 3.7 times the algorithmic bytes).  A cut has to win by more than that
-                // handicap to be taken: 4 % of its time for K ranges, 15 % for stream-K (which wins by 9 % on those 1x1
-                // layers, by 15-20 % on deep 3x3 convolutions and by more on a Dense with few rows).
+                // What a cut costs beyond its own time: partial tiles written and read back, and in the stream-K form every
+                // tile's operands fetched at a K phase of its own, so that tiles of one row block no longer share them in L2.
+                // Here the forms are timed alone, with operands that the launch before left in the caches, hence more than the
+                // 2 to 4 % of the closed rule.  With the closed rule's charges timed passes took longer or the same: ResNet50
+                // batch 64 3870 -> 3904 us, 16 from host memory 1749 -> 1752, MobileNetV2 batch 128 1589 -> 1607, encoder 32 x 256 and
+                // prompts 16 x 128 within 0.1 %.
                 const float score = ms * (mode == 2 ? 1.15f : 1.04f);
                 if (score < best_split_ms) {
                     best_split_ms = score;
@@ -999,7 +999,7 @@ static fdx_status run_igemm(GemmParams& p, bool conv, int batch, const char* fam
         if (cfg < 0)
             cfg = (p.K >= 1024 && p.N % 128 == 0 && blocks(128, 128) >= 2048) ? 13 : 15;
     } else if (p.A2) {
-        // two-source rows: whole tiles of the four-wave fast kernel only, nothing timed
+        // two-source rows: whole tiles (any size) or a few-tiles form, nothing timed
         const int64_t a2_bytes = (int64_t)(p.OH > 0 && p.OW > 0 ? p.M / (p.OH * p.OW) : 0) * p.H2 * p.W2 * p.C2 * 4;
         const bool dual_ok = !conv && batch == 1 && fast_ok && p.a_valid_k == 0 && aligned16(p.A2) && p.C2 % 4 == 0 && p.K1 > 0
             && p.K1 % 16 == 0 && p.K > p.K1 && (p.K - p.K1) % 16 == 0 && p.K - p.K1 <= p.C2 && a2_bytes > 0 && a2_bytes < (1LL << 31)

@@ -5,14 +5,16 @@
 //
 //  * The fp32 MFMA (157 TFLOP/s) is what bounds this work; the bf16 one has 16 times its rate.  An fp32 value is exactly
 //    the sum of three bf16 values (8 + 8 + 8 bits, each the rounding of what the ones before leave), so a product of two
-//    is nine bf16 products, of which the three smallest (a1 b2, a2 b1, a2 b2 with planes counted from 0: 2^-27 of the
-//    result and below) are left out: six MFMAs for sixteen steps of K instead of eight fp32 ones of twice the length.
+//    is nine bf16 products, of which the three smallest (a1 b2, a2 b1, a2 b2 with planes counted from 0) are left out: six
+//    MFMAs for sixteen steps of K instead of eight fp32 ones of twice the length.  They are at most 2^-24 of the product
+//    (2^-24.02 for two operands of 0x1.00fe8p0), 2^-27.5 on average, with either sign: a sum that is one product is off by up to
+//    1.5 roundings of fp32 where the fp32 MFMA is off by one, longer ones are closer than there.
 //    The MFMA adds exact products in fp32, to nearest.  The leading product has accumulators of its own, so a result is
 //    rounded at its own size once per 16 steps of K where the fp32 MFMA does so eight times: against 64-bit sums the
 //    relative error (2-norm, normal operands, K = 64 / 512 / 4608) is 0.5 / 1.3 / 4.2 e-7, with the fp32 MFMA 1.4 / 4.1 / 12 e-7.
-//    8192 x 2048 x 512: 147 -> 93 us, 186 TFLOP/s; with nothing but its MFMAs the kernel runs at 302 and the clock falls to
+//    8192 x 2048 x 512: 147 -> 88.5 us, 194 TFLOP/s; with nothing but its MFMAs the kernel runs at 302 and the clock falls to
 //    1.9 GHz: the power limit, not the issue rate, is the next bound.
-//  * Both operands are split by the threads that stage them, on the way from registers to LDS (5.5 vector instructions a
+//  * Both operands are split by the threads that stage them, on the way from registers to LDS (6.5 vector instructions a
 //    value, hidden behind the MFMAs): operands stay fp32 in memory, nothing is prepared or kept.  Splitting the filter once
 //    at load instead was measured slower (half as many vector instructions, but 6 bytes a value through L2 instead of 4).
 //  * A row of a slab (32 floats) is fetched by four lanes, two 16-byte chunks each (k = 4q.. and 16 + 4q.. for lane q); the
@@ -22,15 +24,16 @@
 //    wave's writes meet each bank once.
 //  * The largest four-wave tile keeps one slab in LDS (two workgroups on a CU then: one's staging beside the other's
 //    products); its operands go to registers in front of a barrier.  The others keep two.
-//  * Workgroups are persistent:
-//
+//  * Registers: 256 a lane bound the larger tiles.  The 256-row tile keeps 4 to 8 values in scratch memory, its halo form 21, none
+//    of them touched in the K loop but one; the four-wave 128 x 128 tile keeps 32 to 60, of which its plain form reads 35 back per
+//    slab and its column-segment form 32.  The cost rule was fitted to them as they are.
 //  * Operands are fetched with raw buffer loads: each lane keeps ONE 32-bit byte offset per
 //    tile row for the whole K loop, the walk along K is a scalar offset shared by the
 //    workgroup (filter tap and channel are uniform within a slab), and a padded or
 //    out-of-range tap is an offset beyond the buffer's extent, which the hardware answers
 //    with zeros -- no branches, no per-slab address arithmetic.  A's base is shifted down by
 //    the top-left padding so offsets stay non-negative.
-//  * A workgroup walks a strided list of output tiles.  Before it writes a finished tile it
+//  * Workgroups are persistent: each walks a strided list of output tiles.  Before it writes a finished tile it
 //    already has the first slab of its next tile in flight, and the tile's stores drain while
 //    the next tile computes: output traffic and first-load latency overlap with MFMA work
 //    instead of adding to it (with one tile per workgroup all workgroups of a round reach
@@ -160,8 +163,8 @@ __device__ __forceinline__ int seg_of(const GemmParams& p, int n0) { return (n0 
 //        rstd * (acc - mean * rowsum(B)) + bias:
 //    no pass over A of its own, and the normalised tensor never exists.
 //  * SEG (GEMM form): the columns of C go to up to three tensors, the rows of each in sequences that lie
-//    apart: the stacked query / key / value projection of prompts, keys and values straight into their cache rows (2048 rows, 768 -> 3 x 768:
-//    69 us instead of three launches of 29.6, which leave 384 tiles on 256 CUs each).
+//    apart: the stacked query / key / value projection of prompts, keys and values straight into their cache rows (2048 rows,
+//    768 -> 3 x 768: 54 us in the stream-K form; three launches of 768 columns each leave 96 tiles of 128 x 128 on 256 CUs).
 //  * HALO (convolution whose map keeps its size, stride 1): K is walked channel slab by channel slab and tap by tap inside a
 //    slab, and a slab of A is the run of input pixels that all taps of the tile's rows touch (rows of a tile are neighbours in
 //    raster order, so is what they read: BM + (kh - 1) dy W + (kw - 1) dx pixels).  It is fetched and split once for all taps
@@ -663,7 +666,7 @@ void igemm_fast_kernel(GemmParams p)
                 read_frags(1, buf);
             multiply(1);
             if (LNF) {
-                // Every slab has passed through store_tiles by now, so every thread has seen 8 * KT values of each of its
+                // Every slab has passed through gather_rows by now, so every thread has seen 8 * KT values of each of its
                 // rows.  The four lanes that share a row (a quad) merge their means and sums of
                 // squared deviations pairwise, equal counts on both sides at each step, on the VALU's lane swaps.  Done here,
                 // behind the last slab's MFMAs and in front of the barrier below, it costs no barrier of its own.
@@ -783,8 +786,8 @@ void igemm_fast_kernel(GemmParams p)
                 continue;
             }
             // Partials are summed in split order.  The own one comes from the workspace like the others where a second
-            // copy of the accumulators would halve the number of resident workgroups (128 x 128 tiles: re-reading it
-            // costs a tile of loads); smaller tiles keep it in registers.
+            // copy of the accumulators would not fit beside them (64 x 64 outputs a wave: of the cut forms the 256-row tile
+            // of the halo form; re-reading it costs a tile of loads); the others keep it in registers.
             constexpr bool REREAD_OWN = TM * TN >= 4;
             f32x16 own[REREAD_OWN ? 1 : TM][REREAD_OWN ? 1 : TN];
             int my_part = -1;

@@ -1795,11 +1795,14 @@ extern "C" fdx_status fdx_debug_force_chain(int mode)
 // Direct sum or Winograd form of a 3x3 stride-1 convolution by predicted cost.  Of 300 timed ones that the costs were not fitted to
 // (maps of 6 to 62 pixels, 8 to 512 channels, batches of 1 to 64) the choice takes 0.6 % longer than the faster form on average, at
 // worst 21 %; Winograd from a gigaflop of direct-sum work on takes 8 %, always the direct kernel 13 % (36 % where the channels
-// are no multiple of 16: 8 images, 56 x 56 x 56 -> 128: direct 49.6 us, Winograd 31.2; 16 of 56 x 56 x 64 -> 64 29.7 / 35.1).  The
-// direct kernel draws more power, which the layers around it pay for with clock: 3 % against it.
+// are no multiple of 16: 8 images, 56 x 56 x 56 -> 128: direct 49.6 us, Winograd 31.2; 16 of 56 x 56 x 64 -> 64 29.7 / 35.1).
+// Nothing is charged for the direct kernel's higher power: ResNet50 passes of 8 / 16 / 24 / 32 / 48 / 64 / 100 images take 964 / 1352 /
+// 1746 / 2075 / 2926 / 3581 / 5429 us, with 3 % charged 963 / 1373 / 1767 / 2074 / 2928 / 3579 / 5361, with 4 % in its favour 964 / 1351 / 1750 /
+// 2071 / 2939 / 3597 / 5453.  It is also closer to 64-bit results (2-norm, 64 / 128 / 256 / 512 channels: 1.1 / 0.8 / 1.1 / 1.3 e-7 against
+// 1.7 / 1.7 / 2.5 / 2.8 e-7; the direct sum on the fp32 MFMA 3.1 / 4.2 / 5.8 / 8.0 e-7).
 static bool winograd_by_rule(int n, int h, int w, int cin, int cout, int oh, int ow, bool residual)
 {
-    return conv2d_winograd_cost(n, cin, cout, oh, ow) < 1.03f * conv3x3_direct_cost(n, h, w, cin, cout, oh, ow, residual);
+    return conv2d_winograd_cost(n, cin, cout, oh, ow) < conv3x3_direct_cost(n, h, w, cin, cout, oh, ow, residual);
 }
 extern "C" int fdx_debug_conv3x3_form(int n, int h, int w, int cin, int cout)
 {
@@ -2930,7 +2933,8 @@ namespace {
         double flops = 0, total = p.flops > 0 ? p.flops : 1;
         // what the pieces behind the first need to travel (55 GB/s over the link) at 50 TFLOP/s, and no more than a quarter of
         // the model: a longer prefix runs more of the model at a quarter of the batch than the copy can hide, a shorter one
-        // leaves the copy uncovered.  ResNet50 from host memory, 16 / 32 / 64 images, us: at 50 TFLOP/s 1711 / 2587 / 4355, 75 1780 / 2639 / 4352,
+        // leaves the copy uncovered.  MobileNetV2, 16 / 32 / 64 / 128 images, us: at 20 TFLOP/s 834 / 1192 / 1867 / 3376, at 50 832 / 1191 / 1848 / 3320,
+        // at 110 828 / 1187 / 1862 / 3364; ResNet50 128 images 8316 / 7688 / 7748.  ResNet50 from host memory, 16 / 32 / 64 images, us: at 50 TFLOP/s 1711 / 2587 / 4355, 75 1780 / 2639 / 4352,
         // 110 1792 / 2648 / 4386, 150 1828 / 2714 / 4454; on another machine 50 1672 / 2484 / 4175, 35 1666 / 2520 / 4318, 20 1684 / 2549 / 4380,
         // 10 1674 / 2536 / 4371.
         const double in_bytes = 4.0 * (double)batch * (double)volume(p.shapes[(size_t)m.inputs[0]]);

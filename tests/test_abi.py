@@ -91,6 +91,7 @@ def test_model_check_runs_without_a_gpu(fdx, modelgen):
     (16, 28, 28, 72, 128, 1),    # 36.8 / 29.2
     (16, 56, 56, 64, 64, 0),     # 29.7 / 35.1
     (16, 28, 28, 128, 128, 0),   # 29.4 / 38.7
+    (16, 14, 14, 256, 256, 0),   # 35.3 / 37.1
     (4, 15, 15, 320, 128, 0),    # 12.7 / 39.6
     (27, 36, 36, 320, 64, 1),    # 107 / 69
 ])

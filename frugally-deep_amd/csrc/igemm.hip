@@ -1187,6 +1187,7 @@ extern "C" fdx_status fdx_debug_force_tile(int cfg)
 }
 
 namespace fdx {
+bool tile_forced() { return g_forced_tile >= 0; }
 // out[M][n] = act(LN(x)[M][k] . w^T + bias + residual), the rows of x normalised over k inside the GEMM (LNF in
 // igemm_fast.hpp): w is the filter with LayerNormalization's gamma folded in ([n][k]), bias the bias with beta folded in,
 // wsum[n] the row sums of w.  FDX_ERR_UNSUPPORTED, with nothing launched, where the fast path does not apply.

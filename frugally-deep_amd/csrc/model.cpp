@@ -1426,6 +1426,12 @@ namespace {
                 bf[(size_t)r] = (float)shift;
             }
         };
+        if (sample_net_keeps_weights(m))
+            for (auto& o : m.ops)
+                if (!o.dead && (o.kind == OpKind::Conv2D || o.kind == OpKind::Dense)) {
+                    o.sample_w = o.hw[0];
+                    o.sample_bias = o.hw[1];
+                }
         for (auto& o : m.ops) {
             if (o.dead) {
                 o.hw.clear();
@@ -1820,6 +1826,20 @@ extern "C" fdx_status fdx_debug_force_winograd(int mode)
     return FDX_OK;
 }
 
+// test hook: -1 = a plan runs a small model as one launch by the rule, 0 = never, 1 = wherever there is a program for it
+static int g_force_sample_net = -1;
+
+extern "C" fdx_status fdx_debug_force_sample_net(int mode)
+{
+    FDX_REQUIRE(mode >= -1 && mode <= 1, "fdx_debug_force_sample_net: mode must be -1, 0 or 1");
+    g_force_sample_net = mode;
+    return FDX_OK;
+}
+extern "C" int fdx_debug_sample_net(const fdx_model* m)
+{
+    return m && !m->plans.empty() && m->plans[0]->sample ? 1 : 0;
+}
+
 fdx_status get_plan(fdx_model* m, int batch, const std::vector<Shape>& in_shapes, Plan** out)
 {
     for (size_t i = 0; i < m->plans.size(); ++i)
@@ -2029,6 +2049,19 @@ fdx_status get_plan(fdx_model* m, int batch, const std::vector<Shape>& in_shapes
             p->conv_form[idx] = (listed ? known == 1
                 : winograd_by_rule(batch, (int)is[0], (int)is[1], (int)is[2], o.cout, g[4], g[5], o.residual >= 0)) ? 1 : 0;
         }
+    // The whole model as one launch: where it is small enough and no form of its operations is asked for.
+    const bool forced = tile_forced() || g_force_winograd >= 0 || g_force_dw_fusion >= 0;
+    if (g_force_sample_net != 0 && (g_force_sample_net == 1 || !forced)) {
+        for (auto& other : m->plans)
+            if (other->sample && other->in_shapes == in_shapes)
+                p->sample = other->sample;
+        if (!p->sample && std::any_of(m->ops.begin(), m->ops.end(), [](const Op& o) { return !o.sample_w.empty(); }))
+            p->sample = sample_net_build(*m, p->order, p->shapes);
+        if (p->sample && g_force_sample_net < 0 && !sample_net_by_rule(*p->sample, *m, p->order, p->shapes, batch))
+            p->sample = nullptr;
+        if (p->sample)
+            p->sample->flops = p->flops / batch;
+    }
     m->plans.insert(m->plans.begin(), std::move(p));
     *out = m->plans[0].get();
     return FDX_OK;
@@ -3030,7 +3063,7 @@ namespace {
         Stager& st = stager();
         std::lock_guard<std::mutex> lock(st.use);
         static const bool no_prefix = [] { const char* e = std::getenv("FDX_STAGE_PREFIX"); return e && e[0] == '0'; }();
-        const int cut = batch >= 8 && !no_prefix ? chunkable_prefix(*m, *p, batch) : 0;
+        const int cut = batch >= 8 && !no_prefix && !p->sample ? chunkable_prefix(*m, *p, batch) : 0;
         static const bool stage_log = [] { const char* e = std::getenv("FDX_STAGE_LOG"); return e && e[0] == '1'; }();
         if (stage_log)
             std::fprintf(stderr, "[fdx stage] %zu bytes, prefix of %d ops (plan has %zu)\n", total, cut, p->order.size());
@@ -3137,7 +3170,14 @@ namespace {
                 }
                 FDX_HIP(hipMemcpyAsync(p->out[m->inputs[i]], in[i], bytes, hipMemcpyDeviceToDevice, stream()));
             }
-        if ((st = execute(*m, *p, done_until)) != FDX_OK)
+        // a model that runs as one launch writes its result where the caller wants it
+        const bool one_launch = p->sample && (g_force_sample_net == 1 || !tile_forced()), direct = one_launch && out_on_device && out[0];
+        if (one_launch) {
+            st = sample_net_launch(*p->sample, p->out[m->inputs[0]], batch, direct ? out[0] : p->out[m->outputs[0]]);
+            m->last_flops = p->flops;
+        } else
+            st = execute(*m, *p, done_until);
+        if (st != FDX_OK)
             return st;
         // Host outputs that fit come back through a pinned buffer of the library (one asynchronous copy each, then a plain
         // memcpy once the stream has drained): a pageable device-to-host copy costs about 0.1 ms however small it is.
@@ -3157,7 +3197,7 @@ namespace {
                 bounce_lock.unlock();
         }
         size_t at = 0;
-        for (size_t i = 0; i < m->outputs.size(); ++i) {
+        for (size_t i = 0; i < m->outputs.size() && !direct; ++i) {
             const size_t bytes = sizeof(float) * (size_t)batch * (size_t)volume(p->shapes[m->outputs[i]]);
             FDX_HIP(hipMemcpyAsync(bounce ? static_cast<void*>(bounce + at) : static_cast<void*>(out[i]), p->out[m->outputs[i]], bytes,
                 out_on_device ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost, stream()));

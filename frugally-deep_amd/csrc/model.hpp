@@ -9,6 +9,7 @@
 
 #include "common.hpp"
 #include "einsum.hpp"
+#include "sample_net.hpp"
 
 namespace fdx {
 
@@ -88,6 +89,7 @@ struct Op {
     std::vector<std::vector<float>> hw;
     // device weights, indexed like hw
     std::vector<float*> dw;
+    std::vector<float> sample_w, sample_bias; // filter [n][k] and bias of a small model, see sample_net_build
 };
 
 struct Block {
@@ -112,6 +114,7 @@ struct Plan {
     std::vector<signed char> ln_fold_on;    // per Dense / attention op with ln_src >= 0: 1 = this plan normalises inside its GEMM
     std::vector<signed char> ln_skip;       // per LayerNormalization op: 1 = every reader normalises for itself, no launch
     std::vector<signed char> chain_done;    // per consumer of such a pair: its result was produced by the producer's launch in this run
+    std::shared_ptr<SampleProgram> sample;  // the whole model as one launch, a workgroup per sample; null: a launch per op
     double flops = 0;
     ~Plan();
 };
@@ -146,6 +149,11 @@ namespace fdx {
 // builds (or reuses) the plan for this batch and these per-sample input shapes
 fdx_status get_plan(fdx_model* m, int batch, const std::vector<Shape>& in_shapes, Plan** out);
 float* plan_alloc(Plan& p, size_t bytes, int* block_index);
+bool sample_net_keeps_weights(const fdx_model& m);
+std::shared_ptr<SampleProgram> sample_net_build(const fdx_model& m, const std::vector<int>& order, const std::vector<Shape>& shapes);
+bool sample_net_by_rule(const SampleProgram& p, const fdx_model& m, const std::vector<int>& order, const std::vector<Shape>& shapes, int batch);
+fdx_status sample_net_launch(const SampleProgram& p, const float* in, int batch, float* out);
+bool tile_forced(); // fdx_debug_force_tile names a configuration
 std::vector<int> topo_order(const fdx_model& m); // producers before consumers, dead ops skipped by callers
 fdx_status positions_launch(float* out, int batch, int t, int start);
 bool chain_supported(int k1, int k2, int n1, int n2);

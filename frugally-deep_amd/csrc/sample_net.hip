@@ -1,0 +1,496 @@
+// A small network as one launch (gfx950): every workgroup takes one sample through all layers, tensors, weights and offset
+// tables in LDS.
+//
+// A network on 32 x 32 images of a few convolutions is a chain of launches of 1.5 to 8 us that each do a fraction of a
+// microsecond of work on a few CUs.  Samples do not meet in any layer, so a workgroup can keep one to itself: what is left is one
+// launch, the image's way in and the sample's arithmetic on one CU (fp32 MFMA, 256 multiply-adds a cycle).
+//
+//  * 16 waves, four per SIMD: a convolution is dealt out as 16-pixel x 16 or 32-channel tiles, each wave walks K on its own; with four
+//    waves a SIMD's matrix pipe stays busy through the two dependent LDS reads in front of a product (offset, then pixel).
+//  * the filter is the MFMA's row operand and the pixels its columns, so that a lane ends up with four neighbouring channels of
+//    a pixel: 16-byte stores.
+//  * an offset table takes the place of the walk over taps and channels: offset of every K element (of every four where the
+//    channels are a multiple of four) from tap (0, 0).  Tensors whose readers pad lie inside a frame of zeros, so no tap is tested.
+//  * a pixel's stride is an odd number of 16-byte pieces: 16 pixels side by side lie in different banks.
+#include "sample_net.hpp"
+
+#include <cfloat>
+
+#include "igemm_params.hpp"
+
+namespace fdx {
+
+// x / d for x and d below 2^16, with ceil(2^32 / d) from the host (exact there: x times the ceiling's excess stays below 2^32)
+__device__ __forceinline__ int quotient(int x, uint32_t by) { return by ? (int)__umulhi((uint32_t)x, by) : x; }
+
+// maximum or sum over the sixteen lanes of a row and over a wave, in every lane
+template <bool MAX>
+__device__ __forceinline__ float both(float a, float b) { return MAX ? fmaxf(a, b) : a + b; }
+template <bool MAX>
+__device__ __forceinline__ float half_row_all(float v)
+{
+    v = both<MAX>(v, dpp_move<0xB1>(v));
+    v = both<MAX>(v, dpp_move<0x4E>(v));
+    return both<MAX>(v, dpp_move<0x141>(v));
+}
+template <bool MAX>
+__device__ __forceinline__ float wave_all(float v)
+{
+    v = half_row_all<MAX>(v);
+    v = both<MAX>(v, dpp_move<0x140>(v));
+    auto lane = [&](int l) { return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), l)); };
+    return both<MAX>(both<MAX>(lane(0), lane(16)), both<MAX>(lane(32), lane(48)));
+}
+
+__device__ __forceinline__ void sample_frame(const SampleStep& s, float* lds, int t)
+{
+    // the frame of zeros around a tensor: its cells are nobody else's
+    const int cells = s.frame_h * s.frame_w;
+    for (int i = t; i < cells; i += kSampleThreads) {
+        const int y = quotient(i, s.by_frame_w), x = i - y * s.frame_w;
+        if ((unsigned)(y - s.frame_top) < (unsigned)s.out_h && (unsigned)(x - s.frame_left) < (unsigned)s.out_w)
+            continue;
+        float* p = lds + s.frame_base + y * s.out_row + x * s.out_pix;
+        int c = 0;
+        if (s.out_pix % 4 == 0)
+            for (; c + 4 <= s.out_c; c += 4)
+                *reinterpret_cast<f32x4*>(p + c) = f32x4 { 0.f, 0.f, 0.f, 0.f };
+        for (; c < s.out_c; ++c)
+            p[c] = 0.f;
+    }
+}
+
+// items of MT x 16 pixels by NT x 16 channels, dealt out to the waves
+template <bool VEC, int MT, int NT>
+__device__ __forceinline__ void sample_conv(const SampleStep& s, float* lds, float* out, int t)
+{
+    typedef int i32x4 __attribute__((ext_vector_type(4)));
+    const int lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6), fr = lane & 15, fg = lane >> 4;
+    const int pixels = s.out_h * s.out_w, m_items = (pixels + 16 * MT - 1) / (16 * MT), groups = s.n_tiles / NT;
+    const int step_y = s.sy * s.in_row, step_x = s.sx * s.in_pix;
+    const int* tab = reinterpret_cast<const int*>(lds) + s.tab + fg * s.tab_stride;
+    int g = 0, mt = wave;
+    for (; mt >= m_items && g < groups; ++g)
+        mt -= m_items;
+    while (g < groups) {
+        const float* w = lds + s.weights + (g * NT * s.chunks * 64 + lane) * 4;
+        f32x4 acc[MT][NT];
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+            acc[0][j] = *reinterpret_cast<const f32x4*>(lds + s.bias + (g * NT + j) * 16 + fg * 4);
+        int oy[MT], ox[MT];
+        const float* a[MT];
+#pragma unroll
+        for (int i = 0; i < MT; ++i) {
+            const int m = (mt * MT + i) * 16 + fr, mm = m < pixels ? m : 0;
+            oy[i] = quotient(mm, s.by_out_w);
+            ox[i] = mm - oy[i] * s.out_w;
+            a[i] = lds + s.in_base + oy[i] * step_y + ox[i] * step_x;
+        }
+#pragma unroll
+        for (int i = 1; i < MT; ++i)
+#pragma unroll
+            for (int j = 0; j < NT; ++j)
+                acc[i][j] = acc[0][j];
+        auto filter = [&](f32x4 (&wv)[NT], int kc) {
+#pragma unroll
+            for (int j = 0; j < NT; ++j)
+                wv[j] = *reinterpret_cast<const f32x4*>(w + (j * s.chunks + kc) * 256);
+        };
+        auto multiply = [&](const f32x4 (&av)[MT], const f32x4 (&wv)[NT]) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int i = 0; i < MT; ++i)
+#pragma unroll
+                    for (int j = 0; j < NT; ++j)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[j][e], av[i][e], acc[i][j], 0, 0, 0);
+        };
+        f32x4 av[MT], wv[NT];
+        if (VEC) { // a lane's offsets of four chunks lie side by side
+            int kc = 0;
+            for (; kc + 4 <= s.whole; kc += 4) {
+                const i32x4 off = *reinterpret_cast<const i32x4*>(tab + kc);
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+#pragma unroll
+                    for (int i = 0; i < MT; ++i)
+                        av[i] = *reinterpret_cast<const f32x4*>(a[i] + off[u]);
+                    filter(wv, kc + u);
+                    multiply(av, wv);
+                }
+            }
+            if (kc < s.chunks) {
+                const i32x4 off = *reinterpret_cast<const i32x4*>(tab + kc); // (the table's rows are whole fours of chunks)
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    if (kc + u >= s.chunks)
+                        break;
+#pragma unroll
+                    for (int i = 0; i < MT; ++i) {
+                        av[i] = *reinterpret_cast<const f32x4*>(a[i] + max(off[u], 0));
+                        if (off[u] < 0) // beyond K: the filter is zero there, and what it meets must be finite
+                            av[i] = f32x4 { 0.f, 0.f, 0.f, 0.f };
+                    }
+                    filter(wv, kc + u);
+                    multiply(av, wv);
+                }
+            }
+        } else {
+            for (int kc = 0; kc < s.whole; ++kc) {
+                const i32x4 off = *reinterpret_cast<const i32x4*>(tab + kc * 4);
+#pragma unroll
+                for (int i = 0; i < MT; ++i)
+                    av[i] = f32x4 { a[i][off[0]], a[i][off[1]], a[i][off[2]], a[i][off[3]] };
+                filter(wv, kc);
+                multiply(av, wv);
+            }
+            if (s.whole < s.chunks) {
+                const i32x4 off = *reinterpret_cast<const i32x4*>(tab + s.whole * 4);
+#pragma unroll
+                for (int i = 0; i < MT; ++i)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const float v = a[i][max(off[e], 0)];
+                        av[i][e] = off[e] < 0 ? 0.f : v;
+                    }
+                filter(wv, s.whole);
+                multiply(av, wv);
+            }
+        }
+        float r[MT * NT * 4];
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int j = 0; j < NT; ++j) {
+                const int n = (g * NT + j) * 16 + fg * 4;
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    r[(i * NT + j) * 4 + e] = acc[i][j][e];
+                if (s.res_base >= 0)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        if (n + e < s.out_c)
+                            r[(i * NT + j) * 4 + e] += lds[s.res_base + oy[i] * s.res_row + ox[i] * s.res_pix + n + e];
+            }
+        if (s.act_kind == FDX_ACT_RELU) // (GELU is a step of its own)
+#pragma unroll
+            for (int z = 0; z < MT * NT * 4; ++z) {
+                const float low = r[z] >= s.act_threshold ? r[z] : s.act_slope * (r[z] - s.act_threshold);
+                r[z] = r[z] >= s.act_max ? s.act_max : low;
+            }
+#pragma unroll
+        for (int i = 0; i < MT; ++i) {
+            const int m = (mt * MT + i) * 16 + fr;
+            if (m >= pixels)
+                continue;
+#pragma unroll
+            for (int j = 0; j < NT; ++j) {
+                const int n = (g * NT + j) * 16 + fg * 4;
+                const float* v = r + (i * NT + j) * 4;
+                if (n >= s.out_c)
+                    continue;
+                if (s.out_base >= 0 && s.out_pix % 4 == 0 && s.out_c % 4 == 0)
+                    *reinterpret_cast<f32x4*>(lds + s.out_base + oy[i] * s.out_row + ox[i] * s.out_pix + n) = f32x4 { v[0], v[1], v[2], v[3] };
+                else {
+                    float* o = s.out_base < 0 ? out + m * s.out_c : lds + s.out_base + oy[i] * s.out_row + ox[i] * s.out_pix;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        if (n + e < s.out_c)
+                            o[n + e] = v[e];
+                }
+            }
+        }
+        for (mt += kSampleThreads / 64; mt >= m_items && g < groups; ++g)
+            mt -= m_items;
+    }
+}
+
+__device__ __forceinline__ float* sample_out(const SampleStep& s, float* lds, float* out, int y, int x)
+{
+    return s.out_base < 0 ? out + (y * s.out_w + x) * s.out_c : lds + s.out_base + y * s.out_row + x * s.out_pix;
+}
+
+// windows in the order of pool2d_kernel: cells outside the image count for neither the maximum nor the average
+template <int VEC, bool MAX>
+__device__ __forceinline__ void sample_pool(const SampleStep& s, float* lds, float* out, int t)
+{
+    const int cv = s.out_c / VEC, total = s.out_h * s.out_w * cv;
+    for (int i = t; i < total; i += kSampleThreads) {
+        const int pix = quotient(i, s.by_out_c), c = (i - pix * cv) * VEC, oy = quotient(pix, s.by_out_w), ox = pix - oy * s.out_w;
+        const int y = oy * s.sy - s.pad_top, x = ox * s.sx - s.pad_left;
+        const int y0 = max(y, 0), y1 = min(y + s.kh, s.in_h), x0 = max(x, 0), x1 = min(x + s.kw, s.in_w);
+        const float* p = lds + s.in_base + y0 * s.in_row + x0 * s.in_pix + c;
+        float val[VEC];
+#pragma unroll
+        for (int v = 0; v < VEC; ++v)
+            val[v] = MAX ? -FLT_MAX : 0.f;
+        for (int fy = y0; fy < y1; ++fy, p += s.in_row) {
+            const float* q = p;
+            for (int fx = x0; fx < x1; fx += 2, q += 2 * s.in_pix) { // two columns on their way at once
+                const float* q1 = fx + 1 < x1 ? q + s.in_pix : q;
+                float z[2][VEC];
+                if constexpr (VEC == 4) {
+                    const f32x4 z0 = *reinterpret_cast<const f32x4*>(q), z1 = *reinterpret_cast<const f32x4*>(q1);
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) {
+                        z[0][v] = z0[v];
+                        z[1][v] = z1[v];
+                    }
+                } else {
+                    z[0][0] = q[0];
+                    z[1][0] = q1[0];
+                }
+#pragma unroll
+                for (int v = 0; v < VEC; ++v) {
+                    val[v] = both<MAX>(val[v], z[0][v]);
+                    val[v] = fx + 1 < x1 ? both<MAX>(val[v], z[1][v]) : val[v];
+                }
+            }
+        }
+        const float count = (float)((y1 - y0) * (x1 - x0));
+        float* o = sample_out(s, lds, out, oy, ox) + c;
+#pragma unroll
+        for (int v = 0; v < VEC; ++v)
+            val[v] = MAX ? val[v] : val[v] / count;
+        if constexpr (VEC == 4)
+            *reinterpret_cast<f32x4*>(o) = f32x4 { val[0], val[1], val[2], val[3] };
+        else
+            o[0] = val[0];
+    }
+}
+
+template <bool MAX>
+__device__ __forceinline__ void sample_global_pool(const SampleStep& s, float* lds, float* out, int t)
+{
+    const int positions = s.in_h * s.in_w, c = s.in_c;
+    float* scratch = lds + s.scratch;
+    for (int c0 = 0; c0 < c; c0 += kSampleThreads) {
+        // a power of two of lanes a slot, so that nothing is divided
+        const int width = c - c0 < kSampleThreads ? c - c0 : kSampleThreads, log2w = width > 1 ? 32 - __builtin_clz((unsigned)width - 1) : 0;
+        const int slots = kSampleThreads >> log2w, slot = t >> log2w, ch = t & ((1 << log2w) - 1);
+        float val = MAX ? -FLT_MAX : 0.f;
+        if (ch < width) {
+            const float* p = lds + s.in_base + c0 + ch;
+            if (s.in_row == s.in_w * s.in_pix)
+                for (int i = slot; i < positions; i += 4 * slots) {
+                    float v[4];
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) // a place beyond the end reads its first one again
+                        v[u] = p[(i + u * slots < positions ? i + u * slots : i) * s.in_pix];
+#pragma unroll
+                    for (int u = 0; u < 4; ++u)
+                        val = i + u * slots < positions ? both<MAX>(val, v[u]) : val;
+                }
+            else
+                for (int i = slot; i < positions; i += slots) {
+                    const int y = quotient(i, s.by_in_w), x = i - y * s.in_w;
+                    val = both<MAX>(val, p[y * s.in_row + x * s.in_pix]);
+                }
+        }
+        scratch[t] = val;
+        __syncthreads();
+        for (int i = t >> 3; i < width; i += kSampleThreads / 8) { // eight neighbouring lanes a channel
+            val = MAX ? -FLT_MAX : 0.f;
+            for (int q = t & 7; q < slots; q += 32) {
+                float v[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+                    v[u] = scratch[((q + 8 * u < slots ? q + 8 * u : q) << log2w) + i];
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+                    val = q + 8 * u < slots ? both<MAX>(val, v[u]) : val;
+            }
+            val = half_row_all<MAX>(val);
+            if ((t & 7) == 0)
+                (s.out_base < 0 ? out : lds + s.out_base)[c0 + i] = MAX ? val : val / (float)positions;
+        }
+        if (c0 + kSampleThreads < c)
+            __syncthreads();
+    }
+}
+
+// a wave per pixel, in the reference's form exp(x - m - log sum) with infinite results as zero
+__device__ __forceinline__ void sample_softmax(const SampleStep& s, float* lds, float* out, int t)
+{
+    const int lane = t & 63;
+    for (int p = __builtin_amdgcn_readfirstlane(t >> 6); p < s.in_h * s.in_w; p += kSampleThreads / 64) {
+        const int y = quotient(p, s.by_in_w), x = p - y * s.in_w;
+        const float* v = lds + s.in_base + y * s.in_row + x * s.in_pix;
+        float* o = sample_out(s, lds, out, y, x);
+        float m = -FLT_MAX, sum = 0.f;
+        for (int i = lane; i < s.in_c; i += 64)
+            m = fmaxf(m, v[i]);
+        m = wave_all<true>(m);
+        for (int i = lane; i < s.in_c; i += 64)
+            sum += expf(v[i] - m);
+        const float ls = logf(wave_all<false>(sum));
+        for (int i = lane; i < s.in_c; i += 64) {
+            const float r = expf(v[i] - m - ls);
+            o[i] = isinf(r) ? 0.f : r;
+        }
+    }
+}
+
+__device__ __forceinline__ void sample_activation(const SampleStep& s, float* lds, float* out, int t)
+{
+    const Act act { s.act_kind, s.act_max, s.act_slope, s.act_threshold };
+    const int total = s.in_h * s.in_w * s.in_c;
+    for (int i = t; i < total; i += kSampleThreads) {
+        const int pix = quotient(i, s.by_out_c), c = i - pix * s.in_c, y = quotient(pix, s.by_in_w), x = pix - y * s.in_w;
+        sample_out(s, lds, out, y, x)[c] = apply_act_full(lds[s.in_base + y * s.in_row + x * s.in_pix + c], act);
+    }
+}
+
+// What bounds it, on the small CNN of 32 x 32 x 3 (two 3x3 convolutions of 16 and 32 channels, pooling, classifier), cycles of a CU per
+// sample: way in 3400, first convolution 11000 (matrix pipes 4100, the rest its scattered 4-byte reads and the epilogue), pooling 3000,
+// second convolution 13000 (9200), global pooling 3000, Dense 2000, softmax 1500.  19.2 us a call up to 256 samples, where seven launches
+// took 27 to 62; eight samples a CU 132 us, 236 before.  With GELU's and softmax's code inside the convolution's epilogue 20 us.
+__global__ __launch_bounds__(kSampleThreads) void sample_net_kernel(const float* __restrict__ in, float* __restrict__ out,
+    const f32x4* __restrict__ image, int image_quads, const SampleStep* __restrict__ program, int steps, int in_volume, int out_volume, int batch)
+{
+    extern __shared__ __attribute__((aligned(16))) float lds[];
+    const int t = threadIdx.x;
+    // a sample on its way in registers: the next one's trip runs under the current one's steps
+    const bool quads = in_volume % 4 == 0; // (the input is 16-byte aligned)
+    f32x4 pre[4];
+    auto fetch = [&](int b) {
+        const float* p = in + (int64_t)b * in_volume;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int i = (t + u * kSampleThreads) * 4;
+            pre[u] = f32x4 { 0.f, 0.f, 0.f, 0.f };
+            if (quads) {
+                if (i < in_volume)
+                    pre[u] = *reinterpret_cast<const f32x4*>(p + i);
+            } else
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (i + e < in_volume)
+                        pre[u][e] = p[i + e];
+        }
+    };
+    fetch(blockIdx.x);
+    {
+        // the first steps' lines into the scalar cache, all on their way at once
+        int lines = 0;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const int* q = reinterpret_cast<const int*>(program + (i < steps ? i : 0));
+            lines |= q[0] | q[16] | q[32];
+        }
+        asm volatile("" ::"s"(lines));
+    }
+    for (int i = t; i < image_quads; i += 4 * kSampleThreads) {
+        f32x4 v[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (i + u * kSampleThreads < image_quads)
+                v[u] = image[i + u * kSampleThreads];
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (i + u * kSampleThreads < image_quads)
+                reinterpret_cast<f32x4*>(lds)[i + u * kSampleThreads] = v[u];
+    }
+    __syncthreads();
+    for (int b = blockIdx.x; b < batch; b += gridDim.x) {
+        float* result = out + (int64_t)b * out_volume;
+        for (int step = 0; step < steps; ++step) {
+            const SampleStep s = program[step];
+            // all of it at once: left alone, every branch below waits for its own fields
+            asm volatile("" ::"s"(s.kind), "s"(s.out_base), "s"(s.frame_h), "s"(s.in_base), "s"(s.kh), "s"(s.tab), "s"(s.weights), "s"(s.res_base),
+                "s"(s.scratch), "s"(s.act_threshold));
+            if (s.frame_h > 0)
+                sample_frame(s, lds, t);
+            switch (s.kind) {
+            case SampleStep::Load: {
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const int i = (t + u * kSampleThreads) * 4;
+                    if (i >= in_volume)
+                        continue;
+                    const int pix = quotient(i, s.by_out_c);
+                    int y = quotient(pix, s.by_out_w), x = pix - y * s.out_w, c = i - pix * s.out_c;
+                    if (s.vec) {
+                        *reinterpret_cast<f32x4*>(lds + s.out_base + y * s.out_row + x * s.out_pix + c) = pre[u];
+                        continue;
+                    }
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        if (i + e < in_volume)
+                            lds[s.out_base + y * s.out_row + x * s.out_pix + c] = pre[u][e];
+                        if (++c == s.out_c) {
+                            c = 0;
+                            if (++x == s.out_w) {
+                                x = 0;
+                                ++y;
+                            }
+                        }
+                    }
+                }
+                if (b + (int)gridDim.x < batch)
+                    fetch(b + gridDim.x);
+                break;
+            }
+            case SampleStep::Conv:
+                switch (s.form) {
+                case 0: sample_conv<false, 1, 1>(s, lds, result, t); break;
+                case 1: sample_conv<false, 4, 1>(s, lds, result, t); break;
+                case 2: sample_conv<true, 1, 1>(s, lds, result, t); break;
+                case 3: sample_conv<true, 4, 1>(s, lds, result, t); break;
+                case 4: sample_conv<true, 1, 2>(s, lds, result, t); break;
+                default: sample_conv<true, 2, 2>(s, lds, result, t); break;
+                }
+                break;
+            case SampleStep::Pool:
+                if (s.vec && s.mode == 0)
+                    sample_pool<4, true>(s, lds, result, t);
+                else if (s.vec)
+                    sample_pool<4, false>(s, lds, result, t);
+                else if (s.mode == 0)
+                    sample_pool<1, true>(s, lds, result, t);
+                else
+                    sample_pool<1, false>(s, lds, result, t);
+                break;
+            case SampleStep::GlobalPool:
+                if (s.mode == 0)
+                    sample_global_pool<true>(s, lds, result, t);
+                else
+                    sample_global_pool<false>(s, lds, result, t);
+                break;
+            case SampleStep::Softmax: sample_softmax(s, lds, result, t); break;
+            default: sample_activation(s, lds, result, t); break;
+            }
+            __syncthreads();
+        }
+    }
+}
+
+SampleProgram::~SampleProgram()
+{
+    if (image)
+        (void)hipFree(image);
+}
+
+fdx_status sample_net_launch(const SampleProgram& p, const float* in, int batch, float* out)
+{
+    FDX_REQUIRE(in && out && batch > 0 && p.image && p.in_volume <= kSampleInput && p.lds_floats <= kSampleLdsFloats
+            && (reinterpret_cast<uintptr_t>(in) & 15) == 0, "sample net: bad arguments");
+    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(sample_net_kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+        kSampleLdsFloats * 4);
+    FDX_HIP(attr);
+    static const int cus = [] {
+        int dev = 0, n = 256;
+        (void)hipGetDevice(&dev);
+        (void)hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev);
+        return n;
+    }();
+    profile_begin();
+    hipLaunchKernelGGL(sample_net_kernel, dim3((unsigned)(batch < cus ? batch : cus)), dim3(kSampleThreads), (size_t)p.lds_floats * 4, stream(),
+        in, out, reinterpret_cast<const f32x4*>(p.image), p.image_floats / 4, p.program, p.steps, p.in_volume, p.out_volume, batch);
+    profile_end("sample_net_f32", p.flops * batch, 4.0 * (p.image_floats + (double)batch * (p.in_volume + p.out_volume)));
+    FDX_LAUNCH_CHECK();
+    return FDX_OK;
+}
+
+} // namespace fdx

@@ -81,6 +81,12 @@ fdx_status fdx_debug_persist_cap(int workgroups);
 fdx_status fdx_debug_force_strips(int strips);
 fdx_status fdx_debug_force_dw_fusion(int mode);
 fdx_status fdx_debug_force_winograd(int mode);
+/* plans built from now on: a small model (one input, one output, convolutions, Dense layers, pooling, activations and softmax whose
+ * tensors and weights fit in a CU's LDS) as one launch, a workgroup per sample: -1 = by the rule of predicted times, unless a form of its
+ * operations is forced (the default), 0 = never, 1 = wherever there is a program for it */
+fdx_status fdx_debug_force_sample_net(int mode);
+/* 1 = the model's last call ran as one launch */
+int fdx_debug_sample_net(const fdx_model* model);
 /* which kernel the rule takes for a 3x3 stride-1 "same" convolution [n][h][w][cin] -> cout: 0 = direct, 1 = Winograd (host only) */
 int fdx_debug_conv3x3_form(int n, int h, int w, int cin, int cout);
 

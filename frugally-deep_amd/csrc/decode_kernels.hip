@@ -983,6 +983,13 @@ fdx_status skinny_gemm_launch(const SkinnyParams& p)
     FDX_REQUIRE(p.n_seg >= 1 && p.n_seg <= 3, "dense_rows: 1 to 3 output segments");
     FDX_REQUIRE(!p.ln || p.K <= SK_WAVES * SK_CHUNK * 16, "dense_rows: the LayerNorm prologue needs K <= %d", SK_WAVES * SK_CHUNK * 16);
     FDX_REQUIRE(!p.residual || p.residual != p.seg[0].ptr, "dense_rows: the residual is read before the output is written; they must not alias");
+    if (!p.packed && gemv_by_rule(p)) {
+        profile_begin();
+        gemv_launch(p);
+        profile_end("dense_rows_f32", 2.0 * p.M * (double)p.N * p.K, 4.0 * ((double)p.N * p.K + (double)p.M * (p.K + p.N)));
+        FDX_LAUNCH_CHECK();
+        return FDX_OK;
+    }
     const int tiles = (p.N + 15) / 16;
     // split K across workgroups when a launch would otherwise leave most CUs idle or a wave would need
     // more than one chunk; LayerNorm launches keep whole rows in one workgroup

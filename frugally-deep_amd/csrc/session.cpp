@@ -687,6 +687,8 @@ bool build_fast_plan(fdx_session* s)
     }
     for (auto& stp : s->steps)
         if (stp.kind == fdx_session::Step::Gemm) {
+            if (gemv_by_rule(stp.g)) // reads the rows as they are
+                continue;
             // decode-time copy of the operand in the order the kernel's lanes read it
             float* packed = alloc((size_t)packed_weight_floats(stp.g.N, stp.g.K));
             if (!packed || pack_weights_launch(stp.g.W, stp.g.N, stp.g.K, stp.g.ldw, packed) != FDX_OK)

@@ -59,6 +59,10 @@ struct SkinnyParams {
 constexpr int kErrSplitExchange = 2; // value of the err cell: the partial tiles of a split launch did not meet
 
 fdx_status skinny_gemm_launch(const SkinnyParams& p);
+// one to six rows against weights row by row (gemv.hip)
+bool gemv_covers(int m, int n, int k, int64_t ldx, int64_t ldw, int64_t ldr, bool ln);
+bool gemv_by_rule(const SkinnyParams& p); // skinny_gemm_launch takes it for these parameters, with the weights not packed
+void gemv_launch(const SkinnyParams& p);
 
 // number of workgroups the launch would use if it takes the wide-output kernel (one that strides over column groups), else 0
 int skinny_wide_grid(const SkinnyParams& p);

@@ -488,6 +488,9 @@ static fdx_status irb_launch(IrbParams& p, int cin, int n_out, int stride, bool 
     return FDX_OK;
 }
 
+// waves of the one workgroup of a CU: tiles of 4 x 8 output pixels that a CU has under way at once
+int irb_block_waves(int cin, int ce, int n_out, int stride) { return irb_waves(cin, ce, n_out, stride); }
+
 static bool al16(const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15) == 0; }
 
 } // namespace fdx

@@ -2669,6 +2669,38 @@ namespace {
         return run_op(m, p, idx);
     }
 
+    // The form of a block by predicted times, in us: a launch costs 4.3 and its tensors' bytes at 4.2 TB/s (3.2 beyond the memory-side cache);
+    // depthwise + projection as one launch walks slabs of 32 channels one after the other, a wave to 32 pixels, and takes that
+    // long however few pixels there are; so does the whole block, in rounds of what is resident.  Over 396 timed blocks (MobileNetV2 of
+    // 128 to 224, batches of 1 to 128) the choice takes 1 % longer than the fastest form, lines drawn by the height of the map
+    // alone (56 and 28 rows, right for batches of 128 images of 224) 13 %: blocks of 28 to 56 rows, one image of 224: layers / pair / block 14.7 /
+    // 23.6 / 26.6, 14.0 / 23.9 / 32.1, 12.3 / 25.1 / 24.9, 8.5 / 22.5 / -.
+    int block_form_by_rule(const fdx_model& m, const Plan& p, int idx)
+    {
+        const Op& c = m.ops[idx];
+        const Op& d = m.ops[c.fuse_dw];
+        const Shape &ds = p.shapes[d.in[0]], &os = p.shapes[idx];
+        if (ds.size() != 3 || os.size() != 3)
+            return 2;
+        const Op* e = c.fuse_exp >= 0 ? &m.ops[c.fuse_exp] : nullptr;
+        if (e && (e->kh != 1 || e->sy != 1))
+            return 3; // a convolution on the image in front: the whole block is the fastest or within 4 us of it
+        const double px_in = (double)p.batch * ds[0] * ds[1], px = (double)p.batch * os[0] * os[1], ce = (double)ds[2], n = (double)os[2];
+        const double x = e ? 4 * px_in * p.shapes[e->in[0]].back() : 0, wide = 4 * px_in * ce, stencil = 4 * px * ce, y = 4 * px * n * (c.residual >= 0 ? 2 : 1);
+        auto traffic = [&](double bytes) { return bytes / (wide > 128e6 ? 3.2e6 : 4.2e6); };
+        const double expand = e ? 4.3 + traffic(x + wide) : 0, slabs = std::ceil(ce / 32);
+        const double layers = expand + 4.3 + traffic(wide + stencil) + 4.3 + traffic(stencil + y);
+        const double pair = expand + std::max({ 3 + slabs * (2.5 + 0.48 * std::ceil(n / 32)), 5 + 0.0023 * (px / 32) * slabs, traffic(wide + y) });
+        double block = 1e30;
+        if (e) {
+            const double tiles = (double)p.batch * ((os[0] + 3) / 4) * ((os[1] + 7) / 8);
+            const int waves = irb_block_waves((int)p.shapes[e->in[0]].back(), (int)ds[2], (int)os[2], d.sy);
+            if (waves > 0) // (two waves a SIMD hold each other up)
+                block = 5 + std::ceil(tiles / (256.0 * waves)) * slabs * (d.sy == 1 ? (waves == 8 ? 4.1 : 3.1) : (waves == 8 ? 8.0 : 5.2));
+        }
+        return block < layers && block < pair ? 3 : pair < layers ? 1 : 2;
+    }
+
     // First execution of a plan: the forms of the block are timed on the real operands (each leaves the same result in the
     // convolution's output buffer) and the plan remembers the fastest; the choice is kept per shape in the tuner's table,
     // so that an exported table pins it too.
@@ -2693,11 +2725,8 @@ namespace {
         int known = 0;
         const bool listed = tune_lookup(key, &known);
         if (listed || tune_frozen()) {
-            // Nothing is timed and the block is not in the table: the forms that win when they are timed (MobileNetV2 at
-            // batch 128: the whole block as one launch on the 112- and 56-row feature maps, depthwise + projection on
-            // the 28-row ones, a launch per layer below that); a form the launchers do not cover falls back inside
-            // run_block_form.
-            const int by_rule = key.M >= 56 ? 3 : key.M >= 28 ? 1 : 2;
+            // nothing is timed and the block is not in the table
+            const int by_rule = block_form_by_rule(m, p, idx);
             const int form = listed ? (known == 1 || known == 3 ? known : 2) : by_rule;
             return run_block_form(m, p, idx, form);
         }

@@ -153,6 +153,7 @@ bool sample_net_keeps_weights(const fdx_model& m);
 std::shared_ptr<SampleProgram> sample_net_build(const fdx_model& m, const std::vector<int>& order, const std::vector<Shape>& shapes);
 bool sample_net_by_rule(const SampleProgram& p, const fdx_model& m, const std::vector<int>& order, const std::vector<Shape>& shapes, int batch);
 fdx_status sample_net_launch(const SampleProgram& p, const float* in, int batch, float* out);
+int irb_block_waves(int cin, int ce, int n_out, int stride); // irb.hip
 bool tile_forced(); // fdx_debug_force_tile names a configuration
 std::vector<int> topo_order(const fdx_model& m); // producers before consumers, dead ops skipped by callers
 fdx_status positions_launch(float* out, int batch, int t, int start);

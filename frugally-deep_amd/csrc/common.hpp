@@ -130,6 +130,24 @@ __device__ __forceinline__ float row16_sum(float v)
     v += dpp_move<0x140>(v); // row_mirror
     return v;
 }
+// Maximum or sum over a wave, in every lane: the sixteen lanes of a row as above, the four rows through scalar registers.
+template <bool MAX>
+__device__ __forceinline__ float either(float a, float b) { return MAX ? fmaxf(a, b) : a + b; }
+template <bool MAX>
+__device__ __forceinline__ float half_row_all(float v) // over eight neighbouring lanes
+{
+    v = either<MAX>(v, dpp_move<0xB1>(v));
+    v = either<MAX>(v, dpp_move<0x4E>(v));
+    return either<MAX>(v, dpp_move<0x141>(v));
+}
+template <bool MAX>
+__device__ __forceinline__ float wave_all(float v)
+{
+    v = half_row_all<MAX>(v);
+    v = either<MAX>(v, dpp_move<0x140>(v));
+    auto lane = [&](int l) { return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), l)); };
+    return either<MAX>(either<MAX>(lane(0), lane(16)), either<MAX>(lane(32), lane(48)));
+}
 #endif
 
 // A column range of a GEMM's output with a tensor of its own (gemm_segments_launch): `cols` columns, rows `ld` floats apart

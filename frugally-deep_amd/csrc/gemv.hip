@@ -27,14 +27,6 @@ struct GemvTail {
     float eps;
 };
 
-// sum over a wave, the same in every lane
-__device__ __forceinline__ float wave_total(float v)
-{
-    v = row16_sum(v);
-    auto lane = [&](int l) { return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), l)); };
-    return (lane(0) + lane(16)) + (lane(32) + lane(48));
-}
-
 // A lane's output of a wave that owns M rows x C columns from n0 on: where it goes, and what is added in front of the activation.
 struct GemvOutput {
     bool ok;
@@ -87,7 +79,7 @@ __device__ __forceinline__ float gemv_sums(const f32x4 (&wa)[C][KQ], int lane, R
     for (int r = 0; r < M; ++r)
 #pragma unroll
         for (int c = 0; c < C; ++c) {
-            const float total = wave_total((s[r][c][0] + s[r][c][1]) + (s[r][c][2] + s[r][c][3]));
+            const float total = wave_all<false>((s[r][c][0] + s[r][c][1]) + (s[r][c][2] + s[r][c][3]));
             v = lane == r * C + c ? total : v;
         }
     return v;
@@ -128,7 +120,7 @@ __global__ __launch_bounds__(64 * kGemvWaves) void gemv_kernel(const float* x, c
 #pragma unroll
             for (int q = 0; q < KQ; ++q)
                 s += (xa[q][0] + xa[q][1]) + (xa[q][2] + xa[q][3]);
-            const float mean = wave_total(s) / (float)k;
+            const float mean = wave_all<false>(s) / (float)k;
             float dev = 0.f;
 #pragma unroll
             for (int q = 0; q < KQ; ++q) {
@@ -139,7 +131,7 @@ __global__ __launch_bounds__(64 * kGemvWaves) void gemv_kernel(const float* x, c
                     dev += xa[q][e] * xa[q][e];
                 }
             }
-            const float rstd = 1.0f / sqrtf(wave_total(dev) / (float)k + tail.eps);
+            const float rstd = 1.0f / sqrtf(wave_all<false>(dev) / (float)k + tail.eps);
             if (lane == 0)
                 row_rstd[wave] = rstd;
         }

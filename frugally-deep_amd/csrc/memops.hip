@@ -13,20 +13,8 @@ namespace fdx {
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-__device__ __forceinline__ float wave_sum(float v)
-{
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1)
-        v += __shfl_xor(v, o, 64);
-    return v;
-}
-__device__ __forceinline__ float wave_max(float v)
-{
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1)
-        v = fmaxf(v, __shfl_xor(v, o, 64));
-    return v;
-}
+__device__ __forceinline__ float wave_sum(float v) { return wave_all<false>(v); }
+__device__ __forceinline__ float wave_max(float v) { return wave_all<true>(v); }
 // block-wide reductions for blocks of up to 1024 threads; every thread gets the result
 template <bool IS_MAX>
 __device__ __forceinline__ float block_reduce(float v, float* smem)
@@ -115,6 +103,7 @@ __global__ __launch_bounds__(256) void dwconv3x3_kernel(const float* __restrict_
     // item index in 32 bits (the host launches this kernel only below 2^31 items): a 64-bit division costs several
     // times the arithmetic of an item
     const unsigned total = (unsigned)n * (unsigned)oh * xt * cv;
+    const __amdgpu_buffer_rsrc_t srd = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(in), 0, (int)((uint32_t)n * (uint32_t)h * (uint32_t)w * (uint32_t)c * 4u), 0x00020000);
     for (unsigned idx = blockIdx.x * blockDim.x + threadIdx.x; idx < total; idx += gridDim.x * blockDim.x) {
         unsigned rest = idx / cv;
         const int cq = (int)(idx - rest * cv);
@@ -132,28 +121,27 @@ __global__ __launch_bounds__(256) void dwconv3x3_kernel(const float* __restrict_
 #pragma unroll
         for (int j = 0; j < TX; ++j)
             acc[j] = b4;
-        const float* ib = in + (int64_t)img * h * w * c + c0;
-        const int ix0 = ox0 * STRIDE - pad_left;
+        // every load of the item on its way before the first is used: a tap outside the image gets an offset beyond the extent
+        // and answers zero.  (Behind a test per row and tap a small map paid the trip to memory row by row: 7 of 11 x 11 x 384 5.4 us against 4.0.)
+        const int ix0 = ox0 * STRIDE - pad_left, iy0 = oy * STRIDE - pad_top;
+        const uint32_t base = (uint32_t)(((img * h + iy0) * w + ix0) * c + c0) * 4u;
+        f32x4 col[3][COLS];
 #pragma unroll
-        for (int fy = 0; fy < 3; ++fy) {
-            const int iy = oy * STRIDE - pad_top + fy;
-            if (iy < 0 || iy >= h)
-                continue;
-            const float* row = ib + (int64_t)iy * w * c;
-            f32x4 col[COLS];
+        for (int fy = 0; fy < 3; ++fy)
 #pragma unroll
             for (int k = 0; k < COLS; ++k) {
-                const int ix = ix0 + k;
-                col[k] = (ix >= 0 && ix < w) ? *reinterpret_cast<const f32x4*>(row + (int64_t)ix * c) : f32x4 { 0.f, 0.f, 0.f, 0.f };
+                const bool ok = (unsigned)(iy0 + fy) < (unsigned)h && (unsigned)(ix0 + k) < (unsigned)w;
+                col[fy][k] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(srd, ok ? (int)(base + (uint32_t)((fy * w + k) * c) * 4u) : (int)0x80000000u, 0, 0));
             }
+#pragma unroll
+        for (int fy = 0; fy < 3; ++fy)
 #pragma unroll
             for (int j = 0; j < TX; ++j)
 #pragma unroll
                 for (int fx = 0; fx < 3; ++fx)
 #pragma unroll
                     for (int v = 0; v < 4; ++v)
-                        acc[j][v] += col[j * STRIDE + fx][v] * wv[fy * 3 + fx][v];
-        }
+                        acc[j][v] += col[fy][j * STRIDE + fx][v] * wv[fy * 3 + fx][v];
         float* op = out + (((int64_t)img * oh + oy) * ow + ox0) * c + c0;
         float r[TX * 4];
 #pragma unroll
@@ -247,6 +235,54 @@ __global__ __launch_bounds__(256) void dwconv3x3_slide_kernel(const float* __res
 
 // ------------------------------------------------------------------ pooling
 // One lane per (output pixel, VEC channels); VEC = 4 moves 16 bytes per access.
+// Windows of PH x PW cells known at compile time, channels in fours: all cells requested before the first is used, addresses clamped into
+// the image.  (Cell by cell behind a test each, 112 x 112 x 64 under 3 x 3 / 2 took 7.1 us for one image against 4.0.)
+template <int PH, int PW, bool MAX>
+__global__ __launch_bounds__(256) void pool2d_small_kernel(const float* __restrict__ in, float* __restrict__ out, int h, int w, int c, int sy, int sx,
+    int pad_top, int pad_left, int zt, int zl, int zb, int zr, int oh, int ow, unsigned total)
+{
+    const unsigned cv = (unsigned)c / 4;
+    for (unsigned idx = blockIdx.x * 256u + threadIdx.x; idx < total; idx += gridDim.x * 256u) {
+        const unsigned pix = idx / cv, row = pix / (unsigned)ow, img = row / (unsigned)oh;
+        const int ch = (int)(idx - pix * cv) * 4, ox = (int)(pix - row * (unsigned)ow), oy = (int)(row - img * (unsigned)oh);
+        const int iy = oy * sy - pad_top, ix = ox * sx - pad_left;
+        const float* p = in + (int64_t)img * h * w * c + ch;
+        f32x4 cell[PH][PW];
+#pragma unroll
+        for (int y = 0; y < PH; ++y)
+#pragma unroll
+            for (int x = 0; x < PW; ++x) {
+                const int cy = min(max(iy + y, 0), h - 1), cx = min(max(ix + x, 0), w - 1);
+                cell[y][x] = *reinterpret_cast<const f32x4*>(p + ((int64_t)cy * w + cx) * c);
+            }
+        f32x4 val;
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+            val[v] = MAX ? -FLT_MAX : 0.f;
+        int div = 0;
+#pragma unroll
+        for (int y = 0; y < PH; ++y)
+#pragma unroll
+            for (int x = 0; x < PW; ++x) {
+                const bool inside = (unsigned)(iy + y) < (unsigned)h && (unsigned)(ix + x) < (unsigned)w;
+                // cells of a folded explicit zero-padding frame are real zeros, others outside are ignored
+                const bool counts = inside || (iy + y >= -zt && iy + y < h + zb && ix + x >= -zl && ix + x < w + zr);
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    const float z = inside ? cell[y][x][v] : 0.f;
+                    const float next = MAX ? fmaxf(val[v], z) : val[v] + z;
+                    val[v] = counts ? next : val[v];
+                }
+                div += counts ? 1 : 0;
+            }
+        if (!MAX)
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+                val[v] = val[v] / (float)div;
+        *reinterpret_cast<f32x4*>(out + (int64_t)pix * c + ch) = val;
+    }
+}
+
 template <int VEC>
 __global__ void pool2d_kernel(const float* __restrict__ in, float* __restrict__ out, int n, int h, int w, int c,
     int ph, int pw, int sy, int sx, int pad_top, int pad_left, int zt, int zl, int zb, int zr, int oh, int ow, int mode)
@@ -549,14 +585,22 @@ __global__ __launch_bounds__(256) void layernorm_wave4_kernel(const float* __res
     if (row >= rows)
         return;
     const float* xr = x + row * depth;
-    f32x4 v[NV];
+    f32x4 v[NV], g[NV], b[NV]; // gamma and beta travel with the row
     float s = 0.f;
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
         const int z = (lane + i * 64) * 4;
         v[i] = z < depth ? *reinterpret_cast<const f32x4*>(xr + z) : f32x4 { 0.f, 0.f, 0.f, 0.f };
-        s += (v[i][0] + v[i][1]) + (v[i][2] + v[i][3]);
     }
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+        const int z = (lane + i * 64) * 4;
+        g[i] = gamma && z < depth ? *reinterpret_cast<const f32x4*>(gamma + z) : f32x4 { 1.f, 1.f, 1.f, 1.f };
+        b[i] = beta && z < depth ? *reinterpret_cast<const f32x4*>(beta + z) : f32x4 { 0.f, 0.f, 0.f, 0.f };
+    }
+#pragma unroll
+    for (int i = 0; i < NV; ++i)
+        s += (v[i][0] + v[i][1]) + (v[i][2] + v[i][3]);
     const float mean = wave_sum(s) / (float)depth;
     float q = 0.f;
 #pragma unroll
@@ -573,13 +617,11 @@ __global__ __launch_bounds__(256) void layernorm_wave4_kernel(const float* __res
     for (int i = 0; i < NV; ++i) {
         const int z = (lane + i * 64) * 4;
         if (z < depth) {
-            const f32x4 g = gamma ? *reinterpret_cast<const f32x4*>(gamma + z) : f32x4 { 1.f, 1.f, 1.f, 1.f };
-            const f32x4 b = beta ? *reinterpret_cast<const f32x4*>(beta + z) : f32x4 { 0.f, 0.f, 0.f, 0.f };
             f32x4 o;
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                const float inv = rs * g[e];
-                o[e] = v[i][e] * inv + (b[e] - mean * inv);
+                const float inv = rs * g[i][e];
+                o[e] = v[i][e] * inv + (b[i][e] - mean * inv);
             }
             *reinterpret_cast<f32x4*>(orow + z) = o;
         }
@@ -820,12 +862,21 @@ extern "C" fdx_status fdx_dwconv2d_nhwc_f32(const float* in, int n, int h, int w
     else if (slide)
         FDX_DW_SLIDE_LAUNCH(8, 4);
 #undef FDX_DW_SLIDE_LAUNCH
-    else if (k3 && sy == 1)
-        hipLaunchKernelGGL((dwconv3x3_kernel<1, 4>), dim3(grid_for((size_t)n * out_h * ((out_w + 3) / 4) * (c / 4), 256)), dim3(256), 0,
-            stream(), in, weights_hwc, bias, out, n, h, w, c, pad_top, pad_left, out_h, out_w, a);
-    else if (k3)
-        hipLaunchKernelGGL((dwconv3x3_kernel<2, 4>), dim3(grid_for((size_t)n * out_h * ((out_w + 3) / 4) * (c / 4), 256)), dim3(256), 0,
-            stream(), in, weights_hwc, bias, out, n, h, w, c, pad_top, pad_left, out_h, out_w, a);
+    else if (k3 && (uint64_t)h * w * c * 4 < (1ull << 31)) { // (offsets of 31 bits: as many images a launch as that holds)
+        const int most = (int)(((1ull << 31) - 1) / ((uint64_t)h * w * c * 4));
+        for (int i = 0; i < n; i += most) {
+            const int count = n - i < most ? n - i : most;
+            const float* x = in + (size_t)i * h * w * c;
+            float* y = out + (size_t)i * out_h * out_w * c;
+            const dim3 grid(grid_for((size_t)count * out_h * ((out_w + 3) / 4) * (c / 4), 256));
+            if (sy == 1)
+                hipLaunchKernelGGL((dwconv3x3_kernel<1, 4>), grid, dim3(256), 0, stream(), x, weights_hwc, bias, y, count, h, w, c, pad_top,
+                    pad_left, out_h, out_w, a);
+            else
+                hipLaunchKernelGGL((dwconv3x3_kernel<2, 4>), grid, dim3(256), 0, stream(), x, weights_hwc, bias, y, count, h, w, c, pad_top,
+                    pad_left, out_h, out_w, a);
+        }
+    }
     else if (vec)
         hipLaunchKernelGGL(dwconv_kernel<4>, dim3(grid_for(items, 256)), dim3(256), 0, stream(), in, weights_hwc, bias,
             out, n, h, w, c, kh, kw, sy, sx, dy, dx, pad_top, pad_left, out_h, out_w, a);
@@ -847,7 +898,20 @@ extern "C" fdx_status fdx_pool2d_nhwc_f32(const float* in, int n, int h, int w, 
     FDX_REQUIRE(mode == 0 || mode == 1, "pool2d: mode must be 0 (max) or 1 (average)");
     const size_t items = (size_t)n * out_h * out_w * c;
     profile_begin();
-    if (c % 4 == 0 && al16(in) && al16(out))
+    const bool small = c % 4 == 0 && al16(in) && al16(out) && ph == pw && (ph == 2 || ph == 3) && items / 4 < (1ull << 31);
+#define FDX_POOL_SMALL(P_, MAX_)                                                                                                            \
+    hipLaunchKernelGGL((pool2d_small_kernel<P_, P_, MAX_>), dim3(grid_for(items / 4, 256)), dim3(256), 0, stream(), in, out, h, w, c, sy, sx, pad_top, \
+        pad_left, zero_top, zero_left, zero_bottom, zero_right, out_h, out_w, (unsigned)(items / 4))
+    if (small && ph == 2 && mode == 0)
+        FDX_POOL_SMALL(2, true);
+    else if (small && ph == 2)
+        FDX_POOL_SMALL(2, false);
+    else if (small && mode == 0)
+        FDX_POOL_SMALL(3, true);
+    else if (small)
+        FDX_POOL_SMALL(3, false);
+#undef FDX_POOL_SMALL
+    else if (c % 4 == 0 && al16(in) && al16(out))
         hipLaunchKernelGGL(pool2d_kernel<4>, dim3(grid_for(items / 4, 256)), dim3(256), 0, stream(), in, out, n, h, w, c, ph, pw,
             sy, sx, pad_top, pad_left, zero_top, zero_left, zero_bottom, zero_right, out_h, out_w, mode);
     else

@@ -23,25 +23,6 @@ namespace fdx {
 // x / d for x and d below 2^16, with ceil(2^32 / d) from the host (exact there: x times the ceiling's excess stays below 2^32)
 __device__ __forceinline__ int quotient(int x, uint32_t by) { return by ? (int)__umulhi((uint32_t)x, by) : x; }
 
-// maximum or sum over the sixteen lanes of a row and over a wave, in every lane
-template <bool MAX>
-__device__ __forceinline__ float both(float a, float b) { return MAX ? fmaxf(a, b) : a + b; }
-template <bool MAX>
-__device__ __forceinline__ float half_row_all(float v)
-{
-    v = both<MAX>(v, dpp_move<0xB1>(v));
-    v = both<MAX>(v, dpp_move<0x4E>(v));
-    return both<MAX>(v, dpp_move<0x141>(v));
-}
-template <bool MAX>
-__device__ __forceinline__ float wave_all(float v)
-{
-    v = half_row_all<MAX>(v);
-    v = both<MAX>(v, dpp_move<0x140>(v));
-    auto lane = [&](int l) { return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), l)); };
-    return both<MAX>(both<MAX>(lane(0), lane(16)), both<MAX>(lane(32), lane(48)));
-}
-
 __device__ __forceinline__ void sample_frame(const SampleStep& s, float* lds, int t)
 {
     // the frame of zeros around a tensor: its cells are nobody else's
@@ -243,8 +224,8 @@ __device__ __forceinline__ void sample_pool(const SampleStep& s, float* lds, flo
                 }
 #pragma unroll
                 for (int v = 0; v < VEC; ++v) {
-                    val[v] = both<MAX>(val[v], z[0][v]);
-                    val[v] = fx + 1 < x1 ? both<MAX>(val[v], z[1][v]) : val[v];
+                    val[v] = either<MAX>(val[v], z[0][v]);
+                    val[v] = fx + 1 < x1 ? either<MAX>(val[v], z[1][v]) : val[v];
                 }
             }
         }
@@ -280,12 +261,12 @@ __device__ __forceinline__ void sample_global_pool(const SampleStep& s, float* l
                         v[u] = p[(i + u * slots < positions ? i + u * slots : i) * s.in_pix];
 #pragma unroll
                     for (int u = 0; u < 4; ++u)
-                        val = i + u * slots < positions ? both<MAX>(val, v[u]) : val;
+                        val = i + u * slots < positions ? either<MAX>(val, v[u]) : val;
                 }
             else
                 for (int i = slot; i < positions; i += slots) {
                     const int y = quotient(i, s.by_in_w), x = i - y * s.in_w;
-                    val = both<MAX>(val, p[y * s.in_row + x * s.in_pix]);
+                    val = either<MAX>(val, p[y * s.in_row + x * s.in_pix]);
                 }
         }
         scratch[t] = val;
@@ -299,7 +280,7 @@ __device__ __forceinline__ void sample_global_pool(const SampleStep& s, float* l
                     v[u] = scratch[((q + 8 * u < slots ? q + 8 * u : q) << log2w) + i];
 #pragma unroll
                 for (int u = 0; u < 4; ++u)
-                    val = q + 8 * u < slots ? both<MAX>(val, v[u]) : val;
+                    val = q + 8 * u < slots ? either<MAX>(val, v[u]) : val;
             }
             val = half_row_all<MAX>(val);
             if ((t & 7) == 0)

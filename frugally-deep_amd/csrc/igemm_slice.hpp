@@ -291,11 +291,14 @@ struct SliceForm {
 };
 constexpr SliceForm kSliceForm[kSliceForms] = { { 1, 1, 8 }, { 1, 2, 8 }, { 2, 2, 8 }, { 2, 2, 4 }, { 4, 2, 8 } };
 
-// The form for a problem, or -1 where the tiled kernel (its cost by tile_pick) is the better one.  The forms were timed on 483
-// problems (M 1-16384, N 16-3072, K 32-4608, up to 6 GFLOP, GEMM and convolution, operands out of memory, launches back to
-// back) and follow, in microseconds, with w = tiles per CU rounded up, to 8-13 % rms
+// The form for a problem, or -1 where the tiled kernel (its cost by tile_pick) is the better one.  The forms were timed on 1000
+// problems (M 1-16384, N 16-3072, K 16-4608, up to 6 GFLOP, GEMM and convolution, weights out of memory, launches back to
+// back) and follow, in microseconds, with w = tiles per CU rounded up, to 13-21 % rms
 //     t0 + w (c1 + c2 (rows + columns of the tile) K / 10^4), c2 larger for a convolution's addressing:
-// a workgroup costs what it pulls through its CU's path from L2, about 36 cycles per KB.  Up to 32 columns the other side is the
+// a workgroup costs what it pulls through its CU's path from L2, about 36 cycles per KB.  With one round of tiles (the first row of a form)
+// K counts up to whole units of all waves: where it is one unit of 32, waves have nothing to do, and the form of four is the fastest (337 x
+// 1144 x 32: 8 / 4 waves 5.0 / 3.8 us); there the choice among the forms takes 0.6 % longer than the best of them, past a round
+// 2.5 %.  Up to 32 columns the other side is the
 // general kernel's narrow tile, which wins from about 600 row blocks of 64 on (N = 32, K = 144-192: 20000 rows 8.2-9.7 against
 // 6.3-7.2 us here, 50000 rows 11.0-14.5 against 11.1-14.0, convolutions 13.9 against 17.1); between 32 and 64 columns the tiled
 // kernel's half empty 64-column tile beats it (97733 x 40 x 288 31.5 against 40.9 us, 24000 x 36 x 512 17.4 / 21.7).
@@ -303,12 +306,16 @@ static int64_t slice_tiles(int M, int N, int bm, int bn) { return (int64_t)((M +
 static float slice_rounds(int64_t tiles) { return (float)((tiles + 255) / 256); }
 static float slice_cost(int form, bool conv, int M, int N, int K)
 {
-    static const float kCost[kSliceForms][4] = { // t0, c1, c2 of a GEMM, c2 of a convolution
-        { 2.18f, 1.29f, 0.42f, 0.59f }, { 2.13f, 1.07f, 0.50f, 0.62f }, { 2.24f, 1.47f, 0.64f, 1.02f }, { 2.52f, 0.71f, 0.76f, 0.92f },
-        { 1.52f, 2.43f, 0.83f, 1.25f }
+    static const float kCost[kSliceForms][2][4] = { // t0, c1, c2 of a GEMM, c2 of a convolution; one round of tiles, more
+        { { 2.46f, 0.64f, 0.39f, 0.89f }, { 2.18f, 1.29f, 0.42f, 0.59f } }, { { 2.73f, 0.25f, 0.47f, 0.78f }, { 2.13f, 1.07f, 0.50f, 0.62f } },
+        { { 2.01f, 0.77f, 0.65f, 1.15f }, { 2.24f, 1.47f, 0.64f, 1.02f } }, { { 2.89f, 0.19f, 0.68f, 1.14f }, { 2.52f, 0.71f, 0.76f, 0.92f } },
+        { { 1.62f, 1.19f, 0.80f, 1.42f }, { 1.52f, 2.43f, 0.83f, 1.25f } }
     };
-    const int bm = 16 * kSliceForm[form].tm, bn = 16 * kSliceForm[form].tn;
-    return kCost[form][0] + slice_rounds(slice_tiles(M, N, bm, bn)) * (kCost[form][1] + kCost[form][conv ? 3 : 2] * 1e-4f * (bm + bn) * K);
+    const int bm = 16 * kSliceForm[form].tm, bn = 16 * kSliceForm[form].tn, unit = 32 * kSliceForm[form].nw;
+    const float rounds = slice_rounds(slice_tiles(M, N, bm, bn));
+    const float* c = kCost[form][rounds > 1.f ? 1 : 0];
+    const int k = rounds > 1.f ? K : (K + unit - 1) / unit * unit;
+    return c[0] + rounds * (c[1] + c[conv ? 3 : 2] * 1e-4f * (bm + bn) * k);
 }
 // whether a launch of this form stays below the 2^32 threads a grid can have
 static bool slice_fits(int form, int M, int N)
@@ -323,7 +330,12 @@ static int slice_pick(bool conv, int M, int N, int K, float tiled_cost)
     if (narrow && t64 > 512)
         return -1;
     int best = -1;
-    float best_cost = narrow ? 1e30f : (t64 <= 256 ? 0.95f : 0.85f) * tiled_cost; // past a round of tiles operands re-read cost the neighbours, too
+    // Below a round of tiles the tiled kernel takes longer than its cost says, which was fitted to 0.2 GFLOP and more: on 600 small problems by
+    // 1.4 us up to K = 128 (4204 x 64 x 64 5.7 against 3.6 us here), convolutions by half (3x3 16 -> 388 on 1001 pixels 9.7 / 7.2), less where
+    // K is long.  Kernel choices then take 1.7 % longer than the best, 5.2 % with 0.95 of the cost.  Past a round operands re-read cost
+    // the neighbours, too.
+    const float fade = 15.f / std::max(15.f, tiled_cost);
+    float best_cost = narrow ? 1e30f : t64 > 256 ? 0.95f * tiled_cost : conv ? (K <= 1024 ? 1.3f : 1.15f) * tiled_cost : tiled_cost + 1.5f * fade * fade;
     for (int i = 0; i < kSliceForms; ++i) {
         const float cost = slice_cost(i, conv, M, N, K);
         if (cost < best_cost && slice_fits(i, M, N)) {

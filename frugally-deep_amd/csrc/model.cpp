@@ -3199,10 +3199,40 @@ namespace {
                 }
                 FDX_HIP(hipMemcpyAsync(p->out[m->inputs[i]], in[i], bytes, hipMemcpyDeviceToDevice, stream()));
             }
-        // a model that runs as one launch writes its result where the caller wants it
-        const bool one_launch = p->sample && (g_force_sample_net == 1 || !tile_forced()), direct = one_launch && out_on_device && out[0];
+        // Results go where the caller wants them as they are produced, where his buffer is aligned like the plan's and meets none of
+        // the inputs or other results (saves the copy's launch: 2 us of a pass): the output op and its views point there for
+        // this call.
+        std::vector<char> direct(m->outputs.size(), 0);
+        const bool one_launch = p->sample && (g_force_sample_net == 1 || !tile_forced());
+        if (out_on_device) {
+            auto root = [&](int i) {
+                while (m->ops[(size_t)i].kind == OpKind::View)
+                    i = m->ops[(size_t)i].in[0];
+                return i;
+            };
+            auto meets = [&](const void* a, size_t an, const void* b, size_t bn) {
+                return reinterpret_cast<uintptr_t>(a) < reinterpret_cast<uintptr_t>(b) + bn && reinterpret_cast<uintptr_t>(b) < reinterpret_cast<uintptr_t>(a) + an;
+            };
+            auto bytes_of = [&](int op) { return sizeof(float) * (size_t)batch * (size_t)volume(p->shapes[(size_t)op]); };
+            for (size_t i = 0; i < m->outputs.size(); ++i) {
+                const int op = root(m->outputs[i]);
+                bool ok = out[i] && (reinterpret_cast<uintptr_t>(out[i]) & 15) == 0 && p->block_of[(size_t)op] >= 0 && m->ops[(size_t)op].kind != OpKind::Input;
+                for (size_t k = 0; k < m->inputs.size() && ok; ++k)
+                    ok = !meets(out[i], bytes_of(op), p->out[(size_t)m->inputs[k]], bytes_of(m->inputs[k]));
+                for (size_t k = 0; k < m->outputs.size() && ok; ++k)
+                    ok = k == i || (root(m->outputs[k]) != op && !meets(out[i], bytes_of(op), out[k], bytes_of(m->outputs[k])));
+                if (!ok)
+                    continue;
+                direct[i] = 1;
+                for (int k : p->order)
+                    if (root(k) == op) {
+                        restore.saved.emplace_back(k, p->out[(size_t)k]);
+                        p->out[(size_t)k] = out[i];
+                    }
+            }
+        }
         if (one_launch) {
-            st = sample_net_launch(*p->sample, p->out[m->inputs[0]], batch, direct ? out[0] : p->out[m->outputs[0]]);
+            st = sample_net_launch(*p->sample, p->out[m->inputs[0]], batch, p->out[m->outputs[0]]);
             m->last_flops = p->flops;
         } else
             st = execute(*m, *p, done_until);
@@ -3226,7 +3256,9 @@ namespace {
                 bounce_lock.unlock();
         }
         size_t at = 0;
-        for (size_t i = 0; i < m->outputs.size() && !direct; ++i) {
+        for (size_t i = 0; i < m->outputs.size(); ++i) {
+            if (direct[i])
+                continue;
             const size_t bytes = sizeof(float) * (size_t)batch * (size_t)volume(p->shapes[m->outputs[i]]);
             FDX_HIP(hipMemcpyAsync(bounce ? static_cast<void*>(bounce + at) : static_cast<void*>(out[i]), p->out[m->outputs[i]], bytes,
                 out_on_device ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost, stream()));

@@ -37,20 +37,23 @@ def test_windows_of_infinities(fdx, oracle):
 
 
 def test_depthwise_beyond_two_gib(fdx):
-    import torch
     n, s, c = 3, 4096, 16  # 1 GiB an image
-    x = torch.randn((n, s, s, c), device="cuda")
-    w, b = torch.randn((3, 3, c), device="cuda"), torch.randn((c,), device="cuda")
-    out, one = torch.full((n, s // 2, s // 2, c), 7.0, device="cuda"), torch.empty((1, s // 2, s // 2, c), device="cuda")
-    torch.cuda.synchronize()
-    p = lambda t, i=0: ctypes.c_void_p(t[i].data_ptr())
-
-    def run(src, count, dst):
-        fdx.check(fdx.lib.fdx_dwconv2d_nhwc_f32(src, count, s, s, c, ctypes.c_void_p(w.data_ptr()), ctypes.c_void_p(b.data_ptr()), 3, 3, 2, 2, 1, 1, 0, 0,
-                                                s // 2, s // 2, None, dst))
-        fdx.sync()
-
-    run(p(x), n, p(out))
+    r = np.random.default_rng(9)
+    some = r.standard_normal(1 << 20).astype(np.float32)
+    x = fdx.DevBuf(4 * n * s * s * c)
     for i in range(n):
-        run(p(x, i), 1, p(one))
-        assert torch.equal(one[0], out[i]), i
+        image = np.tile(np.roll(some, 77 * i), s * s * c >> 20)
+        fdx.check(fdx.lib.fdx_h2d(ctypes.c_void_p(x.ptr.value + 4 * i * s * s * c), image.ctypes.data_as(ctypes.c_void_p), ctypes.c_size_t(image.nbytes)))
+    w, b = fdx.DevBuf.from_host(r.standard_normal((3, 3, c)).astype(np.float32)), fdx.DevBuf.from_host(r.standard_normal(c).astype(np.float32))
+    size = 4 * s * s * c // 4
+    out, one = fdx.DevBuf(n * size), fdx.DevBuf(size)
+
+    def run(image, count, dst):
+        fdx.check(fdx.lib.fdx_dwconv2d_nhwc_f32(ctypes.c_void_p(x.ptr.value + 4 * image * s * s * c), count, s, s, c, fdx._dp(w), fdx._dp(b), 3, 3, 2, 2, 1, 1, 0, 0,
+                                                s // 2, s // 2, None, fdx._dp(dst)))
+
+    run(0, n, out)
+    got = out.to_host((n, size // 4))
+    for i in range(n):
+        run(i, 1, one)
+        assert np.array_equal(one.to_host((size // 4,)), got[i]), i

@@ -9,7 +9,7 @@ namespace fdx {
 // One step of the program that a workgroup runs (read through the scalar cache, three lines each).  Positions (base, tab, weights, bias, ...) count floats
 // from the start of LDS; tensors are rows of pixels of channels with strides of their own.
 struct alignas(64) SampleStep {
-    enum Kind { Load, Conv, Pool, GlobalPool, Softmax, Activation };
+    enum Kind { Load, Conv, Row, Pool, GlobalPool, Softmax, Activation };
     int kind;
     int out_base, out_row, out_pix, out_h, out_w, out_c; // out_base < 0: the sample's row of the result
     int frame_base, frame_h, frame_w, frame_top, frame_left; // output with its frame of zeros, frame_h = 0: none

@@ -39,11 +39,12 @@ namespace {
 
     bool epilogue_kind(const Act& a) { return a.kind == FDX_ACT_NONE || a.kind == FDX_ACT_RELU || a.kind == FDX_ACT_GELU; }
 
-    // Cycles of a CU: the matrix pipes', or the chain of a wave's own items where there are few, and a step's latency.
-    double conv_cycles(int pixels, int n_tiles, int chunks)
+    // Cycles of a CU: the matrix pipes', or the chain of a wave's own items where there are few, and a step's latency, longer where
+    // pixels are read one float at a time.
+    double conv_cycles(int pixels, int n_tiles, int chunks, bool vec)
     {
         const double m_tiles = (pixels + 15) / 16, items = m_tiles * n_tiles;
-        return 2000 + 1500 * std::min(1.0, m_tiles / 16) + 1.25 * std::max(items * chunks * 32, std::ceil(items / 16) * chunks * 350);
+        return (vec ? 2000 : 4000) + 1500 * std::min(1.0, m_tiles / 16) + 1.25 * std::max(items * chunks * 32, std::ceil(items / 16) * chunks * 350);
     }
 
 } // namespace
@@ -287,34 +288,42 @@ std::shared_ptr<SampleProgram> sample_net_build(const fdx_model& m, const std::v
                 s.act_slope = o.act.negative_slope;
                 s.act_threshold = o.act.threshold;
             }
-            const int dy = conv ? o.dy : 1, dx = conv ? o.dx : 1;
-            auto offset = [&](int k) {
-                const int tap = k / cin, fy = tap / kw, fx = tap - fy * kw;
-                return k < k_all ? fy * dy * row + fx * dx * pix + (k - tap * cin) : -1;
-            };
-            // a lane group's offsets side by side, a chunk's four groups one after the other
-            const int per = s.vec ? 4 : 1;
-            s.tab_stride = s.vec ? (s.chunks + 3) / 4 * 4 : s.chunks * 4;
-            s.tab = words((size_t)s.tab_stride * 4);
-            for (int kc = 0; kc < s.chunks; ++kc)
-                for (int fg = 0; fg < 4; ++fg)
-                    for (int e = 0; e < 4; e += per) {
-                        const int v = offset(kc * 16 + fg * 4 + e);
-                        std::memcpy(&image[(size_t)(s.tab + fg * s.tab_stride + (s.vec ? kc : kc * 4 + e))], &v, 4);
-                    }
-            s.weights = words((size_t)s.n_tiles * s.chunks * 256);
-            for (int nt = 0; nt < s.n_tiles; ++nt)
+            if (kh * kw == 1 && x.h * x.w == 1 && me.h * me.w == 1 && !s.pad_top && !s.pad_left) { // one pixel: weights as rows
+                s.kind = SampleStep::Row;
+                const int stride = (cin + 3) / 4 * 4;
+                s.weights = words((size_t)cout * stride);
+                for (int n = 0; n < cout; ++n)
+                    std::memcpy(&image[(size_t)s.weights + (size_t)n * stride], &o.sample_w[(size_t)n * cin], (size_t)cin * 4);
+            } else {
+                const int dy = conv ? o.dy : 1, dx = conv ? o.dx : 1;
+                auto offset = [&](int k) {
+                    const int tap = k / cin, fy = tap / kw, fx = tap - fy * kw;
+                    return k < k_all ? fy * dy * row + fx * dx * pix + (k - tap * cin) : -1;
+                };
+                // a lane group's offsets side by side, a chunk's four groups one after the other
+                const int per = s.vec ? 4 : 1;
+                s.tab_stride = s.vec ? (s.chunks + 3) / 4 * 4 : s.chunks * 4;
+                s.tab = words((size_t)s.tab_stride * 4);
                 for (int kc = 0; kc < s.chunks; ++kc)
-                    for (int lane = 0; lane < 64; ++lane)
-                        for (int e = 0; e < 4; ++e) {
-                            const int n = nt * 16 + (lane & 15), k = kc * 16 + (lane >> 4) * 4 + e;
-                            if (n < cout && k < k_all)
-                                image[(size_t)s.weights + ((size_t)(nt * s.chunks + kc) * 64 + lane) * 4 + e] = o.sample_w[(size_t)n * k_all + k];
+                    for (int fg = 0; fg < 4; ++fg)
+                        for (int e = 0; e < 4; e += per) {
+                            const int v = offset(kc * 16 + fg * 4 + e);
+                            std::memcpy(&image[(size_t)(s.tab + fg * s.tab_stride + (s.vec ? kc : kc * 4 + e))], &v, 4);
                         }
+                s.weights = words((size_t)s.n_tiles * s.chunks * 256);
+                for (int nt = 0; nt < s.n_tiles; ++nt)
+                    for (int kc = 0; kc < s.chunks; ++kc)
+                        for (int lane = 0; lane < 64; ++lane)
+                            for (int e = 0; e < 4; ++e) {
+                                const int n = nt * 16 + (lane & 15), k = kc * 16 + (lane >> 4) * 4 + e;
+                                if (n < cout && k < k_all)
+                                    image[(size_t)s.weights + ((size_t)(nt * s.chunks + kc) * 64 + lane) * 4 + e] = o.sample_w[(size_t)n * k_all + k];
+                            }
+            }
             s.bias = words((size_t)s.n_tiles * 16);
             for (int n = 0; n < cout && n < (int)o.sample_bias.size(); ++n)
                 image[(size_t)(s.bias + n)] = o.sample_bias[(size_t)n];
-            cycles += conv_cycles(me.h * me.w, s.n_tiles, s.chunks);
+            cycles += s.kind == SampleStep::Row ? 1000 + std::ceil(cout / 128.0) * (150 + cin * 2) : conv_cycles(me.h * me.w, s.n_tiles, s.chunks, s.vec);
         }
         if (image.size() > (size_t)kSampleLdsFloats)
             return nullptr;
@@ -389,8 +398,11 @@ std::shared_ptr<SampleProgram> sample_net_build(const fdx_model& m, const std::v
         if (s.kind == SampleStep::Pool) {
             s.vec = s.out_base >= 0 && (s.in_c | s.in_base | s.in_row | s.in_pix | s.out_base | s.out_row | s.out_pix) % 4 == 0;
             s.by_out_c = by(s.vec ? s.out_c / 4 : s.out_c);
+            s.whole = s.kh == 2 && s.kw == 2 && !s.pad_top && !s.pad_left && (s.out_h - 1) * s.sy + 2 <= s.in_h && (s.out_w - 1) * s.sx + 2 <= s.in_w;
         }
-        if (s.kind == SampleStep::Conv) {
+        if (s.kind == SampleStep::Row)
+            s.vec = (s.in_c | s.in_base) % 4 == 0;
+        if (s.kind == SampleStep::Conv || s.kind == SampleStep::Row) {
             s.in_base -= s.pad_top * s.in_row + s.pad_left * s.in_pix;
             if (o.residual >= 0) {
                 const Tensor& r = tensors[(size_t)of[(size_t)o.residual]];
@@ -400,8 +412,10 @@ std::shared_ptr<SampleProgram> sample_net_build(const fdx_model& m, const std::v
                 s.res_pix = r.compact ? rs.c : r.pix;
             }
         }
-        if (s.kind == SampleStep::GlobalPool)
+        if (s.kind == SampleStep::GlobalPool) {
             s.scratch = tensors[(size_t)scratch_of[(size_t)idx]].start;
+            s.vec = (s.in_c | s.in_base | s.in_pix) % 4 == 0 && s.in_row == s.in_w * s.in_pix;
+        }
     }
 
     auto p = std::make_shared<SampleProgram>();
@@ -410,7 +424,7 @@ std::shared_ptr<SampleProgram> sample_net_build(const fdx_model& m, const std::v
     p->steps = (int)steps.size();
     p->in_volume = p_in_volume;
     p->out_volume = (int)volume(shapes[(size_t)m.outputs[0]]);
-    p->us_per_sample = cycles / 2400.0;
+    p->us_per_sample = (cycles + 0.4 * p->out_volume) / 2400.0; // (a result's way out: four floats a cycle at most, 256 CUs at once)
     const size_t step_at = (image.size() + 15) / 16 * 16, step_floats = steps.size() * sizeof(SampleStep) / 4;
     image.resize(step_at + step_floats);
     std::memcpy(&image[step_at], steps.data(), step_floats * 4);
@@ -425,11 +439,11 @@ std::shared_ptr<SampleProgram> sample_net_build(const fdx_model& m, const std::v
 
 // One launch or one per operation, by predicted times: a launch costs what the chain's shortest take (3.7 us), or its traffic and its
 // arithmetic, at 90 TFLOP/s where the tiled kernel has whole slabs and columns and 30 elsewhere, of columns that fill its tile.  Measured, us of a call, launches /
-// one: the small CNN (two 3x3 convolutions of 16 and 32 channels on 32 x 32 x 3) at batch 1 / 256 / 8192 28 / 18.8, 62 / 19.2, 902 /
-// 524; 28 x 28 with 5x5 convolutions of 6 and 16 channels and two Dense layers 48 / 18, 66 / 18.8, 719 / 482; four 3x3
-// convolutions of 16 channels on 16 x 16 33 / 20, 67 / 21, 1060 / 575; strided 3x3 of 32 and 64 channels on 32 x 32 x 3 27 / 16,
-// 37 / 17, 345 / 427 (the rule leaves the last to the launches); three Dense layers of 128 at batch 1 / 256 / 700 16 / 8.7, 16 / 9.4,
-// 17 / 20 (the last left to the launches); one 3x3 convolution 8 -> 32 on 24 x 24 at batch 1 / 256 10 / 13 (left), 28 / 16.
+// one: the small CNN (two 3x3 convolutions of 16 and 32 channels on 32 x 32 x 3) at batch 1 / 256 / 8192 24 / 16.7, 59 / 17.7, 902 /
+// 478; 28 x 28 with 5x5 convolutions of 6 and 16 channels and two Dense layers 44 / 14.9, 61 / 15.9, 717 / 405; four 3x3
+// convolutions of 16 channels on 16 x 16 26 / 19.6, 65 / 20.5, 1060 / 566; strided 3x3 of 32 and 64 channels on 32 x 32 x 3 23 / 15,
+// 40 / 16, 340 / 407 (the rule leaves the last to the launches); three Dense layers of 128 at batch 1 / 256 / 2048 13.5 / 6.8, 13.7 /
+// 7.0, 13.7 / 28 (the last left to the launches); one 3x3 convolution 8 -> 32 on 24 x 24 at batch 1 / 256 8.2 / 12.7 (left), 19.4 / 16.3.
 bool sample_net_by_rule(const SampleProgram& p, const fdx_model& m, const std::vector<int>& order, const std::vector<Shape>& shapes, int batch)
 {
     double launches = 0;

@@ -59,7 +59,31 @@ def wide_pool(b):
     return b.gap(x, "g")
 
 
-NETS = {f.__name__: f for f in (odd_convs, residual, flattened, sequence, wide_pool)}
+def vectors(b):
+    # matrices times one pixel: odd K, more rows than a workgroup takes at once, a K of several rounds; pooled channels that are no
+    # multiple of four; 2 x 2 windows that leave a row and a column over
+    x = b.input((9, 7, 8), "in")
+    x = b.pool(x, "p", 2, 2)
+    x = b.conv2d(x, 13, 3, "a", padding="same", activation="relu", bias_std=0.2)
+    x = b.gap(x, "g")
+    x = b.dense(x, 150, "b", activation="relu", bias_std=0.3)
+    x = b.dense(x, 68, "c", activation="gelu", bias_std=0.3)
+    return b.dense(x, 5, "d", bias_std=0.1)
+
+
+def full_input(b):
+    # the largest input
+    x = b.pool(b.input((64, 64, 4), "in"), "p", 4, 4)
+    return b.gap(b.conv2d(x, 20, 3, "a", activation="relu", bias_std=0.2), "g")
+
+
+def odd_input(b):
+    # a volume that is no multiple of four
+    x = b.pool(b.input((61, 47, 5), "in"), "p", 3, 3, kind="avg")
+    return b.gap(b.conv2d(x, 6, 3, "a", activation="relu", bias_std=0.2), "g", kind="max")
+
+
+NETS = {f.__name__: f for f in (odd_convs, residual, flattened, sequence, wide_pool, vectors, full_input, odd_input)}
 
 
 @pytest.mark.parametrize("batch", [1, 3, 300])  # one sample, fewer than CUs, more than CUs (a workgroup's second sample)

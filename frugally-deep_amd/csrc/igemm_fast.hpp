@@ -172,6 +172,20 @@ __device__ __forceinline__ int seg_of(const GemmParams& p, int n0) { return (n0 
 //    operands are read from LDS at its distance; a lane whose row has no such pixel (the convolution's padding) reads a
 //    pixel of zeros kept behind the run.  64 images: 28 x 28 x 128 -> 128 84 -> 77 us, 14 x 14 x 256 -> 256 87 -> 77,
 //    56 x 56 x 64 -> 64 113 -> 85; 16 images 32 -> 29, 35 (few-tiles ranges) -> 36, 34 -> 26.
+// Bit y * kw + x: filter tap (y, x) lies inside the image, for a row whose tap (0, 0) lies at (iy, ix).  Columns and rows apart and without
+// branches: tap by tap, with lanes taking branches of their own, nine taps of eight rows held up every tile's first load (ResNet50 of 64
+// images 0.5 % longer).
+template <typename Mask>
+__device__ __forceinline__ Mask taps_inside(const GemmParams& p, int iy, int ix)
+{
+    Mask row = 0, all = 0;
+    for (int x = 0; x < p.kw; ++x, ix += p.dx)
+        row |= (Mask)((unsigned)ix < (unsigned)p.W) << x;
+    for (int y = 0, at = 0; y < p.kh; ++y, iy += p.dy, at += p.kw)
+        all |= (unsigned)iy < (unsigned)p.H ? row << at : (Mask)0;
+    return all;
+}
+
 template <int BM, int BN, int WAVES_M, int WAVES_N, bool CONV, bool SPLIT = false, bool STREAMK = false, bool DUAL = false,
     bool LNF = false, bool SEG = false, bool HALO = false>
 __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, split_tile_waves(BM, BN, WAVES_M, WAVES_N))
@@ -313,16 +327,7 @@ void igemm_fast_kernel(GemmParams p)
             for (int i = 0; i < TM; ++i) {
                 const int m = m0 + wm * WTM + i * 32 + fr;
                 const int rm = m % (p.OH * p.OW), oy = rm / p.OW, ox = rm - oy * p.OW;
-                uint32_t mk = 0;
-                for (int y = 0; y < p.kh; ++y) {
-                    const int iy = oy - p.pad_top + y * p.dy;
-                    for (int x = 0; x < p.kw; ++x) {
-                        const int ix = ox - p.pad_left + x * p.dx;
-                        if (m < p.M && iy >= 0 && iy < p.H && ix >= 0 && ix < p.W)
-                            mk |= 1u << (y * p.kw + x);
-                    }
-                }
-                row_mask[i] = mk;
+                row_mask[i] = m < p.M ? taps_inside<uint32_t>(p, oy - p.pad_top, ox - p.pad_left) : 0u;
             }
         } else
 #pragma unroll
@@ -334,19 +339,9 @@ void igemm_fast_kernel(GemmParams p)
                 if (CONV) {
                     const int img = m / (p.OH * p.OW), rm = m - img * (p.OH * p.OW);
                     const int oy = rm / p.OW, ox = rm - oy * p.OW;
-                    const int iy0 = oy * p.sy - p.pad_top, ix0 = ox * p.sx - p.pad_left;
                     // byte offset from the shifted base (shift = (pad_top*W + pad_left)*Cin elements)
                     a_voff[i] = (uint32_t)(((img * p.H + oy * p.sy) * p.W + ox * p.sx) * p.pix_stride) * 4u + kq * 16;
-                    uint64_t mk = 0;
-                    for (int y = 0; y < p.kh; ++y) {
-                        const int iy = iy0 + y * p.dy;
-                        for (int x = 0; x < p.kw; ++x) {
-                            const int ix = ix0 + x * p.dx;
-                            if (iy >= 0 && iy < p.H && ix >= 0 && ix < p.W)
-                                mk |= 1ull << (y * p.kw + x);
-                        }
-                    }
-                    a_mask[HALO ? 0 : i] = mk;
+                    a_mask[HALO ? 0 : i] = taps_inside<uint64_t>(p, oy * p.sy - p.pad_top, ox * p.sx - p.pad_left);
                 } else {
                     a_voff[i] = (uint32_t)((int64_t)m * p.lda) * 4u + kq * 16;
                     a_mask[HALO ? 0 : i] = ~0ull;

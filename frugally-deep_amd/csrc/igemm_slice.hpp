@@ -3,8 +3,8 @@
 //
 // There the tiled kernel leaves most of the chip idle: a 64 x 64 tile of a 14 x 14 map walks K = 2304 slab by slab, each
 // slab a round trip to memory, an LDS pass and a barrier (one image, weights out of memory, per launch: 14 x 14 3x3
-// 256 -> 256 19.6 us, 1x1 1024 -> 256 13.6, 7 x 7 3x3 512 -> 512 26.8; here 9.4, 4.7, 13.2, of which 3.5 are the launch
-// itself; ResNet50 at batch 1 761 -> 390 us).  What bounds it is the path from L2 into a CU.  Here the eight (or four) waves
+// 256 -> 256 19.6 us, 1x1 1024 -> 256 13.6, 7 x 7 3x3 512 -> 512 26.8; here 8.0, 4.6, 10.4, of which 3.5 are the launch
+// itself; ResNet50 at batch 1 761 -> 330 us).  What bounds it is the path from L2 into a CU.  Here the eight (or four) waves
 // of a workgroup share one small output tile and cut its K range between them, every wave on its own:
 //
 //  * a wave loads its units (UK consecutive k of all tile rows) as runs of 64 or 128 bytes per row, DEPTH units in flight from
@@ -62,30 +62,21 @@ __global__ __launch_bounds__(64 * NW) void igemm_slice_kernel(GemmParams p)
     const int m0 = mt * BM, n0 = nt * BN;
 
     uint32_t a_voff[AL], a2_voff[DUAL ? AL : 1], b_voff[BL];
-    uint64_t a_mask[AL];
+    int a_y[CONV ? AL : 1], a_x[CONV ? AL : 1]; // where tap (0, 0) of a row lies in the image
 #pragma unroll
     for (int i = 0; i < AL; ++i) {
         const int m = m0 + i * RPI + lrow;
         a_voff[i] = OOB;
-        a_mask[i] = 0;
+        a_y[CONV ? i : 0] = a_x[CONV ? i : 0] = -(1 << 30);
         if (DUAL)
             a2_voff[i] = OOB;
         if (m < p.M) {
             if (CONV) {
                 const int img = m / (p.OH * p.OW), rm = m - img * (p.OH * p.OW);
                 const int oy = rm / p.OW, ox = rm - oy * p.OW;
-                const int iy0 = oy * p.sy - p.pad_top, ix0 = ox * p.sx - p.pad_left;
+                a_y[CONV ? i : 0] = oy * p.sy - p.pad_top;
+                a_x[CONV ? i : 0] = ox * p.sx - p.pad_left;
                 a_voff[i] = (uint32_t)(((img * p.H + oy * p.sy) * p.W + ox * p.sx) * p.pix_stride) * 4u + lchunk * 16;
-                uint64_t mk = 0;
-                for (int y = 0; y < p.kh; ++y) {
-                    const int iy = iy0 + y * p.dy;
-                    for (int x = 0; x < p.kw; ++x) {
-                        const int ix = ix0 + x * p.dx;
-                        if (iy >= 0 && iy < p.H && ix >= 0 && ix < p.W)
-                            mk |= 1ull << (y * p.kw + x);
-                    }
-                }
-                a_mask[i] = mk;
             } else {
                 a_voff[i] = (uint32_t)((int64_t)m * p.lda) * 4u + lchunk * 16;
                 if (DUAL) {
@@ -105,10 +96,10 @@ __global__ __launch_bounds__(64 * NW) void igemm_slice_kernel(GemmParams p)
     // this wave's units of UK k
     const int units = p.K / UK;
     const int u_lo = (int)((int64_t)units * wave / NW), u_n = (int)((int64_t)units * (wave + 1) / NW) - u_lo;
-    int soff_b = u_lo * (UK * 4), soff_a = soff_b, tap = 0, fx = 0, fy = 0, c0 = 0;
+    int soff_b = u_lo * (UK * 4), soff_a = soff_b, fx = 0, fy = 0, c0 = 0;
     if (CONV) {
         const int k = u_lo * UK;
-        tap = k / p.Cin;
+        const int tap = k / p.Cin;
         c0 = k - tap * p.Cin;
         fy = tap / p.kw;
         fx = tap - fy * p.kw;
@@ -116,11 +107,14 @@ __global__ __launch_bounds__(64 * NW) void igemm_slice_kernel(GemmParams p)
     }
     f32x4 ra[DEPTH][AL], rb[DEPTH][BL];
     uint32_t a_eff[CONV ? AL : 1]; // a_voff under the current filter tap: out of range where the tap lies outside the image
+    // (compared at each tap: a mask of all taps, made in front of the first load, held that up; 3 x 3 launches of ResNet50 on one image 10.2 and 9.6 us with it, 8.4 and 7.2 without)
     auto enter_tap = [&]() {
         if (CONV) {
 #pragma unroll
-            for (int i = 0; i < AL; ++i)
-                a_eff[CONV ? i : 0] = ((a_mask[i] >> tap) & 1) ? a_voff[i] : OOB;
+            for (int i = 0; i < AL; ++i) {
+                const bool inside = (unsigned)(a_y[CONV ? i : 0] + fy * p.dy) < (unsigned)p.H && (unsigned)(a_x[CONV ? i : 0] + fx * p.dx) < (unsigned)p.W;
+                a_eff[CONV ? i : 0] = inside ? a_voff[i] : OOB;
+            }
         }
     };
     enter_tap();
@@ -145,7 +139,6 @@ __global__ __launch_bounds__(64 * NW) void igemm_slice_kernel(GemmParams p)
             c0 += UK;
             if (c0 == p.Cin) {
                 c0 = 0;
-                ++tap;
                 if (++fx == p.kw) {
                     fx = 0;
                     ++fy;
@@ -294,7 +287,7 @@ constexpr SliceForm kSliceForm[kSliceForms] = { { 1, 1, 8 }, { 1, 2, 8 }, { 2, 2
 // The form for a problem, or -1 where the tiled kernel (its cost by tile_pick) is the better one.  The forms were timed on 1000
 // problems (M 1-16384, N 16-3072, K 16-4608, up to 6 GFLOP, GEMM and convolution, weights out of memory, launches back to
 // back) and follow, in microseconds, with w = tiles per CU rounded up, to 13-21 % rms
-//     t0 + w (c1 + c2 (rows + columns of the tile) K / 10^4), c2 larger for a convolution's addressing:
+//     t0 + w (c1 + c2 (rows + columns of the tile) K / 10^4), c2 larger for a convolution:
 // a workgroup costs what it pulls through its CU's path from L2, about 36 cycles per KB.  With one round of tiles (the first row of a form)
 // K counts up to whole units of all waves: where it is one unit of 32, waves have nothing to do, and the form of four is the fastest (337 x
 // 1144 x 32: 8 / 4 waves 5.0 / 3.8 us); there the choice among the forms takes 0.6 % longer than the best of them, past a round
@@ -302,6 +295,8 @@ constexpr SliceForm kSliceForm[kSliceForms] = { { 1, 1, 8 }, { 1, 2, 8 }, { 2, 2
 // general kernel's narrow tile, which wins from about 600 row blocks of 64 on (N = 32, K = 144-192: 20000 rows 8.2-9.7 against
 // 6.3-7.2 us here, 50000 rows 11.0-14.5 against 11.1-14.0, convolutions 13.9 against 17.1); between 32 and 64 columns the tiled
 // kernel's half empty 64-column tile beats it (97733 x 40 x 288 31.5 against 40.9 us, 24000 x 36 x 512 17.4 / 21.7).
+// A convolution's constants are those of a kernel that made a mask of all taps first and put it 1 to 2 us too high, on both sides of the
+// choice: it takes 1.9 % longer than the best of 143 timed convolutions. Fitted again 1.3 %, but ResNet50 of one image 332 against 330 us.
 static int64_t slice_tiles(int M, int N, int bm, int bn) { return (int64_t)((M + bm - 1) / bm) * ((N + bn - 1) / bn); }
 static float slice_rounds(int64_t tiles) { return (float)((tiles + 255) / 256); }
 static float slice_cost(int form, bool conv, int M, int N, int K)

@@ -30,7 +30,7 @@ PEAK_FP32_PRODUCTS_TFLOPS = 419.4
 # kernel families whose products are on the fp32 matrix instructions; in the others the tiled kernel's and the prefill attention's
 # are split products (their launches in the few-tiles and the general form, fp32 too, are counted against that higher peak)
 FP32_MFMA_FAMILIES = {"conv2d_winograd_f32", "inverted_residual_f32", "stem_block_f32", "dwconv_pointwise_f32", "conv1x1_chain_f32",
-                      "dense_rows_f32", "mha_decode_f32", "mha_decode_proj_f32", "einsum_dense_f32"}
+                      "dense_rows_f32", "mha_decode_f32", "mha_decode_proj_f32", "einsum_dense_f32", "sample_net_f32"}
 
 
 def family_peak(family):

@@ -156,3 +156,34 @@ def test_models_without_a_program_keep_their_launches(fdx, modelgen):
             assert fdx.lib.fdx_debug_sample_net(model._h) == 0, f.__name__
     finally:
         fdx.lib.fdx_debug_force_sample_net(-1)
+
+
+@pytest.mark.parametrize("cin,cout,k,h", [(3, 16, 3, 16), (16, 16, 3, 12), (32, 32, 3, 8), (64, 56, 3, 5), (16, 16, 7, 8), (64, 32, 1, 8), (3, 8, 11, 16), (7, 33, 3, 8)])
+def test_sums_as_close_to_64_bits_as_the_launches(fdx, modelgen, cin, cout, k, h):
+    """A convolution's sums: sixteen products in a chain, such chunks by fours (one by one where channels are no multiple of four), then
+    those.  A rounding is off by 2^-24 / sqrt(3) of the value at most in the root mean square; over a chain of n additions, whose sums grow
+    like a square root, n / 2 of the last value's squared add up.  So 2^-24 / sqrt(3) sqrt(16 / 2 + 4 / 2 + chunks / 8 + 1), the one the bias;
+    and no further off than a launch per layer."""
+    b = modelgen.Builder("sums", 3)
+    spec = b.finish([b.conv2d(b.input((h, h, cin), "in"), cout, k, "a", padding="same", bias_std=0.1)])
+    p = spec["trainable_params"]["a"]
+    w = np.asarray(p["weights"], np.float64).reshape(cout, k, k, cin)
+    js = modelgen.dumps(spec)
+    r = np.random.default_rng(21)
+    for x in (r.standard_normal((64, h, h, cin)).astype(np.float32), r.uniform(0, 1, (64, h, h, cin)).astype(np.float32)):
+        framed = np.pad(x.astype(np.float64), ((0, 0), (k // 2, k // 2), (k // 2, k // 2), (0, 0)))
+        want = sum(framed[:, y:y + h, z:z + h] @ w[:, y, z].T for y in range(k) for z in range(k)) + p["bias"]
+        err = {}
+        for mode in (0, 1):
+            fdx.lib.fdx_debug_force_sample_net(mode)
+            try:
+                model = fdx.Model(js, verify=False)
+                got = model.predict([x])[0]
+                assert fdx.lib.fdx_debug_sample_net(model._h) == mode
+            finally:
+                fdx.lib.fdx_debug_force_sample_net(-1)
+            err[mode] = np.linalg.norm(got - want) / np.linalg.norm(want)
+        chunks = -(-k * k * cin // 16)
+        bound = 2.0 ** -24 / 3 ** 0.5 * np.sqrt(8 + (2 + chunks / 8 if cin % 4 == 0 else chunks / 2) + 1)
+        print("sums", cin, cout, k, err, bound, flush=True)
+        assert err[1] <= bound and err[1] <= err[0]

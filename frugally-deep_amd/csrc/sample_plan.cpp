@@ -8,6 +8,8 @@
 
 namespace fdx {
 
+static bool g_fail_sample_memory = false; // test hook
+
 namespace {
 
     // a tensor in LDS: h x w pixels of c channels inside a frame of zeros
@@ -428,12 +430,18 @@ std::shared_ptr<SampleProgram> sample_net_build(const fdx_model& m, const std::v
     const size_t step_at = (image.size() + 15) / 16 * 16, step_floats = steps.size() * sizeof(SampleStep) / 4;
     image.resize(step_at + step_floats);
     std::memcpy(&image[step_at], steps.data(), step_floats * 4);
-    if (hipMalloc(reinterpret_cast<void**>(&p->image), image.size() * 4) != hipSuccess)
+    // (the model then runs as launches, whose checks must not find this call's error)
+    if (hipMalloc(reinterpret_cast<void**>(&p->image), g_fail_sample_memory ? (size_t)1 << 60 : image.size() * 4) != hipSuccess) {
+        (void)hipGetLastError();
+        p->image = nullptr;
         return nullptr;
+    }
     p->program = reinterpret_cast<const SampleStep*>(p->image + step_at);
     if (hipMemcpyAsync(p->image, image.data(), image.size() * 4, hipMemcpyHostToDevice, stream()) != hipSuccess
-        || hipStreamSynchronize(stream()) != hipSuccess)
+        || hipStreamSynchronize(stream()) != hipSuccess) {
+        (void)hipGetLastError();
         return nullptr;
+    }
     return p;
 }
 
@@ -463,3 +471,9 @@ bool sample_net_by_rule(const SampleProgram& p, const fdx_model& m, const std::v
 }
 
 } // namespace fdx
+
+extern "C" fdx_status fdx_debug_fail_sample_memory(int on)
+{
+    fdx::g_fail_sample_memory = on != 0;
+    return FDX_OK;
+}

@@ -187,3 +187,18 @@ def test_sums_as_close_to_64_bits_as_the_launches(fdx, modelgen, cin, cout, k, h
         bound = 2.0 ** -24 / 3 ** 0.5 * np.sqrt(8 + (2 + chunks / 8 if cin % 4 == 0 else chunks / 2) + 1)
         print("sums", cin, cout, k, err, bound, flush=True)
         assert err[1] <= bound and err[1] <= err[0]
+
+
+def test_refused_memory_leaves_the_launches(fdx, modelgen):
+    js = modelgen.dumps(modelgen.small_cnn())
+    x = np.random.default_rng(8).uniform(-1, 1, (3, 32, 32, 3)).astype(np.float32)
+    want = fdx.Model(js, verify=False).predict([x])[0]
+    fdx.lib.fdx_debug_fail_sample_memory(1)
+    try:
+        model = fdx.Model(js, verify=False)
+        got = model.predict([x])[0]
+        assert fdx.lib.fdx_debug_sample_net(model._h) == 0
+        fdx.sync()
+    finally:
+        fdx.lib.fdx_debug_fail_sample_memory(0)
+    assert rel(got, want) <= TOL

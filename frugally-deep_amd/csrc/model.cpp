@@ -2051,16 +2051,20 @@ fdx_status get_plan(fdx_model* m, int batch, const std::vector<Shape>& in_shapes
         }
     // The whole model as one launch: where it is small enough and no form of its operations is asked for.
     const bool forced = tile_forced() || g_force_winograd >= 0 || g_force_dw_fusion >= 0;
-    if (g_force_sample_net != 0 && (g_force_sample_net == 1 || !forced)) {
-        for (auto& other : m->plans)
-            if (other->sample && other->in_shapes == in_shapes)
-                p->sample = other->sample;
-        if (!p->sample && std::any_of(m->ops.begin(), m->ops.end(), [](const Op& o) { return !o.sample_w.empty(); }))
-            p->sample = sample_net_build(*m, p->order, p->shapes);
-        if (p->sample && g_force_sample_net < 0 && !sample_net_by_rule(*p->sample, *m, p->order, p->shapes, batch))
-            p->sample = nullptr;
-        if (p->sample)
+    if (g_force_sample_net != 0 && (g_force_sample_net == 1 || !forced)
+        && std::any_of(m->ops.begin(), m->ops.end(), [](const Op& o) { return !o.sample_w.empty(); })) {
+        auto& made = m->sample_programs;
+        auto at = std::find_if(made.begin(), made.end(), [&](const auto& e) { return e.first == in_shapes; });
+        if (at == made.end()) {
+            if (made.size() >= fdx_model::kMaxPlans)
+                made.pop_back(); // (a plan that runs it keeps it)
+            at = made.emplace(made.begin(), in_shapes, sample_net_build(*m, p->order, p->shapes));
+        }
+        const std::shared_ptr<SampleProgram>& program = at->second;
+        if (program && (g_force_sample_net == 1 || sample_net_by_rule(*program, *m, p->order, p->shapes, batch)) && sample_net_load(*program)) {
+            p->sample = program;
             p->sample->flops = p->flops / batch;
+        }
     }
     m->plans.insert(m->plans.begin(), std::move(p));
     *out = m->plans[0].get();

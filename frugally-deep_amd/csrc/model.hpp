@@ -140,6 +140,8 @@ struct fdx_model {
     // (variable input dimensions, tensor_shape_variable.hpp) keeps up to kMaxPlans of them instead of re-planning
     static constexpr size_t kMaxPlans = 4;
     std::vector<std::unique_ptr<fdx::Plan>> plans;
+    // one-launch programs of the last few input shapes, null where there is none (whatever the batch), most recently made first
+    std::vector<std::pair<std::vector<fdx::Shape>, std::shared_ptr<fdx::SampleProgram>>> sample_programs;
     std::mutex mu;
     double last_flops = 0;
     ~fdx_model();
@@ -151,6 +153,7 @@ fdx_status get_plan(fdx_model* m, int batch, const std::vector<Shape>& in_shapes
 float* plan_alloc(Plan& p, size_t bytes, int* block_index);
 bool sample_net_keeps_weights(const fdx_model& m);
 std::shared_ptr<SampleProgram> sample_net_build(const fdx_model& m, const std::vector<int>& order, const std::vector<Shape>& shapes);
+bool sample_net_load(SampleProgram& p);
 bool sample_net_by_rule(const SampleProgram& p, const fdx_model& m, const std::vector<int>& order, const std::vector<Shape>& shapes, int batch);
 fdx_status sample_net_launch(const SampleProgram& p, const float* in, int batch, float* out);
 int irb_block_waves(int cin, int ce, int n_out, int stride); // irb.hip

@@ -33,12 +33,14 @@ constexpr SampleForm kSampleForms[] = { { false, 1, 1 }, { false, 4, 1 }, { true
 constexpr int kSampleLdsFloats = 40960; // a CU's LDS
 constexpr int kSampleThreads = 1024, kSampleInput = kSampleThreads * 16; // most floats of an input
 
-// A program for one input shape, in device memory: offset tables and weights as they lie in LDS, then the steps.
+// A program for one input shape: offset tables and weights as they lie in LDS, then the steps; in host memory until a plan runs it.
 struct SampleProgram {
+    std::vector<float> host;
+    size_t step_at = 0; // floats in front of the steps
     float* image = nullptr;
     const SampleStep* program = nullptr;
     int image_floats = 0, lds_floats = 0, steps = 0, in_volume = 0, out_volume = 0;
-    double us_per_sample = 0, launches_us = 0, flops = 0; // predicted: one sample on a CU; the layers' own launches, without their arithmetic
+    double us_per_sample = 0, flops = 0; // predicted: one sample on a CU
     ~SampleProgram();
 };
 

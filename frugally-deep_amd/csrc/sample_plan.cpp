@@ -8,7 +8,8 @@
 
 namespace fdx {
 
-static bool g_fail_sample_memory = false; // test hook
+static bool g_fail_sample_memory = false; // test hooks
+static int g_sample_loads = 0;
 
 namespace {
 
@@ -74,7 +75,7 @@ bool sample_net_keeps_weights(const fdx_model& m)
     return floats > 0 && floats <= (size_t)kSampleLdsFloats;
 }
 
-// The program for these shapes, or none where an operation, a layout or the size of LDS speaks against it.
+// The program for these shapes, in host memory, or none where an operation, a layout or the size of LDS speaks against it.
 std::shared_ptr<SampleProgram> sample_net_build(const fdx_model& m, const std::vector<int>& order, const std::vector<Shape>& shapes)
 {
     std::vector<Tensor> tensors;
@@ -427,22 +428,36 @@ std::shared_ptr<SampleProgram> sample_net_build(const fdx_model& m, const std::v
     p->in_volume = p_in_volume;
     p->out_volume = (int)volume(shapes[(size_t)m.outputs[0]]);
     p->us_per_sample = (cycles + 0.4 * p->out_volume) / 2400.0; // (a result's way out: four floats a cycle at most, 256 CUs at once)
-    const size_t step_at = (image.size() + 15) / 16 * 16, step_floats = steps.size() * sizeof(SampleStep) / 4;
-    image.resize(step_at + step_floats);
-    std::memcpy(&image[step_at], steps.data(), step_floats * 4);
-    // (the model then runs as launches, whose checks must not find this call's error)
-    if (hipMalloc(reinterpret_cast<void**>(&p->image), g_fail_sample_memory ? (size_t)1 << 60 : image.size() * 4) != hipSuccess) {
-        (void)hipGetLastError();
-        p->image = nullptr;
-        return nullptr;
-    }
-    p->program = reinterpret_cast<const SampleStep*>(p->image + step_at);
-    if (hipMemcpyAsync(p->image, image.data(), image.size() * 4, hipMemcpyHostToDevice, stream()) != hipSuccess
-        || hipStreamSynchronize(stream()) != hipSuccess) {
-        (void)hipGetLastError();
-        return nullptr;
-    }
+    const size_t step_floats = steps.size() * sizeof(SampleStep) / 4;
+    p->step_at = (image.size() + 15) / 16 * 16;
+    image.resize(p->step_at + step_floats);
+    std::memcpy(&image[p->step_at], steps.data(), step_floats * 4);
+    p->host = std::move(image);
     return p;
+}
+
+// The program into device memory, at the first plan that runs it; false where the memory is refused.
+bool sample_net_load(SampleProgram& p)
+{
+    if (p.image)
+        return true;
+    ++g_sample_loads;
+    float* d = nullptr;
+    const size_t bytes = p.host.size() * sizeof(float);
+    // (the model then runs as launches, whose checks must not find this call's error)
+    if (hipMalloc(reinterpret_cast<void**>(&d), g_fail_sample_memory ? (size_t)1 << 60 : bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    if (hipMemcpyAsync(d, p.host.data(), bytes, hipMemcpyHostToDevice, stream()) != hipSuccess || hipStreamSynchronize(stream()) != hipSuccess) {
+        (void)hipGetLastError();
+        (void)hipFree(d);
+        return false;
+    }
+    p.image = d;
+    p.program = reinterpret_cast<const SampleStep*>(d + p.step_at);
+    p.host = std::vector<float>();
+    return true;
 }
 
 // One launch or one per operation, by predicted times: a launch costs what the chain's shortest take (3.7 us), or its traffic and its
@@ -477,3 +492,4 @@ extern "C" fdx_status fdx_debug_fail_sample_memory(int on)
     fdx::g_fail_sample_memory = on != 0;
     return FDX_OK;
 }
+extern "C" int fdx_debug_sample_loads(void) { return fdx::g_sample_loads; }

@@ -87,6 +87,8 @@ fdx_status fdx_debug_force_winograd(int mode);
 fdx_status fdx_debug_force_sample_net(int mode);
 /* 1 = the device memory of such a launch's program is refused: more is asked for than there is (0 = the default) */
 fdx_status fdx_debug_fail_sample_memory(int on);
+/* programs that went to device memory, or were refused it, since the library was loaded */
+int fdx_debug_sample_loads(void);
 /* 1 = the model's last call ran as one launch */
 int fdx_debug_sample_net(const fdx_model* model);
 /* which kernel the rule takes for a 3x3 stride-1 "same" convolution [n][h][w][cin] -> cout: 0 = direct, 1 = Winograd (host only) */

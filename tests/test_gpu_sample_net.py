@@ -202,3 +202,23 @@ def test_refused_memory_leaves_the_launches(fdx, modelgen):
     finally:
         fdx.lib.fdx_debug_fail_sample_memory(0)
     assert rel(got, want) <= TOL
+
+
+def test_a_program_goes_to_the_device_once_and_only_where_it_runs(fdx, modelgen):
+    # three Dense layers of 128: the rule leaves batches beyond a few hundred to the launches
+    b = modelgen.Builder("dense", 3)
+    x = b.input((128,), "in")
+    for i in range(2):
+        x = b.dense(x, 128, "d%d" % i, activation="relu")
+    model = fdx.Model(modelgen.dumps(b.finish([x])), verify=False)
+    a = np.random.default_rng(4).standard_normal((2100, 128)).astype(np.float32)
+    loads = fdx.lib.fdx_debug_sample_loads
+    before = loads()
+    for n in (2100, 2000, 1900, 1800, 1700, 1600):   # more batches than a model keeps plans
+        model.predict([a[:n]])
+        assert fdx.lib.fdx_debug_sample_net(model._h) == 0 and loads() == before, n
+    want = model.predict([a[:1500]])[0]
+    for n in (1, 2, 3, 4, 5, 6, 1):
+        got = model.predict([a[:n]])[0]
+        assert fdx.lib.fdx_debug_sample_net(model._h) == 1 and loads() == before + 1, n
+        assert rel(got, want[:n]) <= TOL

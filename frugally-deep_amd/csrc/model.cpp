@@ -1837,7 +1837,7 @@ extern "C" fdx_status fdx_debug_force_sample_net(int mode)
 }
 extern "C" int fdx_debug_sample_net(const fdx_model* m)
 {
-    return m && !m->plans.empty() && m->plans[0]->sample ? 1 : 0;
+    return m && m->last_one_launch ? 1 : 0;
 }
 
 fdx_status get_plan(fdx_model* m, int batch, const std::vector<Shape>& in_shapes, Plan** out)
@@ -3235,6 +3235,7 @@ namespace {
                     }
             }
         }
+        m->last_one_launch = one_launch;
         if (one_launch) {
             st = sample_net_launch(*p->sample, p->out[m->inputs[0]], batch, p->out[m->outputs[0]]);
             m->last_flops = p->flops;

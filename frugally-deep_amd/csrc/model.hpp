@@ -144,6 +144,7 @@ struct fdx_model {
     std::vector<std::pair<std::vector<fdx::Shape>, std::shared_ptr<fdx::SampleProgram>>> sample_programs;
     std::mutex mu;
     double last_flops = 0;
+    bool last_one_launch = false; // how the last call ran (test hook)
     ~fdx_model();
 };
 
@@ -155,6 +156,7 @@ bool sample_net_keeps_weights(const fdx_model& m);
 std::shared_ptr<SampleProgram> sample_net_build(const fdx_model& m, const std::vector<int>& order, const std::vector<Shape>& shapes);
 bool sample_net_load(SampleProgram& p);
 bool sample_net_by_rule(const SampleProgram& p, const fdx_model& m, const std::vector<int>& order, const std::vector<Shape>& shapes, int batch);
+int sample_net_cus(); // workgroups that run side by side
 fdx_status sample_net_launch(const SampleProgram& p, const float* in, int batch, float* out);
 int irb_block_waves(int cin, int ce, int n_out, int stride); // irb.hip
 bool tile_forced(); // fdx_debug_force_tile names a configuration

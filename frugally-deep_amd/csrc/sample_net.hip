@@ -592,6 +592,17 @@ SampleProgram::~SampleProgram()
         (void)hipFree(image);
 }
 
+int sample_net_cus()
+{
+    static const int cus = [] {
+        int dev = 0, n = 256;
+        (void)hipGetDevice(&dev);
+        (void)hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev);
+        return n;
+    }();
+    return cus;
+}
+
 fdx_status sample_net_launch(const SampleProgram& p, const float* in, int batch, float* out)
 {
     FDX_REQUIRE(in && out && batch > 0 && p.image && p.in_volume <= kSampleInput && p.lds_floats <= kSampleLdsFloats
@@ -599,12 +610,7 @@ fdx_status sample_net_launch(const SampleProgram& p, const float* in, int batch,
     static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(sample_net_kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
         kSampleLdsFloats * 4);
     FDX_HIP(attr);
-    static const int cus = [] {
-        int dev = 0, n = 256;
-        (void)hipGetDevice(&dev);
-        (void)hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev);
-        return n;
-    }();
+    const int cus = sample_net_cus();
     profile_begin();
     hipLaunchKernelGGL(sample_net_kernel, dim3((unsigned)(batch < cus ? batch : cus)), dim3(kSampleThreads), (size_t)p.lds_floats * 4, stream(),
         in, out, reinterpret_cast<const f32x4*>(p.image), p.image_floats / 4, p.program, p.steps, p.in_volume, p.out_volume, batch);

@@ -482,7 +482,7 @@ bool sample_net_by_rule(const SampleProgram& p, const fdx_model& m, const std::v
         }
         launches += std::max(3.7, us) + (o.softmax ? 3.0 : 0.0);
     }
-    return 3.0 + std::ceil(batch / 256.0) * p.us_per_sample < launches;
+    return 3.0 + std::ceil((double)batch / sample_net_cus()) * p.us_per_sample < launches;
 }
 
 } // namespace fdx

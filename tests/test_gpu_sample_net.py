@@ -222,3 +222,20 @@ def test_a_program_goes_to_the_device_once_and_only_where_it_runs(fdx, modelgen)
         got = model.predict([a[:n]])[0]
         assert fdx.lib.fdx_debug_sample_net(model._h) == 1 and loads() == before + 1, n
         assert rel(got, want[:n]) <= TOL
+
+
+def test_the_hook_tells_how_the_last_call_ran(fdx, modelgen):
+    # a plan made for one launch, and a configuration of the layers' kernels forced behind it
+    model = fdx.Model(modelgen.dumps(modelgen.small_cnn()), verify=False)
+    x = np.random.default_rng(9).uniform(-1, 1, (5, 32, 32, 3)).astype(np.float32)
+    want = model.predict([x])[0]
+    assert fdx.lib.fdx_debug_sample_net(model._h) == 1
+    fdx.check(fdx.lib.fdx_debug_force_tile(0))
+    try:
+        got = model.predict([x])[0]
+        assert fdx.lib.fdx_debug_sample_net(model._h) == 0
+    finally:
+        fdx.check(fdx.lib.fdx_debug_force_tile(-1))
+    assert rel(got, want) <= TOL
+    model.predict([x])
+    assert fdx.lib.fdx_debug_sample_net(model._h) == 1

@@ -3072,10 +3072,10 @@ namespace {
 
     // One host input per model input, each either one contiguous block of `batch` samples or `batch` pointers to single
     // samples; copies them to the plan's input buffers and, where the network starts with a convolution of its own
-    // launch, runs the first ops of the plan piece by piece behind the copy.  *done_until receives the number of leading
-    // positions of the plan's order that have been executed that way.
+    // launch, runs the first ops of the plan piece by piece behind the copy (a small model that is one launch: all of
+    // them).  *done_until receives the number of leading positions of the plan's order that have been executed that way.
     fdx_status stage_host_inputs(fdx_model* m, Plan* p, int batch, const float* const* in, bool per_sample, const std::vector<Shape>& shapes,
-        int* done_until)
+        bool one_launch, int* done_until)
     {
         *done_until = 0;
         size_t total = 0;
@@ -3096,7 +3096,7 @@ namespace {
         Stager& st = stager();
         std::lock_guard<std::mutex> lock(st.use);
         static const bool no_prefix = [] { const char* e = std::getenv("FDX_STAGE_PREFIX"); return e && e[0] == '0'; }();
-        const int cut = batch >= 8 && !no_prefix && !p->sample ? chunkable_prefix(*m, *p, batch) : 0;
+        const int cut = batch < 8 || no_prefix ? 0 : one_launch ? (int)p->order.size() : chunkable_prefix(*m, *p, batch);
         static const bool stage_log = [] { const char* e = std::getenv("FDX_STAGE_LOG"); return e && e[0] == '1'; }();
         if (stage_log)
             std::fprintf(stderr, "[fdx stage] %zu bytes, prefix of %d ops (plan has %zu)\n", total, cut, p->order.size());
@@ -3108,6 +3108,13 @@ namespace {
             int per_piece = std::max(1, (batch + 3) / 4);
             while (per_piece > 1 && sample * (size_t)per_piece > ((size_t)16 << 20))
                 per_piece = (per_piece + 1) / 2;
+            if (one_launch && cut > 0) {
+                // Whole rounds of workgroups, and pieces that begin 16-byte aligned whatever a sample's size.  Us a call of 2048 / 16384 samples, the
+                // layers' launches, one launch behind the whole copy, pieces: small CNN 784 / 5101, 763 / 5172, 674 / 4321; four 3x3
+                // convolutions of 16 channels on 16 x 16 1048 / 7124, 949 / 6587, 830 / 5476.
+                const int round = sample_net_cus();
+                per_piece = per_piece > round ? per_piece / round * round : (per_piece + 3) / 4 * 4;
+            }
             fdx_status fs = st.prepare(sample * (size_t)per_piece);
             if (fs != FDX_OK)
                 return fs;
@@ -3134,6 +3141,13 @@ namespace {
                     const int run_from = run_done;
                     const int run_count = s0 + count - run_done;
                     run_done = s0 + count;
+                    if (one_launch) {
+                        const fdx_status rs = sample_net_launch(*p->sample, p->out[(size_t)m->inputs[0]] + (size_t)run_from * (size_t)volume(shapes[0]), run_count,
+                            p->out[(size_t)m->outputs[0]] + (size_t)run_from * (size_t)p->sample->out_volume);
+                        if (rs != FDX_OK)
+                            return rs;
+                        continue;
+                    }
                     std::vector<std::pair<int, float*>> saved;
                     for (int q = 0; q < cut; ++q) {
                         const int k = p->order[(size_t)q];
@@ -3183,10 +3197,11 @@ namespace {
             }
         } restore{ p, {} };
         int done_until = 0;
+        const bool one_launch = p->sample && (g_force_sample_net == 1 || !tile_forced());
         if (!in_on_device) {
             for (size_t i = 0; i < m->inputs.size() * (per_sample ? (size_t)batch : 1); ++i)
                 FDX_REQUIRE(in[i], "predict: null input %zu", i);
-            if ((st = stage_host_inputs(m, p, batch, in, per_sample, shapes, &done_until)) != FDX_OK)
+            if ((st = stage_host_inputs(m, p, batch, in, per_sample, shapes, one_launch, &done_until)) != FDX_OK)
                 return st;
         } else
             for (size_t i = 0; i < m->inputs.size(); ++i) {
@@ -3207,7 +3222,6 @@ namespace {
         // the inputs or other results (saves the copy's launch: 2 us of a pass): the output op and its views point there for
         // this call.
         std::vector<char> direct(m->outputs.size(), 0);
-        const bool one_launch = p->sample && (g_force_sample_net == 1 || !tile_forced());
         if (out_on_device) {
             auto root = [&](int i) {
                 while (m->ops[(size_t)i].kind == OpKind::View)
@@ -3237,7 +3251,8 @@ namespace {
         }
         m->last_one_launch = one_launch;
         if (one_launch) {
-            st = sample_net_launch(*p->sample, p->out[m->inputs[0]], batch, p->out[m->outputs[0]]);
+            if (done_until == 0)
+                st = sample_net_launch(*p->sample, p->out[m->inputs[0]], batch, p->out[m->outputs[0]]);
             m->last_flops = p->flops;
         } else
             st = execute(*m, *p, done_until);

@@ -239,3 +239,30 @@ def test_the_hook_tells_how_the_last_call_ran(fdx, modelgen):
     assert rel(got, want) <= TOL
     model.predict([x])
     assert fdx.lib.fdx_debug_sample_net(model._h) == 1
+
+
+@pytest.mark.parametrize("net,shape,batch", [("small_cnn", (32, 32, 3), 401), ("small_cnn", (32, 32, 3), 1030), ("odd_input", (61, 47, 5), 77), ("odd_input", (61, 47, 5), 1111)])
+def test_host_arrays_in_pieces(fdx, modelgen, net, shape, batch):
+    """From 4 MB on host arrays arrive in pieces, and each piece runs behind its copy: the bits of the whole batch in device memory.  Pieces below
+    and above a round of workgroups, a last piece of its own size, samples that are no multiple of 16 bytes, more than 16 MB a quarter."""
+    if net == "small_cnn":
+        js = modelgen.dumps(modelgen.small_cnn())
+    else:
+        b = modelgen.Builder(net, 11)
+        js = modelgen.dumps(b.finish([NETS[net](b)]))
+    x = np.random.default_rng(batch).uniform(-1, 1, (batch,) + shape).astype(np.float32)
+    assert x.nbytes >= 4 << 20
+    fdx.lib.fdx_debug_force_sample_net(1)
+    try:
+        model = fdx.Model(js, verify=False)
+        n = int(np.prod(model.output_shapes[0]))
+        got = [model.predict([x])[0], model.predict_samples([[a] for a in x])[0]]
+        assert fdx.lib.fdx_debug_sample_net(model._h) == 1
+        d, out = fdx.DevBuf.from_host(x), fdx.DevBuf(4 * batch * n)
+        model.predict_dev(batch, [d], [shape], [out])
+        fdx.sync()
+        want = out.to_host((batch, n))
+    finally:
+        fdx.lib.fdx_debug_force_sample_net(-1)
+    for g in got:
+        assert np.array_equal(np.asarray(g).reshape(batch, n), want)

@@ -210,15 +210,17 @@ def test_attention_with_output_projection_in_one_launch(fdx, oracle, modelgen, m
         assert rel(lb[0], want) <= TOL
 
 
-def test_embedding_folded_into_its_readers_gives_the_same_tokens(fdx, modelgen):
+@pytest.mark.parametrize("B", [16, 7, 6, 5, 1])
+def test_embedding_folded_into_its_readers_gives_the_same_tokens(fdx, modelgen, B):
     """The opt-in form of the decode step in which the first projection GEMM and the first residual operand form the
-    token + position rows themselves (one launch fewer): same sums in the same order, so logits and tokens are
-    bit-identical to the default step."""
-    print("decode step with the embedding folded into its readers", flush=True)
+    token + position rows themselves (one launch fewer).  From seven sequences on same sums in the same order, so logits and tokens are
+    bit-identical to the default step; up to six the default step's two projections add up in an order of their own, and logits
+    agree to the rounding errors of two layers' sums (so do the tokens, unless two logits are that close)."""
+    print("decode step with the embedding folded into its readers", B, flush=True)
     js = modelgen.dumps(modelgen.gpt2(seed=61, layers=2, d_model=768, heads=12, vocab=50257, max_pos=128, bias_std=0.1,
                                       random_affine=True))
     model = fdx.Model(js, verify=False)
-    B, P, N = 16, 24, 12
+    P, N = 24, 12
     prompts = np.random.default_rng(62).integers(0, 50257, (B, P))
     outs = []
     for mode in (0, 1):
@@ -233,7 +235,10 @@ def test_embedding_folded_into_its_readers_gives_the_same_tokens(fdx, modelgen):
         outs.append((tokens, logits, step_logits, step_next))
         sess.close()
     for a, b in zip(outs[0], outs[1]):
-        assert np.array_equal(a, b)
+        if B > 6:
+            assert np.array_equal(a, b)
+        else:
+            assert a.shape == b.shape and rel(a, b) <= 1e-5
 
 
 def test_greedy_loop_with_the_embedding_in_the_previous_steps_last_launch(fdx, modelgen):

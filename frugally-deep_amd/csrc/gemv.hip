@@ -85,20 +85,20 @@ __device__ __forceinline__ float gemv_sums(const f32x4 (&wa)[C][KQ], int lane, R
     return v;
 }
 
-// K up to 256 KQ: eight waves of C columns each over the whole of K.  The first M waves bring a row each, centred and with its
+// K up to 256 KQ: eight waves of a column each over the whole of K.  The first M waves bring a row each, centred and with its
 // 1 / deviation where it is normalised, into LDS while all waves' weights are on their way: read by every wave for itself
 // the rows took the path from L2 longer than the weights did.
 constexpr int kGemvWaves = 8;
-template <int M, int KQ, int C, bool LN>
+template <int M, int KQ, bool LN>
 __global__ __launch_bounds__(64 * kGemvWaves) void gemv_kernel(const float* x, const float* w, const float* bias, const float* residual, int m, int n,
     int k, int ldx, int ldr, GemvTail tail)
 {
     __shared__ f32x4 rows[M][KQ * 64];
     __shared__ float row_rstd[M];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int n0 = ((int)blockIdx.x * kGemvWaves + wave) * C;
+    const int n0 = (int)blockIdx.x * kGemvWaves + wave;
     const f32x4 zero = { 0.f, 0.f, 0.f, 0.f };
-    f32x4 xa[KQ], wa[C][KQ];
+    f32x4 xa[KQ], wa[1][KQ];
 #pragma unroll
     for (int q = 0; q < KQ; ++q) {
         xa[q] = zero;
@@ -106,14 +106,12 @@ __global__ __launch_bounds__(64 * kGemvWaves) void gemv_kernel(const float* x, c
             xa[q] = *reinterpret_cast<gptr<const f32x4>>(as_global(x) + (int64_t)wave * ldx + (q * 64 + lane) * 4);
     }
 #pragma unroll
-    for (int c = 0; c < C; ++c)
-#pragma unroll
-        for (int q = 0; q < KQ; ++q) {
-            wa[c][q] = zero;
-            if (n0 + c < n && (q * 64 + lane) * 4 < k) // every weight is used once per launch
-                wa[c][q] = __builtin_nontemporal_load(reinterpret_cast<gptr<const f32x4>>(as_global(w) + (int64_t)(n0 + c) * k + (q * 64 + lane) * 4));
-        }
-    const GemvOutput o = gemv_output<M, C>(bias, residual, m, n, ldr, tail, n0, lane);
+    for (int q = 0; q < KQ; ++q) {
+        wa[0][q] = zero;
+        if (n0 < n && (q * 64 + lane) * 4 < k) // every weight is used once per launch
+            wa[0][q] = __builtin_nontemporal_load(reinterpret_cast<gptr<const f32x4>>(as_global(w) + (int64_t)n0 * k + (q * 64 + lane) * 4));
+    }
+    const GemvOutput o = gemv_output<M, 1>(bias, residual, m, n, ldr, tail, n0, lane);
     if (wave < M) {
         if (LN) {
             float s = 0.f;
@@ -140,10 +138,10 @@ __global__ __launch_bounds__(64 * kGemvWaves) void gemv_kernel(const float* x, c
             rows[wave][q * 64 + lane] = xa[q];
     }
     __syncthreads();
-    float v = gemv_sums<M, KQ, C>(wa, lane, [&](int r, int q) { return rows[r][q * 64 + lane]; });
+    float v = gemv_sums<M, KQ, 1>(wa, lane, [&](int r, int q) { return rows[r][q * 64 + lane]; });
     if (o.ok) {
         if (LN)
-            v *= row_rstd[lane / C];
+            v *= row_rstd[lane];
         *as_global(o.dst) = apply_act(v + o.add, tail.act);
     }
 }
@@ -194,37 +192,30 @@ bool gemv_covers(int m, int n, int k, int64_t ldx, int64_t ldw, int64_t ldr, boo
     return m > 0 && m <= kGemvRows && n > 0 && k > 0 && k % 4 == 0 && k <= (ln ? 1024 : kGemvK) && ldw == k && ldx < (1LL << 31) && ldr < (1LL << 31);
 }
 
-// Not where the wide-output kernel strides over thousands of columns, nor with the embedding prologue.  A step of the same decoder, us, tile
-// kernels / here: 1 row 322 / 248, 2 331 / 270, 3 337 / 297, 4 345 / 301, 6 350 / 327, 7 351 / 350, 8 353 / 359.
+// Not where the wide-output kernel strides over thousands of columns, nor with the embedding prologue.  A step of 12 layers of 768, us, tile
+// kernels / here: 1 row 322 / 248, 2 331 / 270, 3 337 / 297, 4 345 / 301, 6 350 / 327, 7 351 / 350, 8 353 / 359.  Of 6 layers, 1 and 6 rows: width 64
+// 138 / 101 and 140 / 119, 128 140 / 103 and 144 / 122, 256 150 / 109 and 155 / 133, 512 160 / 119 and 166 / 145, 1024 208 / 162 and 219 /
+// 217.  Single launches on weights row by row, K 16 to 4096 x N 64 to 12288 x 1 to 6 rows: 0.39 to 0.96 of the tile kernels' time in 575 of
+// 576 (32 x 12288 with six rows 1.01); also where few lanes hold any of K: 16 x 64, one row 2.3 / 4.3, six 2.8 / 3.8, 64 x 4096, six 3.5 / 4.5.
 bool gemv_by_rule(const SkinnyParams& p)
 {
-    return p.M <= kGemvRows && !p.emb_x && !p.emb_res && !p.amax_parts && skinny_wide_grid(p) == 0 && gemv_covers(p.M, p.N, p.K, p.ldx, p.ldw, p.ldr, p.ln != 0);
-}
-
-template <int M, int KQ, int C>
-static void gemv_start(const SkinnyParams& p, const GemvTail& tail)
-{
-    const int groups = (p.N + C - 1) / C;
-    if (p.K > 1024)
-        hipLaunchKernelGGL((gemv_split_kernel<M, KQ, C>), dim3((unsigned)groups), dim3(256), 0, stream(), p.X, p.W, p.bias, p.residual, p.M, p.N, p.K,
-            (int)p.ldx, (int)p.ldr, tail);
-    else if (p.ln)
-        hipLaunchKernelGGL((gemv_kernel<M, KQ, C, true>), dim3((unsigned)((groups + kGemvWaves - 1) / kGemvWaves)), dim3(64 * kGemvWaves), 0, stream(), p.X,
-            p.W, p.bias, p.residual, p.M, p.N, p.K, (int)p.ldx, (int)p.ldr, tail);
-    else
-        hipLaunchKernelGGL((gemv_kernel<M, KQ, C, false>), dim3((unsigned)((groups + kGemvWaves - 1) / kGemvWaves)), dim3(64 * kGemvWaves), 0, stream(), p.X,
-            p.W, p.bias, p.residual, p.M, p.N, p.K, (int)p.ldx, (int)p.ldr, tail);
+    return p.M <= kGemvRows && !p.emb_x && !p.emb_res && !p.amax_parts && gemv_covers(p.M, p.N, p.K, p.ldx, p.ldw, p.ldr, p.ln != 0) && skinny_wide_grid(p) == 0;
 }
 
 template <int M, int KQ>
-static void gemv_rows(const SkinnyParams& p, const GemvTail& tail)
+static void gemv_start(const SkinnyParams& p, const GemvTail& tail)
 {
-    // One column a wave; along a cut K three from three rows on, whose reading they share (a step of 12 layers of 768 with 1 / 2 / 3 columns,
-    // us: one row 248 / 252 / 252, four rows 302 / 303 / 299, six 332 / 332 / 327; two columns a wave everywhere 274, 330, 357).
-    if (M > 2 && p.K > 1024)
-        gemv_start<M, KQ, 3>(p, tail);
+    const dim3 grid((unsigned)((p.N + kGemvWaves - 1) / kGemvWaves)), block(64 * kGemvWaves);
+    if (p.K > 1024) {
+        // A column a workgroup; three from three rows on, which then share the reading of the rows (a step of 12 layers of 768 with 1 / 2 / 3
+        // columns, us: one row 248 / 252 / 252, four rows 302 / 303 / 299, six 332 / 332 / 327).
+        constexpr int C = M > 2 ? 3 : 1;
+        hipLaunchKernelGGL((gemv_split_kernel<M, KQ, C>), dim3((unsigned)((p.N + C - 1) / C)), dim3(256), 0, stream(), p.X, p.W, p.bias, p.residual, p.M,
+            p.N, p.K, (int)p.ldx, (int)p.ldr, tail);
+    } else if (p.ln) // (whole rows: a column a wave; with two everywhere that step took 274, 330 and 357 us)
+        hipLaunchKernelGGL((gemv_kernel<M, KQ, true>), grid, block, 0, stream(), p.X, p.W, p.bias, p.residual, p.M, p.N, p.K, (int)p.ldx, (int)p.ldr, tail);
     else
-        gemv_start<M, KQ, 1>(p, tail);
+        hipLaunchKernelGGL((gemv_kernel<M, KQ, false>), grid, block, 0, stream(), p.X, p.W, p.bias, p.residual, p.M, p.N, p.K, (int)p.ldx, (int)p.ldr, tail);
 }
 
 template <int M>
@@ -232,13 +223,13 @@ static void gemv_k(const SkinnyParams& p, const GemvTail& tail)
 {
     const int per = p.K > 1024 ? (p.K + 3) / 4 : p.K; // of K a wave
     if (per <= 256)
-        gemv_rows<M, 1>(p, tail);
+        gemv_start<M, 1>(p, tail);
     else if (per <= 512)
-        gemv_rows<M, 2>(p, tail);
+        gemv_start<M, 2>(p, tail);
     else if (per <= 768)
-        gemv_rows<M, 3>(p, tail);
+        gemv_start<M, 3>(p, tail);
     else
-        gemv_rows<M, 4>(p, tail);
+        gemv_start<M, 4>(p, tail);
 }
 
 // Launches the rows' kernel for parameters that gemv_covers accepts.
@@ -265,3 +256,10 @@ void gemv_launch(const SkinnyParams& p)
 }
 
 } // namespace fdx
+
+extern "C" int fdx_debug_dense_rows_form(int m, int n, int k, int layernorm)
+{
+    fdx::SkinnyParams p {};
+    p.M = m; p.N = n; p.K = k; p.ldx = p.ldw = k; p.ldr = n; p.ln = layernorm;
+    return fdx::gemv_by_rule(p) ? 1 : 0;
+}

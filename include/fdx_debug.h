@@ -91,6 +91,8 @@ fdx_status fdx_debug_fail_sample_memory(int on);
 int fdx_debug_sample_loads(void);
 /* 1 = the model's last call ran as one launch */
 int fdx_debug_sample_net(const fdx_model* model);
+/* which kernel fdx_dense_rows_f32 (layernorm = 1: fdx_layernorm_dense_rows_f32) takes: 1 = a wave per output column, 0 = the tile kernels */
+int fdx_debug_dense_rows_form(int m, int n, int k, int layernorm);
 /* which kernel the rule takes for a 3x3 stride-1 "same" convolution [n][h][w][cin] -> cout: 0 = direct, 1 = Winograd (host only) */
 int fdx_debug_conv3x3_form(int n, int h, int w, int cin, int cout);
 

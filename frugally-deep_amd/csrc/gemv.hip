@@ -187,9 +187,11 @@ __global__ __launch_bounds__(256) void gemv_split_kernel(const float* x, const f
 
 constexpr int kGemvRows = 6, kGemvK = 4096; // most rows and longest K
 
+// (a grid has fewer than 2^32 threads: 256 a column at most)
 bool gemv_covers(int m, int n, int k, int64_t ldx, int64_t ldw, int64_t ldr, bool ln)
 {
-    return m > 0 && m <= kGemvRows && n > 0 && k > 0 && k % 4 == 0 && k <= (ln ? 1024 : kGemvK) && ldw == k && ldx < (1LL << 31) && ldr < (1LL << 31);
+    return m > 0 && m <= kGemvRows && n > 0 && n < (1 << 24) && k > 0 && k % 4 == 0 && k <= (ln ? 1024 : kGemvK) && ldw == k && ldx < (1LL << 31)
+        && ldr < (1LL << 31);
 }
 
 // Not where the wide-output kernel strides over thousands of columns, nor with the embedding prologue.  A step of 12 layers of 768, us, tile

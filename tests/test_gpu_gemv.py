@@ -56,3 +56,9 @@ def test_non_finite_rows_stay_their_own(fdx, m, k):
     got = out.to_host((m, 40))
     assert np.isfinite(got[:m - 2]).all() and np.isinf(got[m - 2]).all() and np.isnan(got[m - 1]).all()
     assert (np.sign(got[m - 2]) == np.sign(w[:, 5])).all()
+
+
+def test_more_columns_than_a_grid_holds(fdx):
+    # 256 threads a column of a long row: 2^24 columns would be 2^32 threads, which the tile kernels' grid stays below
+    form = fdx.lib.fdx_debug_dense_rows_form
+    assert form(1, (1 << 24) - 1, 1028, 0) == 1 and form(1, 1 << 24, 1028, 0) == 0

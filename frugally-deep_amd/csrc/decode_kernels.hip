@@ -1211,7 +1211,7 @@ extern "C" fdx_status fdx_dense_rows_noalloc_f32(const float* x, int m, int k, c
     p.workspace_floats = fdx::kNoAllocWsFloats;
     p.tickets = reinterpret_cast<int*>(fdx::g_noalloc_ptr + fdx::kNoAllocWsFloats);
     p.ticket_count = fdx::kNoAllocTickets;
-    if (ksplit > 1) {
+    if (ksplit > 1 && !fdx::gemv_by_rule(p)) {
         // every call on this GPU shares the array, which keeps the last call's contents: the tickets this launch counts
         // on start at zero (a fill kernel, not a memset, so that a caller may capture the call)
         hipLaunchKernelGGL(fdx::clear_ints_kernel, dim3((unsigned)((tiles + 255) / 256)), dim3(256), 0, fdx::stream(), p.tickets, tiles);

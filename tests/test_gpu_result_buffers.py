@@ -47,6 +47,7 @@ def test_separate_buffers(fdx, modelgen, odd):
 
 
 def test_result_over_the_input(fdx, modelgen):
+    # "small": one launch, more samples than it has workgroups, which would write rows that others have still to read
     for shift in (0, 4, 400):
         for net in ("layers", "small"):
             b = modelgen.Builder("io", 6)
@@ -55,11 +56,29 @@ def test_result_over_the_input(fdx, modelgen):
             y = b.conv2d(y, 8, 3, "b", padding="same") if net == "small" else b.layernorm(y, "ln")
             m = fdx.Model(modelgen.dumps(b.finish([y])), verify=False)
             a = np.random.default_rng(2).standard_normal((300, 6, 6, 8)).astype(np.float32)
-            want = m.predict([a])[0]
-            t = fdx.DevBuf.from_host(np.concatenate([a.reshape(-1), np.zeros(400, np.float32)]))
-            m.predict_dev(300, [Ptr(t)], [(6, 6, 8)], [Ptr(t, shift)])
-            fdx.sync()
+            fdx.lib.fdx_debug_force_sample_net(1)
+            try:
+                want = m.predict([a])[0]
+                t = fdx.DevBuf.from_host(np.concatenate([a.reshape(-1), np.zeros(400, np.float32)]))
+                m.predict_dev(300, [Ptr(t)], [(6, 6, 8)], [Ptr(t, shift)])
+                fdx.sync()
+                assert fdx.lib.fdx_debug_sample_net(m._h) == (net == "small")
+            finally:
+                fdx.lib.fdx_debug_force_sample_net(-1)
             assert np.array_equal(t.to_host((300 * 288 + 400,))[shift:shift + 300 * 288], want.reshape(-1)), (net, shift)
+
+
+@pytest.mark.parametrize("shift", [4, 288, 860])
+def test_results_that_meet_each_other(fdx, modelgen, shift):
+    # the second one starts inside the first and ends beyond it: written one after the other, each whole
+    m = model(fdx, modelgen)
+    x = np.random.default_rng(7).standard_normal((3, 6, 6, 8)).astype(np.float32)
+    y, f, c = [w.reshape(-1) for w in m.predict([x])]
+    d, t, u = fdx.DevBuf.from_host(x), fdx.DevBuf.from_host(np.full(2 * 864, 9, np.float32)), fdx.DevBuf(4 * 16)
+    run(fdx, m, Ptr(d), [Ptr(t), Ptr(t, shift), Ptr(u)])
+    h = t.to_host((2 * 864,))
+    assert np.array_equal(h[:shift], y[:shift]) and np.array_equal(h[shift:shift + 864], f) and (h[shift + 864:] == 9).all()
+    assert np.array_equal(u.to_host((16,))[:15], c)
 
 
 def test_two_outputs_of_one_layer_and_of_the_input(fdx, modelgen):

@@ -62,7 +62,7 @@ def logits64(p, heads, ids):
 
 def test_prompts_and_steps_far_from_zero(fdx, modelgen):
     """A decoder whose residual stream has a mean of 100 deviations: the last position of a prompt and a decode step on the
-    decode launches (packed filters, rows loaded directly for one sequence, through LDS for sixteen) are about as close to
+    decode launches (filters as they are for one sequence, packed for more; rows loaded directly for seven, through LDS for sixteen) are about as close to
     float64 as the launch-by-launch path of a session too long for them, which normalises in a launch of its own."""
     heads, d_model, vocab = 8, 512, 33000
     spec = modelgen.gpt2(seed=112, layers=1, d_model=d_model, heads=heads, vocab=vocab, max_pos=32, bias_std=0.02)
@@ -73,7 +73,7 @@ def test_prompts_and_steps_far_from_zero(fdx, modelgen):
     for name in ("h0_fc", "lm_head"):
         p[name]["weights"] = zero_sum(p[name]["weights"], 0)
     model = fdx.Model(modelgen.dumps(spec), verify=False)
-    for B in (1, 16):
+    for B in (1, 7, 16):
         print("prompt far from zero", B, flush=True)
         ids = np.random.default_rng(113).integers(0, vocab, (B, 12))
         want = [np.stack([logits64(p, heads, ids[b, :t]) for b in range(B)]) for t in (11, 12)]

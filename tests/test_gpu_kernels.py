@@ -552,9 +552,10 @@ def test_shader_clock_probe(fdx):
 
 
 # (16, 3072, 768), (16, 4096, 1024), (9, 8192, 128): column groups in a multiple of 8, so the K ranges of a group (4, 4 and 8
-# of them) meet inside their XCD's L2; (1, 2048, 48): three column groups, the K ranges meet through memory
+# of them) meet inside their XCD's L2; (7, 2048, 48): three column groups, the K ranges meet through memory; (1, 2048, 48) and
+# (5, 20, 33): the kernels of one to six rows
 DENSE_ROWS = [(16, 768, 2304), (16, 768, 768), (16, 3072, 768), (3, 64, 100), (16, 768, 50257), (5, 20, 33), (7, 1024, 40),
-              (16, 100, 64), (1, 2048, 48), (16, 4096, 1024), (9, 8192, 128)]
+              (16, 100, 64), (1, 2048, 48), (7, 2048, 48), (16, 4096, 1024), (9, 8192, 128)]
 
 
 @pytest.mark.parametrize("m,k,n", DENSE_ROWS)

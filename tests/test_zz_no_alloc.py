@@ -1,6 +1,6 @@
 """The Dense entry point that allocates nothing (its split-K scratch is a fixed device array inside the library)
 against fdx_dense_rows_f32, which allocates its workspace on first use: same kernels, same split, so the results must be
-bit-identical.  Two calls in a row, the second on a smaller input, then the limits."""
+bit-identical.  Calls in a row, the second on a smaller input, then the limits."""
 import numpy as np
 import pytest
 
@@ -20,9 +20,9 @@ def test_no_alloc_dense_rows_equals_the_allocating_entry_point(fdx, oracle):
     fdx.check(fdx.lib.fdx_init(0))
     r = np.random.default_rng(71)
     act = fdx.gelu_act()
-    # (16, 3072, 768): 48 column groups x 4 K ranges through the scratch array; then smaller: (5, 2048, 320), 20 x 2;
-    # then one that needs no scratch at all
-    for m, k, n in [(16, 3072, 768), (5, 2048, 320), (3, 64, 100)]:
+    # (16, 3072, 768): 48 column groups x 4 K ranges through the scratch array; then smaller: (7, 2048, 320), 20 x 8, over the first
+    # one's partial tiles and tickets, and once more behind a call of few rows, (5, 2048, 320), which like (3, 64, 100) needs no scratch
+    for m, k, n in [(16, 3072, 768), (7, 2048, 320), (5, 2048, 320), (7, 2048, 320), (3, 64, 100)]:
         print("no-alloc dense_rows", m, k, n, flush=True)
         x = r.standard_normal((m, k)).astype(np.float32)
         w = (r.standard_normal((n, k)) / np.sqrt(k)).astype(np.float32)

@@ -296,7 +296,7 @@ constexpr SliceForm kSliceForm[kSliceForms] = { { 1, 1, 8 }, { 1, 2, 8 }, { 2, 2
 // The form for a problem, or -1 where the tiled kernel (its cost by tile_pick) is the better one.  The forms were timed on 1000
 // problems (M 1-16384, N 16-3072, K 16-4608, up to 6 GFLOP, GEMM and convolution, weights out of memory, launches back to
 // back) and follow, in microseconds, with w = tiles per CU rounded up, to 13-21 % rms
-//     t0 + w (c1 + c2 (rows + columns of the tile) K / 10^4), c2 larger for a convolution:
+//     t0 + w (c1 + c2 (rows + columns of the tile) K / 10^4):
 // a workgroup costs what it pulls through its CU's path from L2, about 36 cycles per KB.  With one round of tiles (the first row of a form)
 // K counts up to whole units of all waves: where it is one unit of 32, waves have nothing to do, and the form of four is the fastest (337 x
 // 1144 x 32: 8 / 4 waves 5.0 / 3.8 us); there the choice among the forms takes 0.6 % longer than the best of them, past a round
@@ -304,22 +304,33 @@ constexpr SliceForm kSliceForm[kSliceForms] = { { 1, 1, 8 }, { 1, 2, 8 }, { 2, 2
 // general kernel's narrow tile, which wins from about 600 row blocks of 64 on (N = 32, K = 144-192: 20000 rows 8.2-9.7 against
 // 6.3-7.2 us here, 50000 rows 11.0-14.5 against 11.1-14.0, convolutions 13.9 against 17.1); between 32 and 64 columns the tiled
 // kernel's half empty 64-column tile beats it (97733 x 40 x 288 31.5 against 40.9 us, 24000 x 36 x 512 17.4 / 21.7).
-// A convolution's constants are those of a kernel that made a mask of all taps first and put it 1 to 2 us too high, on both sides of the
-// choice: it takes 1.9 % longer than the best of 143 timed convolutions. Fitted again 1.3 %, but ResNet50 of one image 332 against 330 us.
+// A convolution has constants of its own, and two rounds of tiles a row of theirs: the workgroups of both run side by side.  With one
+// round a workgroup takes longer where more CUs pull at once:
+//     t0 + (rows + columns of the tile) K / 10^4 (c2 + c1 tiles / CUs).
+// Fitted to 1000 timed convolutions (3x3, 3x3 and 1x1 of stride 2, 5x5; M 20-30000, K 16-8000, weights from the memory-side cache), 5 to 7 %
+// rms.  Over 1000 others the choice of form and kernel takes 0.4 % longer than the best (0.8 % with constants that were
+// 13 to 24 % too high in one round, 0.7 % without the last term), and with Winograd beside them, 478 problems, 0.3 %.
 static int64_t slice_tiles(int M, int N, int bm, int bn) { return (int64_t)((M + bm - 1) / bm) * ((N + bn - 1) / bn); }
 static float slice_rounds(int64_t tiles) { return (float)((tiles + 255) / 256); }
 static float slice_cost(int form, bool conv, int M, int N, int K)
 {
-    static const float kCost[kSliceForms][2][4] = { // t0, c1, c2 of a GEMM, c2 of a convolution; one round of tiles, more
-        { { 2.46f, 0.64f, 0.39f, 0.89f }, { 2.18f, 1.29f, 0.42f, 0.59f } }, { { 2.73f, 0.25f, 0.47f, 0.78f }, { 2.13f, 1.07f, 0.50f, 0.62f } },
-        { { 2.01f, 0.77f, 0.65f, 1.15f }, { 2.24f, 1.47f, 0.64f, 1.02f } }, { { 2.89f, 0.19f, 0.68f, 1.14f }, { 2.52f, 0.71f, 0.76f, 0.92f } },
-        { { 1.62f, 1.19f, 0.80f, 1.42f }, { 1.52f, 2.43f, 0.83f, 1.25f } }
+    static const float kGemm[2][kSliceForms][3] = { // t0, c1, c2; one round of tiles, more
+        { { 2.46f, 0.64f, 0.39f }, { 2.73f, 0.25f, 0.47f }, { 2.01f, 0.77f, 0.65f }, { 2.89f, 0.19f, 0.68f }, { 1.62f, 1.19f, 0.80f } },
+        { { 2.18f, 1.29f, 0.42f }, { 2.13f, 1.07f, 0.50f }, { 2.24f, 1.47f, 0.64f }, { 2.52f, 0.71f, 0.76f }, { 1.52f, 2.43f, 0.83f } }
+    };
+    static const float kConv[3][kSliceForms][3] = { // one round, two, more
+        { { 3.53f, 0.07f, 0.45f }, { 3.34f, 0.08f, 0.52f }, { 3.49f, 0.08f, 0.69f }, { 3.78f, 0.06f, 0.78f }, { 4.54f, 0.06f, 0.86f } },
+        { { 4.95f, 0.f, 0.50f }, { 4.35f, 0.f, 0.50f }, { 6.84f, 0.f, 0.70f }, { 4.83f, 0.f, 0.69f }, { 11.35f, 0.f, 0.86f } },
+        { { 2.27f, 1.37f, 0.51f }, { 2.93f, 1.08f, 0.48f }, { 1.95f, 2.36f, 0.74f }, { 3.09f, 0.97f, 0.68f }, { 1.71f, 4.60f, 0.91f } }
     };
     const int bm = 16 * kSliceForm[form].tm, bn = 16 * kSliceForm[form].tn, unit = 32 * kSliceForm[form].nw;
-    const float rounds = slice_rounds(slice_tiles(M, N, bm, bn));
-    const float* c = kCost[form][rounds > 1.f ? 1 : 0];
-    const int k = rounds > 1.f ? K : (K + unit - 1) / unit * unit;
-    return c[0] + rounds * (c[1] + c[conv ? 3 : 2] * 1e-4f * (bm + bn) * k);
+    const int64_t tiles = slice_tiles(M, N, bm, bn);
+    const float rounds = slice_rounds(tiles);
+    const float pulled = 1e-4f * (float)(bm + bn) * (float)(rounds > 1.f ? K : (K + unit - 1) / unit * unit);
+    const float* c = conv ? kConv[rounds > 2.f ? 2 : rounds > 1.f ? 1 : 0][form] : kGemm[rounds > 1.f][form];
+    if (conv && rounds <= 1.f)
+        return c[0] + pulled * (c[2] + c[1] * (float)tiles / 256.f);
+    return c[0] + rounds * (c[1] + c[2] * pulled);
 }
 // whether a launch of this form stays below the 2^32 threads a grid can have
 static bool slice_fits(int form, int M, int N)
@@ -335,11 +346,11 @@ static int slice_pick(bool conv, int M, int N, int K, float tiled_cost)
         return -1;
     int best = -1;
     // Below a round of tiles the tiled kernel takes longer than its cost says, which was fitted to 0.2 GFLOP and more: on 600 small problems by
-    // 1.4 us up to K = 128 (4204 x 64 x 64 5.7 against 3.6 us here), convolutions by half (3x3 16 -> 388 on 1001 pixels 9.7 / 7.2), less where
-    // K is long.  Kernel choices then take 1.7 % longer than the best, 5.2 % with 0.95 of the cost.  Past a round operands re-read cost
-    // the neighbours, too.
+    // 1.4 us up to K = 128 (4204 x 64 x 64 5.7 against 3.6 us here), on 1700 convolutions by 2 us up to a cost of 9, 1.2 at 16, 0.4 at 25.  Kernel
+    // choices then take 1.7 % (convolutions 0.4 %) longer than the best; GEMMs 5.2 % with 0.95 of the cost.  Past a round operands
+    // re-read cost the neighbours, too.
     const float fade = 15.f / std::max(15.f, tiled_cost);
-    float best_cost = narrow ? 1e30f : t64 > 256 ? 0.95f * tiled_cost : conv ? (K <= 1024 ? 1.3f : 1.15f) * tiled_cost : tiled_cost + 1.5f * fade * fade;
+    float best_cost = narrow ? 1e30f : t64 > 256 ? 0.95f * tiled_cost : tiled_cost + 1.5f * fade * fade;
     for (int i = 0; i < kSliceForms; ++i) {
         const float cost = slice_cost(i, conv, M, N, K);
         if (cost < best_cost && slice_fits(i, M, N)) {

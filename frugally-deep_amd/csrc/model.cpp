@@ -1802,6 +1802,7 @@ extern "C" fdx_status fdx_debug_force_chain(int mode)
 // (maps of 6 to 62 pixels, 8 to 512 channels, batches of 1 to 64) the choice takes 0.6 % longer than the faster form on average, at
 // worst 21 %; Winograd from a gigaflop of direct-sum work on takes 8 %, always the direct kernel 13 % (36 % where the channels
 // are no multiple of 16: 8 images, 56 x 56 x 56 -> 128: direct 49.6 us, Winograd 31.2; 16 of 56 x 56 x 64 -> 64 29.7 / 35.1).
+// Of 478 up to 4 GFLOP, timed with the few-tiles kernel as it is now, it takes 0.3 %, at worst 15 %; the Winograd form is the faster one of 4 % there.
 // Nothing is charged for the direct kernel's higher power: ResNet50 passes of 8 / 16 / 24 / 32 / 48 / 64 / 100 images take 964 / 1352 /
 // 1746 / 2075 / 2926 / 3581 / 5429 us, with 3 % charged 963 / 1373 / 1767 / 2074 / 2928 / 3579 / 5361, with 4 % in its favour 964 / 1351 / 1750 /
 // 2071 / 2939 / 3597 / 5453.  It is also closer to 64-bit results (2-norm, 64 / 128 / 256 / 512 channels: 1.1 / 0.8 / 1.1 / 1.3 e-7 against

@@ -1372,6 +1372,38 @@ float conv3x3_direct_cost(int n, int h, int w, int cin, int cout, int oh, int ow
     const bool halo = oh == h && ow == w && cin % kSlab == 0 && 2 * w + 2 <= kHaloSpan;
     return fast_pick(true, (int)m, cout, 9 * cin, a_floats, residual, 1, closed_cuts(), halo).cost;
 }
+
+// Predicted time (us) of any convolution or Dense layer (conv = false: `rows` rows of cin) as run_igemm launches it, for layers of small
+// networks.  The general kernel's by tile and by whether its operands come in fours:
+//     t0 + a k w + t (e + b k) + g k,  t = tiles / CUs, w = t rounded up, k = K / 1000 in whole slabs,
+// fitted to 1050 timed layers (1 to 64 input channels, 4 to 64 output channels, filters of 1, 3 and 5, maps of 3 to 40, 1 to 8192 images; Dense
+// layers of 8 to 128), 6 to 17 % rms.
+float layer_cost(bool conv, int64_t rows, int cin, int taps, int cout, int64_t a_floats, bool residual, bool halo)
+{
+    const int m = (int)std::min<int64_t>(rows, INT32_MAX), k = taps * cin;
+    const float out_mb = 4e-6f * (float)((double)a_floats + (residual ? 2. : 1.) * (double)rows * cout);
+    if (cin % 16 == 0 && cout % 4 == 0 && a_floats < (1LL << 29)) {
+        const TileChoice c = fast_pick(conv, m, cout, k, a_floats, residual, 1, closed_cuts(), halo);
+        if (c.cfg < kSliceCfg && !conv && k <= 32 && cout <= 160 && m >= 65536)
+            return std::min(c.cost, 4.f + out_mb / 3.5f); // the row-streaming kernel
+        const float fade = 15.f / std::max(15.f, c.cost); // (see slice_pick)
+        if (c.cfg >= kSliceCfg || cout > 32)
+            return c.cost + (c.cfg < kSliceCfg ? 1.5f * fade * fade : 0.f);
+    }
+    const int cfg = general_pick(m, cout, 1);
+    if (cfg == 0)
+        return general_cost(m, cout, k);
+    static const float kCost[3][2][5] = { // tiles of 128 x 64, 128 x 32, 64 x 64; in fours, one by one
+        { { 3.36f, 26.3f, 1.82f, 8.9f, 46.9f }, { 5.31f, 58.6f, 1.39f, 0.f, 54.8f } },
+        { { 3.92f, 18.0f, 0.68f, 3.9f, 27.5f }, { 4.04f, 15.9f, 0.53f, 27.8f, 74.7f } },
+        { { 3.94f, 11.9f, 0.82f, 6.8f, 18.0f }, { 4.41f, 46.4f, 0.59f, 0.f, 0.6f } }
+    };
+    const int bm = cfg == 3 ? 64 : 128, bn = cfg == 2 ? 32 : 64;
+    const int64_t tiles = (int64_t)((m + bm - 1) / bm) * ((cout + bn - 1) / bn);
+    const float ks = 1e-3f * BK * (float)((k + BK - 1) / BK), t = (float)tiles / 256.f, w = (float)((tiles + 255) / 256);
+    const float* c = kCost[cfg - 1][cin % 4 == 0 ? 0 : 1];
+    return c[0] + c[1] * ks * w + t * (c[2] + c[3] * ks) + c[4] * ks;
+}
 } // namespace fdx
 
 extern "C" fdx_status fdx_conv2d_nhwc_f32(const float* in, int n, int h, int w, int cin,

@@ -150,6 +150,20 @@ __device__ __forceinline__ uint32_t seg_offset(const GemmParams& p, int sg, int 
 }
 __device__ __forceinline__ int seg_of(const GemmParams& p, int n0) { return (n0 >= p.seg_col[0]) + (n0 >= p.seg_col[1]); }
 
+// Bit y * kw + x: filter tap (y, x) lies inside the image, for a row whose tap (0, 0) lies at (iy, ix).  Columns and rows apart and without
+// branches: tap by tap, with lanes taking branches of their own, nine taps of eight rows held up every tile's first load (ResNet50 of 64
+// images 0.5 % longer).
+template <typename Mask>
+__device__ __forceinline__ Mask taps_inside(const GemmParams& p, int iy, int ix)
+{
+    Mask row = 0, all = 0;
+    for (int x = 0; x < p.kw; ++x, ix += p.dx)
+        row |= (Mask)((unsigned)ix < (unsigned)p.W) << x;
+    for (int y = 0, at = 0; y < p.kh; ++y, iy += p.dy, at += p.kw)
+        all |= (unsigned)iy < (unsigned)p.H ? row << at : (Mask)0;
+    return all;
+}
+
 //  * DUAL (GEMM form, whole tiles only): the rows of A come from two tensors -- the first K1 columns from A with row
 //    stride lda, the other K - K1 from A2, whose row for output pixel (image, y, x) is pixel (y * s2y, x * s2x) of an
 //    [H2][W2][C2] map.  That is the sum of two pointwise convolutions as one GEMM over the concatenated channels
@@ -172,20 +186,6 @@ __device__ __forceinline__ int seg_of(const GemmParams& p, int n0) { return (n0 
 //    operands are read from LDS at its distance; a lane whose row has no such pixel (the convolution's padding) reads a
 //    pixel of zeros kept behind the run.  64 images: 28 x 28 x 128 -> 128 84 -> 77 us, 14 x 14 x 256 -> 256 87 -> 77,
 //    56 x 56 x 64 -> 64 113 -> 85; 16 images 32 -> 29, 35 (few-tiles ranges) -> 36, 34 -> 26.
-// Bit y * kw + x: filter tap (y, x) lies inside the image, for a row whose tap (0, 0) lies at (iy, ix).  Columns and rows apart and without
-// branches: tap by tap, with lanes taking branches of their own, nine taps of eight rows held up every tile's first load (ResNet50 of 64
-// images 0.5 % longer).
-template <typename Mask>
-__device__ __forceinline__ Mask taps_inside(const GemmParams& p, int iy, int ix)
-{
-    Mask row = 0, all = 0;
-    for (int x = 0; x < p.kw; ++x, ix += p.dx)
-        row |= (Mask)((unsigned)ix < (unsigned)p.W) << x;
-    for (int y = 0, at = 0; y < p.kh; ++y, iy += p.dy, at += p.kw)
-        all |= (unsigned)iy < (unsigned)p.H ? row << at : (Mask)0;
-    return all;
-}
-
 template <int BM, int BN, int WAVES_M, int WAVES_N, bool CONV, bool SPLIT = false, bool STREAMK = false, bool DUAL = false,
     bool LNF = false, bool SEG = false, bool HALO = false>
 __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, split_tile_waves(BM, BN, WAVES_M, WAVES_N))

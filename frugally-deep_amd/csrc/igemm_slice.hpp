@@ -14,6 +14,7 @@
 //  * the waves' partial tiles meet once in LDS and are added in wave order (the sum does not depend on timing), the
 //    epilogue runs on the sum.  Bias and residual are requested in front of the K walk.
 //  * tiles are numbered so that an XCD owns neighbours that share the larger operand's rows: it passes through one L2.
+
 // f with n, at most MOST, as a compile-time constant
 template <int MOST, typename F>
 __device__ __forceinline__ void by_count(int n, F&& f)

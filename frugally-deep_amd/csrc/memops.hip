@@ -234,7 +234,6 @@ __global__ __launch_bounds__(256) void dwconv3x3_slide_kernel(const float* __res
 }
 
 // ------------------------------------------------------------------ pooling
-// One lane per (output pixel, VEC channels); VEC = 4 moves 16 bytes per access.
 // Windows of PH x PW cells known at compile time, channels in fours: all cells requested before the first is used, addresses clamped into
 // the image.  (Cell by cell behind a test each, 112 x 112 x 64 under 3 x 3 / 2 took 7.1 us for one image against 4.0.)
 template <int PH, int PW, bool MAX>
@@ -283,6 +282,7 @@ __global__ __launch_bounds__(256) void pool2d_small_kernel(const float* __restri
     }
 }
 
+// One lane per (output pixel, VEC channels); VEC = 4 moves 16 bytes per access.
 template <int VEC>
 __global__ void pool2d_kernel(const float* __restrict__ in, float* __restrict__ out, int n, int h, int w, int c,
     int ph, int pw, int sy, int sx, int pad_top, int pad_left, int zt, int zl, int zb, int zr, int oh, int ow, int mode)

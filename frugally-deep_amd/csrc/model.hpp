@@ -176,6 +176,8 @@ fdx_status gemm_ln_launch(const float* x, int64_t m, int k, const float* w, cons
 // predicted times of a 3x3 stride-1 convolution as a direct sum and in the Winograd form (igemm.hip, wino.hip)
 float conv3x3_direct_cost(int n, int h, int w, int cin, int cout, int oh, int ow, bool residual);
 float conv2d_winograd_cost(int n, int cin, int cout, int oh, int ow);
+// predicted time of a small network's layer (igemm.hip)
+float layer_cost(bool conv, int64_t rows, int cin, int taps, int cout, int64_t a_floats, bool residual, bool halo);
 fdx_status conv1x1_dual_launch(const float* in1, int n, int oh, int ow, int c1, const float* in2, int h2, int w2, int c2, int s2y, int s2x,
     const float* w_cat, const float* bias, int cout, const fdx_act* act, float* out);
 fdx_status conv1x1_padded_launch(const float* in, int64_t rows, int cin, const float* w_padded, int k_padded, const float* bias,

@@ -42,12 +42,13 @@ namespace {
 
     bool epilogue_kind(const Act& a) { return a.kind == FDX_ACT_NONE || a.kind == FDX_ACT_RELU || a.kind == FDX_ACT_GELU; }
 
-    // Cycles of a CU: the matrix pipes', or the chain of a wave's own items where there are few, and a step's latency, longer where
-    // pixels are read one float at a time.
+    // Cycles of a CU.  A convolution: the matrix pipes', or the chain of a wave's own items where there are few, longer where pixels are
+    // read one float at a time, and an epilogue a tile.  These and the other steps' constants below, of 100 timed models with 300
+    // convolutions, predict 100 others to 9 % rms (1 to 5 convolutions of 4 to 64 channels on maps of 6 to 40, or Dense layers).
     double conv_cycles(int pixels, int n_tiles, int chunks, bool vec)
     {
-        const double m_tiles = (pixels + 15) / 16, items = m_tiles * n_tiles;
-        return (vec ? 2000 : 4000) + 1500 * std::min(1.0, m_tiles / 16) + 1.25 * std::max(items * chunks * 32, std::ceil(items / 16) * chunks * 350);
+        const double tiles = (pixels + 15) / 16 * (double)n_tiles, chain = std::max(tiles * chunks * 32, std::ceil(tiles / 16) * chunks * 350);
+        return (vec ? 1450 + 0.93 * chain : 1750 + 1.14 * chain) + 110 * tiles;
     }
 
 } // namespace
@@ -221,17 +222,17 @@ std::shared_ptr<SampleProgram> sample_net_build(const fdx_model& m, const std::v
         const Tensor& me = seen[(size_t)r.op];
         if ((r.behind && o.softmax) || o.kind == OpKind::Softmax) {
             s.kind = SampleStep::Softmax;
-            cycles += 700 + std::ceil(me.h * me.w / 16.0) * (1000 + me.c * 3);
+            cycles += 900 + std::ceil(me.h * me.w / 16.0) * (1270 + me.c * 3.8);
         } else if (o.kind == OpKind::Input) {
             s.kind = SampleStep::Load;
-            cycles += 3000 + volume(shapes[(size_t)r.op]) * 0.2;
+            cycles += 1600 + volume(shapes[(size_t)r.op]) * 0.42;
         } else if (r.behind || o.kind == OpKind::Act) {
             s.kind = SampleStep::Activation;
             s.act_kind = o.act.kind;
             s.act_max = o.act.max_value;
             s.act_slope = o.act.negative_slope;
             s.act_threshold = o.act.threshold;
-            cycles += 700 + (double)me.h * me.w * me.c * 0.5;
+            cycles += 900 + (double)me.h * me.w * me.c * 0.64;
         } else if (o.kind == OpKind::Pool) {
             const Tensor& x = seen[(size_t)o.in[0]];
             int g[6];
@@ -245,12 +246,12 @@ std::shared_ptr<SampleProgram> sample_net_build(const fdx_model& m, const std::v
             s.pad_top = g[0];
             s.pad_left = g[2];
             s.mode = o.pool_mode;
-            cycles += 1500 + (double)me.h * me.w * me.c * o.kh * o.kw * 0.1;
+            cycles += 1900 + (double)me.h * me.w * me.c * o.kh * o.kw * 0.13;
         } else if (o.kind == OpKind::GlobalPool) {
             const Tensor& x = seen[(size_t)o.in[0]];
             s.kind = SampleStep::GlobalPool;
             s.mode = o.pool_mode;
-            cycles += 2000 + (double)x.h * x.w * x.c * 0.15;
+            cycles += 2500 + (double)x.h * x.w * x.c * 0.19;
         } else { // convolution; a Dense layer is one of 1 x 1
             const bool conv = o.kind == OpKind::Conv2D;
             const Tensor& x = seen[(size_t)o.in[0]];
@@ -326,7 +327,7 @@ std::shared_ptr<SampleProgram> sample_net_build(const fdx_model& m, const std::v
             s.bias = words((size_t)s.n_tiles * 16);
             for (int n = 0; n < cout && n < (int)o.sample_bias.size(); ++n)
                 image[(size_t)(s.bias + n)] = o.sample_bias[(size_t)n];
-            cycles += s.kind == SampleStep::Row ? 1000 + std::ceil(cout / 128.0) * (150 + cin * 2) : conv_cycles(me.h * me.w, s.n_tiles, s.chunks, s.vec);
+            cycles += s.kind == SampleStep::Row ? 1400 + std::ceil(cout / 128.0) * (210 + cin * 2.8) : conv_cycles(me.h * me.w, s.n_tiles, s.chunks, s.vec);
         }
         if (image.size() > (size_t)kSampleLdsFloats)
             return nullptr;
@@ -427,7 +428,7 @@ std::shared_ptr<SampleProgram> sample_net_build(const fdx_model& m, const std::v
     p->steps = (int)steps.size();
     p->in_volume = p_in_volume;
     p->out_volume = (int)volume(shapes[(size_t)m.outputs[0]]);
-    p->us_per_sample = (cycles + 0.4 * p->out_volume) / 2400.0; // (a result's way out: four floats a cycle at most, 256 CUs at once)
+    p->us_per_sample = (cycles + 0.68 * p->out_volume) / 2400.0; // (a result's way out)
     const size_t step_floats = steps.size() * sizeof(SampleStep) / 4;
     p->step_at = (image.size() + 15) / 16 * 16;
     image.resize(p->step_at + step_floats);
@@ -460,13 +461,15 @@ bool sample_net_load(SampleProgram& p)
     return true;
 }
 
-// One launch or one per operation, by predicted times: a launch costs what the chain's shortest take (3.7 us), or its traffic and its
-// arithmetic, at 90 TFLOP/s where the tiled kernel has whole slabs and columns and 30 elsewhere, of columns that fill its tile.  Measured, us of a call, launches /
-// one: the small CNN (two 3x3 convolutions of 16 and 32 channels on 32 x 32 x 3) at batch 1 / 256 / 8192 24 / 16.7, 59 / 17.7, 902 /
-// 478; 28 x 28 with 5x5 convolutions of 6 and 16 channels and two Dense layers 44 / 14.9, 61 / 15.9, 717 / 405; four 3x3
-// convolutions of 16 channels on 16 x 16 26 / 19.6, 65 / 20.5, 1060 / 566; strided 3x3 of 32 and 64 channels on 32 x 32 x 3 23 / 15,
-// 40 / 16, 340 / 407 (the rule leaves the last to the launches); three Dense layers of 128 at batch 1 / 256 / 2048 13.5 / 6.8, 13.7 /
-// 7.0, 13.7 / 28 (the last left to the launches); one 3x3 convolution 8 -> 32 on 24 x 24 at batch 1 / 256 8.2 / 12.7 (left), 19.4 / 16.3.
+// One launch or one per operation, by predicted times: a convolution or Dense layer's own launch as layer_cost has it, any other by its traffic,
+// 3.7 us at least.  Over 1200 timed calls (200 models of 1 to 5 convolutions of 4 to 64 channels or 1 to 4 Dense layers, 1 to 8192 samples) the
+// choice takes 0.4 % longer than the faster form, at worst 32 %; with one rate for all convolutions it took 10 %, and 2.1 times as
+// long where 8192 samples of two convolutions to 24 and 64 channels went into one launch.  Measured, us of a call, launches / one: the small CNN (two 3x3
+// convolutions of 16 and 32 channels on 32 x 32 x 3) at batch 1 / 256 / 8192 24 / 17.2, 59 / 17.9, 906 / 490; 28 x 28 with 5x5 convolutions of 6 and 16
+// channels and two Dense layers 44 / 15.5, 62 / 16.1, 717 / 414; four 3x3 convolutions of 16 channels on 16 x 16 25 / 20.7, 66 / 21.6, 1060 /
+// 600; strided 3x3 of 32 and 64 channels on 32 x 32 x 3 22 / 15.6, 34 / 16.6, 335 / 427 (the last left to the launches); two
+// Dense layers of 128 at batch 1 / 256 / 2048 13.2 / 6.7, 13.6 / 7.0, 13.5 / 28 (left); one 3x3 convolution 8 -> 32 on 24 x 24 at batch 1 / 256 / 8192 8.2 / 13.1
+// (left), 19.3 / 16.6, 387 / 397 (left).
 bool sample_net_by_rule(const SampleProgram& p, const fdx_model& m, const std::vector<int>& order, const std::vector<Shape>& shapes, int batch)
 {
     double launches = 0;
@@ -474,13 +477,23 @@ bool sample_net_by_rule(const SampleProgram& p, const fdx_model& m, const std::v
         const Op& o = m.ops[(size_t)idx];
         if (o.dead || o.kind == OpKind::Input || o.kind == OpKind::View)
             continue;
-        const double in = (double)batch * volume(shapes[(size_t)o.in[0]]), out = (double)batch * volume(shapes[(size_t)idx]);
-        double us = (in + out) * 4 / 3e6;
+        const Shape &is = shapes[(size_t)o.in[0]], &os = shapes[(size_t)idx];
+        const double in = (double)batch * volume(is), out = (double)batch * volume(os);
+        double us = std::max(3.7, (in + out) * 4 / 3e6);
         if (o.kind == OpKind::Conv2D || o.kind == OpKind::Dense) {
-            const double n = (double)shapes[(size_t)idx].back(), rate = o.n_in % 16 == 0 && n >= 64 ? 90e6 : 30e6 * std::min(1.0, n / 32);
-            us = std::max(us, 2 * out * o.n_in * o.kh * o.kw / rate);
+            const int n = (int)os.back();
+            const int64_t rows = (int64_t)batch * (volume(os) / n), a_floats = (int64_t)in;
+            int d[3], e[3];
+            (void)hwc_of(is, d);
+            (void)hwc_of(os, e);
+            const bool same = o.kind == OpKind::Conv2D && o.sy == 1 && o.sx == 1 && d[0] == e[0] && d[1] == e[1];
+            const bool pointwise = o.kind == OpKind::Dense || (same && o.kh == 1 && o.kw == 1);
+            const int taps = o.kind == OpKind::Dense ? 1 : o.kh * o.kw;
+            us = layer_cost(!pointwise, rows, o.n_in, taps, n, a_floats, o.residual >= 0, same && taps >= 6 && o.n_in % 32 == 0 && d[1] <= 63);
+            if (same && o.kh == 3 && o.kw == 3 && fdx_conv2d_winograd_supported(o.n_in, n))
+                us = std::min(us, (double)conv2d_winograd_cost(batch, o.n_in, n, e[0], e[1]));
         }
-        launches += std::max(3.7, us) + (o.softmax ? 3.0 : 0.0);
+        launches += us + (o.softmax ? 3.0 : 0.0);
     }
     return 3.0 + std::ceil((double)batch / sample_net_cus()) * p.us_per_sample < launches;
 }

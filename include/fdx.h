@@ -404,7 +404,10 @@ fdx_status fdx_model_io_shape(const fdx_model* m, int is_output, int index, int*
  * tensor_shape.hpp:246-250).  Outputs: out[i] receives batch * volume floats; out_dims/out_ranks are
  * written per output.  Host-pointer and device-pointer variants.  The device-pointer variant returns with its work
  * queued on the library's stream (fdx_sync waits for it) and reads inputs that are 16-byte aligned where they lie
- * (others are copied first): such an input must stay unchanged until that work has completed.
+ * (others are copied first): such an input must stay unchanged until that work has completed.  Results are written to out_dev
+ * while the work runs, not by a copy at its end (except into buffers that are not 16-byte aligned, or that overlap an input or
+ * each other): the buffers must be left alone until it has completed, and after a failed call, or one whose work
+ * fails, they may hold part of a result.
  */
 fdx_status fdx_model_predict(fdx_model* m, int batch, const float* const* in, const int64_t* in_dims,
     const int* in_ranks, float* const* out, int64_t* out_dims, int* out_ranks);

@@ -205,7 +205,7 @@ def test_refused_memory_leaves_the_launches(fdx, modelgen):
 
 
 def test_a_program_goes_to_the_device_once_and_only_where_it_runs(fdx, modelgen):
-    # three Dense layers of 128: the rule leaves batches beyond a few hundred to the launches
+    # two Dense layers of 128: the rule leaves batches beyond a few hundred to the launches
     b = modelgen.Builder("dense", 3)
     x = b.input((128,), "in")
     for i in range(2):
@@ -266,3 +266,22 @@ def test_host_arrays_in_pieces(fdx, modelgen, net, shape, batch):
         fdx.lib.fdx_debug_force_sample_net(-1)
     for g in got:
         assert np.array_equal(np.asarray(g).reshape(batch, n), want)
+
+
+def test_the_rule_follows_the_layers_own_times(fdx, modelgen):
+    """Two convolutions of 5x5 / 2 and 3x3 to 24 and 64 channels on 12 x 12: as one launch twice as fast up to a few hundred samples, twice as slow
+    for 8192 (267 us against 126).  Three convolutions with six channels in the middle on 8 x 8: 13 against 44 us for one sample."""
+    def wide(b):
+        return b.conv2d(b.conv2d(b.input((12, 12, 8), "in"), 24, 5, "a", strides=2, padding="same", activation="relu"), 64, 3, "b", padding="same")
+
+    def thin(b):
+        x = b.conv2d(b.input((8, 8, 4), "in"), 48, 3, "a", padding="same", activation="relu")
+        x = b.pool(b.conv2d(x, 6, 3, "b", padding="same", activation="relu"), "p", 2, 2)
+        return b.conv2d(x, 48, 5, "c", padding="same")
+
+    for f, shape, forms in ((wide, (12, 12, 8), {1: 1, 64: 1, 8192: 0}), (thin, (8, 8, 4), {1: 1, 256: 1})):
+        b = modelgen.Builder(f.__name__, 3)
+        model = fdx.Model(modelgen.dumps(b.finish([f(b)])), verify=False)
+        for n, form in forms.items():
+            model.predict([np.zeros((n,) + shape, np.float32)])
+            assert fdx.lib.fdx_debug_sample_net(model._h) == form, (f.__name__, n)

@@ -5,7 +5,7 @@
 // microsecond of work on a few CUs.  Samples do not meet in any layer, so a workgroup can keep one to itself: what is left is one
 // launch, the image's way in and the sample's arithmetic on one CU (fp32 MFMA, 256 multiply-adds a cycle).
 //
-//  * 16 waves, four per SIMD: a convolution is dealt out as 16-pixel x 16 or 32-channel tiles, each wave walks K on its own; with four
+//  * 16 waves, four per SIMD: a convolution is dealt out as 16-pixel x 16 or 32-channel tiles, each wave walks K on its own in short chains; with four
 //    waves a SIMD's matrix pipe stays busy through the two dependent LDS reads in front of a product (offset, then pixel).
 //  * the filter is the MFMA's row operand and the pixels its columns, so that a lane ends up with four neighbouring channels of
 //    a pixel: 16-byte stores.
@@ -28,7 +28,7 @@ __device__ __forceinline__ int product(int a, int b) { return (int)__umul24((uns
 __device__ __forceinline__ int position(int y, int x, int row, int pix) { return product(y, row) + product(x, pix); }
 
 // ReLU of N values.  Without slope and threshold one instruction a value, and one that finds what is not finite (0 * value is zero
-// otherwise): that takes the general form, six a value.  With the 24-bit positions the small CNN's first convolution 11300 -> 10700 cycles.
+// otherwise): that takes the general form, six a value.  With the 24-bit positions the small CNN's first convolution took 600 of 11300 cycles less.
 template <int N>
 __device__ __forceinline__ void sample_relu(const SampleStep& s, float* r)
 {
@@ -426,10 +426,10 @@ __device__ __forceinline__ void sample_activation(const SampleStep& s, float* ld
 }
 
 // What bounds it, on the small CNN of 32 x 32 x 3 (two 3x3 convolutions of 16 and 32 channels, pooling, classifier), cycles of a CU per
-// sample: way in 5000, first convolution 10700 (matrix pipes 4100, the rest its scattered 4-byte reads and the epilogue), pooling 1700,
-// second convolution 13000 (7500), global pooling 2400, Dense 1300, softmax 1800.  17.7 us a call up to 256 samples, where seven launches
-// took 27 to 62; eight samples a CU 121 us, 234 before.  Image and input on their way together, Dense off the matrix
-// instructions and 2 x 2 windows and pooled channels by fours: 18.9 -> 17.7.  Nothing may go to scratch memory: 20 bytes a lane of it
+// sample: way in 5800, first convolution 10200 (matrix pipes 4100, the rest its scattered 4-byte reads and the epilogue), pooling 1900,
+// second convolution 14000 (9200), global pooling 2600, Dense 1300, softmax 1700.  16.7 us a call for one sample and 17.6 up to 256, where
+// seven launches take 24 and 59; 8192 samples 490 us, 906 as launches.  Image and input on their way together, Dense off the matrix
+// instructions, 2 x 2 windows and pooled channels by fours took 1.2 us off it.  Nothing may go to scratch memory: 20 bytes a lane of it
 // cost 7 us a launch.
 __global__ __launch_bounds__(kSampleThreads) void sample_net_kernel(const float* __restrict__ in, float* __restrict__ out,
     const f32x4* __restrict__ image, int image_quads, const SampleStep* __restrict__ program, int steps, int in_volume, int out_volume, int batch)

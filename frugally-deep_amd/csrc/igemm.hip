@@ -1380,7 +1380,7 @@ float conv3x3_direct_cost(int n, int h, int w, int cin, int cout, int oh, int ow
 // layers of 8 to 128), 6 to 17 % rms.
 float layer_cost(bool conv, int64_t rows, int cin, int taps, int cout, int64_t a_floats, bool residual, bool halo)
 {
-    const int m = (int)std::min<int64_t>(rows, INT32_MAX), k = taps * cin;
+    const int m = (int)std::min<int64_t>(rows, 1 << 30), k = taps * cin; // (rows up to the next tile stay within an int)
     const float out_mb = 4e-6f * (float)((double)a_floats + (residual ? 2. : 1.) * (double)rows * cout);
     if (cin % 16 == 0 && cout % 4 == 0 && a_floats < (1LL << 29)) {
         const TileChoice c = fast_pick(conv, m, cout, k, a_floats, residual, 1, closed_cuts(), halo);
@@ -1388,7 +1388,7 @@ float layer_cost(bool conv, int64_t rows, int cin, int taps, int cout, int64_t a
             return std::min(c.cost, 4.f + out_mb / 3.5f); // the row-streaming kernel
         const float fade = 15.f / std::max(15.f, c.cost); // (see slice_pick)
         if (c.cfg >= kSliceCfg || cout > 32)
-            return c.cost + (c.cfg < kSliceCfg ? 1.5f * fade * fade : 0.f);
+            return c.cost + (c.cfg < kSliceCfg ? (conv ? 2.2f : 1.5f) * fade * fade : 0.f);
     }
     const int cfg = general_pick(m, cout, 1);
     if (cfg == 0)

@@ -347,11 +347,11 @@ static int slice_pick(bool conv, int M, int N, int K, float tiled_cost)
         return -1;
     int best = -1;
     // Below a round of tiles the tiled kernel takes longer than its cost says, which was fitted to 0.2 GFLOP and more: on 600 small problems by
-    // 1.4 us up to K = 128 (4204 x 64 x 64 5.7 against 3.6 us here), on 1700 convolutions by 2 us up to a cost of 9, 1.2 at 16, 0.4 at 25.  Kernel
+    // 1.4 us up to K = 128 (4204 x 64 x 64 5.7 against 3.6 us here), on 1700 convolutions by 2.2 us up to a cost of 9, 1.2 at 16, 0.4 at 25.  Kernel
     // choices then take 1.7 % (convolutions 0.4 %) longer than the best; GEMMs 5.2 % with 0.95 of the cost.  Past a round operands
     // re-read cost the neighbours, too.
     const float fade = 15.f / std::max(15.f, tiled_cost);
-    float best_cost = narrow ? 1e30f : t64 > 256 ? 0.95f * tiled_cost : tiled_cost + 1.5f * fade * fade;
+    float best_cost = narrow ? 1e30f : t64 > 256 ? 0.95f * tiled_cost : tiled_cost + (conv ? 2.2f : 1.5f) * fade * fade;
     for (int i = 0; i < kSliceForms; ++i) {
         const float cost = slice_cost(i, conv, M, N, K);
         if (cost < best_cost && slice_fits(i, M, N)) {

@@ -108,18 +108,24 @@ __device__ __forceinline__ void sample_conv(const SampleStep& s, float* lds, flo
         };
         // One chain over all of K rounds the whole sum at every step: 2-norm error against 64 bits of 3x3 filters on 16 / 32 / 64 channels 2.1 /
         // 2.9 / 3.9 e-7, 1.2 / 1.3 / 1.6 as launches.  So a chunk's products start from zero, and chunks add up by fours before they join the
-        // rest: 0.9 / 1.0 / 1.0 e-7, small CNN 17.3 -> 17.6 us a call.  (Tile by tile: the chains of all tiles at once spill.)
+        // rest: 0.9 / 1.0 / 1.0 e-7, small CNN 17.35 -> 17.55 us a call.  (The chains of up to two tiles at once; of four they spill, two by two as well.)
         auto multiply = [&](const f32x4 (&av)[MT], const f32x4 (&wv)[NT], f32x4 (&sum)[MT][NT], bool first) {
+            constexpr int SIDE = MT * NT <= 2 ? MT * NT : 1; // tiles side by side
 #pragma unroll
-            for (int i = 0; i < MT; ++i)
+            for (int z = 0; z < MT * NT; z += SIDE) {
+                f32x4 part[SIDE];
 #pragma unroll
-                for (int j = 0; j < NT; ++j) {
-                    f32x4 part = { 0.f, 0.f, 0.f, 0.f };
+                for (int q = 0; q < SIDE; ++q)
+                    part[q] = f32x4 { 0.f, 0.f, 0.f, 0.f };
 #pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        part = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[j][e], av[i][e], part, 0, 0, 0);
-                    sum[i][j] = first ? part : sum[i][j] + part;
-                }
+                for (int e = 0; e < 4; ++e)
+#pragma unroll
+                    for (int q = 0; q < SIDE; ++q)
+                        part[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[(z + q) % NT][e], av[(z + q) / NT][e], part[q], 0, 0, 0);
+#pragma unroll
+                for (int q = 0; q < SIDE; ++q)
+                    sum[(z + q) / NT][(z + q) % NT] = first ? part[q] : sum[(z + q) / NT][(z + q) % NT] + part[q];
+            }
         };
         auto join = [&](const f32x4 (&sum)[MT][NT]) {
 #pragma unroll
@@ -427,8 +433,8 @@ __device__ __forceinline__ void sample_activation(const SampleStep& s, float* ld
 
 // What bounds it, on the small CNN of 32 x 32 x 3 (two 3x3 convolutions of 16 and 32 channels, pooling, classifier), cycles of a CU per
 // sample: way in 5800, first convolution 10200 (matrix pipes 4100, the rest its scattered 4-byte reads and the epilogue), pooling 1900,
-// second convolution 14000 (9200), global pooling 2600, Dense 1300, softmax 1700.  16.7 us a call for one sample and 17.6 up to 256, where
-// seven launches take 24 and 59; 8192 samples 490 us, 906 as launches.  Image and input on their way together, Dense off the matrix
+// second convolution 14000 (9200), global pooling 2600, Dense 1300, softmax 1700.  16.6 us a call for one sample and 17.5 up to 256, where
+// seven launches take 24 and 59; 8192 samples 485 us, 906 as launches.  Image and input on their way together, Dense off the matrix
 // instructions, 2 x 2 windows and pooled channels by fours took 1.2 us off it.  Nothing may go to scratch memory: 20 bytes a lane of it
 // cost 7 us a launch.
 __global__ __launch_bounds__(kSampleThreads) void sample_net_kernel(const float* __restrict__ in, float* __restrict__ out,

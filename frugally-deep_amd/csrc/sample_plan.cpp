@@ -464,12 +464,12 @@ bool sample_net_load(SampleProgram& p)
 // One launch or one per operation, by predicted times: a convolution or Dense layer's own launch as layer_cost has it, any other by its traffic,
 // 3.7 us at least.  Over 1200 timed calls (200 models of 1 to 5 convolutions of 4 to 64 channels or 1 to 4 Dense layers, 1 to 8192 samples) the
 // choice takes 0.4 % longer than the faster form, at worst 32 %; with one rate for all convolutions it took 10 %, and 2.1 times as
-// long where 8192 samples of two convolutions to 24 and 64 channels went into one launch.  Measured, us of a call, launches / one: the small CNN (two 3x3
-// convolutions of 16 and 32 channels on 32 x 32 x 3) at batch 1 / 256 / 8192 24 / 17.2, 59 / 17.9, 906 / 490; 28 x 28 with 5x5 convolutions of 6 and 16
-// channels and two Dense layers 44 / 15.5, 62 / 16.1, 717 / 414; four 3x3 convolutions of 16 channels on 16 x 16 25 / 20.7, 66 / 21.6, 1060 /
-// 600; strided 3x3 of 32 and 64 channels on 32 x 32 x 3 22 / 15.6, 34 / 16.6, 335 / 427 (the last left to the launches); two
-// Dense layers of 128 at batch 1 / 256 / 2048 13.2 / 6.7, 13.6 / 7.0, 13.5 / 28 (left); one 3x3 convolution 8 -> 32 on 24 x 24 at batch 1 / 256 / 8192 8.2 / 13.1
-// (left), 19.3 / 16.6, 387 / 397 (left).
+// long where 8192 samples of two convolutions to 24 and 64 channels went into one launch.  Measured, us of a call, launches / one: the small
+// CNN (two 3x3 convolutions of 16 and 32 channels on 32 x 32 x 3) at batch 1 / 256 / 8192 24 / 17.0, 59 / 17.8, 903 / 485; 28 x 28 with 5x5
+// convolutions of 6 and 16 channels and two Dense layers 44 / 15.3, 62 / 16.1, 717 / 411; four 3x3 convolutions of 16 channels on 16 x 16 25 /
+// 20.6, 65 / 21.5, 1059 / 597; strided 3x3 of 32 and 64 channels on 32 x 32 x 3 22 / 15.6, 34 / 16.6, 335 / 427 (the last left to the
+// launches); three Dense layers, 64 -> 128 -> 128 -> 4, at batch 1 / 256 / 2048 13.2 / 6.7, 13.6 / 7.0, 13.5 / 28 (left); one 3x3 convolution 8 -> 32 on
+// 24 x 24 at batch 1 / 256 / 8192 8.1 / 13.0, 19.3 / 16.4, 385 / 396 (all left, the second wrongly).
 bool sample_net_by_rule(const SampleProgram& p, const fdx_model& m, const std::vector<int>& order, const std::vector<Shape>& shapes, int batch)
 {
     double launches = 0;
